@@ -317,6 +317,37 @@ def test_gemm_gated(M, H, D, dtype, simple, act):
         k.FORCE_SIMPLE = False
 
 
+# float32 on the matrix cores: the edges of its tiles (16 and 32 rows, 32 to 128 columns), of its rules (16 | 17 and 32 | 33
+# rows, 4,096 and 8,192 columns) and of its k tiles, K short of one round of the waves, operands 4 bytes off
+@pytest.mark.parametrize("M,N,Kd,off", [
+    (1, 48, 32, 0), (15, 33, 64, 0), (16, 4096, 96, 0), (16, 8192, 64, 0), (17, 4097, 288, 0), (17, 4096, 288, 0), (32, 80, 544, 0),
+    (33, 200, 128, 0), (64, 96, 1056, 0), (65, 129, 32, 0), (129, 160, 64, 0), (161, 3000, 160, 0), (700, 3072, 128, 0),
+    (300, 7000, 96, 0), (7, 40, 64, 1), (70, 96, 64, 1)])
+def test_gemm_float32_on_the_matrix_cores(M, N, Kd, off):
+    k = K()
+    a = rnd((M * Kd + off,), 91).to(DEV)[off:].view(M, Kd)
+    w = rnd((N, Kd), 92).to(DEV)
+    x = rnd((M, N), 93).to(DEV)
+    want = a.double() @ w.double().t()
+    # K products and K additions in any order: each is off by at most 2^-24 of what it holds, which the sum of the
+    # products' sizes bounds; the residual's addition once more
+    bound = (2.0 * Kd + 2.0) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t() + x.double().abs())
+    out = torch.empty((M, N), dtype=torch.float32, device=DEV)
+    assert bool(((k.gemm(a, w, out, k.EPI_STORE_F32).double() - want).abs() <= bound).all())
+    got = k.gemm(a, w, x.clone(), k.EPI_ADD_F32).double()
+    assert bool(((got - want - x.double()).abs() <= bound).all())
+    if N >= 32:                                      # gate and up rows in blocks of 16
+        H = N // 32 * 16 - 3 if N > 64 else N // 32 * 16
+        rows = w[:32 * ((H + 15) // 16)].contiguous()
+        p = (a.double() @ rows.double().t()).view(M, -1, 2, 16)
+        gt, up = (p[:, :, i].reshape(M, -1)[:, :H] for i in (0, 1))
+        got = k.gemm(a, rows, torch.empty((M, H), dtype=torch.float32, device=DEV), k.EPI_GATED, hidden=H).double()
+        b = bound[:, :rows.shape[0]].reshape(M, -1, 2, 16)
+        bg, bu = (b[:, :, i].reshape(M, -1)[:, :H] for i in (0, 1))
+        # silu's slope is at most 1.1; its own and the product's rounding: a few units of the last place
+        assert bool(((got - R.silu(gt) * up).abs() <= 1.1 * bg * (up.abs() + bu) + gt.abs() * bu + 16 * 2.0 ** -24 * (gt * up).abs()).all())
+
+
 def test_gemm_vector_of_the_reference():
     """src/test.cpp:157-168: n = 256 inputs, d = 16 outputs, N(0,1), absolute 1e-4."""
     k = K()

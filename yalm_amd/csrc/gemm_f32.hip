@@ -1,0 +1,412 @@
+// C = epilogue(A[M,K] * W[N,K]^T) in float32 on the matrix cores (v_mfma_f32_16x16x4_f32: products and sums in
+// float32, as a chain of fused multiply-adds): the products of the true 32-bit path.
+//
+// gemm_f32_kernel, from some 64 rows on bound by the matrix cores (157 TFLOP/s: the vector units' own rate, but an operand
+// register serves 16 products where gemm_simple_kernel reads LDS for every eight).  A workgroup of four waves owns a
+// tile of 32 FA x 32 FB; a wave FA x FB products of 16 x 16.  k tiles of 32 floats go straight into LDS (128-byte rows,
+// 16-byte chunks XOR-swizzled by the row, as in gemm_dma.hip); a lane reads four consecutive k of a row at once and feeds
+// them to four products one after the other: which k stands in which place of a product does not matter as long as both
+// operands agree.  It reaches 119 to 138 TFLOP/s (rocBLAS 129 to 153); 701 rows against gemm_simple_kernel: 16,384 x 3,072
+// 2,250 -> 552 us, 128,256 x 3,072 16.3 -> 4.0 ms, 3,072 x 8,192 1,740 -> 290 us.
+//
+// gemm_few_f32_kernel and small tiles take a decode step's rows, which the vector units' kernel (gemm_rows_f32_kernel) had
+// multiplied at a fraction of memory's rate: 16 rows, 4,096 x 4,096 55 -> 20 us, 128,256 x 3,072 729 -> 278 us; one row,
+// 4,096 x 4,096 24 -> 16 us.
+//
+// Sums over short runs of k join a total of their own: two short chains of additions lie closer to 64 bits than one over K
+// (a relative error of 3.0e-7 at 701 rows and K 8,192, where gemm_simple_kernel's was 1.6e-6; at most 64 rows 0.8 to 1.4e-7,
+// gemm_rows_f32_kernel's 0.8 to 2.2e-7).
+#include "common.h"
+#include "yalm_hip.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr int TK = 32;                           // floats of k a tile
+constexpr int ROWB = TK * 4;
+constexpr int CPR = ROWB / 16;                   // 16-byte chunks a row
+constexpr int RPI = WAVE / CPR;                  // rows one wave instruction brings
+constexpr int NW = 4;
+
+__device__ __forceinline__ int swizzle_of(int row) { return (row >> 1) & (CPR - 1); }
+
+// at most N_ of this wave's loads in flight, and none of its LDS reads
+template <int N_>
+__device__ __forceinline__ void wait_loads() {
+  __builtin_amdgcn_s_waitcnt((N_ & 0xF) | ((N_ >> 4) << 14) | (0x7 << 4) | (0x0 << 8));
+}
+
+// stages of LDS: as many as leave room for two workgroups a CU, four at most
+constexpr int stages_of(int FA, int FB) { return 640 / (32 * (FA + FB)) < 4 ? 640 / (32 * (FA + FB)) : 4; }
+constexpr int GROUP = 4;                         // tile columns that an XCD walks together
+
+// FINE: four chains of sums, one for each of the k that a lane holds side by side, joined and added to the total every four k
+// tiles: chains of 32 and of K / 128 additions.  Else one chain, added to the total every eight k tiles.
+template <int EPI, int FA, int FB, bool FINE>
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                          float* __restrict__ C, int M, int N, int K, GateOut H) {
+  constexpr int TM = 32 * FA, TN = 32 * FB, ROWS = TM + TN, STAGE_B = ROWS * ROWB, S = stages_of(FA, FB);
+  constexpr int L = ROWS / (RPI * NW);           // load instructions a wave and stage
+  constexpr int CH = FINE ? 4 : 1, FOLD = FINE ? 4 : 8;
+  static_assert(S >= 2 && (S - 1) * L < 64, "vmcnt holds 6 bits");
+  static_assert(!gated(EPI) || FB % 2 == 0, "the gated epilogue pairs column tiles");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char stages[];
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int wm = wave / 2, wn = wave % 2;
+  const int l16 = lane % 16, lq = lane / 16;
+  // Workgroup i runs on XCD i mod 8: every XCD takes a run of the tiles (groups of GROUP columns, in a group the columns
+  // fastest), so that the tiles it works on at a time share rows and columns in its second-level cache.
+  const int mt = (M + TM - 1) / TM, nt = (N + TN - 1) / TN, tiles = mt * nt, chunk = (tiles + 7) / 8;
+  const int i0 = blockIdx.x, t = (i0 % 8) * chunk + i0 / 8;
+  if (t >= tiles || i0 / 8 >= chunk) return;
+  const int per_group = mt * GROUP, g = t / per_group, r0 = t % per_group, width = min(GROUP, nt - g * GROUP);
+  const int m0 = (r0 / width) * TM, n0 = (g * GROUP + r0 % width) * TN;
+
+  const float* gp[L];
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int row = (i * NW + wave) * RPI + lane / CPR;
+    const float* base = row < TM ? A + (size_t)min(m0 + row, M - 1) * K          // rows past the edge repeat the last
+                                 : W + (size_t)min(n0 + row - TM, N - 1) * K;    // one and are never stored
+    gp[i] = base + ((lane % CPR) ^ swizzle_of(row)) * 4;
+  }
+  auto issue = [&](int kt, int stage, int i) {
+#if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops a template that names this builtin, and its launch stub with it
+    __builtin_amdgcn_global_load_lds(gp[i] + (size_t)kt * TK, stages + stage * STAGE_B + (i * NW + wave) * 1024, 16, 0, 0);
+#endif
+  };
+  auto issue_all = [&](int kt, int stage) {
+#pragma unroll
+    for (int i = 0; i < L; ++i) issue(kt, stage, i);
+  };
+
+  f32x4 acc[CH][FA][FB], total[FA][FB];
+#pragma unroll
+  for (int a = 0; a < FA; ++a)
+#pragma unroll
+    for (int b = 0; b < FB; ++b) {
+      total[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < CH; ++c) acc[c][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+
+  // fragments: address in a stage row * 128 + ((4 s + lq) ^ swizzle) * 16 for step s; tiles 16 rows apart share the swizzle
+  const int a_row = wm * (TM / 2) + l16, w_row = wn * (TN / 2) + l16;
+  int a_at[2], w_at[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    a_at[s] = a_row * ROWB + (((4 * s + lq) ^ swizzle_of(a_row)) << 4);
+    w_at[s] = (TM + w_row) * ROWB + (((4 * s + lq) ^ swizzle_of(TM + w_row)) << 4);
+  }
+
+  // Tile kt lies in stage kt mod S; S tiles are in LDS or on their way.  The barrier of a tile stands between its two
+  // steps: the second step's fragments are in registers by then, so nobody reads the tile's stage any more and tile
+  // kt + S is asked for at once, a load behind every few products; the first fragments of tile kt + 1 are read in front
+  // of the last products of tile kt.
+  const int nk = K / TK;
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < nk) issue_all(s, s);
+  if (nk >= S) wait_loads<(S - 1) * L>(); else wait_loads<0>();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  f32x4 fa[2][FA], fw[2][FB];
+  auto read_frags = [&](int stage, int s) {
+    const unsigned char* at = stages + stage * STAGE_B;
+#pragma unroll
+    for (int a = 0; a < FA; ++a) fa[s][a] = *reinterpret_cast<const f32x4*>(at + a_at[s] + a * 16 * ROWB);
+#pragma unroll
+    for (int b = 0; b < FB; ++b) fw[s][b] = *reinterpret_cast<const f32x4*>(at + w_at[s] + b * 16 * ROWB);
+  };
+  read_frags(0, 0);
+  int stage = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    const int next = stage + 1 == S ? 0 : stage + 1;
+    read_frags(stage, 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int a = 0; a < FA; ++a)
+#pragma unroll
+        for (int b = 0; b < FB; ++b)
+          acc[e % CH][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[0][a][e], fw[0][b][e], acc[e % CH][a][b], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // tile kt + 1 has landed when at most the loads of the S - 2 tiles behind it are in flight
+    if (kt + S - 1 < nk) wait_loads<(S - 2) * L>(); else wait_loads<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read_frags(next, 0);                           // behind the last tile: whatever lies there, never used
+    const bool more = kt + S < nk;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int a = 0; a < FA; ++a)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+          acc[e % CH][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[1][a][e], fw[1][b][e], acc[e % CH][a][b], 0, 0, 0);
+          const int j = (e * FA + a) * FB + b;
+#pragma unroll
+          for (int i = 0; i < L; ++i)
+            if (j == (i + 1) * 4 * FA * FB / (L + 1) - 1) {
+              if (more) issue(kt + S, stage, i);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    stage = next;
+    if ((kt + 1) % FOLD == 0 || kt + 1 == nk) {
+#pragma unroll
+      for (int a = 0; a < FA; ++a)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+          if constexpr (FINE) total[a][b] += (acc[0][a][b] + acc[1][a][b]) + (acc[2][a][b] + acc[3][a][b]);
+          else total[a][b] += acc[0][a][b];
+#pragma unroll
+          for (int c = 0; c < CH; ++c) acc[c][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+
+  // lane (lq, l16) holds rows 4 lq .. 4 lq + 3 of column l16 of every 16 x 16
+#pragma unroll
+  for (int a = 0; a < FA; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + wm * (TM / 2) + a * 16 + 4 * lq + r;
+      if (m >= M) continue;
+      if (gated(EPI)) {                              // weight rows: 16 gate rows, 16 up rows, ...: even tiles gate, odd tiles up
+#pragma unroll
+        for (int p = 0; p < FB / 2; ++p) {
+          const int hcol = (n0 + wn * (TN / 2)) / 2 + p * 16 + l16;
+          if (hcol < H) C[(size_t)m * H + hcol] = gate_unit<EPI>(total[a][2 * p][r], total[a][2 * p + 1][r], H);
+        }
+      } else {
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+          const int n = n0 + wn * (TN / 2) + b * 16 + l16;
+          if (n >= N) continue;
+          const size_t o = (size_t)m * N + n;
+          if (EPI == 2) C[o] += total[a][b][r];
+          else C[o] = total[a][b][r];
+        }
+      }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// At most 64 rows (a decode step of the 32-bit path): bound by the weights' one trip from memory.  A workgroup owns
+// 16 NB weight rows and all (16 MB) rows of A; its waves take every NWV-th block of 32 k (128 bytes of each row, whole
+// lines) and their sums are added in LDS in the waves' order.  Weights and A go from memory straight into registers, the
+// next block's while one is multiplied (two blocks ahead measured the same).
+// ---------------------------------------------------------------------------
+constexpr int NWV = 8;
+
+template <int EPI, int MB, int NB>
+__global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                    float* __restrict__ C, int M, int N, int K, GateOut H) {
+  static_assert(!gated(EPI) || NB == 2, "a block of gate rows and its up rows");
+  __shared__ f32x4 sums[NWV][MB * NB][WAVE];
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int l16 = lane % 16, lq = lane / 16;
+  const int n0 = blockIdx.x * 16 * NB;
+  const float* wp[NB];
+  const float* ap[MB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) wp[b] = W + (size_t)min(n0 + b * 16 + l16, N - 1) * K + lq * 4;    // rows past the edge repeat the
+#pragma unroll
+  for (int a = 0; a < MB; ++a) ap[a] = A + (size_t)min(a * 16 + l16, M - 1) * K + lq * 4;         // last one, never stored
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  const int blocks = K / TK, mine = (blocks - wave + NWV - 1) / NWV;     // this wave's: wave, wave + NWV, ...
+  f32x4 w[2][NB][2], x[2][MB][2];
+  auto load = [&](int buf, int i) {                // block i of this wave
+    const size_t k = (size_t)(i * NWV + wave) * TK;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) w[buf][b][h] = __builtin_nontemporal_load((const f32x4*)(wp[b] + k + h * 16));
+#pragma unroll
+      for (int a = 0; a < MB; ++a) x[buf][a][h] = *(const f32x4*)(ap[a] + k + h * 16);
+    }
+  };
+  auto multiply = [&](int buf) {                   // a sum of its own for each of the four k that a lane holds side by side
+    f32x4 part[4][MB][NB];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) part[e][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int a = 0; a < MB; ++a)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+            part[e][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[buf][a][h][e], w[buf][b][h][e], part[e][a][b], 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[a][b] += (part[0][a][b] + part[1][a][b]) + (part[2][a][b] + part[3][a][b]);
+  };
+  if (mine > 0) {
+    load(0, 0);
+    int i = 0;
+    for (; i + 2 < mine; i += 2) {
+      load(1, i + 1);
+      multiply(0);
+      load(0, i + 2);
+      multiply(1);
+    }
+    if (i + 1 < mine) load(1, i + 1);
+    multiply(0);
+    if (i + 1 < mine) multiply(1);
+  }
+#pragma unroll
+  for (int a = 0; a < MB; ++a)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) sums[wave][a * NB + b][lane] = acc[a][b];
+  __syncthreads();
+
+  // lane (lq, l16) of a 16 x 16 holds rows 4 lq .. 4 lq + 3 of column l16
+  constexpr int UNITS = gated(EPI) ? MB : MB * NB;
+  for (int e = tid; e < UNITS * WAVE; e += NWV * WAVE) {
+    const int at = e % WAVE, unit = e / WAVE, col = at % 16, row = 4 * (at / 16);
+    auto total = [&](int t) {
+      f32x4 v = sums[0][t][at];
+#pragma unroll
+      for (int i = 1; i < NWV; ++i) v += sums[i][t][at];
+      return v;
+    };
+    if constexpr (gated(EPI)) {
+      const f32x4 gt = total(unit * 2), up = total(unit * 2 + 1);
+      const int hcol = blockIdx.x * 16 + col;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = unit * 16 + row + r;
+        if (m < M && hcol < H) C[(size_t)m * H + hcol] = gate_unit<EPI>(gt[r], up[r], H);
+      }
+    } else {
+      const f32x4 v = total(unit);
+      const int n = n0 + (unit % NB) * 16 + col;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = (unit / NB) * 16 + row + r;
+        if (m >= M || n >= N) continue;
+        const size_t o = (size_t)m * N + n;
+        if (EPI == 2) C[o] += v[r];
+        else C[o] = v[r];
+      }
+    }
+  }
+}
+
+template <int EPI, int MB, int NB>
+int launch_few(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
+  gemm_few_f32_kernel<EPI, MB, NB><<<ceil_div(N, 16 * NB), NWV * WAVE, 0, stream>>>(A, W, C, M, N, K, H);
+  return launch_status();
+}
+
+template <int EPI, int FA, int FB, bool FINE>
+int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
+  if constexpr (gated(EPI) && FB % 2 != 0) {
+    return YALM_ERR_ARG;
+  } else {
+    const int tiles = ceil_div(M, 32 * FA) * ceil_div(N, 32 * FB), lds = stages_of(FA, FB) * 32 * (FA + FB) * ROWB;
+    auto kernel = &gemm_f32_kernel<EPI, FA, FB, FINE>;
+    if (lds > 64 * 1024) {
+      static LdsAllowance allowed;
+      if (int rc = allow_dynamic_lds(allowed, (const void*)kernel, lds); rc != YALM_OK) return rc;
+    }
+    kernel<<<8 * ceil_div(tiles, 8), 256, lds, stream>>>(A, W, C, M, N, K, H);
+    return launch_status();
+  }
+}
+
+// Estimated time in us of one of the tile's kernel: f = FA FB products of 16 x 16 a wave.  Measured: a k tile takes 0.13 +
+// 0.116 f us of a workgroup that has a CU to itself and 0.055 + 0.118 f of a CU's time where several share it (K 3,072 and
+// 4,096: 4x4 249 us, 3x3 111, 2x4 102, 2x2 73, 2x1 45, 1x1 32 alone); a last round on a fraction of the CUs costs half a
+// round and half its fraction.
+double tile_time(int M, int N, int K, int fa, int fb) {
+  const double f = fa * fb, per = (double)ceil_div(M, 32 * fa) * ceil_div(N, 32 * fb) / 256.0, k = K / TK;
+  if (per <= 1.0) return (0.13 + 0.116 * f) * k;
+  const long whole = (long)per;
+  const double rest = per - (double)whole;
+  return (0.055 + 0.118 * f) * k * ((double)whole + (rest > 0.0 ? 0.5 + 0.5 * rest : 0.0));
+}
+
+// The tile for a shape: the fastest by that estimate (701 rows, N x K: 16,384 x 3,072 takes 2x4 555 us, 128,256 x 3,072 2x4
+// 4.0 ms, 3,072 x 8,192 3x3 288 us on exactly 256 tiles, 2x4 would be 24 % slower).  Up to 64 rows the small tiles' FINE
+// form: there the products were summed more finely before (gemm_rows_f32_kernel), and memory is what bounds them.
+template <int EPI>
+int launch_tiles(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
+  static constexpr int shapes[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 3}, {3, 4}, {4, 4}};
+  const bool fine = M <= 64;
+  int best = -1;
+  double best_t = 0.0;
+  for (int i = 0; i < (fine ? 5 : 8); ++i) {
+    if (gated(EPI) && shapes[i][1] % 2) continue;
+    const double t = tile_time(M, N, K, shapes[i][0], shapes[i][1]);
+    if (best < 0 || t < best_t) { best = i; best_t = t; }
+  }
+#define YALM_F32_TILE(FA_, FB_) \
+  return fine ? launch_f32<EPI, FA_, FB_, true>(A, W, C, M, N, K, H, stream) : launch_f32<EPI, FA_, FB_, false>(A, W, C, M, N, K, H, stream)
+  switch (best) {
+    case 0: YALM_F32_TILE(1, 1);
+    case 1: YALM_F32_TILE(1, 2);
+    case 2: YALM_F32_TILE(2, 1);
+    case 3: YALM_F32_TILE(2, 2);
+    case 4: YALM_F32_TILE(2, 4);
+    case 5: return launch_f32<EPI, 3, 3, false>(A, W, C, M, N, K, H, stream);
+    case 6: return launch_f32<EPI, 3, 4, false>(A, W, C, M, N, K, H, stream);
+    default: return launch_f32<EPI, 4, 4, false>(A, W, C, M, N, K, H, stream);
+  }
+#undef YALM_F32_TILE
+}
+
+// Up to 64 rows of up to 4,096 columns (16 rows: 8,191) go to gemm_few_f32_kernel: the tiles' kernel would leave CUs without
+// work, and walks K alone where eight waves share it (16 rows, 4,096 x 4,096 20 against 32 us, 3,072 x 8,192 36 against 60,
+// 512 x 256 3.5 against 4.4; at 64 rows 43, 81 and 5.2 against 33, 61 and 4.4, but summed more finely, as before).  Wider
+// products go to the tiles, which read A once for 32 weight rows and more (16 rows, 16,384 x 3,072: 44 against 54 us,
+// 128,256 x 3,072: 278 against 392).
+template <int EPI>
+int launch(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
+  constexpr int NB = gated(EPI) ? 2 : 1;
+  if (M <= 64 && N <= 4096) {
+    if (M <= 16) return launch_few<EPI, 1, NB>(A, W, C, M, N, K, H, stream);
+    if (M <= 32) return launch_few<EPI, 2, NB>(A, W, C, M, N, K, H, stream);
+    return launch_few<EPI, 4, NB>(A, W, C, M, N, K, H, stream);
+  }
+  if (M <= 16 && N < 8192) return launch_few<EPI, 1, 2>(A, W, C, M, N, K, H, stream);
+  return launch_tiles<EPI>(A, W, C, M, N, K, H, stream);
+}
+
+}  // namespace
+
+// K a multiple of 32 and 16-byte aligned operands; YALM_ERR_ARG: not taken.  Nor are up to four rows of a wide product: the
+// vector units' kernel keeps up with memory there (one row, 128,256 x 3,072 271 against 290 us, 16,384 x 3,072 44 against 47).
+int yalm_gemm_f32_mfma(const void* A, const void* W, void* C, int M, int N, int K, int epilogue, GateOut H, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) ||
+      (M <= 4 && N >= 8192))
+    return YALM_ERR_ARG;
+  const float *a = (const float*)A, *w = (const float*)W;
+  float* c = (float*)C;
+  switch (epilogue) {
+    case 0:
+    case 1: return launch<0>(a, w, c, M, N, K, H, stream);
+    case 2: return launch<2>(a, w, c, M, N, K, H, stream);
+    case 3: return launch<3>(a, w, c, M, N, K, H, stream);
+    case 5: return launch<5>(a, w, c, M, N, K, H, stream);
+  }
+  return YALM_ERR_ARG;
+}

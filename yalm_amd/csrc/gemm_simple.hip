@@ -2,12 +2,16 @@
 // true 32-bit path and the fallback of the bfloat16 path for shapes the MFMA kernels
 // refuse.  gemm_simple: 64x64 tile, 16-deep k steps through LDS, 256 threads with a 4x4
 // register tile each; any M, N, K.  gemm_rows_f32: at most 64 rows of float32, a pass over
-// the weights for every 16 of them (below).
+// the weights for every 16 of them (below).  Float32 with K a multiple of 32 goes to the matrix cores (gemm_f32.hip), but for
+// up to four rows of a wide product.
 #include "common.h"
 #include "yalm_hip.h"
 
 int yalm_gemm_bf16_mfma(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N,
                         int K, int epilogue, GateOut H, hipStream_t stream);   // gemm_mfma.hip; YALM_ERR_ARG: shape refused
+
+int yalm_gemm_f32_mfma(const void* A, const void* W, void* C, int M, int N, int K, int epilogue, GateOut H,
+                       hipStream_t stream);                                    // gemm_f32.hip; the same
 
 namespace {
 constexpr int BM = 64, BN = 64, BK = 16;
@@ -244,7 +248,9 @@ extern "C" int yalm_gemm(const void* A, const void* W, void* C, float* workspace
   if (gated(epilogue) && (H <= 0 || N != 32 * ((H + 15) / 16))) return YALM_ERR_ARG;
   if (dtype == YALM_F32) {
     if (!force_simple) {
-      int rc = gemm_rows_f32(A, W, C, M, N, K, epilogue, H, stream);
+      int rc = yalm_gemm_f32_mfma(A, W, C, M, N, K, epilogue, H, stream);
+      if (rc != YALM_ERR_ARG) return rc;
+      rc = gemm_rows_f32(A, W, C, M, N, K, epilogue, H, stream);
       if (rc != YALM_ERR_ARG) return rc;
     }
     return gemm_simple<float>(A, W, C, M, N, K, epilogue, H, stream);
