@@ -744,6 +744,59 @@ def test_attn_decode_with_the_length_of_the_longest_sequence(n_heads, n_kv, hd, 
     _attn_decode_case(n_heads, n_kv, hd, window, lens, splits, torch.bfloat16, False, max(lens) if said == "longest" else said)
 
 
+# float32 on the matrix cores against the general kernels: head sizes with pages in rows and in blocks, one tile and many, a
+# window, blocks of positions, every shape of the scores, one split and several, more than 16 heads a group, rows in another
+# order with splits of the longest sequence's size, a value that is infinite (a query that does not see it must not notice)
+@pytest.mark.parametrize("shape", ["plain", "bias", "softcap", "sink", "slopes", "log", "infinite"])
+@pytest.mark.parametrize("n_heads,n_kv,hd,window,block,lens,splits", [
+    (4, 2, 16, 0, 0, [5, 64, 65], 1), (6, 3, 48, 100, 0, [130, 300], 3), (8, 2, 128, 0, 0, [200, 1, 129], 2),
+    (18, 1, 64, 70, 0, [150, 64], 1), (3, 3, 32, 0, 96, [257, 17], 2), (2, 1, 112, 0, 0, [66], 1)])
+def test_attention_float32_on_the_matrix_cores(n_heads, n_kv, hd, window, block, lens, splits, shape):
+    k = K()
+    T, B = sum(lens), len(lens)
+    more = {"bias": {"score_bias": rnd((n_heads, 50), 61).to(DEV)}, "softcap": {"softcap": 2.5},
+            "sink": {"sink_logit": rnd((n_heads,), 62).to(DEV)}, "slopes": {"slopes": rnd((n_heads,), 63, scale=0.1).abs().to(DEV)},
+            "log": {"log_distance": (rnd((n_heads,), 64).abs().to(DEV), rnd((n_heads,), 65).abs().to(DEV))}}.get(shape, {})
+    q, kk, v = (rnd((T, n * hd), 66 + i) for i, n in enumerate((n_heads, n_kv, n_kv)))
+    if shape == "infinite":
+        v[lens[0] - 1, 0] = float("inf")             # the first sequence's last position, which only its last query sees
+        v[T - lens[-1], -1] = float("-inf")          # the last sequence's first position
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    seq = np.repeat(np.arange(B), lens)
+    pos = np.concatenate([np.arange(n) for n in lens])
+    ks, vs, tile0 = stage(kk, v, lens, n_kv, hd, torch.float32)
+    kp, vp, bt, slots, ring, _, _ = paged_case(lens, n_kv, hd, window, torch.float32, 20, stored=False)
+    if shape == "infinite":
+        for b, n in enumerate(lens):                 # the longest sequence's last value, and one a page or so before it
+            for at in {n - 1, max(0, n - 70)}:
+                vp[bt[slots[b], at // 64 % ring], 0, 3, at % 64] = float("inf")
+    kp, vp = pages_as_stored(kp, vp)
+    qd = rnd((B, n_heads * hd), 70)
+    got = {}
+    for simple in (False, True):
+        out, o32, lse = (torch.full((T, n), 7.0, device=DEV) for n in (n_heads * hd, n_heads * hd, n_heads))
+        dec, dlse = (torch.full((B, n), 7.0, device=DEV) for n in (n_heads * hd, n_heads))
+        partial = torch.empty(k.attn_decode_workspace_floats(B, n_heads, hd, splits), device=DEV)
+        k.FORCE_SIMPLE = simple
+        try:
+            k.attn_prefill(q.to(DEV), ks.to(DEV), vs.to(DEV), out, i32(cu), i32(tile0), i32(seq), i32(pos), n_heads, n_kv, hd,
+                           window, lse=lse, out_f32=o32, block=block, **more)
+            k.attn_decode(qd.to(DEV), kp.to(DEV), vp.to(DEV), bt.to(DEV), ring, i32(slots), i32(lens), dec, partial, n_heads,
+                          n_kv, hd, window, splits, lse=dlse, block=block, step_max_len=None if simple else i32([max(lens)]),
+                          seq_order=None if simple else i32(list(range(B))[::-1]), **more)
+        finally:
+            k.FORCE_SIMPLE = False
+        got[simple] = [t.cpu().double() for t in (out, o32, lse, dec, dlse)]
+    # both sum the same terms in float32 in another order: scores of a few tens off by 1e-5 of themselves at most, and the
+    # probabilities with them
+    for what, a, b in zip(("prefill", "prefill unrounded", "prefill lse", "decode", "decode lse"), got[False], got[True]):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a[a.isinf()], b[a.isinf()]) and torch.equal(a.isinf(), b.isinf()), what
+        fine = b.isfinite()
+        err = ((a - b).abs()[fine] / b[fine].abs().clamp(min=1.0)).max().item()
+        assert err <= 2e-5, "%s: %.3e" % (what, err)
+    assert shape == "infinite" or got[False][0].isfinite().all()
+
+
 def _attn_decode_case(n_heads, n_kv, hd, window, lens, splits, dtype, simple, step_max_len):
     k = K()
     B = len(lens)

@@ -1,5 +1,5 @@
-// Attention in float32 arithmetic for every storage type: the kernels of the
-// true 32-bit path and the fallback of the bfloat16 path.  One wave per
+// Attention in float32 arithmetic for every storage type: the fallback of the matrix-core
+// kernels (attention_f32.hip, attention_mfma_*.hip) for the head sizes they refuse.  One wave per
 // (query, head); keys are taken 64 at a time, a lane per key for the scores
 // and a lane per output element for the mix; softmax state in float32.
 #include <float.h>
@@ -13,6 +13,14 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
                                 const int* cu_seqlens, const int* seq_tile0, const int* tile_order, int n_order,
                                 int T, int B, int n_tiles, int n_heads, int n_kv_heads, int head_dim, int window,
                                 const ScoreShape& shape, hipStream_t stream);
+int yalm_attn_prefill_f32_mfma(const void* q, const void* k_stage, const void* v_stage, void* out, float* out_f32, float* lse,
+                               const int* cu_seqlens, const int* seq_tile0, int B, int n_tiles, int n_heads,
+                               int n_kv_heads, int head_dim, int window, const ScoreShape& shape, hipStream_t stream);
+int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
+                              int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out, float* lse,
+                              float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window, int n_splits,
+                              int n_pages, int page_layout, const int* step_max_len, const int* seq_order,
+                              const ScoreShape& shape, hipStream_t stream);
 int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
                                int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
                                float* lse, float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window,
@@ -350,6 +358,11 @@ extern "C" int yalm_attn_prefill_lse(const void* q, const void* k_stage, const v
   const ScoreShape shape = {score_bias, n_bias, softcap, sink_logit, slopes, block, log_a, log_b};
   dim3 grid(T, n_heads);
   if (dtype == YALM_F32) {
+    if (!force_simple) {
+      int rc = yalm_attn_prefill_f32_mfma(q, k_stage, v_stage, out, out_f32, lse, cu_seqlens, seq_tile0, B, n_tiles,
+                                          n_heads, n_kv_heads, head_dim, window, shape, stream);
+      if (rc != YALM_ERR_ARG) return rc;
+    }
     if (head_dim <= ACC_SMALL * WAVE)
       attn_prefill_simple_kernel<float, ACC_SMALL><<<grid, WAVE, 0, stream>>>(
           (const float*)q, (const float*)k_stage, (const float*)v_stage, (float*)out, out_f32, lse, seq_tile0, tok_seq,
@@ -423,6 +436,18 @@ int attn_decode_any(const void* q, const void* k_pages, const void* v_pages, con
     return YALM_ERR_ARG;
   dim3 grid(B, n_heads, n_splits), cgrid(B, n_heads);
   if (dtype == YALM_F32) {
+    if (!force_simple) {
+      const bool merge = n_splits > 1 || sinks.n_sinks > 0;     // with sinks the merge kernel always runs: it takes them in
+      int rc = yalm_attn_decode_f32_mfma(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len,
+                                         merge ? nullptr : out, lse, partial, B, n_heads, n_kv_heads, head_dim, window,
+                                         n_splits, n_pages, page_layout, step_max_len, seq_order, shape, stream);
+      if (rc != YALM_ERR_ARG) {
+        if (rc != YALM_OK || !merge) return rc;
+        attn_decode_combine_kernel<float><<<cgrid, COMBINE_THREADS, 0, stream>>>(partial, (float*)out, lse, n_heads,
+                                                                                 head_dim, n_splits, sinks, sink_logit);
+        return launch_status();
+      }
+    }
     if (head_dim <= ACC_SMALL * WAVE) {
       attn_decode_simple_kernel<float, ACC_SMALL><<<grid, WAVE, 0, stream>>>(
           (const float*)q, (const float*)k_pages, (const float*)v_pages, block_table, table_stride, ring_pages,
