@@ -12,9 +12,10 @@
 // Probabilities of zero still multiply their value there, and 0 times infinity is no number.  Keys whose values are not all
 // finite are mixed one by one instead, zeros left out.
 //
-// 701 tokens, 24 heads of 128: 2,590 -> PREFILL_US us a layer; a decode step of 4 sequences of 20 to 36 tokens, 4 heads of 128:
-// 24 -> DECODE_US us, and no kernel that merges splits behind it where there is one.
+// 701 tokens, 24 heads of 128: 2,590 -> 87 us a layer; a decode step of 4 sequences of 20 to 36 tokens, 4 heads of 128:
+// 24 -> 8 us, and no kernel that merges splits behind it where there is one.
 #include <float.h>
+#include <type_traits>
 #include "common.h"
 #include "sinks.h"
 #include "yalm_hip.h"
@@ -221,8 +222,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_f32_kernel(
 // ---------------------------------------------------------------------------
 // decode: one query a sequence over the pages of the cache; grid (split, KV head and up to 16 of its query heads, sequence).
 // Each of the four waves takes a quarter of every page of the split (the 16 key rows that lie together where pages are in
-// blocks), so that a short context is worked by all of them; the next page's keys and values are in flight meanwhile, and
-// the waves' results are merged in LDS.  Bound by memory for long contexts, by a page's chain of loads, products and
+// blocks), so that a short context is worked by all of them; the next page's keys are in flight while a page is mixed, and the
+// waves' results are merged in LDS.  Bound by memory for long contexts, by a page's chain of loads, products and
 // exponentials for short ones.
 // ---------------------------------------------------------------------------
 template <int HD, bool BLOCKS, bool SHAPED>
@@ -262,29 +263,38 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
     // the wave's key rows: row0 + 8 (i / 4) + i mod 4 for i < 16 (page_row_place's 16 wave ... 16 wave + 15)
     const int row0 = 32 * (wave >> 1) + 4 * (wave & 1);
     const int k_row = row0 + 8 * (l16 >> 2) + (l16 & 3), v_row = row0 + 8 * lq;
-    f32x4 qv[DT], kf[2][DT], vf[2][DT];
+    f32x4 qv[DT], kf[DT], vf[DT];
 #pragma unroll
     for (int s = 0; s < DT; ++s) qv[s] = ld4(q + ((size_t)b * n_heads + h) * HD + s * 16 + lq * 4);
     auto page_at = [&](int ap) {
       return (size_t)min(max(table[ap % ring_pages], 0), n_pages - 1) * page_elems + (size_t)g * PAGE * HD;
     };
-    auto load = [&](int buf, int ap) {
-      const size_t at = page_at(ap);
+    auto load_keys = [&](size_t at) {
 #pragma unroll
-      for (int s = 0; s < DT; ++s) kf[buf][s] = ld4(k_pages + at + page_k_offset(LAYOUT, k_row, s * 16 + lq * 4, HD));
-#pragma unroll
-      for (int d = 0; d < DT; ++d) vf[buf][d] = ld4(v_pages + at + page_v_offset(LAYOUT, v_row, d * 16 + l16, HD));
+      for (int s = 0; s < DT; ++s) kf[s] = ld4(k_pages + at + page_k_offset(LAYOUT, k_row, s * 16 + lq * 4, HD));
     };
-    auto mix = [&](int buf, int ap) {
+    size_t at = 0;                                 // the page's place
+    // one page; has_next is a compile-time tag (std::true_type: the next page's keys are asked for)
+    auto one_page = [&](int ap, auto has_next) {
+      constexpr bool NEXT = decltype(has_next)::value;
+      const size_t at_next = NEXT ? page_at(ap + 1) : 0, at_v = at;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) vf[d] = ld4(v_pages + at_v + page_v_offset(LAYOUT, v_row, d * 16 + l16, HD));
+      __builtin_amdgcn_sched_barrier(0);           // the values are asked for before the keys are waited for
       f32x4 even = {0.f, 0.f, 0.f, 0.f}, uneven = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < DT; ++s)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if (s % 2 == 0) even = mfma4(kf[buf][s][e], qv[s][e], even);
-          else uneven = mfma4(kf[buf][s][e], qv[s][e], uneven);
+          if (s % 2 == 0) even = mfma4(kf[s][e], qv[s][e], even);
+          else uneven = mfma4(kf[s][e], qv[s][e], uneven);
         }
       f32x4 sc = even + uneven;
+      if constexpr (NEXT) {
+        load_keys(at_next);                        // in flight while this page is mixed
+        at = at_next;
+        __builtin_amdgcn_sched_barrier(0);
+      }
       const int pos0 = ap * PAGE + v_row;          // lane (lq, l16) holds the keys pos0 + r of head l16
       float mx = -FLT_MAX;
 #pragma unroll
@@ -296,7 +306,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
         mx = fmaxf(mx, sc[r]);
 #pragma unroll
         for (int d = 0; d < DT; ++d)               // rows that nobody sees may hold anything
-          if (!seen) vf[buf][d][r] = 0.f;
+          if (!seen) vf[d][r] = 0.f;
       }
       mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
       mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
@@ -315,12 +325,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
       for (int d = 0; d < DT; ++d) {
         part[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) part[d] = mfma4(vf[buf][d][r], sc[r], part[d]);
+        for (int r = 0; r < 4; ++r) part[d] = mfma4(vf[d][r], sc[r], part[d]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) z = fmaf(part[d][r], 0.f, z);
       }
       if (__any(z != 0.f)) {                       // key by key, probabilities of zero left out
-        const size_t at = page_at(ap);
 #pragma unroll
         for (int d = 0; d < DT; ++d) part[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < 4; ++k)
@@ -332,7 +341,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
               for (int d = 0; d < DT; ++d)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                  part[d][e] = fmaf(p, v_pages[at + page_v_offset(LAYOUT, row0 + 8 * k + r, d * 16 + lq * 4 + e, HD)], part[d][e]);
+                  part[d][e] = fmaf(p, v_pages[at_v + page_v_offset(LAYOUT, row0 + 8 * k + r, d * 16 + lq * 4 + e, HD)], part[d][e]);
             }
           }
       }
@@ -342,17 +351,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
         for (int r = 0; r < 4; ++r) o[d][r] = fmaf(o[d][r], corr, part[d][r]);
     };
     if (p_begin < p_end) {
-      load(0, p_begin);
+      at = page_at(p_begin);
+      load_keys(at);
       int ap = p_begin;
-      for (; ap + 2 < p_end; ap += 2) {
-        load(1, ap + 1);
-        mix(0, ap);
-        load(0, ap + 2);
-        mix(1, ap + 1);
-      }
-      if (ap + 1 < p_end) load(1, ap + 1);
-      mix(0, ap);
-      if (ap + 1 < p_end) mix(1, ap + 1);
+      for (; ap + 1 < p_end; ++ap) one_page(ap, std::true_type{});
+      one_page(ap, std::false_type{});
     }
   }
 
