@@ -42,6 +42,7 @@ class _BucketBuffers:
         self.copied = [None, None]    # the event after the last upload of each host copy
         self.turn = 0
         self.meta = torch.zeros(n_meta, dtype=torch.int32, device=engine.device)
+        self._device_index = self.meta.device.index      # a plain number: torch looks the current stream up sooner
 
     def host(self):
         """The host copy to fill for the next upload."""
@@ -53,7 +54,7 @@ class _BucketBuffers:
         self.meta.copy_(self.meta_host[self.turn], non_blocking=True)
         if self.copied[self.turn] is None:
             self.copied[self.turn] = torch.cuda.Event()
-        self.copied[self.turn].record()
+        self.copied[self.turn].record(torch.cuda.current_stream(self._device_index))
         self.turn ^= 1
 
 
@@ -111,6 +112,7 @@ class Engine:
         self.use_graphs = use_graphs
         self.max_graphs = max(1, int(max_graphs))
         self._widest_row = model.widest_row()
+        self._weight_bytes = model.weight_bytes()       # the weights are loaded: counted once, not every step
         self._prompt_tables = model.prompt_tables()     # index tables that parts want made for a step of whole prompts
         self._segments = model.decode_segments()        # the parts are fixed from here on: asked once, not every step
         self._any_graph = any(safe for safe, _, _ in self._segments)
@@ -137,7 +139,7 @@ class Engine:
         and the keys and values the sequences hold (a window's worth where a line keeps a window).
         The reference's Config::active_bytes (src/model.cpp:71-96) for a batch, with the head at
         its stored width."""
-        total = self.model.weight_bytes() + (len(slots) - 1) * self.model.embedding.weight_bytes()
+        total = self._weight_bytes + (len(slots) - 1) * self.model.embedding.weight_bytes()
         for g in self.cache.kv_groups:
             per_token = g.bytes_per_token()
             for s in slots:

@@ -86,7 +86,7 @@ class Sampler:
             u.copy_(host_u[:R], non_blocking=True)          # from pinned memory: the host does not wait for the queue
             kernels.sample(logits, u, float(temperature), out)
         host[:R].copy_(out, non_blocking=True)
-        landed.record()
+        landed.record(torch.cuda.current_stream(out.device.index))
         self._turn += 1
         return Drawn(out, host[:R], landed, self, self._turn)
 
