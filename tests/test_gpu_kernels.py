@@ -744,6 +744,46 @@ def test_attn_decode_with_the_length_of_the_longest_sequence(n_heads, n_kv, hd, 
     _attn_decode_case(n_heads, n_kv, hd, window, lens, splits, torch.bfloat16, False, max(lens) if said == "longest" else said)
 
 
+# the splits merged by the last workgroup to arrive: against the kernel that merges them, launch after launch with the same
+# counters; splits that find nothing to do, a padding row, more splits than lanes, several groups of 16 heads, a sink logit
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n_heads,n_kv,hd,window,lens,splits,sink", [
+    (4, 2, 16, 0, [5, 640], 2, False), (8, 2, 128, 0, [3000, 3, 700], 16, False), (34, 2, 64, 0, [300, 65], 3, True),
+    (5, 1, 80, 100, [700, 64], 5, True), (2, 1, 32, 0, [70 * 64 * 4], 70, False), (40, 1, 128, 0, [900], 9, False),
+    (3, 1, 256, 0, [400, 1], 4, False)])
+def test_attn_decode_merged_by_the_last_workgroup(n_heads, n_kv, hd, window, lens, splits, sink, dtype):
+    k = K()
+    B = len(lens)
+    kp, vp, bt, slots, ring, keys, vals = paged_case(lens, n_kv, hd, window, dtype, 20)
+    kp, vp, bt = kp.to(DEV), vp.to(DEV), bt.to(DEV)
+    logit = rnd((n_heads,), 62).to(DEV) if sink else None
+    counters = torch.zeros(k.attn_decode_counters(B + 1, n_heads, n_kv), dtype=torch.int32, device=DEV)
+    for turn in range(3):
+        q = torch.cat([rnd((B, n_heads * hd), 80 + turn, dtype), torch.zeros((1, n_heads * hd), dtype=dtype)]).to(DEV)
+        got = []
+        for c in (None, counters):
+            out = torch.full((B + 1, n_heads * hd), 7.0, dtype=dtype, device=DEV)
+            lse = torch.full((B + 1, n_heads), 7.0, device=DEV)
+            partial = torch.full((k.attn_decode_workspace_floats(B + 1, n_heads, hd, splits),), float("nan"), device=DEV)
+            k.attn_decode(q, kp, vp, bt, ring, i32(slots + [-1]), i32(lens + [0]), out, partial, n_heads, n_kv, hd, window, splits,
+                          lse=lse, sink_logit=logit, counters=c)
+            got.append((out.double(), lse.double()))
+        # The same partial results, added in another order.  Each side's sum over the splits is off by at most (splits + 4)
+        # 2^-24 of the sum of its terms' sizes (a rounding a term, the weights' exponential and the division), and those,
+        # weights of values that sum to one, are at most the largest value; a bfloat16 result is rounded on top, 2^-8 of
+        # itself a side.  The lse: the logarithm of a sum that is off by as much, and its own rounding.
+        biggest = max(v.abs().max().item() for v in vals)
+        off = 2 * (splits + 4) * 2.0 ** -24
+        rounding = 2.0 ** -7 if dtype == torch.bfloat16 else 0.0
+        (a, la), (b, lb) = got
+        assert torch.isfinite(b).all() and bool(((a - b).abs() <= off * biggest + rounding * b.abs()).all())
+        assert bool(((la - lb).abs() <= off + 2.0 ** -21 * lb.abs()).all())
+        assert int(counters.abs().sum()) == 0
+    with pytest.raises(ValueError):
+        k.attn_decode(q, kp, vp, bt, ring, i32(slots + [-1]), i32(lens + [0]), out, partial, n_heads, n_kv, hd, window, splits,
+                      counters=counters[:-1])
+
+
 # float32 on the matrix cores against the general kernels: head sizes with pages in rows and in blocks, one tile and many, a
 # window, blocks of positions, every shape of the scores, one split and several, more than 16 heads a group, rows in another
 # order with splits of the longest sequence's size, a value that is infinite (a query that does not see it must not notice)

@@ -17,6 +17,7 @@
 #include <float.h>
 #include <type_traits>
 #include "common.h"
+#include "attention_merge.h"
 #include "sinks.h"
 #include "yalm_hip.h"
 
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
     const int* __restrict__ block_table, int table_stride, int ring_pages, const int* __restrict__ seq_slot,
     const int* __restrict__ seq_len, float* __restrict__ partial, float* __restrict__ out, float* __restrict__ lse,
     int n_heads, int n_kv_heads, int window, int n_splits, int n_pages, const int* __restrict__ step_max_len,
-    const int* __restrict__ seq_order, ScoreShape sh) {
+    const int* __restrict__ seq_order, ScoreShape sh, int* __restrict__ counters) {
   constexpr int DT = HD / 16, NW = 4, LAYOUT = BLOCKS ? YALM_PAGE_BLOCKS : YALM_PAGE_ROWS;
   __shared__ float sm_m[NW][16], sm_l[NW][16];
   __shared__ f32x4 sm_o[NW][DT][WAVE];
@@ -371,11 +372,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
   for (int d = 0; d < DT; ++d) sm_o[wave][d][lane] = o[d] * scale;
   if (lq == 0) sm_l[wave][l16] = l * scale;
   __syncthreads();
-  if (l16 >= G) return;
   float lt = (sm_l[0][l16] + sm_l[1][l16]) + (sm_l[2][l16] + sm_l[3][l16]);
   float keep = 1.0f;
   float* to;
-  if (out != nullptr) {                            // one split: this is the result
+  if (n_splits == 1 && out != nullptr) {           // one split: this is the result
     to = out + ((size_t)b * n_heads + h) * HD;
     if (SHAPED && sh.sink_logit != nullptr && lt > 0.f) {     // the learned logit: in the denominator only
       const float sk = sh.sink_logit[h], m_new = fmaxf(m_all, sk);
@@ -384,21 +384,32 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
       m_all = m_new;
     }
     keep = lt > 0.f ? keep / lt : 0.f;
-    if (lse != nullptr && wave == 0 && lq == 0) lse[(size_t)b * n_heads + h] = lt > 0.f ? m_all + logf(lt) : -FLT_MAX;
+    if (lse != nullptr && wave == 0 && lq == 0 && l16 < G) lse[(size_t)b * n_heads + h] = lt > 0.f ? m_all + logf(lt) : -FLT_MAX;
   } else {
     to = partial + (((size_t)b * n_heads + h) * n_splits + split) * (HD + 2);
-    if (wave == 0 && lq == 0) {
-      to[HD] = m_all;
-      to[HD + 1] = lt;
+    if (wave == 0 && lq == 0 && l16 < G) {
+      if (counters != nullptr) {
+        store_pair(to + HD, m_all, lt);
+      } else {
+        to[HD] = m_all;
+        to[HD + 1] = lt;
+      }
     }
   }
 #pragma unroll
   for (int d = 0; d < DT; ++d)
-    if (d % NW == wave) {
+    if (d % NW == wave && l16 < G) {
       const f32x4 v = (sm_o[0][d][lane] + sm_o[1][d][lane]) + (sm_o[2][d][lane] + sm_o[3][d][lane]);
+      if (counters != nullptr) {
+        store_pair(to + d * 16 + lq * 4, v[0], v[1]);
+        store_pair(to + d * 16 + lq * 4 + 2, v[2], v[3]);
+      } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) to[d * 16 + lq * 4 + r] = v[r] * keep;       // a partial row need not lie on 16 bytes
+        for (int r = 0; r < 4; ++r) to[d * 16 + lq * 4 + r] = v[r] * keep;       // a partial row need not lie on 16 bytes
+      }
     }
+  if (counters != nullptr && last_to_arrive(counters + (size_t)blockIdx.z * gridDim.y + blockIdx.y, n_splits))
+    merge_splits<HD, NW, false>(partial, out, lse, b, n_heads, h0, G, n_splits, sh.sink_logit, wave, lane);
 }
 
 template <int HD>
@@ -449,22 +460,22 @@ int yalm_attn_prefill_f32_mfma(const void* q, const void* k_stage, const void* v
   return YALM_ERR_ARG;
 }
 
-// out null: the splits' partial results are merged by the caller.  YALM_ERR_ARG: not taken
+// out null: the splits' partial results are merged by the caller; with counters the kernel merges them.  YALM_ERR_ARG: not taken
 int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
                               int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out, float* lse,
                               float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window, int n_splits,
                               int n_pages, int page_layout, const int* step_max_len, const int* seq_order,
-                              const ScoreShape& shape, hipStream_t stream) {
+                              const ScoreShape& shape, int* counters, hipStream_t stream) {
   const int parts_g = (n_heads / n_kv_heads + 15) / 16;
   const bool blocks = page_layout == YALM_PAGE_BLOCKS;
   if (!takes(head_dim, q, k_pages, v_pages, nullptr) || (long)n_kv_heads * parts_g > 65535 || B > 65535 ||
-      (blocks && head_dim % 32 != 0) || (out == nullptr && partial == nullptr))
+      (blocks && head_dim % 32 != 0) || (out == nullptr && partial == nullptr) || (out == nullptr && counters != nullptr))
     return YALM_ERR_ARG;
   const dim3 grid(n_splits, n_kv_heads * parts_g, B);
 #define YALM_RUN(HD_, BLOCKS_, SHAPED_)                                                                                  \
   attn_decode_f32_kernel<HD_, BLOCKS_, SHAPED_><<<grid, 256, 0, stream>>>(                                               \
       (const float*)q, (const float*)k_pages, (const float*)v_pages, block_table, table_stride, ring_pages, seq_slot,    \
-      seq_len, partial, (float*)out, lse, n_heads, n_kv_heads, window, n_splits, n_pages, step_max_len, seq_order, shape)
+      seq_len, partial, (float*)out, lse, n_heads, n_kv_heads, window, n_splits, n_pages, step_max_len, seq_order, shape, counters)
 #define YALM_HD16(HD_)                                                                                                   \
   case HD_:                                                                                                              \
     if (shape.any()) YALM_RUN(HD_, false, true);                                                                         \

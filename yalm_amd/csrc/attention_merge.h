@@ -1,0 +1,97 @@
+// The merge of a decode step's attention splits inside the attention kernel: the workgroup that arrives last of a (sequence,
+// KV head)'s splits merges their partial results, in the splits' order whoever is last, so that no kernel of its own does
+// (4.7 us a layer of a decode step, most of it a launch).  counters: an int for each (sequence, blockIdx.y), zero before
+// the launch and behind it.
+//
+// The partial results pass between XCDs, whose second-level caches do not see each other's lines: they are stored and loaded
+// as relaxed atomics of agent scope, which go through to where all XCDs see them and are not served from a cache that does
+// not; every wave waits until its stores have got there before the workgroup's barrier, and the counter is raised behind
+// that.  (An acquire-release exchange instead writes back and drops the whole cache, once a workgroup: a step of
+// thirty-two layers at batch 8 took 3.60 ms that way, with the kernel that merges 3.40.)
+#pragma once
+#include <float.h>
+#include "common.h"
+
+typedef unsigned long long pair_bits;            // two floats
+
+__device__ __forceinline__ void store_pair(float* p, float a, float b) {
+  const pair_bits v = (pair_bits)__float_as_uint(a) | ((pair_bits)__float_as_uint(b) << 32);
+  __hip_atomic_store(reinterpret_cast<pair_bits*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_pair(const float* p) {
+  const pair_bits v = __hip_atomic_load(reinterpret_cast<const pair_bits*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return make_float2(__uint_as_float((unsigned)v), __uint_as_float((unsigned)(v >> 32)));
+}
+
+// True in every thread of the one workgroup that arrives last of `n`; what the others stored with store_pair is there then.
+__device__ __forceinline__ bool last_to_arrive(int* counter, int n) {
+  __shared__ int last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    if (last) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // for the next launch
+  }
+  __syncthreads();
+  return last;
+}
+
+// partial: [B, n_heads, n_splits, HD + 2] = (sum[HD], maximum, denominator), on 8 bytes; BASE2: maxima are exponents of 2, else
+// of e.  The workgroup's NW waves take the heads h0 ... h0 + G - 1 of row b in turn.
+template <int HD, int NW, bool BASE2, typename T>
+__device__ __forceinline__ void merge_splits(const float* partial, T* __restrict__ out, float* __restrict__ lse, int b, int n_heads,
+                                             int h0, int G, int n_splits, const float* __restrict__ sink_logit, int wave, int lane) {
+  constexpr int EL = (HD / 2 + WAVE - 1) / WAVE, PRE = 8;      // pairs of elements a lane; splits asked for together
+  auto weight = [](float d) { return BASE2 ? __builtin_amdgcn_exp2f(d) : expf(d); };
+  for (int hh = wave; hh < G; hh += NW) {
+    const int h = h0 + hh;
+    const float* part = partial + ((size_t)b * n_heads + h) * n_splits * (HD + 2);
+    const float logit = sink_logit != nullptr ? sink_logit[h] * (BASE2 ? 1.4426950408889634f : 1.0f) : -FLT_MAX;
+    float m = logit, l = 0.f;
+    float2 acc[EL];
+#pragma unroll
+    for (int e = 0; e < EL; ++e) acc[e] = make_float2(0.f, 0.f);
+    for (int s0 = 0; s0 < n_splits; s0 += PRE) {
+      float2 v[PRE][EL], ml[PRE];
+#pragma unroll
+      for (int u = 0; u < PRE; ++u) {
+        const float* ps = part + (size_t)min(s0 + u, n_splits - 1) * (HD + 2);
+        ml[u] = load_pair(ps + HD);
+#pragma unroll
+        for (int e = 0; e < EL; ++e) v[u][e] = load_pair(ps + 2 * min(lane + e * WAVE, HD / 2 - 1));
+      }
+      float m_new = m;
+#pragma unroll
+      for (int u = 0; u < PRE; ++u) m_new = fmaxf(m_new, ml[u].x);
+      const float corr = weight(m - m_new);
+      l *= corr;
+#pragma unroll
+      for (int e = 0; e < EL; ++e) acc[e].x *= corr, acc[e].y *= corr;
+#pragma unroll
+      for (int u = 0; u < PRE; ++u)
+        if (s0 + u < n_splits) {
+          const float f = weight(ml[u].x - m_new);
+          l = fmaf(ml[u].y, f, l);
+#pragma unroll
+          for (int e = 0; e < EL; ++e) {
+            acc[e].x = fmaf(v[u][e].x, f, acc[e].x);
+            acc[e].y = fmaf(v[u][e].y, f, acc[e].y);
+          }
+        }
+      m = m_new;
+    }
+    if (sink_logit != nullptr && l > 0.f) l += weight(logit - m);
+    const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+    T* row = out + ((size_t)b * n_heads + h) * HD;
+#pragma unroll
+    for (int e = 0; e < EL; ++e) {
+      const int p = lane + e * WAVE;
+      if (p < HD / 2) {
+        row[2 * p] = from_f32<T>(acc[e].x * inv_l);
+        row[2 * p + 1] = from_f32<T>(acc[e].y * inv_l);
+      }
+    }
+    if (lse != nullptr && lane == 0)
+      lse[(size_t)b * n_heads + h] = l > 0.f ? (BASE2 ? m * 0.6931471805599453f : m) + logf(l) : -FLT_MAX;
+  }
+}

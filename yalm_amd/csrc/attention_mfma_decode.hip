@@ -1,6 +1,7 @@
 // Decode attention on the matrix cores: one query a sequence over the pages of the cache (see attention_mfma.h for the
 // products' layout).
 #include "attention_mfma.h"
+#include "attention_merge.h"
 
 // attention_simple.hip; base2: the partial results' maxima are exponents of 2, not of e
 int yalm_attn_decode_combine_bf16(const float* partial, void* out, float* lse, int B, int n_heads, int head_dim,
@@ -26,7 +27,7 @@ __global__ __launch_bounds__(NW * WAVE, NW == 4 && HD <= 128 ? 2 : 1) void attn_
     const int* __restrict__ block_table, int table_stride, int ring_pages, const int* __restrict__ seq_slot,
     const int* __restrict__ seq_len, float* __restrict__ partial, bf16* __restrict__ out, float* __restrict__ lse,
     int n_heads, int n_kv_heads, int window, int n_splits, int n_pages, const int* __restrict__ step_max_len,
-    const int* __restrict__ seq_order, ScoreShape shape) {
+    const int* __restrict__ seq_order, ScoreShape shape, int* __restrict__ counters) {
   const float* __restrict__ bias = shape.bias;
   const int n_bias = shape.n_bias;
   // A head size that is no multiple of 32 (pages in rows then): the last step of the scores' product is half empty.
@@ -233,15 +234,27 @@ __global__ __launch_bounds__(NW * WAVE, NW == 4 && HD <= 128 ? 2 : 1) void attn_
         f32x4 v = sm_o[0][dt][lane];
 #pragma unroll
         for (int w = 1; w < NW; ++w) v += sm_o[w][dt][lane];
+        float* to = part + dt * 16 + 4 * qd;
+        if (counters != nullptr) {
+          store_pair(to, v[0], v[1]);
+          store_pair(to + 2, v[2], v[3]);
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) part[dt * 16 + 4 * qd + r] = v[r];
+          for (int r = 0; r < 4; ++r) to[r] = v[r];
+        }
       }
       if (wave == 0 && qd == 0) {
-        part[HD] = m_all;
-        part[HD + 1] = lt;
+        if (counters != nullptr) {
+          store_pair(part + HD, m_all, lt);
+        } else {
+          part[HD] = m_all;
+          part[HD + 1] = lt;
+        }
       }
     }
   }
+  if (counters != nullptr && last_to_arrive(counters + (size_t)blockIdx.z * gridDim.y + blockIdx.y, n_splits))
+    merge_splits<HD, NW, true>(partial, out, lse, b, n_heads, h0, G, n_splits, shape.sink_logit, wave, lane);
 }
 
 }  // namespace
@@ -250,13 +263,14 @@ int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v
                                int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
                                float* lse, float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window,
                                int n_splits, int n_pages, int page_layout, const SinkArgs& sinks,
-                               const int* step_max_len, const int* seq_order, const ScoreShape& shape,
+                               const int* step_max_len, const int* seq_order, const ScoreShape& shape, int* counters,
                                hipStream_t stream) {
   const float* bias = shape.bias;
   const int n_bias = shape.n_bias;
   const bool shaped = shape.any();
   // with sinks the merge kernel always runs: it takes them in, also where there is one split
   const bool merge = n_splits > 1 || sinks.n_sinks > 0;
+  if (n_splits == 1 || sinks.n_sinks > 0 || ((uintptr_t)partial & 7)) counters = nullptr;      // the kernel merges splits, and no sinks
   if (!mfma_shape_ok(n_heads, n_kv_heads, head_dim, shaped)) return YALM_ERR_ARG;
   // a score bias: the engine's layout of the pages only (blocks where the head size allows), and no sinks (they are
   // scored without it)
@@ -269,8 +283,8 @@ int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v
 #define YALM_DECODE(HD_, NW_, BLOCKS_, BIAS_)                                                                       \
   attn_decode_mfma_kernel<HD_, NW_, BLOCKS_, BIAS_><<<grid, NW_ * WAVE, 0, stream>>>(                               \
       (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, block_table, table_stride, ring_pages, seq_slot, \
-      seq_len, partial, merge ? nullptr : (bf16*)out, lse, n_heads, n_kv_heads, window, n_splits, n_pages, \
-      step_max_len, seq_order, shape)
+      seq_len, partial, merge && counters == nullptr ? nullptr : (bf16*)out, lse, n_heads, n_kv_heads, window, n_splits, n_pages, \
+      step_max_len, seq_order, shape, counters)
   // 4 waves a workgroup: 8 measured no faster with one split and slower with more (a CU draws about
   // 33 GB/s whatever its number of waves, so a small batch needs its workgroups spread over all CUs)
   // pages in blocks for the head sizes that are multiples of 32, in rows for the others (and for yalm_attn_decode)
@@ -321,6 +335,6 @@ int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v
 #undef YALM_DECODE_HD16
 #undef YALM_DECODE
   int rc = launch_status();
-  if (rc != YALM_OK || !merge) return rc;          // one split writes the result itself
+  if (rc != YALM_OK || !merge || counters != nullptr) return rc;      // one split, or the last to arrive, writes the result itself
   return yalm_attn_decode_combine_bf16(partial, out, lse, B, n_heads, head_dim, n_splits, 1, sinks, shape.sink_logit, stream);
 }

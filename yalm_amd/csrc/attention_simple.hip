@@ -20,12 +20,12 @@ int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_
                               int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out, float* lse,
                               float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window, int n_splits,
                               int n_pages, int page_layout, const int* step_max_len, const int* seq_order,
-                              const ScoreShape& shape, hipStream_t stream);
+                              const ScoreShape& shape, int* counters, hipStream_t stream);
 int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
                                int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
                                float* lse, float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window,
                                int n_splits, int n_pages, int page_layout, const SinkArgs& sinks,
-                               const int* step_max_len, const int* seq_order, const ScoreShape& shape,
+                               const int* step_max_len, const int* seq_order, const ScoreShape& shape, int* counters,
                                hipStream_t stream);
 
 namespace {
@@ -425,7 +425,7 @@ int attn_decode_any(const void* q, const void* k_pages, const void* v_pages, con
                     int page_layout, int dtype, int force_simple, const SinkArgs& sinks, const int* step_max_len,
                     const int* seq_order, const float* score_bias, int n_bias, float softcap,
                     const float* sink_logit, const float* slopes, int block, const float* log_a, const float* log_b,
-                                 hipStream_t stream) {
+                    int* counters, hipStream_t stream) {
   if (B <= 0) return YALM_OK;
   const ScoreShape shape = {score_bias, n_bias, softcap, sink_logit, slopes, block, log_a, log_b};
   if ((score_bias != nullptr && n_bias <= 0) || softcap < 0.f || block < 0 || ((shape.any() || block > 0) && sinks.n_sinks > 0))
@@ -438,11 +438,13 @@ int attn_decode_any(const void* q, const void* k_pages, const void* v_pages, con
   if (dtype == YALM_F32) {
     if (!force_simple) {
       const bool merge = n_splits > 1 || sinks.n_sinks > 0;     // with sinks the merge kernel always runs: it takes them in
+      int* arrived = n_splits > 1 && sinks.n_sinks == 0 && ((uintptr_t)partial & 7) == 0 ? counters : nullptr;
       int rc = yalm_attn_decode_f32_mfma(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len,
-                                         merge ? nullptr : out, lse, partial, B, n_heads, n_kv_heads, head_dim, window,
-                                         n_splits, n_pages, page_layout, step_max_len, seq_order, shape, stream);
+                                         merge && arrived == nullptr ? nullptr : out, lse, partial, B, n_heads, n_kv_heads,
+                                         head_dim, window, n_splits, n_pages, page_layout, step_max_len, seq_order, shape,
+                                         arrived, stream);
       if (rc != YALM_ERR_ARG) {
-        if (rc != YALM_OK || !merge) return rc;
+        if (rc != YALM_OK || !merge || arrived != nullptr) return rc;
         attn_decode_combine_kernel<float><<<cgrid, COMBINE_THREADS, 0, stream>>>(partial, (float*)out, lse, n_heads,
                                                                                  head_dim, n_splits, sinks, sink_logit);
         return launch_status();
@@ -467,7 +469,7 @@ int attn_decode_any(const void* q, const void* k_pages, const void* v_pages, con
   if (!force_simple) {
     int rc = yalm_attn_decode_bf16_mfma(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len,
                                         out, lse, partial, B, n_heads, n_kv_heads, head_dim, window, n_splits,
-                                        n_pages, page_layout, sinks, step_max_len, seq_order, shape, stream);
+                                        n_pages, page_layout, sinks, step_max_len, seq_order, shape, counters, stream);
     if (rc != YALM_ERR_ARG) return rc;
   }
   if (head_dim <= ACC_SMALL * WAVE) {
@@ -495,11 +497,25 @@ extern "C" int yalm_attn_decode_lse(const void* q, const void* k_pages, const vo
                                     const float* score_bias, int n_bias, float softcap, const float* sink_logit,
                                     const float* slopes, int block, const float* log_a, const float* log_b,
                                  hipStream_t stream) {
+  return yalm_attn_decode_merged(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len, out, lse, partial,
+                                 nullptr, B, n_heads, n_kv_heads, head_dim, window, n_splits, n_pages, page_layout, dtype,
+                                 force_simple, step_max_len, seq_order, score_bias, n_bias, softcap, sink_logit, slopes, block,
+                                 log_a, log_b, stream);
+}
+
+extern "C" int yalm_attn_decode_merged(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
+                                       int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
+                                       float* lse, float* partial, int* counters, int B, int n_heads, int n_kv_heads,
+                                       int head_dim, int window, int n_splits, int n_pages, int page_layout, int dtype,
+                                       int force_simple, const int* step_max_len, const int* seq_order,
+                                       const float* score_bias, int n_bias, float softcap, const float* sink_logit,
+                                       const float* slopes, int block, const float* log_a, const float* log_b,
+                                       hipStream_t stream) {
   SinkArgs none = {};
   return attn_decode_any(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len, out, lse,
                          partial, B, n_heads, n_kv_heads, head_dim, window, n_splits, n_pages, page_layout, dtype,
                          force_simple, none, step_max_len, seq_order, score_bias, n_bias, softcap, sink_logit, slopes, block,
-                         log_a, log_b, stream);
+                         log_a, log_b, counters, stream);
 }
 
 extern "C" int yalm_attn_decode(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
@@ -544,7 +560,7 @@ extern "C" int yalm_attn_decode_sinks(const void* q, const void* k_pages, const 
   sk.n_sinks = n_sinks;
   return attn_decode_any(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len, out, nullptr,
                          partial, B, n_heads, n_kv_heads, head_dim, window, n_splits, n_pages, page_layout, dtype,
-                         force_simple, sk, step_max_len, seq_order, nullptr, 0, 0.f, nullptr, nullptr, 0, nullptr, nullptr, stream);
+                         force_simple, sk, step_max_len, seq_order, nullptr, 0, 0.f, nullptr, nullptr, 0, nullptr, nullptr, nullptr, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -205,6 +205,17 @@ int yalm_attn_decode_lse(const void* q, const void* k_pages, const void* v_pages
 //   out[t, h] = (e^lse out + sum_j e^s_j v_j) / (e^lse + sum_j e^s_j), s_j = q . k_j / sqrt(hd); with src_f32 (the
 //   out_f32 of yalm_attn_prefill_lse; may be null) the unrounded result is read from there, so that the mixed row
 //   is rounded once.
+// yalm_attn_decode_lse with an int32 for each (sequence, KV head and up to 16 of its query heads), zero before the first call
+//   and left so: where a matrix-core kernel takes the call, its last workgroup of a row merges the splits, and no kernel of
+//   its own does (null: as yalm_attn_decode_lse).  Calls that may run at the same time need counters of their own, as they
+//   need a `partial` of their own.
+int yalm_attn_decode_merged(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
+                            int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
+                            float* lse, float* partial, int* counters, int B, int n_heads, int n_kv_heads, int head_dim,
+                            int window, int n_splits, int n_pages, int page_layout, int dtype, int force_simple,
+                            const int* step_max_len, const int* seq_order, const float* score_bias, int n_bias,
+                            float softcap, const float* sink_logit, const float* slopes, int block, const float* log_a,
+                            const float* log_b, hipStream_t stream);
 // A decode step: yalm_attn_decode_sinks is yalm_attn_decode whose merge of the splits takes those sinks in
 //   as further splits of one key each (no rounding in between, no launch more; the merge runs with one
 //   split too); with store != 0 a token at a position < n_sinks first stores its own key and value from its

@@ -660,15 +660,22 @@ def attn_decode_workspace_floats(B, n_heads, head_dim, n_splits):
     return library.lib().yalm_attn_decode_workspace(B, n_heads, head_dim, n_splits) // 4
 
 
+def attn_decode_counters(B, n_heads, n_kv_heads):
+    """The int32 elements that attn_decode's `counters` must hold: one for each sequence, KV head and 16 of its heads."""
+    return B * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
+
+
 def attn_decode(q, k_pages, v_pages, block_table, ring_pages, seq_slot, seq_len, out, partial, n_heads, n_kv_heads,
                 head_dim, window, n_splits, lse=None, sinks=None, layout=None, step_max_len=None, seq_order=None,
-                score_bias=None, softcap=0.0, sink_logit=None, slopes=None, block=0, log_distance=None):
+                score_bias=None, softcap=0.0, sink_logit=None, slopes=None, block=0, log_distance=None, counters=None):
     """One query per sequence over the cache pages (laid out as `layout` says, default page_layout(head_dim));
     seq_len counts the new key.  lse as in attn_prefill.  step_max_len (int32 [1] on the device, optional): the
     length of the step's longest sequence, with which sequences of unequal lengths are cut into splits of equal
     size; seq_order (int32 [B] on the device, a permutation of the rows, optional): the order in which the
     workgroups take the rows (both change the division of the work and no result).  score_bias: see _bias; softcap,
-    sink_logit: see _shape; block: see attn_prefill (none of these with sinks).
+    sink_logit: see _shape; block: see attn_prefill (none of these with sinks).  counters (optional; int32, at least
+    attn_decode_counters elements, zero and left so): the attention kernel's last workgroup of a row merges the splits,
+    instead of a kernel behind it; not shared with a call that may run at the same time.
     sinks = (sink_k, sink_v [slots, n_kv_heads, n_sinks, head_dim], cos_sin or None, rotary_dim, store):
     the attention sinks that a query's window no longer covers are taken in where the splits are merged
     (their keys turned by max(0, position - window - n_sinks + 1) positions with the table cos_sin); with
@@ -696,8 +703,14 @@ def attn_decode(q, k_pages, v_pages, block_table, ring_pages, seq_slot, seq_len,
     p_ord = _opt(seq_order, "seq_order", torch.int32, (B,))
     if sinks is None:
         p_lse = None if lse is None else _need(lse, "lse", torch.float32, (B, n_heads))
-        library.check(library.lib().yalm_attn_decode_lse(
-            p_q, p_kp, p_vp, p_bt, stride, ring_pages, p_ss, p_sl, p_o, p_lse, p_w, B, n_heads, n_kv_heads, head_dim,
+        p_cnt = None
+        if counters is not None:
+            p_cnt = _need(counters, "counters", torch.int32)
+            if counters.numel() < attn_decode_counters(B, n_heads, n_kv_heads):
+                raise ValueError("attn_decode: %d counters, %d needed"
+                                 % (counters.numel(), attn_decode_counters(B, n_heads, n_kv_heads)))
+        library.check(library.lib().yalm_attn_decode_merged(
+            p_q, p_kp, p_vp, p_bt, stride, ring_pages, p_ss, p_sl, p_o, p_lse, p_w, p_cnt, B, n_heads, n_kv_heads, head_dim,
             int(window), int(n_splits), n_pages, _layout(layout, head_dim), dtype_code(dt), force, p_max, p_ord,
             *_bias(score_bias, n_heads), *_shape(softcap, sink_logit, n_heads, slopes), int(block),
             *_log_distance(log_distance, n_heads), _stream()), "attn_decode")

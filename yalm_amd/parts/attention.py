@@ -68,6 +68,13 @@ def decode_splits(n_heads, n_kv_heads, head_dim, B, max_pages, ragged=False, sha
     return max(1, min(max_pages, TARGET_WORKGROUPS // max(1, B * n_heads)))
 
 
+def decode_counters(ctx, B, n_heads, n_kv_heads, n_splits):
+    """What lets the attention kernel of a decode step merge its splits itself (None: there is nothing to merge)."""
+    if n_splits == 1:
+        return None
+    return ctx.ws.get_zeroed("attn.counters", (kernels.attn_decode_counters(B, n_heads, n_kv_heads),), torch.int32)
+
+
 @part("mixer", "gqa_attention")
 class GQAttention(Part):
     prompt_tables = (kv_tiles,)
@@ -244,7 +251,8 @@ class GQAttention(Part):
             sinks = (sink_k, sink_v, self.position.table, self.position.rotary_dim, writes_cache)
         kernels.attn_decode(q, k_pages, v_pages, group.table, group.ring_pages, ctx.seq_slot, ctx.seq_len, o, partial,
                             self.n_heads, self.n_kv_heads, self.head_dim, self.window, n_splits, sinks=sinks,
-                            step_max_len=ctx.step_max_len, seq_order=ctx.seq_order, score_bias=self.score_bias)
+                            step_max_len=ctx.step_max_len, seq_order=ctx.seq_order, score_bias=self.score_bias,
+                            counters=decode_counters(ctx, T, self.n_heads, self.n_kv_heads, n_splits))
 
     def forward(self, h, x, ctx, line, writes_cache=True, emit_for=None):
         T = h.shape[0]

@@ -31,7 +31,7 @@ import torch
 from ..cache.manager import KVRequest
 from ..ops import kernels
 from ..weights.loader import ParamSpec, place
-from .attention import ROPE_TILES_MIN_TOKENS, decode_splits, kv_tiles
+from .attention import ROPE_TILES_MIN_TOKENS, decode_counters, decode_splits, kv_tiles
 from .base import Part, build_part, part
 from .rope import interleave_rows
 
@@ -214,7 +214,8 @@ class LatentAttention(Part):
             n_splits = decode_splits(H, 1, P, T, min(group.ring_pages, ctx.pages_bucket), ctx.ragged)
             partial = ws.get("attn.partial", (kernels.attn_decode_workspace_floats(T, H, P, n_splits),), torch.float32)
             kernels.attn_decode(q, k_pages, v_pages, group.table, group.ring_pages, ctx.seq_slot, ctx.seq_len, o, partial,
-                                H, 1, P, self.window, n_splits, step_max_len=ctx.step_max_len, seq_order=ctx.seq_order)
+                                H, 1, P, self.window, n_splits, step_max_len=ctx.step_max_len, seq_order=ctx.seq_order,
+                                counters=decode_counters(ctx, T, H, 1, n_splits))
         # 4. the heads' values from their latent results, the gate, the output projection
         values = ws.get("latent.values", (T, H * self.v_dim), act)
         gate = proj[:, kv_at + self.kv_cols:] if self.gated else None
