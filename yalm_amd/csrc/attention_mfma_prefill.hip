@@ -24,6 +24,10 @@ namespace {
 // workgroup, 32 key tiles at 2,048 tokens, while the mean is 17).
 // BIAS: the scores are shaped (ScoreShape: a cap, a term by the distance of query and key, bias[head][min(distance,
 // n_bias - 1)], a learned logit in the denominator; each optional).
+__host__ __device__ constexpr bool prefill_dma(int hd) { return hd == 128; }
+// the place (0..15) at which a fragment read takes key row `row` (key_row's inverse): its chunks are swizzled by it
+__device__ __forceinline__ int key_swizzle(int row) { return (row & 3) | ((row >> 3) & 3) << 2; }
+
 template <int HD, int NC, int KSPL, bool BIAS>
 __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void attn_prefill_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_stage, const bf16* __restrict__ v_stage,
@@ -36,8 +40,12 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
   // lanes, the row's last 8 elements once more in the keys'), and the tile's chunks do not divide evenly over the threads.
   constexpr int KS = (HD + 31) / 32, DT = HD / 16;
   static_assert(HD % 16 == 0, "head sizes in steps of 16");
-  constexpr int KROW = HD + 8;                    // LDS row strides (elements): 16 bytes of padding
-  constexpr int VROW = PAGE + 8;
+  // DMA (head size 128): the tiles go from memory straight into LDS, rows unpadded, the 16-byte chunks of a row XOR-swizzled
+  // by the place at which the fragment reads take the row, so that sixteen lanes read from all banks; else through registers
+  // into rows with 16 bytes of padding.
+  constexpr bool DMA = prefill_dma(HD);
+  constexpr int KROW = DMA ? HD : HD + 8;         // LDS row strides (elements)
+  constexpr int VROW = DMA ? PAGE : PAGE + 8;
   constexpr int KTILE = PAGE * KROW, VTILE = HD * VROW;
   constexpr int CHUNKS = PAGE * HD / 8;           // 16-byte chunks of a tile
   constexpr int NLOAD = (CHUNKS + 255) / 256;     // chunks per thread and tile
@@ -57,7 +65,7 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
   }
   // half: which group of four waves (which key tiles); tid, wave: the thread's place inside its group
   const int half = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 256), tid = threadIdx.x % 256;
-  const int wave = tid / WAVE, lane = tid % WAVE, qd = lane / 16, j = lane % 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE, qd = lane / 16, j = lane % 16;
   int b = 0;
   {
     int lo_b = 0, hi_b = B - 1;
@@ -117,7 +125,22 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
   const int wave_last = min(pos0 + 16 * NC - 1, len - 1);
   const size_t tile_elems = (size_t)n_kv_heads * PAGE * HD;
 
-  // global -> registers -> LDS; key rows are stored at the index the MFMA row reads them at
+  // global -> LDS, a wave's instructions 1 KB each: keys 4 rows, values 8; a lane asks for the chunk that belongs in its place.
+  // Or global -> registers -> LDS; key rows are then stored at the index the MFMA row reads them at
+  auto dma_tile = [&](int kt, int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops a template that names this builtin, and its launch stub with it
+    const bf16* kp = k_stage + (tile0 + kt) * tile_elems + (size_t)g * PAGE * HD;
+    const bf16* vp = v_stage + (tile0 + kt) * tile_elems + (size_t)g * PAGE * HD;
+    unsigned char* to = smem_raw + (size_t)(buf * KSPL + half) * (KTILE + VTILE) * sizeof(bf16);
+#pragma unroll
+    for (int p = 0; p < NLOAD; ++p) {
+      const int c = tid + p * 256, row = c / (HD / 8), vrow = c / 8;
+      __builtin_amdgcn_global_load_lds(kp + row * HD + ((c % (HD / 8)) ^ key_swizzle(row)) * 8, to + (wave + p * 4) * 1024, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(vp + vrow * PAGE + ((c % 8) ^ ((vrow >> 1) & 7)) * 8,
+                                       to + KTILE * sizeof(bf16) + (wave + p * 4) * 1024, 16, 0, 0);
+    }
+#endif
+  };
   bf16x8 rk[NLOAD], rv[NLOAD];
   auto load_tile = [&](int kt) {
     const bf16* kp = k_stage + (tile0 + kt) * tile_elems + (size_t)g * PAGE * HD;
@@ -145,15 +168,23 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
   };
 
   if (kt_lo + half <= kt_hi) {
-    load_tile(kt_lo + half);
-    store_tile(0);
+    if constexpr (DMA) {
+      dma_tile(kt_lo + half, 0);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+      load_tile(kt_lo + half);
+      store_tile(0);
+    }
   }
   __syncthreads();
   for (int kt0 = kt_lo; kt0 <= kt_hi; kt0 += KSPL) {        // every group its own tile of the round
     const int kt = kt0 + half;
     const int cur = ((kt0 - kt_lo) / KSPL) & 1;
     const bool next = kt + KSPL <= kt_hi;
-    if (next) load_tile(kt + KSPL);
+    if (next) {
+      if constexpr (DMA) dma_tile(kt + KSPL, cur ^ 1);      // that buffer was read before the last barrier
+      else load_tile(kt + KSPL);
+    }
     const int base = kt * PAGE;
     const bool visible = kt <= kt_hi && wave_live && base <= wave_last && base + PAGE - 1 >= wave_lo;
     if (visible) {
@@ -168,7 +199,9 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(ks_l + (t * 16 + j) * KROW + min(ks * 32 + qd * 8, HD - 8));
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(
+              DMA ? ks_l + key_row(t, j) * KROW + ((ks * 4 + qd) ^ j) * 8
+                  : ks_l + (t * 16 + j) * KROW + min(ks * 32 + qd * 8, HD - 8));
 #pragma unroll
           for (int c = 0; c < NC; ++c)
             sc[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qv[c][ks], sc[c][t], 0, 0, 0);
@@ -244,7 +277,8 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
       for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          bf16x8 vf = *reinterpret_cast<const bf16x8*>(vs_l + (dt * 16 + j) * VROW + s2 * 32 + qd * 8);
+          bf16x8 vf = *reinterpret_cast<const bf16x8*>(
+              vs_l + (dt * 16 + j) * VROW + (DMA ? ((s2 * 4 + qd) ^ ((j >> 1) & 7)) * 8 : s2 * 32 + qd * 8));
           if (tail) {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
@@ -256,7 +290,8 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
         }
       }
     }
-    if (next) store_tile(cur ^ 1);
+    if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this wave's share of the next tile has landed
+    else if (next) store_tile(cur ^ 1);
     __syncthreads();
   }
   if constexpr (KSPL == 2) {
@@ -391,7 +426,8 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
   if (tile_order && (n_order <= 0 || n_order > n_tiles)) return YALM_ERR_ARG;
   dim3 grid(n_heads, tile_order ? n_order : n_tiles);
   const long total = (long)grid.x * grid.y;
-  const size_t tile_bytes = ((size_t)PAGE * (head_dim + 8) + (size_t)head_dim * (PAGE + 8)) * sizeof(bf16);
+  const size_t pad = prefill_dma(head_dim) ? 0 : 8;
+  const size_t tile_bytes = ((size_t)PAGE * (head_dim + pad) + (size_t)head_dim * (PAGE + pad)) * sizeof(bf16);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k_stage, *vp = (const bf16*)v_stage;
   // A wide head: two buffers of keys and values fill up to 141 KB of LDS, so four waves a workgroup are the one form.
   if (head_dim > 128)
