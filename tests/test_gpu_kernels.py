@@ -789,8 +789,8 @@ def test_attn_decode_merged_by_the_last_workgroup(n_heads, n_kv, hd, window, len
 # order with splits of the longest sequence's size, a value that is infinite (a query that does not see it must not notice)
 @pytest.mark.parametrize("shape", ["plain", "bias", "softcap", "sink", "slopes", "log", "infinite"])
 @pytest.mark.parametrize("n_heads,n_kv,hd,window,block,lens,splits", [
-    (4, 2, 16, 0, 0, [5, 64, 65], 1), (6, 3, 48, 100, 0, [130, 300], 3), (8, 2, 128, 0, 0, [200, 1, 129], 2),
-    (18, 1, 64, 70, 0, [150, 64], 1), (3, 3, 32, 0, 96, [257, 17], 2), (2, 1, 112, 0, 0, [66], 1)])
+    (4, 2, 64, 0, 0, [5, 64, 65], 1), (6, 3, 80, 100, 0, [130, 300], 3), (8, 2, 128, 0, 0, [200, 1, 129], 2),
+    (18, 1, 64, 70, 0, [150, 64], 1), (3, 3, 96, 0, 96, [257, 17], 2), (2, 1, 112, 0, 0, [66], 1)])
 def test_attention_float32_on_the_matrix_cores(n_heads, n_kv, hd, window, block, lens, splits, shape):
     k = K()
     T, B = sum(lens), len(lens)

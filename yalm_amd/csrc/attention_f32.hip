@@ -1,5 +1,6 @@
 // Attention of the true 32-bit path on the matrix cores (v_mfma_f32_16x16x4_f32), softmax state and expf in float32:
-// head sizes of 16 to 128 in steps of 16, every shape of the scores.  The kernels of attention_simple.hip take the others.
+// head sizes of 64 to 128 in steps of 16, every shape of the scores.  The kernels of attention_simple.hip take the others:
+// on smaller heads the products are too few to matter beside a page's exponentials and exchanges.
 //
 //   scores^T[key, query] = K[key, :] . Q[query, :]        A = 16 key rows x 4 elements, B = 16 queries
 //   out^T[elem, query]  += V^T[elem, key] P^T[key, query]  A = 16 elements x 4 keys, B = P^T
@@ -431,7 +432,7 @@ int launch_prefill(const float* q, const float* k_stage, const float* v_stage, f
 }
 
 bool takes(int head_dim, const void* a, const void* b, const void* c, const void* d) {
-  return head_dim >= 16 && head_dim <= 128 && head_dim % 16 == 0 &&
+  return head_dim >= 64 && head_dim <= 128 && head_dim % 16 == 0 &&
          (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) & 15) == 0;
 }
 
@@ -447,9 +448,6 @@ int yalm_attn_prefill_f32_mfma(const void* q, const void* k_stage, const void* v
     return launch_prefill<HD_>((const float*)q, (const float*)k_stage, (const float*)v_stage, (float*)out, out_f32, lse, \
                                cu_seqlens, seq_tile0, B, n_tiles, n_heads, n_kv_heads, window, shape, stream)
   switch (head_dim) {
-    YALM_HD(16);
-    YALM_HD(32);
-    YALM_HD(48);
     YALM_HD(64);
     YALM_HD(80);
     YALM_HD(96);
@@ -489,9 +487,6 @@ int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_
     else YALM_RUN(HD_, false, false);                                                                                    \
     break
   switch (head_dim) {
-    YALM_HD16(16);
-    YALM_HD32(32);
-    YALM_HD16(48);
     YALM_HD32(64);
     YALM_HD16(80);
     YALM_HD32(96);
