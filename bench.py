@@ -122,7 +122,7 @@ KERNEL_FACES = ("embed", "rmsnorm", "gemm", "gemm_norm", "gemm_norm_qkv_rope", "
                 "attn_decode", "sink_store", "attn_sink_mix", "argmax", "cast", "norm_add", "polynorm", "head_matmul",
                 "latent_pack", "moe_route", "moe_select", "moe_pair_gate_up", "moe_pair_down", "moe_grouped", "embed_sinusoid",
                 "qkv_pack", "v_tiles", "mlstm_scan", "mlstm_chunks", "gated_delta", "embed_learned", "activate", "gated_add",
-                "time_conv", "gated_bias_act", "sigmoid_gate", "loop_pack", "hgrn2", "layer_norm", "layer_norm_sum", "embed_pairs",
+                "time_conv", "gated_bias_act", "sigmoid_gate", "loop_pack", "hgrn2", "norm_add_pair", "layer_norm", "layer_norm_sum", "embed_pairs",
                 "latent_norm", "moe_select_groups", "gla", "gla_tiles", "squash", "squash_add", "rms_gate", "head_gate", "softcap",
                 "lightning", "lightning_tiles", "lru", "lru_step")
 FP32_FACES = ("mlstm_scan", "mlstm_chunks", "gated_delta", "hgrn2", "gla", "gla_tiles", "lightning", "lightning_tiles")     # kernels of float32 multiply-adds whatever the model's dtype: priced against that peak
@@ -198,6 +198,8 @@ def kernel_cost(name, a, kw, kv_tokens, torch):
             2.0 * T * H * K * N
     if name == "latent_pack":
         return "latent_pack %d tokens" % a[0].shape[0], nbytes(a[7]), 0.0
+    if name == "norm_add_pair":
+        return "norm_add_pair %dx%d" % tuple(a[0].shape), 4 * nbytes(a[0]) + (nbytes(a[6]) if len(a) > 6 and a[6] is not None else 0), 0.0
     if name == "norm_add":
         return "norm_add %dx%d" % tuple(a[0].shape), 3 * nbytes(a[0]), 0.0
     if name == "layer_norm_sum":

@@ -58,6 +58,31 @@ def test_norm_add(R_, D, out_dtype):
     assert torch.allclose(xd.cpu().to(F64), x.to(F64) + P.rms_norm(y.to(F64), wb.to(F64), 1e-5), rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("R_,D", [(1, 8), (5, 80), (33, 1000), (2, 2048), (3, 4097), (2, 9001)])       # the kernel's forms by width
+@pytest.mark.parametrize("out_dtype", [None, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("then_norm", [False, True])
+def test_norm_add_pair(R_, D, out_dtype, then_norm):
+    from yalm_amd.ops import kernels
+    y, y2, x = randn(R_, D, seed=1, scale=3.0), randn(R_, D, seed=4, scale=0.2), randn(R_, D, seed=2)
+    w, w2, wn = (1.0 + 0.1 * randn(D, seed=s) for s in (3, 5, 13))
+    want = x.to(F64) + P.rms_norm(y.to(F64), w.to(F64), 1e-5) + P.rms_norm(y2.to(F64), w2.to(F64), 1e-5)
+    xd = x.to(DEV)
+    h = None if out_dtype is None else torch.zeros(R_, D, dtype=out_dtype, device=DEV)
+    args = (y.to(DEV), w.to(DEV), y2.to(DEV), w2.to(DEV), 1e-5, xd, h, (wn.to(DEV), 3e-6) if then_norm else None)
+    if then_norm and h is None:
+        with pytest.raises(ValueError):
+            kernels.norm_add_pair(*args)
+        return
+    kernels.norm_add_pair(*args)
+    # D squares summed in float32 and a few roundings of numbers up to 12: as for one result above
+    assert torch.allclose(xd.cpu().to(F64), want, rtol=1e-5, atol=1e-5)
+    if h is not None and not then_norm:
+        assert torch.equal(h.cpu(), xd.cpu().to(out_dtype))
+    elif h is not None:
+        tol = 1e-5 if out_dtype == torch.float32 else 1e-2
+        assert torch.allclose(h.cpu().to(F64), P.rms_norm(want, wn.to(F64), 3e-6), rtol=tol, atol=tol)
+
+
 @pytest.mark.parametrize("R_,F", [(1, 4), (7, 112), (20, 1500), (3, 8200), (2, 40001)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_polynorm(R_, F, out_dtype):

@@ -17,39 +17,49 @@ __global__ __launch_bounds__(ROW_THREADS) void cast_kernel(const float* __restri
   for (; i < n; i += step) out[i] = from_f32<T>(x[i]);
 }
 
-// x[r] += y[r] * rsqrt(mean(y[r]^2) + eps) * w; if h is given: h[r] = T(x[r]), or with next_w the norm that reads
-// the stream next, h[r] = T(x[r] * rsqrt(mean(x[r]^2) + next_eps) * next_w)
-template <typename W, typename T, int NT, int PER>
-__global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ y, const W* __restrict__ w, float eps,
+// x[r] += y[r] * rsqrt(mean(y[r]^2) + eps) * w, with PAIR then the same of y2 and w2; if h is given: h[r] = T(x[r]), or with
+// next_w the norm that reads the stream next, h[r] = T(x[r] * rsqrt(mean(x[r]^2) + next_eps) * next_w).  Bound by memory in a
+// prompt (x, y, y2 once each way: a second launch for y2 and a norm kernel behind it would read and write x twice more:
+// 1,909 rows of 4,096 24 + 24 + 10 -> 42 us), by the launch in a decode step (three of 4.6 us -> one of 6.5).
+template <typename W, typename T, int NT, int PER, bool PAIR>
+__global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ y, const W* __restrict__ w,
+                                                      const float* __restrict__ y2, const W* __restrict__ w2, float eps,
                                                       float* __restrict__ x, T* __restrict__ h, const float* __restrict__ next_w,
                                                       float next_eps, int D) {
   // PER > 0: the row fits PER values a thread; y is read once and the new x stays in registers for the second norm
   __shared__ float red[NT / WAVE];
   const size_t row = (size_t)blockIdx.x * D;
-  float keep[PER > 0 ? PER : 1];
-  float ss = 0.f;
+  float keep[PER > 0 ? PER : 1], keep2[PER > 0 && PAIR ? PER : 1];
+  float ss = 0.f, sp = 0.f;
   if (PER > 0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
       keep[j] = i < D ? y[row + i] : 0.f;
       ss += keep[j] * keep[j];
+      if constexpr (PAIR) {
+        keep2[j] = i < D ? y2[row + i] : 0.f;
+        sp += keep2[j] * keep2[j];
+      }
     }
   } else {
     for (int i = threadIdx.x; i < D; i += NT) {
       const float v = y[row + i];
       ss += v * v;
+      if constexpr (PAIR) sp += y2[row + i] * y2[row + i];
     }
   }
   ss = block_sum<NT / WAVE>(ss, red);
-  const float scale = 1.0f / sqrtf(ss / (float)D + eps);
+  if constexpr (PAIR) sp = block_sum<NT / WAVE>(sp, red);
+  const float scale = 1.0f / sqrtf(ss / (float)D + eps), scale_p = PAIR ? 1.0f / sqrtf(sp / (float)D + eps) : 0.f;
   float ss2 = 0.f;
   if (PER > 0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
       if (i < D) {
-        const float v = x[row + i] + keep[j] * scale * to_f32(w[i]);
+        float v = x[row + i] + keep[j] * scale * to_f32(w[i]);
+        if constexpr (PAIR) v += keep2[j] * scale_p * to_f32(w2[i]);
         x[row + i] = v;
         keep[j] = v;
         ss2 += v * v;
@@ -58,7 +68,8 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
     }
   } else {
     for (int i = threadIdx.x; i < D; i += NT) {
-      const float v = x[row + i] + y[row + i] * scale * to_f32(w[i]);
+      float v = x[row + i] + y[row + i] * scale * to_f32(w[i]);
+      if constexpr (PAIR) v += y2[row + i] * scale_p * to_f32(w2[i]);
       x[row + i] = v;
       ss2 += v * v;
       if (h != nullptr && next_w == nullptr) h[row + i] = from_f32<T>(v);
@@ -307,15 +318,15 @@ extern "C" int yalm_cast(const float* x, void* out, long n, int out_dtype, hipSt
   return launch_status();
 }
 
-template <typename W, typename T>
-static int norm_add_launch(const float* y, const void* w, float eps, float* x, void* h, const float* next_w, float next_eps,
-                           int R, int D, hipStream_t stream) {
-  if (D < 2048)
-    norm_add_kernel<W, T, 256, 8><<<R, 256, 0, stream>>>(y, (const W*)w, eps, x, (T*)h, next_w, next_eps, D);
-  else if (D <= 8192)
-    norm_add_kernel<W, T, 1024, 8><<<R, 1024, 0, stream>>>(y, (const W*)w, eps, x, (T*)h, next_w, next_eps, D);
-  else
-    norm_add_kernel<W, T, 1024, 0><<<R, 1024, 0, stream>>>(y, (const W*)w, eps, x, (T*)h, next_w, next_eps, D);
+template <typename W, typename T, bool PAIR>
+static int norm_add_launch(const float* y, const void* w, const float* y2, const void* w2, float eps, float* x, void* h,
+                           const float* next_w, float next_eps, int R, int D, hipStream_t stream) {
+#define NA(NT_, PER_) \
+  norm_add_kernel<W, T, NT_, PER_, PAIR><<<R, NT_, 0, stream>>>(y, (const W*)w, y2, (const W*)w2, eps, x, (T*)h, next_w, next_eps, D)
+  if (D < 2048) NA(256, 8);
+  else if (D <= 8192) NA(1024, 8);
+  else NA(1024, 0);
+#undef NA
   return launch_status();
 }
 
@@ -327,10 +338,20 @@ extern "C" int yalm_norm_add(const float* y, const void* w, int w_dtype, float e
   if (h_out != nullptr && h_dtype != YALM_F32 && h_dtype != YALM_BF16) return YALM_ERR_DTYPE;
   const bool hb = h_out != nullptr && h_dtype == YALM_BF16;
   if (w_dtype == YALM_F32)
-    return hb ? norm_add_launch<float, bf16>(y, w, eps, x, h_out, next_w, next_eps, R, D, stream)
-              : norm_add_launch<float, float>(y, w, eps, x, h_out, next_w, next_eps, R, D, stream);
-  return hb ? norm_add_launch<bf16, bf16>(y, w, eps, x, h_out, next_w, next_eps, R, D, stream)
-            : norm_add_launch<bf16, float>(y, w, eps, x, h_out, next_w, next_eps, R, D, stream);
+    return hb ? norm_add_launch<float, bf16, false>(y, w, nullptr, nullptr, eps, x, h_out, next_w, next_eps, R, D, stream)
+              : norm_add_launch<float, float, false>(y, w, nullptr, nullptr, eps, x, h_out, next_w, next_eps, R, D, stream);
+  return hb ? norm_add_launch<bf16, bf16, false>(y, w, nullptr, nullptr, eps, x, h_out, next_w, next_eps, R, D, stream)
+            : norm_add_launch<bf16, float, false>(y, w, nullptr, nullptr, eps, x, h_out, next_w, next_eps, R, D, stream);
+}
+
+extern "C" int yalm_norm_add_pair(const float* y, const float* w, const float* y2, const float* w2, float eps, float* x,
+                                  void* h_out, int h_dtype, const float* next_w, float next_eps, int R, int D, hipStream_t stream) {
+  if (R <= 0) return YALM_OK;
+  if (D <= 0) return YALM_ERR_ARG;
+  if (h_out != nullptr && h_dtype != YALM_F32 && h_dtype != YALM_BF16) return YALM_ERR_DTYPE;
+  return h_out != nullptr && h_dtype == YALM_BF16
+             ? norm_add_launch<float, bf16, true>(y, w, y2, w2, eps, x, h_out, next_w, next_eps, R, D, stream)
+             : norm_add_launch<float, float, true>(y, w, y2, w2, eps, x, h_out, next_w, next_eps, R, D, stream);
 }
 
 template <typename T, bool STORE_X>

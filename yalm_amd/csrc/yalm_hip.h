@@ -269,6 +269,9 @@ int yalm_token_prob(const float* logits, const int* index, float* prob, int R, i
 int yalm_cast(const float* x, void* out, long n, int out_dtype, hipStream_t stream);
 int yalm_norm_add(const float* y, const void* w, int w_dtype, float eps, float* x, void* h_out, int h_dtype,
                   const float* next_w, float next_eps, int R, int D, hipStream_t stream);
+// yalm_norm_add_pair: yalm_norm_add of y and w (float32), then of y2 and w2, in one pass over the stream.
+int yalm_norm_add_pair(const float* y, const float* w, const float* y2, const float* w2, float eps, float* x, void* h_out,
+                       int h_dtype, const float* next_w, float next_eps, int R, int D, hipStream_t stream);
 // yalm_layer_norm: n[r] = LN(alpha * x[row(r)] + y[r]), LN(v) = (v - mean) / sqrt(mean of the squared deviations + eps) * w + b,
 // row(r) = row_index ? row_index[r] : r; y may be null.  store_x (no row_index then): x[r] = n[r].  h (optional with
 // store_x): dtype(n[r]), or with next_w, next_b the layer norm with those of n[r].  All weights float32 [D].

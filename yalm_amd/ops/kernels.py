@@ -819,6 +819,24 @@ def norm_add(y, weight, eps, x, h_out=None, next_norm=None):
     return x
 
 
+def norm_add_pair(y, weight, y2, weight2, eps, x, h_out=None, next_norm=None):
+    """norm_add of y and its weight, then of y2 and its own (both weights float32), in one pass over the stream."""
+    R, D = y.shape
+    p_h, h_code = None, 0
+    if h_out is not None:
+        p_h, h_code = _need(h_out, "h_out", None, (R, D)), dtype_code(h_out.dtype)
+    p_n, n_eps = None, 0.0
+    if next_norm is not None:
+        if h_out is None:
+            raise ValueError("norm_add_pair: the next norm's output needs h_out")
+        p_n, n_eps = _need(next_norm[0], "next norm weight", torch.float32, (D,)), float(next_norm[1])
+    library.check(library.lib().yalm_norm_add_pair(
+        _need(y, "y", torch.float32, (R, D)), _need(weight, "weight", torch.float32, (D,)), _need(y2, "y2", torch.float32, (R, D)),
+        _need(weight2, "weight2", torch.float32, (D,)), float(eps), _need(x, "x", torch.float32, (R, D)), p_h, h_code, p_n, n_eps,
+        R, D, _stream()), "norm_add_pair")
+    return x
+
+
 def layer_norm(x, weight, bias, eps, out, row_index=None):
     """out[r] = LN(x[row(r)]) * weight + bias, LN(v) = (v - mean) / sqrt(mean of the squared deviations + eps); x, weight and
     bias float32, out [R, D] in the compute dtype, row(r) = row_index[r] (int32) or r."""

@@ -51,6 +51,7 @@ _SIGNATURES = {
     "yalm_gemm_partial_scaled": (_I, [_P, _P, _P, ctypes.c_long, _I, _I, _I, _P, _P, _I, _F, _P]),
     "yalm_cast": (_I, [_P, _P, ctypes.c_long, _I, _P]),
     "yalm_norm_add": (_I, [_P, _P, _I, _F, _P, _P, _I, _P, _F, _I, _I, _P]),
+    "yalm_norm_add_pair": (_I, [_P, _P, _P, _P, _F, _P, _P, _I, _P, _F, _I, _I, _P]),
     "yalm_polynorm": (_I, [_P, _P, _F, _P, _I, _I, _I, _P]),
     "yalm_head_matmul": (_I, [_P, _I, ctypes.c_long, _I, _I, _P, _I, _P, _I, ctypes.c_long, _I, _I, _F, _P, ctypes.c_long,
                               _I, _I, _I, _I, _P]),
@@ -99,7 +100,7 @@ _SIGNATURES = {
     "yalm_probe_mfma": (_I, [_I, _I, _I, _P, _P, _P]),
 }
 
-ABI_VERSION = 38
+ABI_VERSION = 39
 
 
 class KernelError(RuntimeError):

@@ -13,6 +13,7 @@ class PreNormResidualBlock(Part):
         p = layer_spec.prefix
         self.mixer_norm = build_part("norm", layer_spec.mixer_norm, dim, p)
         self.mixer = build_part("mixer", layer_spec.mixer, dim, p)
+        self.mixer_emits = getattr(self.mixer, "emits_norm", False)
         self.feed_forward = self.feed_forward_norm = None             # a layer may have no feed-forward
         if layer_spec.part("feed_forward") is not None:
             self.feed_forward_norm = build_part("norm", layer_spec.feed_forward_norm, dim, p)
@@ -37,6 +38,13 @@ class PreNormResidualBlock(Part):
         may prepare its activations), or None."""
         return self.mixer_norm
 
+    def _mix(self, h, x, ctx, line, writes_cache):
+        """The mixer on its input; one that takes emit_for may leave the feed-forward's norm ready."""
+        if self.mixer_emits and self.feed_forward is not None and not self.feed_forward.fuses_norm(self.feed_forward_norm, x, ctx):
+            self.mixer.forward(h, x, ctx, line, writes_cache, emit_for=self.feed_forward_norm)
+        else:
+            self.mixer.forward(h, x, ctx, line, writes_cache)
+
     def forward(self, x, ctx, line, writes_cache=True, next_norm=None):
         plain_end = False                 # whether the layer's last sublayer ran behind a norm kernel of its own
         if self.mixer_input is not None:
@@ -48,7 +56,7 @@ class PreNormResidualBlock(Part):
                 self.mixer_norm.forward(x, h, ctx)
             filtered = ctx.ws.get("block.filtered", (x.shape[0], self.dim), ctx.act_dtype)
             self.mixer_input.forward(h, filtered, ctx, (line, "input"))
-            self.mixer.forward(filtered, x, ctx, (line, "mixer"), writes_cache)
+            self._mix(filtered, x, ctx, (line, "mixer"), writes_cache)
             plain_end = self.feed_forward is None
         elif self.mixer.fuses_norm(self.mixer_norm, x, ctx):
             self.mixer.forward_prenorm(x, self.mixer_norm, ctx, line, writes_cache,
@@ -60,14 +68,18 @@ class PreNormResidualBlock(Part):
             else:
                 h = ctx.ws.get("block.h", (x.shape[0], self.dim), ctx.act_dtype)
                 self.mixer_norm.forward(x, h, ctx)
-            self.mixer.forward(h, x, ctx, line, writes_cache)
+            self._mix(h, x, ctx, line, writes_cache)
             plain_end = self.feed_forward is None
         if self.feed_forward is not None:
             if self.feed_forward.fuses_norm(self.feed_forward_norm, x, ctx):
                 self.feed_forward.forward_prenorm(x, self.feed_forward_norm, ctx, emit_for=next_norm)
             else:
-                h = ctx.ws.get("block.h", (x.shape[0], self.dim), ctx.act_dtype)
-                self.feed_forward_norm.forward(x, h, ctx)
+                left = ctx.normed.pop(id(self.feed_forward_norm), None)
+                if left is not None and left[1] is None:      # the mixer has left this norm's output
+                    h = left[0]
+                else:
+                    h = ctx.ws.get("block.h", (x.shape[0], self.dim), ctx.act_dtype)
+                    self.feed_forward_norm.forward(x, h, ctx)
                 self.feed_forward.forward(h, x, ctx)
                 plain_end = True
         # sublayers that fold no norm into their products leave nothing for whoever reads the stream next: in a decode

@@ -18,6 +18,8 @@ from .base import JoinableMixer, Part, build_part, part
 
 @part("mixer", "side_by_side")
 class SideBySide(Part):
+    emits_norm = True                 # forward takes emit_for
+
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
         p = spec.params
@@ -100,14 +102,20 @@ class SideBySide(Part):
         r.between(h, proj[:, l.n_in:], o[:, l.n_out:], ctx, (line, "right"), writes_cache, r.share)
         self._gemm(ctx, o, self.wo, x, epilogue)
 
-    def forward(self, h, x, ctx, line, writes_cache=True):
+    def forward(self, h, x, ctx, line, writes_cache=True, emit_for=None):
+        """emit_for: the norm that reads the stream next; two normed results leave its output for whoever takes it."""
         T = h.shape[0]
         if self.scales is not None:
             if self.late_bias is not None:
                 raise ValueError("a mixer whose last product has a bias writes its result (forward_to); it does not add to the stream")
             return self._joint(h, x, ctx, line, writes_cache, kernels.EPI_ADD_F32)
-        y = ctx.ws.get("side.y", (T, self.dim), torch.float32)
+        y, y2 = (ctx.ws.get(name, (T, self.dim), torch.float32) for name in ("side.y", "side.y2"))
         self.left.forward_to(h, y, ctx, (line, "left"), writes_cache)
-        kernels.norm_add(y, self.w_left, self.eps, x)
-        self.right.forward_to(h, y, ctx, (line, "right"), writes_cache)
-        kernels.norm_add(y, self.w_right, self.eps, x)
+        self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache)
+        if emit_for is None or not hasattr(emit_for, "fused") or ctx.act_dtype == torch.float32:   # its sums run in another order:
+            # in float32 the norm's own kernel keeps its bits, which a faint read-out behind it magnifies a thousandfold
+            kernels.norm_add_pair(y, self.w_left, y2, self.w_right, self.eps, x)
+            return
+        ahead = ctx.ws.get("block.h", (T, self.dim), ctx.act_dtype)           # both members have read what lay there
+        kernels.norm_add_pair(y, self.w_left, y2, self.w_right, self.eps, x, ahead, emit_for.fused())
+        ctx.normed[id(emit_for)] = (ahead, None, None)
