@@ -174,7 +174,7 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
       if (r >= M) break;
       const int pos = max(rope_pos[r], 0);
       rope_cs[r] = make_float2(1.f, 0.f);
-      if (ra.cos_sin != nullptr && half > 0)
+      if (ra.cos_sin != nullptr && half > 0 && ra.n_positions > 0)
         rope_cs[r] = ra.cos_sin[(size_t)min(pos, ra.n_positions - 1) * half + min(nn >> 1, half - 1)];
       rope_phys[r] = ra.block_table[(size_t)max(rope_slot[r], 0) * ra.table_stride + (pos / PAGE) % ra.ring_pages];
     }
