@@ -750,7 +750,7 @@ def test_attn_decode_with_the_length_of_the_longest_sequence(n_heads, n_kv, hd, 
 @pytest.mark.parametrize("n_heads,n_kv,hd,window,lens,splits,sink", [
     (4, 2, 16, 0, [5, 640], 2, False), (8, 2, 128, 0, [3000, 3, 700], 16, False), (34, 2, 64, 0, [300, 65], 3, True),
     (5, 1, 80, 100, [700, 64], 5, True), (2, 1, 32, 0, [70 * 64 * 4], 70, False), (40, 1, 128, 0, [900], 9, False),
-    (3, 1, 256, 0, [400, 1], 4, False)])
+    (3, 1, 256, 0, [400, 1], 4, False), (8, 2, 64, 0, [64 * 17, 200], 17, True), (2, 2, 192, 0, [64 * 33, 64 * 66], 33, False)])
 def test_attn_decode_merged_by_the_last_workgroup(n_heads, n_kv, hd, window, lens, splits, sink, dtype):
     k = K()
     B = len(lens)
@@ -768,16 +768,9 @@ def test_attn_decode_merged_by_the_last_workgroup(n_heads, n_kv, hd, window, len
             k.attn_decode(q, kp, vp, bt, ring, i32(slots + [-1]), i32(lens + [0]), out, partial, n_heads, n_kv, hd, window, splits,
                           lse=lse, sink_logit=logit, counters=c)
             got.append((out.double(), lse.double()))
-        # The same partial results, added in another order.  Each side's sum over the splits is off by at most (splits + 4)
-        # 2^-24 of the sum of its terms' sizes (a rounding a term, the weights' exponential and the division), and those,
-        # weights of values that sum to one, are at most the largest value; a bfloat16 result is rounded on top, 2^-8 of
-        # itself a side.  The lse: the logarithm of a sum that is off by as much, and its own rounding.
-        biggest = max(v.abs().max().item() for v in vals)
-        off = 2 * (splits + 4) * 2.0 ** -24
-        rounding = 2.0 ** -7 if dtype == torch.bfloat16 else 0.0
+        # the same partial results, added in the same order: the same bits
         (a, la), (b, lb) = got
-        assert torch.isfinite(b).all() and bool(((a - b).abs() <= off * biggest + rounding * b.abs()).all())
-        assert bool(((la - lb).abs() <= off + 2.0 ** -21 * lb.abs()).all())
+        assert torch.isfinite(b).all() and torch.equal(a, b) and torch.equal(la, lb)
         assert int(counters.abs().sum()) == 0
     with pytest.raises(ValueError):
         k.attn_decode(q, kp, vp, bt, ring, i32(slots + [-1]), i32(lens + [0]), out, partial, n_heads, n_kv, hd, window, splits,

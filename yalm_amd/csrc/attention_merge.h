@@ -1,5 +1,5 @@
 // The merge of a decode step's attention splits inside the attention kernel: the workgroup that arrives last of a (sequence,
-// KV head)'s splits merges their partial results, in the splits' order whoever is last, so that no kernel of its own does
+// KV head)'s splits merges their partial results, in one order whoever is last, so that no kernel of its own does
 // (4.7 us a layer of a decode step, most of it a launch).  counters: an int for each (sequence, blockIdx.y), zero before
 // the launch and behind it.
 //
@@ -37,58 +37,79 @@ __device__ __forceinline__ bool last_to_arrive(int* counter, int n) {
 }
 
 // partial: [B, n_heads, n_splits, HD + 2] = (sum[HD], maximum, denominator), on 8 bytes; BASE2: maxima are exponents of 2, else
-// of e.  The workgroup's NW waves take the heads h0 ... h0 + G - 1 of row b in turn.
+// of e.  The workgroup's NW waves take the heads h0 ... h0 + G - 1 of row b in turn.  The sums run in the order of
+// attn_decode_combine_kernel, so that it does not show in a result which of the two merged: the denominators a lane a split,
+// the weighted sums in four chains of every fourth split.
 template <int HD, int NW, bool BASE2, typename T>
 __device__ __forceinline__ void merge_splits(const float* partial, T* __restrict__ out, float* __restrict__ lse, int b, int n_heads,
                                              int h0, int G, int n_splits, const float* __restrict__ sink_logit, int wave, int lane) {
-  constexpr int EL = (HD / 2 + WAVE - 1) / WAVE, PRE = 8;      // pairs of elements a lane; splits asked for together
-  auto weight = [](float d) { return BASE2 ? __builtin_amdgcn_exp2f(d) : expf(d); };
+  constexpr int EL = (HD / 2 + WAVE - 1) / WAVE, PRE = 8, CHAINS = 4;      // pairs of elements a lane; splits asked for together
+  static_assert(PRE % CHAINS == 0 && WAVE % PRE == 0, "a split's chain and its lane follow from its place in a run");
+  auto weight = [](float d) { return BASE2 ? exp2f(d) : expf(d); };
   for (int hh = wave; hh < G; hh += NW) {
     const int h = h0 + hh;
     const float* part = partial + ((size_t)b * n_heads + h) * n_splits * (HD + 2);
-    const float logit = sink_logit != nullptr ? sink_logit[h] * (BASE2 ? 1.4426950408889634f : 1.0f) : -FLT_MAX;
-    float m = logit, l = 0.f;
-    float2 acc[EL];
-#pragma unroll
-    for (int e = 0; e < EL; ++e) acc[e] = make_float2(0.f, 0.f);
-    for (int s0 = 0; s0 < n_splits; s0 += PRE) {
-      float2 v[PRE][EL], ml[PRE];
+    auto maximum_of = [&](int s) { return s < n_splits ? load_pair(part + (size_t)s * (HD + 2) + HD) : make_float2(-FLT_MAX, 0.f); };
+    float2 v[2][PRE][EL];
+    auto ask = [&](int buf, int s0) {
 #pragma unroll
       for (int u = 0; u < PRE; ++u) {
         const float* ps = part + (size_t)min(s0 + u, n_splits - 1) * (HD + 2);
-        ml[u] = load_pair(ps + HD);
 #pragma unroll
-        for (int e = 0; e < EL; ++e) v[u][e] = load_pair(ps + 2 * min(lane + e * WAVE, HD / 2 - 1));
+        for (int e = 0; e < EL; ++e) v[buf][u][e] = load_pair(ps + 2 * min(lane + e * WAVE, HD / 2 - 1));
       }
-      float m_new = m;
+    };
+    float2 ml = maximum_of(lane);                  // of split lane
+    ask(0, 0);
+    if (n_splits > PRE) ask(1, PRE);
+    float m = ml.x;
+    for (int s = lane + WAVE; s < n_splits; s += WAVE) m = fmaxf(m, maximum_of(s).x);
+    m = wave_max(m);
+    const float logit = sink_logit != nullptr ? sink_logit[h] * (BASE2 ? 1.4426950408889634f : 1.0f) : -FLT_MAX;
+    if (sink_logit != nullptr) m = fmaxf(m, logit);
+    float f = weight(ml.x - m);                    // of split lane
+    float l = lane < n_splits ? ml.y * f : 0.f;
+    for (int s = lane + WAVE; s < n_splits; s += WAVE) {
+      const float2 other = maximum_of(s);
+      l = fmaf(other.y, weight(other.x - m), l);
+    }
+    l = wave_sum(l);
+    if (sink_logit != nullptr && l > 0.f) l += weight(logit - m);
+    float2 acc[CHAINS][EL];
 #pragma unroll
-      for (int u = 0; u < PRE; ++u) m_new = fmaxf(m_new, ml[u].x);
-      const float corr = weight(m - m_new);
-      l *= corr;
+    for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-      for (int e = 0; e < EL; ++e) acc[e].x *= corr, acc[e].y *= corr;
+      for (int e = 0; e < EL; ++e) acc[c][e] = make_float2(0.f, 0.f);
+    auto add = [&](int buf, int s0) {
+      if (s0 != 0 && s0 % WAVE == 0) f = weight(maximum_of(s0 + lane).x - m);
 #pragma unroll
-      for (int u = 0; u < PRE; ++u)
+      for (int u = 0; u < PRE; ++u) {
+        const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), (s0 + u) % WAVE));
         if (s0 + u < n_splits) {
-          const float f = weight(ml[u].x - m_new);
-          l = fmaf(ml[u].y, f, l);
 #pragma unroll
           for (int e = 0; e < EL; ++e) {
-            acc[e].x = fmaf(v[u][e].x, f, acc[e].x);
-            acc[e].y = fmaf(v[u][e].y, f, acc[e].y);
+            acc[u % CHAINS][e].x = fmaf(v[buf][u][e].x, fs, acc[u % CHAINS][e].x);
+            acc[u % CHAINS][e].y = fmaf(v[buf][u][e].y, fs, acc[u % CHAINS][e].y);
           }
         }
-      m = m_new;
+      }
+    };
+    for (int s0 = 0; s0 < n_splits; s0 += 2 * PRE) {
+      add(0, s0);
+      if (s0 + 2 * PRE < n_splits) ask(0, s0 + 2 * PRE);
+      if (s0 + PRE < n_splits) {
+        add(1, s0 + PRE);
+        if (s0 + 3 * PRE < n_splits) ask(1, s0 + 3 * PRE);
+      }
     }
-    if (sink_logit != nullptr && l > 0.f) l += weight(logit - m);
     const float inv_l = l > 0.f ? 1.0f / l : 0.f;
     T* row = out + ((size_t)b * n_heads + h) * HD;
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
       const int p = lane + e * WAVE;
       if (p < HD / 2) {
-        row[2 * p] = from_f32<T>(acc[e].x * inv_l);
-        row[2 * p + 1] = from_f32<T>(acc[e].y * inv_l);
+        row[2 * p] = from_f32<T>((((acc[0][e].x + acc[1][e].x) + acc[2][e].x) + acc[3][e].x) * inv_l);
+        row[2 * p + 1] = from_f32<T>((((acc[0][e].y + acc[1][e].y) + acc[2][e].y) + acc[3][e].y) * inv_l);
       }
     }
     if (lse != nullptr && lane == 0)
