@@ -750,7 +750,7 @@ def test_attn_decode_with_the_length_of_the_longest_sequence(n_heads, n_kv, hd, 
 @pytest.mark.parametrize("n_heads,n_kv,hd,window,lens,splits,sink", [
     (4, 2, 16, 0, [5, 640], 2, False), (8, 2, 128, 0, [3000, 3, 700], 16, False), (34, 2, 64, 0, [300, 65], 3, True),
     (5, 1, 80, 100, [700, 64], 5, True), (2, 1, 32, 0, [70 * 64 * 4], 70, False), (40, 1, 128, 0, [900], 9, False),
-    (3, 1, 256, 0, [400, 1], 4, False), (8, 2, 64, 0, [64 * 17, 200], 17, True), (2, 2, 192, 0, [64 * 33, 64 * 66], 33, False)])
+    (3, 1, 256, 0, [400, 1], 4, False), (4, 2, 256, 0, [400, 1], 4, False), (8, 2, 64, 0, [64 * 17, 200], 17, True), (2, 2, 192, 0, [64 * 33, 64 * 66], 33, False)])
 def test_attn_decode_merged_by_the_last_workgroup(n_heads, n_kv, hd, window, lens, splits, sink, dtype):
     k = K()
     B = len(lens)
@@ -775,6 +775,26 @@ def test_attn_decode_merged_by_the_last_workgroup(n_heads, n_kv, hd, window, len
     with pytest.raises(ValueError):
         k.attn_decode(q, kp, vp, bt, ring, i32(slots + [-1]), i32(lens + [0]), out, partial, n_heads, n_kv, hd, window, splits,
                       counters=counters[:-1])
+
+
+# more heads than a workgroup has waves: the kernel behind merges (inside, the waves would take the heads in turn), so whatever
+# the counters hold is left alone
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(5, 1, 64), (16, 2, 128), (40, 1, 96), (3, 1, 256), (16, 1, 192)])
+def test_attn_decode_of_many_heads_is_merged_behind(n_heads, n_kv, hd, dtype):
+    k = K()
+    lens, splits = [700, 64], 3
+    kp, vp, bt, slots, ring, _, _ = paged_case(lens, n_kv, hd, 0, dtype, 21)
+    q = rnd((2, n_heads * hd), 22, dtype).to(DEV)
+    partial = torch.empty(k.attn_decode_workspace_floats(2, n_heads, hd, splits), device=DEV)
+    counters = torch.full((k.attn_decode_counters(2, n_heads, n_kv),), 1000, dtype=torch.int32, device=DEV)
+    got = []
+    for c in (None, counters):
+        out = torch.full((2, n_heads * hd), 7.0, dtype=dtype, device=DEV)
+        k.attn_decode(q, kp.to(DEV), vp.to(DEV), bt.to(DEV), ring, i32(slots), i32(lens), out, partial, n_heads, n_kv, hd, 0, splits,
+                      counters=c)
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and int((counters - 1000).abs().sum()) == 0
 
 
 # float32 on the matrix cores against the general kernels: head sizes with pages in rows and in blocks, one tile and many, a

@@ -411,7 +411,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
         for (int r = 0; r < 4; ++r) to[d * 16 + lq * 4 + r] = v[r] * keep;       // a partial row need not lie on 16 bytes
       }
     }
-  if (counters != nullptr && last_to_arrive(counters + (size_t)blockIdx.z * gridDim.y + blockIdx.y, n_splits))
+  if (counters != nullptr && last_to_arrive(counters + ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * COUNTER_STRIDE, n_splits))
     merge_splits<HD, NW, false>(partial, out, lse, b, n_heads, h0, G, n_splits, sh.sink_logit, wave, lane);
 }
 

@@ -1,7 +1,8 @@
 // The merge of a decode step's attention splits inside the attention kernel: the workgroup that arrives last of a (sequence,
 // KV head)'s splits merges their partial results, in one order whoever is last, so that no kernel of its own does
 // (4.7 us a layer of a decode step, most of it a launch).  counters: an int for each (sequence, blockIdx.y), zero before
-// the launch and behind it.
+// the launch and behind it, each in a line of memory of its own (arrivals at counters of one line wait for each other: eight rows
+// in 16 splits 9.1 us with them side by side, 8.4 apart).
 //
 // The partial results pass between XCDs, whose second-level caches do not see each other's lines: they are stored and loaded
 // as relaxed atomics of agent scope, which go through to where all XCDs see them and are not served from a cache that does
@@ -12,7 +13,15 @@
 #include <float.h>
 #include "common.h"
 
+constexpr int COUNTER_STRIDE = 32;               // ints
 typedef unsigned long long pair_bits;            // two floats
+
+// Whether the last workgroup to arrive should merge the splits of its heads (of `heads` of a KV head, at most 16): a wave takes
+// a head, so where there is one for each the merge costs the last workgroup less than a launch behind it, and where the waves
+// take several in turn more.  Merged inside against by the kernel behind, us, at 4 / 16 / 64 splits of 256 keys and one sequence:
+// four waves and 4 heads of 128 7.5 / 8.0 / 11.8 against 8.1 / 8.5 / 18.4; 8 heads 8.6 / 9.5 / 15.6 against 8.0 / 8.4 / 17.9;
+// 16 heads 11.1 / 12.8 / 24.3 against 8.1 / 8.6 / 18.1; two waves and 4 heads of 256 11.5 / 12.8 / 21.4 against 10.9 / 11.4 / 27.0.
+inline bool merges_inside(int heads, int waves) { return heads <= waves; }
 
 __device__ __forceinline__ void store_pair(float* p, float a, float b) {
   const pair_bits v = (pair_bits)__float_as_uint(a) | ((pair_bits)__float_as_uint(b) << 32);

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(NW * WAVE, NW == 4 && HD <= 128 ? 2 : 1) void attn_
       }
     }
   }
-  if (counters != nullptr && last_to_arrive(counters + (size_t)blockIdx.z * gridDim.y + blockIdx.y, n_splits))
+  if (counters != nullptr && last_to_arrive(counters + ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * COUNTER_STRIDE, n_splits))
     merge_splits<HD, NW, true>(partial, out, lse, b, n_heads, h0, G, n_splits, shape.sink_logit, wave, lane);
 }
 
@@ -270,13 +270,15 @@ int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v
   const bool shaped = shape.any();
   // with sinks the merge kernel always runs: it takes them in, also where there is one split
   const bool merge = n_splits > 1 || sinks.n_sinks > 0;
-  if (n_splits == 1 || sinks.n_sinks > 0 || ((uintptr_t)partial & 7)) counters = nullptr;      // the kernel merges splits, and no sinks
   if (!mfma_shape_ok(n_heads, n_kv_heads, head_dim, shaped)) return YALM_ERR_ARG;
   // a score bias: the engine's layout of the pages only (blocks where the head size allows), and no sinks (they are
   // scored without it)
   if ((bias != nullptr && n_bias <= 0) ||
       (shaped && ((page_layout != YALM_PAGE_BLOCKS && head_dim % 32 == 0) || sinks.n_sinks > 0)))
     return YALM_ERR_ARG;
+  // the attention kernel merges splits, and no sinks
+  if (n_splits == 1 || sinks.n_sinks > 0 || ((uintptr_t)partial & 7) || !merges_inside(n_heads / n_kv_heads, head_dim == 256 ? 2 : 4))
+    counters = nullptr;
   const int parts_g = (n_heads / n_kv_heads + 15) / 16;      // workgroups a KV head: 16 query heads each
   if ((long)n_kv_heads * parts_g > 65535) return YALM_ERR_ARG;
   dim3 grid(n_splits, n_kv_heads * parts_g, B);

@@ -5,6 +5,7 @@
 #include <float.h>
 #include <mutex>
 #include "common.h"
+#include "attention_merge.h"
 #include "sinks.h"
 #include "yalm_hip.h"
 
@@ -438,7 +439,8 @@ int attn_decode_any(const void* q, const void* k_pages, const void* v_pages, con
   if (dtype == YALM_F32) {
     if (!force_simple) {
       const bool merge = n_splits > 1 || sinks.n_sinks > 0;     // with sinks the merge kernel always runs: it takes them in
-      int* arrived = n_splits > 1 && sinks.n_sinks == 0 && ((uintptr_t)partial & 7) == 0 ? counters : nullptr;
+      int* arrived = n_splits > 1 && sinks.n_sinks == 0 && ((uintptr_t)partial & 7) == 0 && merges_inside(n_heads / n_kv_heads, 4)
+                         ? counters : nullptr;
       int rc = yalm_attn_decode_f32_mfma(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len,
                                          merge && arrived == nullptr ? nullptr : out, lse, partial, B, n_heads, n_kv_heads,
                                          head_dim, window, n_splits, n_pages, page_layout, step_max_len, seq_order, shape,

@@ -205,7 +205,7 @@ int yalm_attn_decode_lse(const void* q, const void* k_pages, const void* v_pages
 //   out[t, h] = (e^lse out + sum_j e^s_j v_j) / (e^lse + sum_j e^s_j), s_j = q . k_j / sqrt(hd); with src_f32 (the
 //   out_f32 of yalm_attn_prefill_lse; may be null) the unrounded result is read from there, so that the mixed row
 //   is rounded once.
-// yalm_attn_decode_lse with an int32 for each (sequence, KV head and up to 16 of its query heads), zero before the first call
+// yalm_attn_decode_lse with 32 int32 for each (sequence, KV head and up to 16 of its query heads), zero before the first call
 //   and left so: where a matrix-core kernel takes the call, its last workgroup of a row merges the splits, and no kernel of
 //   its own does (null: as yalm_attn_decode_lse).  Calls that may run at the same time need counters of their own, as they
 //   need a `partial` of their own.

@@ -661,8 +661,8 @@ def attn_decode_workspace_floats(B, n_heads, head_dim, n_splits):
 
 
 def attn_decode_counters(B, n_heads, n_kv_heads):
-    """The int32 elements that attn_decode's `counters` must hold: one for each sequence, KV head and 16 of its heads."""
-    return B * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
+    """The int32 elements that attn_decode's `counters` must hold: a line of memory for each sequence, KV head and 16 of its heads."""
+    return 32 * B * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
 
 
 def attn_decode(q, k_pages, v_pages, block_table, ring_pages, seq_slot, seq_len, out, partial, n_heads, n_kv_heads,
@@ -674,8 +674,8 @@ def attn_decode(q, k_pages, v_pages, block_table, ring_pages, seq_slot, seq_len,
     size; seq_order (int32 [B] on the device, a permutation of the rows, optional): the order in which the
     workgroups take the rows (both change the division of the work and no result).  score_bias: see _bias; softcap,
     sink_logit: see _shape; block: see attn_prefill (none of these with sinks).  counters (optional; int32, at least
-    attn_decode_counters elements, zero and left so): the attention kernel's last workgroup of a row merges the splits,
-    instead of a kernel behind it; not shared with a call that may run at the same time.
+    attn_decode_counters elements, zero and left so): the attention kernel's last workgroup of a row may merge the splits,
+    instead of a kernel behind it (it does where that is sooner; the results are the same, to the bit); not shared with a call that may run at the same time.
     sinks = (sink_k, sink_v [slots, n_kv_heads, n_sinks, head_dim], cos_sin or None, rotary_dim, store):
     the attention sinks that a query's window no longer covers are taken in where the splits are merged
     (their keys turned by max(0, position - window - n_sinks + 1) positions with the table cos_sin); with

@@ -100,7 +100,7 @@ _SIGNATURES = {
     "yalm_probe_mfma": (_I, [_I, _I, _I, _P, _P, _P]),
 }
 
-ABI_VERSION = 39
+ABI_VERSION = 40
 
 
 class KernelError(RuntimeError):
