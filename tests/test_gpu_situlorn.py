@@ -83,6 +83,23 @@ def test_norm_add_pair(R_, D, out_dtype, then_norm):
         assert torch.allclose(h.cpu().to(F64), P.rms_norm(want, wn.to(F64), 3e-6), rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("R_,D", [(1, 8), (5, 1024), (4, 1025), (3, 1028), (9, 2048), (2, 4096), (3, 4097), (7, 8192), (2, 8196), (2, 9001)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("off", [0, 1])                            # 1: a stream that does not lie on 16 bytes
+def test_norm_add_pair_has_the_bits_of_its_three_steps(R_, D, dtype, off):
+    from yalm_amd.ops import kernels
+    y, y2 = randn(R_, D, seed=1, scale=3.0).to(DEV), randn(R_, D, seed=4, scale=0.2).to(DEV)
+    flat = randn(R_ * D + off, seed=2).to(DEV)
+    w, w2, wn = ((1.0 + 0.1 * randn(D, seed=s)).to(DEV) for s in (3, 5, 13))
+    one, both = flat.clone()[off:].view(R_, D), flat.clone()[off:].view(R_, D)
+    h1, h2 = (torch.zeros(R_, D, dtype=dtype, device=DEV) for _ in range(2))
+    kernels.norm_add(y, w, 1e-5, one)
+    kernels.norm_add(y2, w2, 1e-5, one)
+    kernels.rmsnorm(one, wn, h1, 3e-6)
+    kernels.norm_add_pair(y, w, y2, w2, 1e-5, both, h2, (wn, 3e-6))
+    assert torch.equal(one, both) and torch.equal(h1, h2)
+
+
 @pytest.mark.parametrize("R_,F", [(1, 4), (7, 112), (20, 1500), (3, 8200), (2, 40001)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_polynorm(R_, F, out_dtype):

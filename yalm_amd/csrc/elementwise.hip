@@ -2,6 +2,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "rms_row.h"
 #include "yalm_hip.h"
 
 // ---------------------------------------------------------------------------
@@ -92,19 +93,12 @@ __global__ void rmsnorm_kernel(const float* __restrict__ x, const TW* __restrict
     return;
   }
   const float* xr = x + (size_t)src * D;
-  float ss = 0.f;
-  for (int i = threadIdx.x; i < D; i += NW * WAVE) {
-    float v = xr[i];
-    ss += v * v;
-  }
-  ss = block_sum<NW>(ss, red);
+  const float ss = block_sum<NW>(rms_part(xr, D, threadIdx.x, NW * WAVE), red);
   float scale = 1.0f / sqrtf(ss / (float)D + eps);
   for (int i = threadIdx.x; i < D; i += NW * WAVE) o[i] = from_f32<TO>(xr[i] * scale * to_f32(w[i]));
 }
 
-// The same with the row kept in registers between the two passes (read once, 16 bytes a load):
-// D a multiple of 4, at most 256 threads x 8 x 4 elements.
-constexpr int RMS_VEC_MAX = 8;
+// The same with the row kept in registers between the two passes (read once, 16 bytes a load): rms_row_vec.
 __device__ __forceinline__ void store4(float* o, float a, float b, float c, float d) {
   *reinterpret_cast<float4*>(o) = make_float4(a, b, c, d);
 }
@@ -133,7 +127,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float* __restric
   for (int u = 0; u < RMS_VEC_MAX; ++u) {
     const int i = threadIdx.x + u * 256;
     v[u] = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    ss += v[u].x * v[u].x + v[u].y * v[u].y + v[u].z * v[u].z + v[u].w * v[u].w;
+    ss = rms_add4(ss, v[u]);
   }
   ss = block_sum<4>(ss, red);
   const float scale = 1.0f / sqrtf(ss / (float)D + eps);
@@ -150,9 +144,7 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float* __restric
 template <typename TW, typename TO>
 static int rmsnorm_launch(const float* x, const void* w, void* out, const int* row_index, int R, int D, float eps,
                           hipStream_t stream) {
-  const bool vec = D % 4 == 0 && D > 1024 && D <= 256 * 4 * RMS_VEC_MAX && !((uintptr_t)x & 15) &&
-                   !((uintptr_t)out & 15);
-  if (vec)
+  if (rms_row_vec(x, out, D))
     rmsnorm_vec_kernel<TW, TO><<<R, 256, 0, stream>>>(x, (const TW*)w, (TO*)out, row_index, D, eps);
   else if (D > 1024)
     rmsnorm_kernel<TW, TO, 4><<<R, 256, 0, stream>>>(x, (const TW*)w, (TO*)out, row_index, D, eps);

@@ -3,6 +3,7 @@
 // a norm's place (tanh(alpha x) * w + b), and of a row's RMS norm under a sigmoid gate.  Everything is float32 arithmetic, on a
 // row per workgroup where a row has sums; inputs from GEMMs are float32, outputs go to the compute dtype.
 #include "common.h"
+#include "rms_row.h"
 #include "yalm_hip.h"
 
 namespace {
@@ -18,14 +19,15 @@ __global__ __launch_bounds__(ROW_THREADS) void cast_kernel(const float* __restri
 }
 
 // x[r] += y[r] * rsqrt(mean(y[r]^2) + eps) * w, with PAIR then the same of y2 and w2; if h is given: h[r] = T(x[r]), or with
-// next_w the norm that reads the stream next, h[r] = T(x[r] * rsqrt(mean(x[r]^2) + next_eps) * next_w).  Bound by memory in a
+// next_w the norm that reads the stream next, h[r] = T(x[r] * rsqrt(mean(x[r]^2) + next_eps) * next_w); with PAIR it has the
+// bits of the norm's own kernel (next_vec: rms_row_vec; the row goes through LDS to the threads that sum it there).  Bound by memory in a
 // prompt (x, y, y2 once each way: a second launch for y2 and a norm kernel behind it would read and write x twice more:
 // 1,909 rows of 4,096 24 + 24 + 10 -> 42 us), by the launch in a decode step (three of 4.6 us -> one of 6.5).
 template <typename W, typename T, int NT, int PER, bool PAIR>
 __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ y, const W* __restrict__ w,
                                                       const float* __restrict__ y2, const W* __restrict__ w2, float eps,
                                                       float* __restrict__ x, T* __restrict__ h, const float* __restrict__ next_w,
-                                                      float next_eps, int D) {
+                                                      float next_eps, bool next_vec, int D) {
   // PER > 0: the row fits PER values a thread; y is read once and the new x stays in registers for the second norm
   __shared__ float red[NT / WAVE];
   const size_t row = (size_t)blockIdx.x * D;
@@ -76,7 +78,15 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
     }
   }
   if (h == nullptr || next_w == nullptr) return;
-  ss2 = block_sum<NT / WAVE>(ss2, red);
+  if constexpr (PAIR && PER > 0) {
+    __shared__ __attribute__((aligned(16))) float new_x[NT * PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) new_x[threadIdx.x + j * NT] = keep[j];
+    __syncthreads();
+    ss2 = rms_sum_of_lds(new_x, D, next_vec, red);
+  } else {
+    ss2 = block_sum<NT / WAVE>(ss2, red);
+  }
   const float scale2 = 1.0f / sqrtf(ss2 / (float)D + next_eps);
   if (PER > 0) {
 #pragma unroll
@@ -322,7 +332,9 @@ template <typename W, typename T, bool PAIR>
 static int norm_add_launch(const float* y, const void* w, const float* y2, const void* w2, float eps, float* x, void* h,
                            const float* next_w, float next_eps, int R, int D, hipStream_t stream) {
 #define NA(NT_, PER_) \
-  norm_add_kernel<W, T, NT_, PER_, PAIR><<<R, NT_, 0, stream>>>(y, (const W*)w, y2, (const W*)w2, eps, x, (T*)h, next_w, next_eps, D)
+  norm_add_kernel<W, T, NT_, PER_, PAIR><<<R, NT_, 0, stream>>>(y, (const W*)w, y2, (const W*)w2, eps, x, (T*)h, next_w, next_eps, \
+                                                          next_vec, D)
+  const bool next_vec = rms_row_vec(x, h, D);
   if (D < 2048) NA(256, 8);
   else if (D <= 8192) NA(1024, 8);
   else NA(1024, 0);
@@ -349,6 +361,10 @@ extern "C" int yalm_norm_add_pair(const float* y, const float* w, const float* y
   if (R <= 0) return YALM_OK;
   if (D <= 0) return YALM_ERR_ARG;
   if (h_out != nullptr && h_dtype != YALM_F32 && h_dtype != YALM_BF16) return YALM_ERR_DTYPE;
+  if (D > 8192 && h_out != nullptr && next_w != nullptr) {      // a row that no workgroup keeps: the norm's own kernel behind
+    const int rc = norm_add_launch<float, float, true>(y, w, y2, w2, eps, x, nullptr, nullptr, 0.f, R, D, stream);
+    return rc != YALM_OK ? rc : yalm_rmsnorm(x, next_w, YALM_F32, h_out, h_dtype, nullptr, R, D, next_eps, stream);
+  }
   return h_out != nullptr && h_dtype == YALM_BF16
              ? norm_add_launch<float, bf16, true>(y, w, y2, w2, eps, x, h_out, next_w, next_eps, R, D, stream)
              : norm_add_launch<float, float, true>(y, w, y2, w2, eps, x, h_out, next_w, next_eps, R, D, stream);

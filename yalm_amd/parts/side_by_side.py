@@ -112,8 +112,7 @@ class SideBySide(Part):
         y, y2 = (ctx.ws.get(name, (T, self.dim), torch.float32) for name in ("side.y", "side.y2"))
         self.left.forward_to(h, y, ctx, (line, "left"), writes_cache)
         self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache)
-        if emit_for is None or not hasattr(emit_for, "fused") or ctx.act_dtype == torch.float32:   # its sums run in another order:
-            # in float32 the norm's own kernel keeps its bits, which a faint read-out behind it magnifies a thousandfold
+        if emit_for is None or not hasattr(emit_for, "fused"):
             kernels.norm_add_pair(y, self.w_left, y2, self.w_right, self.eps, x)
             return
         ahead = ctx.ws.get("block.h", (T, self.dim), ctx.act_dtype)           # both members have read what lay there
