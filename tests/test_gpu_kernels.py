@@ -317,6 +317,25 @@ def test_gemm_gated(M, H, D, dtype, simple, act):
         k.FORCE_SIMPLE = False
 
 
+# float32: a row's results have the same bits whatever the rows beside it, up to 64 of them (narrow and wide products, short and
+# long sums, sums of no whole k tiles)
+@pytest.mark.parametrize("epi", ["store", "add", "gated"])
+@pytest.mark.parametrize("N,Kd", [(64, 32), (96, 36), (96, 544), (4096, 288), (4128, 96), (8192, 2048), (8192, 2080), (16416, 4128)])
+def test_gemm_float32_rows_do_not_depend_on_their_number(N, Kd, epi):
+    k = K()
+    a, w, x = rnd((64, Kd), 95).to(DEV), rnd((N, Kd), 96).to(DEV), rnd((64, N), 97).to(DEV)
+    H = N // 2 - 3 if N > 64 else N // 2
+
+    def product(lo, hi):
+        if epi == "gated":
+            return k.gemm(a[lo:hi], w, torch.empty((hi - lo, H), device=DEV), k.EPI_GATED, hidden=H)
+        return k.gemm(a[lo:hi], w, x[lo:hi].clone(), k.EPI_ADD_F32 if epi == "add" else k.EPI_STORE_F32)
+
+    whole = product(0, 64)
+    for lo, hi in [(0, n) for n in (1, 2, 4, 5, 7, 8, 15, 16, 17, 31, 32, 33, 48, 63)] + [(20, 21), (50, 64)]:
+        assert torch.equal(product(lo, hi), whole[lo:hi]), (lo, hi)
+
+
 # float32 on the matrix cores: the edges of its tiles (16 and 32 rows, 32 to 128 columns), of its rules (16 | 17 and 32 | 33
 # rows, 4,096 and 8,192 columns) and of its k tiles, K short of one round of the waves, operands 4 bytes off
 @pytest.mark.parametrize("M,N,Kd,off", [

@@ -10,12 +10,12 @@
 // 2,250 -> 552 us, 128,256 x 3,072 16.3 -> 4.0 ms, 3,072 x 8,192 1,740 -> 290 us.
 //
 // gemm_few_f32_kernel and small tiles take a decode step's rows, which the vector units' kernel (gemm_rows_f32_kernel) had
-// multiplied at a fraction of memory's rate: 16 rows, 4,096 x 4,096 55 -> 20 us, 128,256 x 3,072 729 -> 278 us; one row,
-// 4,096 x 4,096 24 -> 16 us.
+// multiplied at a fraction of memory's rate: 16 rows, 4,096 x 4,096 54 -> 19 us, 128,256 x 3,072 725 -> 276 us; one row,
+// 4,096 x 4,096 23 -> 16 us, 128,256 x 3,072 263 -> 257 us.
 //
-// Sums over short runs of k join a total of their own: two short chains of additions lie closer to 64 bits than one over K
-// (a relative error of 3.0e-7 at 701 rows and K 8,192, where gemm_simple_kernel's was 1.6e-6; at most 64 rows 0.8 to 1.4e-7,
-// gemm_rows_f32_kernel's 0.8 to 2.2e-7).
+// Sums over short runs of k join a total of their own: short chains of additions lie closer to 64 bits than one over K (a relative
+// error of 3.0e-7 at 701 rows and K 8,192, where gemm_simple_kernel's was 1.6e-6; at most 64 rows 0.6e-7 at K 32 to 1.3e-7 at K
+// 3,072 and 1.6e-7 at K 14,336, gemm_rows_f32_kernel's 0.6e-7, 1.4e-7 and 2.8e-7).
 #include "common.h"
 #include "yalm_hip.h"
 
@@ -31,6 +31,16 @@ constexpr int NW = 4;
 
 __device__ __forceinline__ int swizzle_of(int row) { return (row >> 1) & (CPR - 1); }
 
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// The products of the 16 k that a wave's lanes hold, four by four, joined in a tree
+__device__ __forceinline__ f32x4 sum_of_products(f32x4 a, f32x4 b) {
+  f32x4 p[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = mfma4(a[e], b[e], (f32x4){0.f, 0.f, 0.f, 0.f});
+  return (p[0] + p[1]) + (p[2] + p[3]);
+}
+
 // at most N_ of this wave's loads in flight, and none of its LDS reads
 template <int N_>
 __device__ __forceinline__ void wait_loads() {
@@ -41,8 +51,8 @@ __device__ __forceinline__ void wait_loads() {
 constexpr int stages_of(int FA, int FB) { return 640 / (32 * (FA + FB)) < 4 ? 640 / (32 * (FA + FB)) : 4; }
 constexpr int GROUP = 4;                         // tile columns that an XCD walks together
 
-// FINE: four chains of sums, one for each of the k that a lane holds side by side, joined and added to the total every four k
-// tiles: chains of 32 and of K / 128 additions.  Else one chain, added to the total every eight k tiles.
+// FINE: four chains of sums, one for each of the k that a lane holds side by side, joined every four k tiles and added to a sum
+// that joins the total every sixteen: chains of 32, 4 and K / 512 additions.  Else one chain, added to the total every eight k tiles.
 template <int EPI, int FA, int FB, bool FINE>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                           float* __restrict__ C, int M, int N, int K, GateOut H) {
@@ -74,7 +84,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
   }
   auto issue = [&](int kt, int stage, int i) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops a template that names this builtin, and its launch stub with it
-    __builtin_amdgcn_global_load_lds(gp[i] + (size_t)kt * TK, stages + stage * STAGE_B + (i * NW + wave) * 1024, 16, 0, 0);
+    const float* from = gp[i] + (size_t)kt * TK;
+    unsigned char* to = stages + stage * STAGE_B + (i * NW + wave) * 1024;
+    // weights that at most 64 rows need are not kept in the caches (2: non-temporal): 4 rows, 128,256 x 3,072 273 -> 254 us
+    if (FINE && i >= TM / (RPI * NW)) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);
+    else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
 #endif
   };
   auto issue_all = [&](int kt, int stage) {
@@ -82,12 +96,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
     for (int i = 0; i < L; ++i) issue(kt, stage, i);
   };
 
-  f32x4 acc[CH][FA][FB], total[FA][FB];
+  f32x4 acc[CH][FA][FB], some[FINE ? FA : 1][FINE ? FB : 1], total[FA][FB];
 #pragma unroll
   for (int a = 0; a < FA; ++a)
 #pragma unroll
     for (int b = 0; b < FB; ++b) {
       total[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      if constexpr (FINE) some[a][b] = total[a][b];
 #pragma unroll
       for (int c = 0; c < CH; ++c) acc[c][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
@@ -132,7 +147,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
       for (int a = 0; a < FA; ++a)
 #pragma unroll
         for (int b = 0; b < FB; ++b)
-          acc[e % CH][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[0][a][e], fw[0][b][e], acc[e % CH][a][b], 0, 0, 0);
+          acc[e % CH][a][b] = mfma4(fa[0][a][e], fw[0][b][e], acc[e % CH][a][b]);
     __builtin_amdgcn_sched_barrier(0);
     // tile kt + 1 has landed when at most the loads of the S - 2 tiles behind it are in flight
     if (kt + S - 1 < nk) wait_loads<(S - 2) * L>(); else wait_loads<0>();
@@ -147,7 +162,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
       for (int a = 0; a < FA; ++a)
 #pragma unroll
         for (int b = 0; b < FB; ++b) {
-          acc[e % CH][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[1][a][e], fw[1][b][e], acc[e % CH][a][b], 0, 0, 0);
+          acc[e % CH][a][b] = mfma4(fa[1][a][e], fw[1][b][e], acc[e % CH][a][b]);
           const int j = (e * FA + a) * FB + b;
 #pragma unroll
           for (int i = 0; i < L; ++i)
@@ -162,8 +177,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
       for (int a = 0; a < FA; ++a)
 #pragma unroll
         for (int b = 0; b < FB; ++b) {
-          if constexpr (FINE) total[a][b] += (acc[0][a][b] + acc[1][a][b]) + (acc[2][a][b] + acc[3][a][b]);
-          else total[a][b] += acc[0][a][b];
+          if constexpr (FINE) {
+            some[a][b] += (acc[0][a][b] + acc[1][a][b]) + (acc[2][a][b] + acc[3][a][b]);
+            if ((kt + 1) % (4 * FOLD) == 0 || kt + 1 == nk) {
+              total[a][b] += some[a][b];
+              some[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+          } else {
+            total[a][b] += acc[0][a][b];
+          }
 #pragma unroll
           for (int c = 0; c < CH; ++c) acc[c][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
         }
@@ -198,9 +220,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
 
 // ---------------------------------------------------------------------------
 // At most 64 rows (a decode step of the 32-bit path): bound by the weights' one trip from memory.  A workgroup owns
-// 16 NB weight rows and all (16 MB) rows of A; its waves take every NWV-th block of 32 k (128 bytes of each row, whole
-// lines) and their sums are added in LDS in the waves' order.  Weights and A go from memory straight into registers, the
-// next block's while one is multiplied (two blocks ahead measured the same).
+// 16 NB weight rows and 16 MB rows of A; its waves take every NWV-th block of 32 k (128 bytes of each row, whole
+// lines), a block's eight products are joined in a tree, and the waves' sums in a tree in LDS: at K 32 NWV, chains of 4 + 3 + 3
+// additions.  Weights and A go from memory straight into registers, the next block's while one is multiplied (two blocks ahead
+// measured the same).
 // ---------------------------------------------------------------------------
 constexpr int NWV = 8;
 
@@ -212,7 +235,10 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int l16 = lane % 16, lq = lane / 16;
-  const int n0 = blockIdx.x * 16 * NB;
+  const int n0 = blockIdx.x * 16 * NB, m0 = blockIdx.y * 16 * MB;
+  A += (size_t)m0 * K;
+  C += (size_t)m0 * (gated(EPI) ? (int)H : N);
+  M -= m0;
   const float* wp[NB];
   const float* ap[MB];
 #pragma unroll
@@ -237,27 +263,12 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
       for (int a = 0; a < MB; ++a) x[buf][a][h] = *(const f32x4*)(ap[a] + k + h * 16);
     }
   };
-  auto multiply = [&](int buf) {                   // a sum of its own for each of the four k that a lane holds side by side
-    f32x4 part[4][MB][NB];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int a = 0; a < MB; ++a)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) part[e][a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int a = 0; a < MB; ++a)
-#pragma unroll
-          for (int b = 0; b < NB; ++b)
-            part[e][a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[buf][a][h][e], w[buf][b][h][e], part[e][a][b], 0, 0, 0);
+  auto multiply = [&](int buf) {
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc[a][b] += (part[0][a][b] + part[1][a][b]) + (part[2][a][b] + part[3][a][b]);
+      for (int b = 0; b < NB; ++b)
+        acc[a][b] += sum_of_products(x[buf][a][0], w[buf][b][0]) + sum_of_products(x[buf][a][1], w[buf][b][1]);
   };
   if (mine > 0) {
     load(0, 0);
@@ -283,10 +294,8 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
   for (int e = tid; e < UNITS * WAVE; e += NWV * WAVE) {
     const int at = e % WAVE, unit = e / WAVE, col = at % 16, row = 4 * (at / 16);
     auto total = [&](int t) {
-      f32x4 v = sums[0][t][at];
-#pragma unroll
-      for (int i = 1; i < NWV; ++i) v += sums[i][t][at];
-      return v;
+      return ((sums[0][t][at] + sums[1][t][at]) + (sums[2][t][at] + sums[3][t][at])) +
+             ((sums[4][t][at] + sums[5][t][at]) + (sums[6][t][at] + sums[7][t][at]));
     };
     if constexpr (gated(EPI)) {
       const f32x4 gt = total(unit * 2), up = total(unit * 2 + 1);
@@ -313,7 +322,7 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
 
 template <int EPI, int MB, int NB>
 int launch_few(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  gemm_few_f32_kernel<EPI, MB, NB><<<ceil_div(N, 16 * NB), NWV * WAVE, 0, stream>>>(A, W, C, M, N, K, H);
+  gemm_few_f32_kernel<EPI, MB, NB><<<dim3(ceil_div(N, 16 * NB), ceil_div(M, 16 * MB)), NWV * WAVE, 0, stream>>>(A, W, C, M, N, K, H);
   return launch_status();
 }
 
@@ -347,14 +356,14 @@ double tile_time(int M, int N, int K, int fa, int fb) {
 
 // The tile for a shape: the fastest by that estimate (701 rows, N x K: 16,384 x 3,072 takes 2x4 555 us, 128,256 x 3,072 2x4
 // 4.0 ms, 3,072 x 8,192 3x3 288 us on exactly 256 tiles, 2x4 would be 24 % slower).  Up to 64 rows the small tiles' FINE
-// form: there the products were summed more finely before (gemm_rows_f32_kernel), and memory is what bounds them.
+// form (2x4 would spill registers: 128,256 x 3,072 at 64 rows 446 against 459 us with 2x2, 16,384 x 3,072 114 against 66).
 template <int EPI>
 int launch_tiles(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
   static constexpr int shapes[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 3}, {3, 4}, {4, 4}};
   const bool fine = M <= 64;
   int best = -1;
   double best_t = 0.0;
-  for (int i = 0; i < (fine ? 5 : 8); ++i) {
+  for (int i = 0; i < (fine ? 4 : 8); ++i) {
     if (gated(EPI) && shapes[i][1] % 2) continue;
     const double t = tile_time(M, N, K, shapes[i][0], shapes[i][1]);
     if (best < 0 || t < best_t) { best = i; best_t = t; }
@@ -366,7 +375,7 @@ int launch_tiles(const float* A, const float* W, float* C, int M, int N, int K, 
     case 1: YALM_F32_TILE(1, 2);
     case 2: YALM_F32_TILE(2, 1);
     case 3: YALM_F32_TILE(2, 2);
-    case 4: YALM_F32_TILE(2, 4);
+    case 4: return launch_f32<EPI, 2, 4, false>(A, W, C, M, N, K, H, stream);
     case 5: return launch_f32<EPI, 3, 3, false>(A, W, C, M, N, K, H, stream);
     case 6: return launch_f32<EPI, 3, 4, false>(A, W, C, M, N, K, H, stream);
     default: return launch_f32<EPI, 4, 4, false>(A, W, C, M, N, K, H, stream);
@@ -374,31 +383,43 @@ int launch_tiles(const float* A, const float* W, float* C, int M, int N, int K, 
 #undef YALM_F32_TILE
 }
 
-// Up to 64 rows of up to 4,096 columns (16 rows: 8,191) go to gemm_few_f32_kernel: the tiles' kernel would leave CUs without
-// work, and walks K alone where eight waves share it (16 rows, 4,096 x 4,096 20 against 32 us, 3,072 x 8,192 36 against 60,
-// 512 x 256 3.5 against 4.4; at 64 rows 43, 81 and 5.2 against 33, 61 and 4.4, but summed more finely, as before).  Wider
-// products go to the tiles, which read A once for 32 weight rows and more (16 rows, 16,384 x 3,072: 44 against 54 us,
-// 128,256 x 3,072: 278 against 392).
+// How many of the rows and weight rows a workgroup of gemm_few_f32_kernel takes (no sum depends on it).  Every 16 rows by
+// themselves where that leaves no CU two workgroups (64 rows, 1,024 x 1,024 6.8 us; 2 and 4 times 16 8.9 and 13.1), else 32, and
+// 64 of up to 4,096 columns (64 rows, 4,096 x 4,096 42 against 51 us with 32).  Two blocks of weight rows save reading A, which
+// pays from 8 rows of many columns on (5,120 x 3,072: 4 rows 22.1 us with one, 22.8 with two, 16 rows 28.1 and 25.7).
+template <int EPI>
+int launch_few_rows(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
+  constexpr bool G = gated(EPI);
+  const bool alone = M <= 16 || (long)ceil_div(N, G ? 32 : 16) * ceil_div(M, 16) <= 256;
+  if constexpr (G) {
+    if (alone) return launch_few<EPI, 1, 2>(A, W, C, M, N, K, H, stream);
+    return launch_few<EPI, 2, 2>(A, W, C, M, N, K, H, stream);
+  } else {
+    if (alone && M > 7 && N > 4096) return launch_few<EPI, 1, 2>(A, W, C, M, N, K, H, stream);
+    if (alone) return launch_few<EPI, 1, 1>(A, W, C, M, N, K, H, stream);
+    if (N > 4096) return launch_few<EPI, 2, 2>(A, W, C, M, N, K, H, stream);
+    if (M <= 32) return launch_few<EPI, 2, 1>(A, W, C, M, N, K, H, stream);
+    return launch_few<EPI, 4, 1>(A, W, C, M, N, K, H, stream);
+  }
+}
+
+// Up to 64 rows the form of a sum follows from N and K alone, so that a row's results do not change with the number of rows
+// beside it.  gemm_few_f32_kernel takes what is narrow (the tiles' kernel would leave CUs without work, and walks K alone where
+// eight waves share it: 16 rows, 4,096 x 4,096 19 against 33 us, 3,072 x 8,192 34 against 60; 64 rows 42 and 81 against 33 and 61)
+// and short sums, where the FINE chains would lie further from 64 bits than gemm_rows_f32_kernel's (a relative error at K 1,024 of
+// 1.2e-7 against 1.0e-7, its own 0.9e-7; at K 2,560 1.26e-7 against 1.33e-7).  The rest goes to the tiles, which read A once for 32
+// weight rows and more (16,384 x 3,072: one row 43 us, 16 rows 42, 64 rows 66; gemm_few_f32_kernel 45, 51 and 127).
 template <int EPI>
 int launch(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  constexpr int NB = gated(EPI) ? 2 : 1;
-  if (M <= 64 && N <= 4096) {
-    if (M <= 16) return launch_few<EPI, 1, NB>(A, W, C, M, N, K, H, stream);
-    if (M <= 32) return launch_few<EPI, 2, NB>(A, W, C, M, N, K, H, stream);
-    return launch_few<EPI, 4, NB>(A, W, C, M, N, K, H, stream);
-  }
-  if (M <= 16 && N < 8192) return launch_few<EPI, 1, 2>(A, W, C, M, N, K, H, stream);
+  if (M <= 64 && (N < 8192 || K <= 2048)) return launch_few_rows<EPI>(A, W, C, M, N, K, H, stream);
   return launch_tiles<EPI>(A, W, C, M, N, K, H, stream);
 }
 
 }  // namespace
 
-// K a multiple of 32 and 16-byte aligned operands; YALM_ERR_ARG: not taken.  Nor are up to four rows of a wide product: the
-// vector units' kernel keeps up with memory there (one row, 128,256 x 3,072 271 against 290 us, 16,384 x 3,072 44 against 47).
+// K a multiple of 32 and 16-byte aligned operands; YALM_ERR_ARG: not taken.
 int yalm_gemm_f32_mfma(const void* A, const void* W, void* C, int M, int N, int K, int epilogue, GateOut H, hipStream_t stream) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) ||
-      (M <= 4 && N >= 8192))
-    return YALM_ERR_ARG;
+  if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return YALM_ERR_ARG;
   const float *a = (const float*)A, *w = (const float*)W;
   float* c = (float*)C;
   switch (epilogue) {

@@ -2,8 +2,7 @@
 // true 32-bit path and the fallback of the bfloat16 path for shapes the MFMA kernels
 // refuse.  gemm_simple: 64x64 tile, 16-deep k steps through LDS, 256 threads with a 4x4
 // register tile each; any M, N, K.  gemm_rows_f32: at most 64 rows of float32, a pass over
-// the weights for every 16 of them (below).  Float32 with K a multiple of 32 goes to the matrix cores (gemm_f32.hip), but for
-// up to four rows of a wide product.
+// the weights for every 16 of them (below).  Float32 with K a multiple of 32 goes to the matrix cores (gemm_f32.hip).
 #include "common.h"
 #include "yalm_hip.h"
 
