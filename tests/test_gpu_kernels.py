@@ -763,6 +763,26 @@ def test_attn_decode_with_the_length_of_the_longest_sequence(n_heads, n_kv, hd, 
     _attn_decode_case(n_heads, n_kv, hd, window, lens, splits, torch.bfloat16, False, max(lens) if said == "longest" else said)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,window,lens,splits", [
+    (8, 2, 128, 0, [1000, 3, 517, 64, 65], 4), (4, 1, 64, 0, [40, 900], 7), (5, 5, 80, 150, [700, 64, 164], 3), (2, 1, 32, 0, [400, 9], 2)])
+def test_attn_decode_float32_of_a_row_does_not_depend_on_the_others(n_heads, n_kv, hd, window, lens, splits):
+    k = K()
+    B = len(lens)
+    kp, vp, bt, slots, ring, _, _ = paged_case(lens, n_kv, hd, window, torch.float32, 24)
+    kp, vp, bt, q = kp.to(DEV), vp.to(DEV), bt.to(DEV), rnd((B, n_heads * hd), 25).to(DEV)
+    partial = torch.empty(k.attn_decode_workspace_floats(B, n_heads, hd, splits), device=DEV)
+
+    def decode(rows, longest):
+        out = torch.full((len(rows), n_heads * hd), 7.0, device=DEV)
+        return k.attn_decode(q[rows], kp, vp, bt, ring, i32([slots[r] for r in rows]), i32([lens[r] for r in rows]), out, partial,
+                             n_heads, n_kv, hd, window, splits, step_max_len=None if longest is None else i32([longest]))
+
+    together = decode(list(range(B)), max(lens))
+    assert torch.equal(decode(list(range(B)), None), together) and torch.equal(decode(list(range(B)), 100000), together)
+    for r in range(B):
+        assert torch.equal(decode([r], lens[r])[0], together[r])
+
+
 # the splits merged by the last workgroup to arrive: against the kernel that merges them, launch after launch with the same
 # counters; splits that find nothing to do, a padding row, more splits than lanes, several groups of 16 heads, a sink logit
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -235,8 +235,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_stride, int ring_pages, const int* __restrict__ seq_slot,
     const int* __restrict__ seq_len, float* __restrict__ partial, float* __restrict__ out, float* __restrict__ lse,
-    int n_heads, int n_kv_heads, int window, int n_splits, int n_pages, const int* __restrict__ step_max_len,
-    const int* __restrict__ seq_order, ScoreShape sh, int* __restrict__ counters) {
+    int n_heads, int n_kv_heads, int window, int n_splits, int n_pages, const int* __restrict__ seq_order, ScoreShape sh, int* __restrict__ counters) {
   constexpr int DT = HD / 16, NW = 4, LAYOUT = BLOCKS ? YALM_PAGE_BLOCKS : YALM_PAGE_ROWS;
   __shared__ float sm_m[NW][16], sm_l[NW][16];
   __shared__ f32x4 sm_o[NW][DT][WAVE];
@@ -255,11 +254,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
 
   if (L > 0) {
     const int lo = first_visible(L - 1, window, sh.block), first_page = lo / PAGE, last_page = (L - 1) / PAGE;
-    int per = (last_page - first_page + n_splits) / n_splits;
-    if (step_max_len != nullptr) {                 // every split as many pages as the longest sequence's (attention_mfma_decode.hip)
-      const int Lm = max(step_max_len[0], 1);
-      per = max(per, ((Lm - 1) / PAGE - first_visible(Lm - 1, window, sh.block) / PAGE + n_splits) / n_splits);
-    }
+    // cut by the sequence's own length: in float32 its sums hang on no other sequence of the step
+    const int per = (last_page - first_page + n_splits) / n_splits;
     const int p_begin = first_page + split * per, p_end = min(last_page + 1, p_begin + per);
     const float inv = sqrtf((float)HD);
     const size_t page_elems = (size_t)n_kv_heads * PAGE * HD;
@@ -464,8 +460,8 @@ int yalm_attn_prefill_f32_mfma(const void* q, const void* k_stage, const void* v
 int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
                               int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out, float* lse,
                               float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window, int n_splits,
-                              int n_pages, int page_layout, const int* step_max_len, const int* seq_order,
-                              const ScoreShape& shape, int* counters, hipStream_t stream) {
+                              int n_pages, int page_layout, const int* seq_order, const ScoreShape& shape, int* counters,
+                              hipStream_t stream) {
   const int parts_g = (n_heads / n_kv_heads + 15) / 16;
   const bool blocks = page_layout == YALM_PAGE_BLOCKS;
   if (!takes(head_dim, q, k_pages, v_pages, nullptr) || (long)n_kv_heads * parts_g > 65535 || B > 65535 ||
@@ -475,7 +471,7 @@ int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_
 #define YALM_RUN(HD_, BLOCKS_, SHAPED_)                                                                                  \
   attn_decode_f32_kernel<HD_, BLOCKS_, SHAPED_><<<grid, 256, 0, stream>>>(                                               \
       (const float*)q, (const float*)k_pages, (const float*)v_pages, block_table, table_stride, ring_pages, seq_slot,    \
-      seq_len, partial, (float*)out, lse, n_heads, n_kv_heads, window, n_splits, n_pages, step_max_len, seq_order, shape, counters)
+      seq_len, partial, (float*)out, lse, n_heads, n_kv_heads, window, n_splits, n_pages, seq_order, shape, counters)
 #define YALM_HD16(HD_)                                                                                                   \
   case HD_:                                                                                                              \
     if (shape.any()) YALM_RUN(HD_, false, true);                                                                         \

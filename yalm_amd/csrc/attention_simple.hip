@@ -20,8 +20,8 @@ int yalm_attn_prefill_f32_mfma(const void* q, const void* k_stage, const void* v
 int yalm_attn_decode_f32_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
                               int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out, float* lse,
                               float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window, int n_splits,
-                              int n_pages, int page_layout, const int* step_max_len, const int* seq_order,
-                              const ScoreShape& shape, int* counters, hipStream_t stream);
+                              int n_pages, int page_layout, const int* seq_order, const ScoreShape& shape, int* counters,
+                              hipStream_t stream);
 int yalm_attn_decode_bf16_mfma(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
                                int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
                                float* lse, float* partial, int B, int n_heads, int n_kv_heads, int head_dim, int window,
@@ -443,8 +443,7 @@ int attn_decode_any(const void* q, const void* k_pages, const void* v_pages, con
                          ? counters : nullptr;
       int rc = yalm_attn_decode_f32_mfma(q, k_pages, v_pages, block_table, table_stride, ring_pages, seq_slot, seq_len,
                                          merge && arrived == nullptr ? nullptr : out, lse, partial, B, n_heads, n_kv_heads,
-                                         head_dim, window, n_splits, n_pages, page_layout, step_max_len, seq_order, shape,
-                                         arrived, stream);
+                                         head_dim, window, n_splits, n_pages, page_layout, seq_order, shape, arrived, stream);
       if (rc != YALM_ERR_ARG) {
         if (rc != YALM_OK || !merge || arrived != nullptr) return rc;
         attn_decode_combine_kernel<float><<<cgrid, COMBINE_THREADS, 0, stream>>>(partial, (float*)out, lse, n_heads,

@@ -77,8 +77,9 @@ def generate(engine, prompts, max_new_tokens=256, temperature=0.0, seed=0, stop_
     ahead: queue each step before the host has read the tokens of the step before
     (default: if the engine has step_from and the sampler has draw).  A request that has ended
     leaves the batch a step later then, so a step may run with another number of rows and take other
-    kernels: the tokens are the same either way up to choices between logits that lie within rounding of
-    each other (in float32 the last bits of a sum, in bfloat16 more)."""
+    kernels: in float32 the tokens are the same either way (a row's sums do not depend on the rows beside it, up to 64 of
+    them; but the attention of contexts beyond 256 tokens is cut by their number, which moves its last bits), in bfloat16
+    up to choices between logits that lie within rounding of each other."""
     from .sampling import Sampler
     sampler = sampler or Sampler(seed)
     stats = stats if stats is not None else GenerationStats()

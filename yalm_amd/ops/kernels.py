@@ -672,7 +672,8 @@ def attn_decode(q, k_pages, v_pages, block_table, ring_pages, seq_slot, seq_len,
     seq_len counts the new key.  lse as in attn_prefill.  step_max_len (int32 [1] on the device, optional): the
     length of the step's longest sequence, with which sequences of unequal lengths are cut into splits of equal
     size; seq_order (int32 [B] on the device, a permutation of the rows, optional): the order in which the
-    workgroups take the rows (both change the division of the work and no result).  score_bias: see _bias; softcap,
+    workgroups take the rows (both change the division of the work and no result but by the order of its sums; in float32 a
+    sequence is cut by its own length, and not a bit depends on the others).  score_bias: see _bias; softcap,
     sink_logit: see _shape; block: see attn_prefill (none of these with sinks).  counters (optional; int32, at least
     attn_decode_counters elements, zero and left so): the attention kernel's last workgroup of a row may merge the splits,
     instead of a kernel behind it (it does where that is sooner; the results are the same, to the bit); not shared with a call that may run at the same time.
