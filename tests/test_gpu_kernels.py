@@ -783,6 +783,30 @@ def test_attn_decode_float32_of_a_row_does_not_depend_on_the_others(n_heads, n_k
         assert torch.equal(decode([r], lens[r])[0], together[r])
 
 
+@pytest.mark.parametrize("missing", [-1, -7, 1 << 20])
+@pytest.mark.parametrize("hd", [32, 64, 112, 128])
+def test_attn_decode_float32_passes_over_a_page_that_does_not_exist(hd, missing):
+    """As the general kernel does: the page's keys are not among those that a query sees."""
+    k = K()
+    lens, n_heads, n_kv, splits = [300, 64, 130], 4, 2, 2
+    kp, vp, bt, slots, ring, _, _ = paged_case(lens, n_kv, hd, 0, torch.float32, 26)
+    bt[slots[0], 1] = missing
+    bt[slots[2], 0] = missing
+    q = rnd((3, n_heads * hd), 27).to(DEV)
+    partial = torch.empty(k.attn_decode_workspace_floats(3, n_heads, hd, splits), device=DEV)
+    got = []
+    for simple in (False, True):
+        k.FORCE_SIMPLE = simple
+        try:
+            out = torch.full((3, n_heads * hd), 7.0, device=DEV)
+            k.attn_decode(q, kp.to(DEV), vp.to(DEV), bt.to(DEV), ring, i32(slots), i32(lens), out, partial, n_heads, n_kv, hd, 0, splits)
+        finally:
+            k.FORCE_SIMPLE = False
+        got.append(out)
+    # sums of at most 300 terms, weights that sum to one, in two orders
+    assert torch.isfinite(got[1]).all() and bool(((got[0] - got[1]).abs() <= 2 * 300 * 2.0 ** -24 * 5.0).all())
+
+
 # the splits merged by the last workgroup to arrive: against the kernel that merges them, launch after launch with the same
 # counters; splits that find nothing to do, a padding row, more splits than lanes, several groups of 16 heads, a sink logit
 @pytest.mark.parametrize("dtype", DTYPES)

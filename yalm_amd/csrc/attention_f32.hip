@@ -266,18 +266,19 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
     f32x4 qv[DT], kf[DT], vf[DT];
 #pragma unroll
     for (int s = 0; s < DT; ++s) qv[s] = ld4(q + ((size_t)b * n_heads + h) * HD + s * 16 + lq * 4);
-    auto page_at = [&](int ap) {
-      return (size_t)min(max(table[ap % ring_pages], 0), n_pages - 1) * page_elems + (size_t)g * PAGE * HD;
-    };
+    // a page that does not exist (never the case for a live sequence) is seen by nobody; some other is read in its place
+    auto page_at = [&](int phys) { return (size_t)min(max(phys, 0), n_pages - 1) * page_elems + (size_t)g * PAGE * HD; };
     auto load_keys = [&](size_t at) {
 #pragma unroll
       for (int s = 0; s < DT; ++s) kf[s] = ld4(k_pages + at + page_k_offset(LAYOUT, k_row, s * 16 + lq * 4, HD));
     };
-    size_t at = 0;                                 // the page's place
+    int phys = 0;                                  // the page
     // one page; has_next is a compile-time tag (std::true_type: the next page's keys are asked for)
     auto one_page = [&](int ap, auto has_next) {
       constexpr bool NEXT = decltype(has_next)::value;
-      const size_t at_next = NEXT ? page_at(ap + 1) : 0, at_v = at;
+      const int phys_next = NEXT ? table[(ap + 1) % ring_pages] : 0;
+      const size_t at_v = page_at(phys);
+      const bool there = phys >= 0 && phys < n_pages;
 #pragma unroll
       for (int d = 0; d < DT; ++d) vf[d] = ld4(v_pages + at_v + page_v_offset(LAYOUT, v_row, d * 16 + l16, HD));
       __builtin_amdgcn_sched_barrier(0);           // the values are asked for before the keys are waited for
@@ -291,15 +292,15 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
         }
       f32x4 sc = even + uneven;
       if constexpr (NEXT) {
-        load_keys(at_next);                        // in flight while this page is mixed
-        at = at_next;
+        load_keys(page_at(phys_next));             // in flight while this page is mixed
+        phys = phys_next;
         __builtin_amdgcn_sched_barrier(0);
       }
       const int pos0 = ap * PAGE + v_row;          // lane (lq, l16) holds the keys pos0 + r of head l16
       float mx = -FLT_MAX;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const bool seen = pos0 + r >= lo && pos0 + r < L;
+        const bool seen = there && pos0 + r >= lo && pos0 + r < L;
         float s = sc[r] / inv;
         if constexpr (SHAPED) s = shaped(sh, s, h, L - 1 - pos0 - r);
         sc[r] = seen ? s : -INFINITY;
@@ -351,8 +352,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
         for (int r = 0; r < 4; ++r) o[d][r] = fmaf(o[d][r], corr, part[d][r]);
     };
     if (p_begin < p_end) {
-      at = page_at(p_begin);
-      load_keys(at);
+      phys = table[p_begin % ring_pages];
+      load_keys(page_at(phys));
       int ap = p_begin;
       for (; ap + 1 < p_end; ++ap) one_page(ap, std::true_type{});
       one_page(ap, std::false_type{});
