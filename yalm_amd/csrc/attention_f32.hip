@@ -333,18 +333,18 @@ __global__ __launch_bounds__(256, 2) void attn_decode_f32_kernel(
       if (__any(z != 0.f)) {                       // key by key, probabilities of zero left out
 #pragma unroll
         for (int d = 0; d < DT; ++d) part[d] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < 4; ++k)
+#pragma unroll 1
+        for (int key = 0; key < 16; ++key) {       // key 4 k + r in lane (k, l16), place r
+          const int r = key & 3;
+          const float p = __shfl(r < 2 ? (r == 0 ? sc[0] : sc[1]) : (r == 2 ? sc[2] : sc[3]), key / 4 * 16 + l16, WAVE);
+          if (p != 0.f) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float p = __shfl(sc[r], k * 16 + l16, WAVE);
-            if (p != 0.f) {
+            for (int d = 0; d < DT; ++d)
 #pragma unroll
-              for (int d = 0; d < DT; ++d)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  part[d][e] = fmaf(p, v_pages[at_v + page_v_offset(LAYOUT, row0 + 8 * k + r, d * 16 + lq * 4 + e, HD)], part[d][e]);
-            }
+              for (int e = 0; e < 4; ++e)
+                part[d][e] = fmaf(p, v_pages[at_v + page_v_offset(LAYOUT, row0 + 8 * (key / 4) + r, d * 16 + lq * 4 + e, HD)], part[d][e]);
           }
+        }
       }
 #pragma unroll
       for (int d = 0; d < DT; ++d)

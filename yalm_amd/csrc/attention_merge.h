@@ -19,7 +19,7 @@ typedef unsigned long long pair_bits;            // two floats
 // Whether the last workgroup to arrive should merge the splits of its heads (of `heads` of a KV head, at most 16): a wave takes
 // a head, so where there is one for each the merge costs the last workgroup less than a launch behind it, and where the waves
 // take several in turn more.  Merged inside against by the kernel behind, us, at 4 / 16 / 64 splits of 256 keys and one sequence:
-// four waves and 4 heads of 128 7.5 / 8.0 / 11.8 against 8.1 / 8.5 / 18.4; 8 heads 8.6 / 9.5 / 15.6 against 8.0 / 8.4 / 17.9;
+// four waves and 4 heads of 128 7.1 / 7.6 / 11.3 against 8.0 / 8.4 / 18.6; 8 heads 8.6 / 9.5 / 15.6 against 8.0 / 8.4 / 17.9;
 // 16 heads 11.1 / 12.8 / 24.3 against 8.1 / 8.6 / 18.1; two waves and 4 heads of 256 11.5 / 12.8 / 21.4 against 10.9 / 11.4 / 27.0.
 inline bool merges_inside(int heads, int waves) { return heads <= waves; }
 
@@ -60,12 +60,14 @@ __device__ __forceinline__ void merge_splits(const float* partial, T* __restrict
     const float* part = partial + ((size_t)b * n_heads + h) * n_splits * (HD + 2);
     auto maximum_of = [&](int s) { return s < n_splits ? load_pair(part + (size_t)s * (HD + 2) + HD) : make_float2(-FLT_MAX, 0.f); };
     float2 v[2][PRE][EL];
+    int none = 0;                                  // zero in a vector register: the splits' places are worked out a lane, from one
+    asm("" : "+v"(none));                          // base, and take no scalar registers from the attention's loops
     auto ask = [&](int buf, int s0) {
 #pragma unroll
       for (int u = 0; u < PRE; ++u) {
-        const float* ps = part + (size_t)min(s0 + u, n_splits - 1) * (HD + 2);
+        const int ps = min(s0 + u + none, n_splits - 1) * (HD + 2);
 #pragma unroll
-        for (int e = 0; e < EL; ++e) v[buf][u][e] = load_pair(ps + 2 * min(lane + e * WAVE, HD / 2 - 1));
+        for (int e = 0; e < EL; ++e) v[buf][u][e] = load_pair(part + (unsigned)(ps + 2 * min(lane + e * WAVE, HD / 2 - 1)));
       }
     };
     float2 ml = maximum_of(lane);                  // of split lane
