@@ -162,8 +162,8 @@ long yalm_attn_decode_workspace(int B, int n_heads, int head_dim, int n_splits);
 // sum of exp(score) over the keys the query saw (-FLT_MAX for a padding row), so that further keys can be
 // mixed in afterwards (yalm_attn_sink_mix).  out_f32 (prefill only; float32 [T, n_heads, hd], may be null) receives
 // the result before its rounding to `dtype`, for the same purpose.  step_max_len (device, one int, may be null): the length of the step's
-// longest sequence; the matrix-core decode kernel then cuts every sequence into splits of that sequence's split size,
-// so that sequences of unequal lengths give workgroups of equal work (no result depends on it).  seq_order (device,
+// longest sequence; the bfloat16 matrix-core decode kernel then cuts every sequence into splits of that sequence's split size,
+// so that sequences of unequal lengths give workgroups of equal work (no result depends on it but by the order of its sums).  seq_order (device,
 // B ints, a permutation of the rows; may be null): the order in which that kernel's workgroups take the rows.
 // score_bias (device, float32 [n_heads, n_bias]; may be null): a term added to every score (after the 1/sqrt(head_dim)
 // scaling) by the distance between query and key, score_bias[head, min(distance, n_bias - 1)]: what a position
@@ -189,6 +189,19 @@ int yalm_attn_decode_lse(const void* q, const void* k_pages, const void* v_pages
                          float softcap, const float* sink_logit, const float* slopes, int block, const float* log_a,
                           const float* log_b, hipStream_t stream);
 
+// yalm_attn_decode_lse with 32 int32 for each (sequence, KV head and up to 16 of its query heads), zero before the first call
+// and left so: where a matrix-core kernel takes the call, its last workgroup of a row merges the splits, and no kernel of
+// its own does (null: as yalm_attn_decode_lse).  Calls that may run at the same time need counters of their own, as they
+// need a `partial` of their own.  `partial` lies on 8 bytes then, or the counters are left alone and the kernel behind merges; so
+// they are with more heads a KV head than a workgroup has waves, where that is sooner.  The results are the same, to the bit.
+int yalm_attn_decode_merged(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
+                            int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
+                            float* lse, float* partial, int* counters, int B, int n_heads, int n_kv_heads, int head_dim,
+                            int window, int n_splits, int n_pages, int page_layout, int dtype, int force_simple,
+                            const int* step_max_len, const int* seq_order, const float* score_bias, int n_bias,
+                            float softcap, const float* sink_logit, const float* slopes, int block, const float* log_a,
+                            const float* log_b, hipStream_t stream);
+
 // Attention sinks beside a window (src/infer.cpp:305-319, 486-488): the first n_sinks positions of a
 // sequence stay visible when the window has moved past them, and each then counts as lying
 // window + n_sinks - 1 - j positions behind the query, however long the sequence is.  The reference
@@ -205,17 +218,6 @@ int yalm_attn_decode_lse(const void* q, const void* k_pages, const void* v_pages
 //   out[t, h] = (e^lse out + sum_j e^s_j v_j) / (e^lse + sum_j e^s_j), s_j = q . k_j / sqrt(hd); with src_f32 (the
 //   out_f32 of yalm_attn_prefill_lse; may be null) the unrounded result is read from there, so that the mixed row
 //   is rounded once.
-// yalm_attn_decode_lse with 32 int32 for each (sequence, KV head and up to 16 of its query heads), zero before the first call
-//   and left so: where a matrix-core kernel takes the call, its last workgroup of a row merges the splits, and no kernel of
-//   its own does (null: as yalm_attn_decode_lse).  Calls that may run at the same time need counters of their own, as they
-//   need a `partial` of their own.
-int yalm_attn_decode_merged(const void* q, const void* k_pages, const void* v_pages, const int* block_table,
-                            int table_stride, int ring_pages, const int* seq_slot, const int* seq_len, void* out,
-                            float* lse, float* partial, int* counters, int B, int n_heads, int n_kv_heads, int head_dim,
-                            int window, int n_splits, int n_pages, int page_layout, int dtype, int force_simple,
-                            const int* step_max_len, const int* seq_order, const float* score_bias, int n_bias,
-                            float softcap, const float* sink_logit, const float* slopes, int block, const float* log_a,
-                            const float* log_b, hipStream_t stream);
 // A decode step: yalm_attn_decode_sinks is yalm_attn_decode whose merge of the splits takes those sinks in
 //   as further splits of one key each (no rounding in between, no launch more; the merge runs with one
 //   split too); with store != 0 a token at a position < n_sinks first stores its own key and value from its
