@@ -13,6 +13,10 @@
 #include <float.h>
 #include "common.h"
 
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "this exchange rests on how gfx950 carries out accesses of agent scope, not on the order of the language"
+#endif
+
 constexpr int COUNTER_STRIDE = 32;               // ints
 typedef unsigned long long pair_bits;            // two floats
 
