@@ -336,8 +336,50 @@ def test_gemm_float32_rows_do_not_depend_on_their_number(N, Kd, epi):
         assert torch.equal(product(lo, hi), whole[lo:hi]), (lo, hi)
 
 
-# float32 on the matrix cores: the edges of its tiles (16 and 32 rows, 32 to 128 columns), of its rules (16 | 17 and 32 | 33
-# rows, 4,096 and 8,192 columns) and of its k tiles, K short of one round of the waves, operands 4 bytes off
+# Every kernel and tile of the float32 products on the matrix cores (yalm_gemm_f32_choice), with edges of 1 to 31 rows and columns
+# and K of 37 or 69 k tiles: each ring of two to four stages turns many times, and sums are folded in whole and broken runs
+@pytest.mark.parametrize("M,N,Kd,choice", [
+    (1, 40, 1184, 11), (9, 4100, 1184, 12), (17, 3000, 1184, 21), (33, 4100, 1184, 22), (47, 2001, 1184, 41),
+    (3, 8200, 2208, 111), (1, 20001, 2208, 112), (33, 11999, 2208, 121), (47, 40001, 2208, 122),
+    (70, 41, 1184, 211), (129, 4001, 1184, 212), (97, 5130, 1184, 221), (161, 8201, 1184, 222), (161, 16401, 1184, 224),
+    (161, 12001, 1184, 233), (513, 5131, 1184, 234), (321, 20001, 1184, 244)])
+def test_gemm_float32_every_tile(M, N, Kd, choice):
+    from yalm_amd.ops import library
+    k = K()
+    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 0) == choice
+    a, w, x = rnd((M, Kd), 101).to(DEV), rnd((N, Kd), 102).to(DEV), rnd((M, N), 103).to(DEV)
+    want = a.double() @ w.double().t()
+    # K products and K additions in any order, the residual's addition once more (as below)
+    bound = (2.0 * Kd + 2.0) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t() + x.double().abs())
+    out = k.gemm(a, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32)
+    assert bool(((out.double() - want).abs() <= bound).all())
+    # those bounds are of the worst case: the sums' own errors are chance's, some of a rounding's size, and a k tile left out or
+    # taken twice (a thirty-seventh of the products) is a thousand times that
+    assert float((out.double() - want).norm() / want.norm()) <= 1e-6
+    got = k.gemm(a, w, x.clone(), k.EPI_ADD_F32).double() - x.double()
+    assert bool(((got - want).abs() <= bound).all()) and float((got - want).norm() / want.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("M,N,Kd,choice", [
+    (1, 64, 1184, 12), (33, 3008, 1184, 22), (3, 8224, 2208, 112), (47, 40000, 2208, 122), (65, 64, 1184, 212), (161, 8224, 1184, 222),
+    (161, 16416, 1184, 224), (513, 5152, 1184, 234), (321, 20000, 1184, 244)])
+def test_gemm_float32_every_gated_tile(M, N, Kd, choice):
+    from yalm_amd.ops import library
+    k = K()
+    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 1) == choice
+    H = N // 2 - 3
+    a, w = rnd((M, Kd), 104).to(DEV), rnd((N, Kd), 105, scale=Kd ** -0.5).to(DEV)
+    p = (a.double() @ w.double().t()).view(M, -1, 2, 16)
+    gate, up = p[:, :, 0].reshape(M, -1)[:, :H], p[:, :, 1].reshape(M, -1)[:, :H]
+    want = gate / (1.0 + torch.exp(-gate)) * up
+    got = k.gemm(a, w, torch.full((M, H), 7.0, device=DEV), k.EPI_GATED, hidden=H).double()
+    # gate and up are sums about 1e-6 off at sizes of 1 that the unit multiplies (its slope is at most 1.1), and its own roundings
+    assert float((got - want).norm() / want.norm()) <= 4e-6
+    assert float((got - want).abs().max()) <= 1e-4
+
+
+# float32 on the matrix cores: the edges of the smallest tiles and of the rules (16 | 17 and 32 | 33 rows, 4,096 and 8,192
+# columns), of one k tile and a few, K short of one round of the waves, operands 4 bytes off
 @pytest.mark.parametrize("M,N,Kd,off", [
     (1, 48, 32, 0), (15, 33, 64, 0), (16, 4096, 96, 0), (16, 8192, 64, 0), (17, 4097, 288, 0), (17, 4096, 288, 0), (32, 80, 544, 0),
     (33, 200, 128, 0), (64, 96, 1056, 0), (65, 129, 32, 0), (129, 160, 64, 0), (161, 3000, 160, 0), (700, 3072, 128, 0),

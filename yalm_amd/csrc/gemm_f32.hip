@@ -328,18 +328,14 @@ int launch_few(const float* A, const float* W, float* C, int M, int N, int K, Ga
 
 template <int EPI, int FA, int FB, bool FINE>
 int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  if constexpr (gated(EPI) && FB % 2 != 0) {
-    return YALM_ERR_ARG;
-  } else {
-    const int tiles = ceil_div(M, 32 * FA) * ceil_div(N, 32 * FB), lds = stages_of(FA, FB) * 32 * (FA + FB) * ROWB;
-    auto kernel = &gemm_f32_kernel<EPI, FA, FB, FINE>;
-    if (lds > 64 * 1024) {
-      static LdsAllowance allowed;
-      if (int rc = allow_dynamic_lds(allowed, (const void*)kernel, lds); rc != YALM_OK) return rc;
-    }
-    kernel<<<8 * ceil_div(tiles, 8), 256, lds, stream>>>(A, W, C, M, N, K, H);
-    return launch_status();
+  const int tiles = ceil_div(M, 32 * FA) * ceil_div(N, 32 * FB), lds = stages_of(FA, FB) * 32 * (FA + FB) * ROWB;
+  auto kernel = &gemm_f32_kernel<EPI, FA, FB, FINE>;
+  if (lds > 64 * 1024) {
+    static LdsAllowance allowed;
+    if (int rc = allow_dynamic_lds(allowed, (const void*)kernel, lds); rc != YALM_OK) return rc;
   }
+  kernel<<<8 * ceil_div(tiles, 8), 256, lds, stream>>>(A, W, C, M, N, K, H);
+  return launch_status();
 }
 
 // Estimated time in us of one of the tile's kernel: f = FA FB products of 16 x 16 a wave.  Measured: a k tile takes 0.13 +
@@ -354,53 +350,37 @@ double tile_time(int M, int N, int K, int fa, int fb) {
   return (0.055 + 0.118 * f) * k * ((double)whole + (rest > 0.0 ? 0.5 + 0.5 * rest : 0.0));
 }
 
-// The tile for a shape: the fastest by that estimate (701 rows, N x K: 16,384 x 3,072 takes 2x4 555 us, 128,256 x 3,072 2x4
-// 4.0 ms, 3,072 x 8,192 3x3 288 us on exactly 256 tiles, 2x4 would be 24 % slower).  Up to 64 rows the small tiles' FINE
-// form (2x4 would spill registers: 128,256 x 3,072 at 64 rows 446 against 459 us with 2x2, 16,384 x 3,072 114 against 66).
-template <int EPI>
-int launch_tiles(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  static constexpr int shapes[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 3}, {3, 4}, {4, 4}};
-  const bool fine = M <= 64;
-  int best = -1;
-  double best_t = 0.0;
-  for (int i = 0; i < (fine ? 4 : 8); ++i) {
-    if (gated(EPI) && shapes[i][1] % 2) continue;
-    const double t = tile_time(M, N, K, shapes[i][0], shapes[i][1]);
-    if (best < 0 || t < best_t) { best = i; best_t = t; }
-  }
-#define YALM_F32_TILE(FA_, FB_) \
-  return fine ? launch_f32<EPI, FA_, FB_, true>(A, W, C, M, N, K, H, stream) : launch_f32<EPI, FA_, FB_, false>(A, W, C, M, N, K, H, stream)
-  switch (best) {
-    case 0: YALM_F32_TILE(1, 1);
-    case 1: YALM_F32_TILE(1, 2);
-    case 2: YALM_F32_TILE(2, 1);
-    case 3: YALM_F32_TILE(2, 2);
-    case 4: return launch_f32<EPI, 2, 4, false>(A, W, C, M, N, K, H, stream);
-    case 5: return launch_f32<EPI, 3, 3, false>(A, W, C, M, N, K, H, stream);
-    case 6: return launch_f32<EPI, 3, 4, false>(A, W, C, M, N, K, H, stream);
-    default: return launch_f32<EPI, 4, 4, false>(A, W, C, M, N, K, H, stream);
-  }
-#undef YALM_F32_TILE
-}
+struct Choice {
+  enum Kernel { FEW, FINE, COARSE } kernel;
+  int a, b;                                        // MB and NB, or FA and FB
+};
 
 // How many of the rows and weight rows a workgroup of gemm_few_f32_kernel takes (no sum depends on it).  Every 16 rows by
 // themselves where that leaves no CU two workgroups (64 rows, 1,024 x 1,024 6.8 us; 2 and 4 times 16 8.9 and 13.1), else 32, and
 // 64 of up to 4,096 columns (64 rows, 4,096 x 4,096 42 against 51 us with 32).  Two blocks of weight rows save reading A, which
 // pays from 8 rows of many columns on (5,120 x 3,072: 4 rows 22.1 us with one, 22.8 with two, 16 rows 28.1 and 25.7).
-template <int EPI>
-int launch_few_rows(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  constexpr bool G = gated(EPI);
-  const bool alone = M <= 16 || (long)ceil_div(N, G ? 32 : 16) * ceil_div(M, 16) <= 256;
-  if constexpr (G) {
-    if (alone) return launch_few<EPI, 1, 2>(A, W, C, M, N, K, H, stream);
-    return launch_few<EPI, 2, 2>(A, W, C, M, N, K, H, stream);
-  } else {
-    if (alone && M > 7 && N > 4096) return launch_few<EPI, 1, 2>(A, W, C, M, N, K, H, stream);
-    if (alone) return launch_few<EPI, 1, 1>(A, W, C, M, N, K, H, stream);
-    if (N > 4096) return launch_few<EPI, 2, 2>(A, W, C, M, N, K, H, stream);
-    if (M <= 32) return launch_few<EPI, 2, 1>(A, W, C, M, N, K, H, stream);
-    return launch_few<EPI, 4, 1>(A, W, C, M, N, K, H, stream);
+Choice choose_few(int M, int N, bool gate) {
+  const bool alone = M <= 16 || (long)ceil_div(N, gate ? 32 : 16) * ceil_div(M, 16) <= 256;
+  if (gate) return {Choice::FEW, alone ? 1 : 2, 2};
+  if (alone) return {Choice::FEW, 1, M > 7 && N > 4096 ? 2 : 1};
+  if (N > 4096) return {Choice::FEW, 2, 2};
+  return {Choice::FEW, M <= 32 ? 2 : 4, 1};
+}
+
+// The fastest tile by the estimate (701 rows, N x K: 16,384 x 3,072 takes 2x4 555 us, 128,256 x 3,072 2x4 4.0 ms, 3,072 x 8,192
+// 3x3 288 us on exactly 256 tiles, 2x4 would be 24 % slower).  Up to 64 rows the small tiles' FINE form (2x4 would spill
+// registers: 128,256 x 3,072 at 64 rows 446 against 459 us with 2x2, 16,384 x 3,072 114 against 66).
+Choice choose_tile(int M, int N, int K, bool gate) {
+  static constexpr int shapes[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 3}, {3, 4}, {4, 4}};
+  const bool fine = M <= 64;
+  int best = -1;
+  double best_t = 0.0;
+  for (int i = 0; i < (fine ? 4 : 8); ++i) {
+    if (gate && shapes[i][1] % 2) continue;
+    const double t = tile_time(M, N, K, shapes[i][0], shapes[i][1]);
+    if (best < 0 || t < best_t) { best = i; best_t = t; }
   }
+  return {fine ? Choice::FINE : Choice::COARSE, shapes[best][0], shapes[best][1]};
 }
 
 // Up to 64 rows the form of a sum follows from N and K alone, so that a row's results do not change with the number of rows
@@ -409,13 +389,46 @@ int launch_few_rows(const float* A, const float* W, float* C, int M, int N, int 
 // and short sums, where the FINE chains would lie further from 64 bits than gemm_rows_f32_kernel's (a relative error at K 1,024 of
 // 1.2e-7 against 1.0e-7, its own 0.9e-7; at K 2,560 1.26e-7 against 1.33e-7).  The rest goes to the tiles, which read A once for 32
 // weight rows and more (16,384 x 3,072: one row 43 us, 16 rows 42, 64 rows 66; gemm_few_f32_kernel 45, 51 and 127).
+Choice choose(int M, int N, int K, bool gate) {
+  return M <= 64 && (N < 8192 || K <= 2048) ? choose_few(M, N, gate) : choose_tile(M, N, K, gate);
+}
+
 template <int EPI>
 int launch(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  if (M <= 64 && (N < 8192 || K <= 2048)) return launch_few_rows<EPI>(A, W, C, M, N, K, H, stream);
-  return launch_tiles<EPI>(A, W, C, M, N, K, H, stream);
+  const Choice c = choose(M, N, K, gated(EPI));
+#define YALM_TAKE(KERNEL_, A_, B_, CALL_) \
+  if (c.kernel == Choice::KERNEL_ && c.a == A_ && c.b == B_) return CALL_(A, W, C, M, N, K, H, stream)
+  YALM_TAKE(FEW, 1, 2, (launch_few<EPI, 1, 2>));
+  YALM_TAKE(FEW, 2, 2, (launch_few<EPI, 2, 2>));
+  YALM_TAKE(FINE, 1, 2, (launch_f32<EPI, 1, 2, true>));
+  YALM_TAKE(FINE, 2, 2, (launch_f32<EPI, 2, 2, true>));
+  YALM_TAKE(COARSE, 1, 2, (launch_f32<EPI, 1, 2, false>));
+  YALM_TAKE(COARSE, 2, 2, (launch_f32<EPI, 2, 2, false>));
+  YALM_TAKE(COARSE, 2, 4, (launch_f32<EPI, 2, 4, false>));
+  YALM_TAKE(COARSE, 3, 4, (launch_f32<EPI, 3, 4, false>));
+  YALM_TAKE(COARSE, 4, 4, (launch_f32<EPI, 4, 4, false>));
+  if constexpr (!gated(EPI)) {                     // an odd number of column tiles
+    YALM_TAKE(FEW, 1, 1, (launch_few<EPI, 1, 1>));
+    YALM_TAKE(FEW, 2, 1, (launch_few<EPI, 2, 1>));
+    YALM_TAKE(FEW, 4, 1, (launch_few<EPI, 4, 1>));
+    YALM_TAKE(FINE, 1, 1, (launch_f32<EPI, 1, 1, true>));
+    YALM_TAKE(FINE, 2, 1, (launch_f32<EPI, 2, 1, true>));
+    YALM_TAKE(COARSE, 1, 1, (launch_f32<EPI, 1, 1, false>));
+    YALM_TAKE(COARSE, 2, 1, (launch_f32<EPI, 2, 1, false>));
+    YALM_TAKE(COARSE, 3, 3, (launch_f32<EPI, 3, 3, false>));
+  }
+#undef YALM_TAKE
+  return YALM_ERR_ARG;
 }
 
 }  // namespace
+
+// Which kernel and tile a product takes: 100 kernel (0 gemm_few_f32_kernel, 1 FINE tiles, 2 tiles) + 10 a + b
+extern "C" int yalm_gemm_f32_choice(int M, int N, int K, int gate) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0) return -1;
+  const Choice c = choose(M, N, K, gate != 0);
+  return 100 * c.kernel + 10 * c.a + c.b;
+}
 
 // K a multiple of 32 and 16-byte aligned operands; YALM_ERR_ARG: not taken.
 int yalm_gemm_f32_mfma(const void* A, const void* W, void* C, int M, int N, int K, int epilogue, GateOut H, hipStream_t stream) {
