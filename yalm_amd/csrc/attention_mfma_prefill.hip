@@ -351,19 +351,6 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
   }
 }
 
-// compute units of the current device (asked once: this library drives one device a process)
-int compute_units() {
-  static int n = 0;
-  if (n == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    n = v;
-  }
-  return n;
-}
-
 // launches attn_prefill_mfma_kernel<head_dim, NC, KSPL> (more than 64 KB of LDS is asked for once a device)
 template <int HD, int NC, int KSPL, bool BIAS>
 int launch_prefill(dim3 grid, int threads, size_t lds, hipStream_t stream, const bf16* qp, const bf16* kp, const bf16* vp,

@@ -125,6 +125,19 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// compute units of the current device (asked once: this library drives one device a process)
+inline int compute_units() {
+  static int n = 0;
+  if (n == 0) {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
+      v = 256;
+    n = v;
+  }
+  return n;
+}
+
 // More than 64 KB of dynamic LDS has to be allowed for a kernel before its first launch, on every device it is
 // launched on.  One LdsAllowance (a static of the launcher) per kernel: a bit per device, set under a lock.
 struct LdsAllowance {

@@ -343,7 +343,7 @@ int launch_f32(const float* A, const float* W, float* C, int M, int N, int K, Ga
 // 4,096: 4x4 249 us, 3x3 111, 2x4 102, 2x2 73, 2x1 45, 1x1 32 alone); a last round on a fraction of the CUs costs half a
 // round and half its fraction.
 double tile_time(int M, int N, int K, int fa, int fb) {
-  const double f = fa * fb, per = (double)ceil_div(M, 32 * fa) * ceil_div(N, 32 * fb) / 256.0, k = K / TK;
+  const double f = fa * fb, per = (double)ceil_div(M, 32 * fa) * ceil_div(N, 32 * fb) / compute_units(), k = K / TK;
   if (per <= 1.0) return (0.13 + 0.116 * f) * k;
   const long whole = (long)per;
   const double rest = per - (double)whole;
@@ -360,7 +360,7 @@ struct Choice {
 // 64 of up to 4,096 columns (64 rows, 4,096 x 4,096 42 against 51 us with 32).  Two blocks of weight rows save reading A, which
 // pays from 8 rows of many columns on (5,120 x 3,072: 4 rows 22.1 us with one, 22.8 with two, 16 rows 28.1 and 25.7).
 Choice choose_few(int M, int N, bool gate) {
-  const bool alone = M <= 16 || (long)ceil_div(N, gate ? 32 : 16) * ceil_div(M, 16) <= 256;
+  const bool alone = M <= 16 || (long)ceil_div(N, gate ? 32 : 16) * ceil_div(M, 16) <= compute_units();
   if (gate) return {Choice::FEW, alone ? 1 : 2, 2};
   if (alone) return {Choice::FEW, 1, M > 7 && N > 4096 ? 2 : 1};
   if (N > 4096) return {Choice::FEW, 2, 2};
