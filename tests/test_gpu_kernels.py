@@ -730,6 +730,33 @@ def test_attn_prefill_in_a_given_tile_order(n_heads, n_kv, hd, window, lens):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("off", [(1, 0), (0, 2), (3, 5)])
+def test_attn_prefill_with_stages_off_sixteen_bytes(off):
+    """At head size 128 tiles that go straight into LDS have to lie on 16 bytes; others are taken by the general kernel."""
+    k = K()
+    lens, n_heads, n_kv, hd, dtype = [200, 33], 4, 2, 128, torch.bfloat16
+    T = sum(lens)
+    q, kk, v = rnd((T, n_heads * hd), 43, dtype), rnd((T, n_kv * hd), 44, dtype), rnd((T, n_kv * hd), 45, dtype)
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    seq = np.repeat(np.arange(len(lens)), lens)
+    pos = np.concatenate([np.arange(n) for n in lens])
+    ks, vs, tile0 = stage(kk, v, lens, n_kv, hd, dtype)
+
+    def moved(t, by):
+        flat = torch.empty(t.numel() + 8, dtype=dtype, device=DEV)
+        view = flat[by:by + t.numel()].view(t.shape)
+        view.copy_(t)
+        return view
+
+    out = torch.empty((T, n_heads * hd), dtype=dtype, device=DEV)
+    k.attn_prefill(q.to(DEV), moved(ks, off[0]), moved(vs, off[1]), out, i32(cu), i32(tile0), i32(seq), i32(pos), n_heads, n_kv, hd, 0)
+    want, o = [], 0
+    for n in lens:
+        want.append(masked_attention_float64(q[o:o + n], kk[o:o + n], v[o:o + n], n_heads, n_kv, hd, 0))
+        o += n
+    close(out, torch.cat(want), dtype, "prefill attention")
+
+
 def paged_case(lens, n_kv, hd, window, dtype, seed, poison=True, stored=True):
     """Random keys/values of sequences of the given lengths laid out in pages the way
     the cache does (ring for a window), the rest of the pool poisoned with NaN.  stored=False: the pages in

@@ -411,6 +411,7 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
   if (!mfma_shape_ok(n_heads, n_kv_heads, head_dim, biased) || n_tiles > 65535) return YALM_ERR_ARG;
   if (shape.bias != nullptr && shape.n_bias <= 0) return YALM_ERR_ARG;
   if (tile_order && (n_order <= 0 || n_order > n_tiles)) return YALM_ERR_ARG;
+  if (prefill_dma(head_dim) && (((uintptr_t)k_stage | (uintptr_t)v_stage) & 15)) return YALM_ERR_ARG;    // 16 bytes a lane into LDS
   dim3 grid(n_heads, tile_order ? n_order : n_tiles);
   const long total = (long)grid.x * grid.y;
   const size_t pad = prefill_dma(head_dim) ? 0 : 8;
