@@ -732,7 +732,7 @@ def test_attn_prefill_in_a_given_tile_order(n_heads, n_kv, hd, window, lens):
 
 @pytest.mark.parametrize("off", [(1, 0), (0, 2), (3, 5)])
 def test_attn_prefill_with_stages_off_sixteen_bytes(off):
-    """At head size 128 tiles that go straight into LDS have to lie on 16 bytes; others are taken by the general kernel."""
+    """At head size 128 tiles that go straight into LDS have to lie on 16 bytes; others go through registers, with the same bits."""
     k = K()
     lens, n_heads, n_kv, hd, dtype = [200, 33], 4, 2, 128, torch.bfloat16
     T = sum(lens)
@@ -748,8 +748,10 @@ def test_attn_prefill_with_stages_off_sixteen_bytes(off):
         view.copy_(t)
         return view
 
-    out = torch.empty((T, n_heads * hd), dtype=dtype, device=DEV)
+    out, on_sixteen = (torch.empty((T, n_heads * hd), dtype=dtype, device=DEV) for _ in range(2))
     k.attn_prefill(q.to(DEV), moved(ks, off[0]), moved(vs, off[1]), out, i32(cu), i32(tile0), i32(seq), i32(pos), n_heads, n_kv, hd, 0)
+    k.attn_prefill(q.to(DEV), moved(ks, 0), moved(vs, 0), on_sixteen, i32(cu), i32(tile0), i32(seq), i32(pos), n_heads, n_kv, hd, 0)
+    assert torch.equal(out, on_sixteen)
     want, o = [], 0
     for n in lens:
         want.append(masked_attention_float64(q[o:o + n], kk[o:o + n], v[o:o + n], n_heads, n_kv, hd, 0))

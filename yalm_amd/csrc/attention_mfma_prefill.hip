@@ -24,11 +24,11 @@ namespace {
 // workgroup, 32 key tiles at 2,048 tokens, while the mean is 17).
 // BIAS: the scores are shaped (ScoreShape: a cap, a term by the distance of query and key, bias[head][min(distance,
 // n_bias - 1)], a learned logit in the denominator; each optional).
-__host__ __device__ constexpr bool prefill_dma(int hd) { return hd == 128; }
+constexpr bool prefill_dma(int hd) { return hd == 128; }       // built with DMA too
 // the place (0..15) at which a fragment read takes key row `row` (key_row's inverse): its chunks are swizzled by it
 __device__ __forceinline__ int key_swizzle(int row) { return (row & 3) | ((row >> 3) & 3) << 2; }
 
-template <int HD, int NC, int KSPL, bool BIAS>
+template <int HD, int NC, int KSPL, bool BIAS, bool DMA>
 __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void attn_prefill_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_stage, const bf16* __restrict__ v_stage,
     bf16* __restrict__ out, float* __restrict__ out_f32, float* __restrict__ lse, const int* __restrict__ cu_seqlens,
@@ -40,10 +40,9 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
   // lanes, the row's last 8 elements once more in the keys'), and the tile's chunks do not divide evenly over the threads.
   constexpr int KS = (HD + 31) / 32, DT = HD / 16;
   static_assert(HD % 16 == 0, "head sizes in steps of 16");
-  // DMA (head size 128): the tiles go from memory straight into LDS, rows unpadded, the 16-byte chunks of a row XOR-swizzled
-  // by the place at which the fragment reads take the row, so that sixteen lanes read from all banks; else through registers
-  // into rows with 16 bytes of padding.
-  constexpr bool DMA = prefill_dma(HD);
+  // DMA (head size 128, staged keys and values on 16 bytes): the tiles go from memory straight into LDS, rows unpadded, the
+  // 16-byte chunks of a row XOR-swizzled by the place at which the fragment reads take the row, so that sixteen lanes read from
+  // all banks; else through registers, which no alignment binds, into rows with 16 bytes of padding.
   constexpr int KROW = DMA ? HD : HD + 8;         // LDS row strides (elements)
   constexpr int VROW = DMA ? PAGE : PAGE + 8;
   constexpr int KTILE = PAGE * KROW, VTILE = HD * VROW;
@@ -352,12 +351,12 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 && HD <= 144 ? 2 : 1) void at
 }
 
 // launches attn_prefill_mfma_kernel<head_dim, NC, KSPL> (more than 64 KB of LDS is asked for once a device)
-template <int HD, int NC, int KSPL, bool BIAS>
+template <int HD, int NC, int KSPL, bool BIAS, bool DMA>
 int launch_prefill(dim3 grid, int threads, size_t lds, hipStream_t stream, const bf16* qp, const bf16* kp, const bf16* vp,
                    bf16* out, float* out_f32, float* lse, const int* cu_seqlens, const int* seq_tile0,
                    const int* tile_order, int fold_at, int B, int n_heads, int n_kv_heads, int window,
                    const ScoreShape& shape) {
-  auto kernel = &attn_prefill_mfma_kernel<HD, NC, KSPL, BIAS>;
+  auto kernel = &attn_prefill_mfma_kernel<HD, NC, KSPL, BIAS, DMA>;
   if (lds > 64 * 1024) {
     static LdsAllowance allowed;
     if (int rc = allow_dynamic_lds(allowed, (const void*)kernel, 150 * 1024); rc != YALM_OK) return rc;
@@ -367,10 +366,12 @@ int launch_prefill(dim3 grid, int threads, size_t lds, hipStream_t stream, const
   return launch_status();
 }
 template <int NC, int KSPL, typename... Args>
-int launch_prefill_hd(int head_dim, bool biased, Args... args) {
-#define YALM_PREFILL_HD(HD_)                                                        \
-  case HD_:                                                                         \
-    return biased ? launch_prefill<HD_, NC, KSPL, true>(args...) : launch_prefill<HD_, NC, KSPL, false>(args...)
+int launch_prefill_hd(int head_dim, bool biased, bool dma, Args... args) {
+#define YALM_PREFILL_HD(HD_)                                                                         \
+  case HD_:                                                                                          \
+    if constexpr (prefill_dma(HD_))                                                                  \
+      if (dma) return biased ? launch_prefill<HD_, NC, KSPL, true, true>(args...) : launch_prefill<HD_, NC, KSPL, false, true>(args...); \
+    return biased ? launch_prefill<HD_, NC, KSPL, true, false>(args...) : launch_prefill<HD_, NC, KSPL, false, false>(args...)
   switch (head_dim) {
     YALM_PREFILL_HD(16);
     YALM_PREFILL_HD(32);
@@ -386,7 +387,7 @@ int launch_prefill_hd(int head_dim, bool biased, Args... args) {
 }
 template <typename... Args>
 int launch_prefill_wide(int head_dim, Args... args) {
-#define YALM_PREFILL_WIDE(HD_) case HD_: return launch_prefill<HD_, 2, 1, false>(args...)
+#define YALM_PREFILL_WIDE(HD_) case HD_: return launch_prefill<HD_, 2, 1, false, false>(args...)
   switch (head_dim) {
     YALM_PREFILL_WIDE(144);
     YALM_PREFILL_WIDE(160);
@@ -411,10 +412,10 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
   if (!mfma_shape_ok(n_heads, n_kv_heads, head_dim, biased) || n_tiles > 65535) return YALM_ERR_ARG;
   if (shape.bias != nullptr && shape.n_bias <= 0) return YALM_ERR_ARG;
   if (tile_order && (n_order <= 0 || n_order > n_tiles)) return YALM_ERR_ARG;
-  if (prefill_dma(head_dim) && (((uintptr_t)k_stage | (uintptr_t)v_stage) & 15)) return YALM_ERR_ARG;    // 16 bytes a lane into LDS
   dim3 grid(n_heads, tile_order ? n_order : n_tiles);
   const long total = (long)grid.x * grid.y;
-  const size_t pad = prefill_dma(head_dim) ? 0 : 8;
+  const bool dma = prefill_dma(head_dim) && (((uintptr_t)k_stage | (uintptr_t)v_stage) & 15) == 0;      // 16 bytes a lane into LDS
+  const size_t pad = dma ? 0 : 8;
   const size_t tile_bytes = ((size_t)PAGE * (head_dim + pad) + (size_t)head_dim * (PAGE + pad)) * sizeof(bf16);
   const bf16 *qp = (const bf16*)q, *kp = (const bf16*)k_stage, *vp = (const bf16*)v_stage;
   // A wide head: two buffers of keys and values fill up to 141 KB of LDS, so four waves a workgroup are the one form.
@@ -430,7 +431,7 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
   if (n_tiles == B) {
     // every sequence has one tile of keys: nothing to take in halves and to merge (33 tokens with 32 heads 8.3 -> 7.9
     // us, four times 64 8.1 -> 7.2, forty times 50 with 24 heads, which took 128 queries a workgroup, 22.5 -> 20.7)
-    return launch_prefill_hd<1, 1>(head_dim, biased, dim3(n_heads, n_tiles), 256, 2 * tile_bytes, stream, qp, kp, vp,
+    return launch_prefill_hd<1, 1>(head_dim, biased, dma, dim3(n_heads, n_tiles), 256, 2 * tile_bytes, stream, qp, kp, vp,
                                    (bf16*)out, out_f32, lse, cu_seqlens, seq_tile0, (const int*)nullptr, (int)total, B,
                                    n_heads, n_kv_heads, window, shape);
   }
@@ -438,13 +439,13 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
     // a short step: a workgroup of eight waves for every tile of 64 queries (not 128), so that twice as many
     // compute units work (512 tokens with 32 heads: 19.6 -> 15.9 us a layer); all of them run at once, so their order
     // does not matter
-    return launch_prefill_hd<1, 2>(head_dim, biased, dim3(n_heads, n_tiles), 512, 4 * tile_bytes, stream, qp, kp, vp,
+    return launch_prefill_hd<1, 2>(head_dim, biased, dma, dim3(n_heads, n_tiles), 512, 4 * tile_bytes, stream, qp, kp, vp,
                                    (bf16*)out, out_f32, lse, cu_seqlens, seq_tile0, (const int*)nullptr, 0, B, n_heads,
                                    n_kv_heads, window, shape);
   }
   if (working <= 2L * compute_units()) {
     // a workgroup of eight waves a compute unit, the workgroups that see the most keys first
-    return launch_prefill_hd<2, 2>(head_dim, biased, grid, 512, 4 * tile_bytes, stream, qp, kp, vp, (bf16*)out, out_f32,
+    return launch_prefill_hd<2, 2>(head_dim, biased, dma, grid, 512, 4 * tile_bytes, stream, qp, kp, vp, (bf16*)out, out_f32,
                                    lse, cu_seqlens, seq_tile0, tile_order, (int)total, B, n_heads, n_kv_heads, window,
                                    shape);
   }
@@ -452,6 +453,6 @@ int yalm_attn_prefill_bf16_mfma(const void* q, const void* k_stage, const void* 
   // half of the launch runs from the shortest workgroup up
   const int cus = compute_units();
   const int fold_at = total > cus && total <= 2 * cus ? cus : (int)total;
-  return launch_prefill_hd<2, 1>(head_dim, biased, grid, 256, 2 * tile_bytes, stream, qp, kp, vp, (bf16*)out, out_f32,
+  return launch_prefill_hd<2, 1>(head_dim, biased, dma, grid, 256, 2 * tile_bytes, stream, qp, kp, vp, (bf16*)out, out_f32,
                                  lse, cu_seqlens, seq_tile0, tile_order, fold_at, B, n_heads, n_kv_heads, window, shape);
 }
