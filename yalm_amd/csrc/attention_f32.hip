@@ -1,8 +1,9 @@
 // Attention of the true 32-bit path on the matrix cores (v_mfma_f32_16x16x4_f32), softmax state and expf in float32:
 // head sizes of 64 to 128 in steps of 16, every shape of the scores.  The kernels of attention_simple.hip take the others.
-// Smaller heads stay there for their bits, not for their time: both sum to about 3e-7, in another order, and a model of such
-// heads (of 8 to 24, a recurrent head beside the attention) read a nearly empty recurrent state there, which magnifies a last
-// bit a thousandfold: 1.1e-4 off in the logits with these kernels, 2.7e-5 with the general ones.
+// Smaller heads stay there for their bits, not for their time: both sum to about 3e-7, in another order, and a model of heads of 8
+// to 24 with a recurrent head beside the attention read a nearly empty recurrent state there, which magnifies a last bit a
+// thousandfold: 1.1e-4 off in the logits with these kernels, 2.7e-5 with the general ones.  Heads of 32 and 48 have not been
+// compared and stay with them too.
 //
 //   scores^T[key, query] = K[key, :] . Q[query, :]        A = 16 key rows x 4 elements, B = 16 queries
 //   out^T[elem, query]  += V^T[elem, key] P^T[key, query]  A = 16 elements x 4 keys, B = P^T
@@ -15,7 +16,7 @@
 // Probabilities of zero still multiply their value there, and 0 times infinity is no number.  Keys whose values are not all
 // finite are mixed one by one instead, zeros left out.
 //
-// 701 tokens, 24 heads of 128: 2,590 -> 87 us a layer; a decode step of 4 sequences of 20 to 36 tokens, 4 heads of 128:
+// 701 tokens, 24 heads of 128: 2,564 -> 87 us a layer; a decode step of 4 sequences of 20 to 36 tokens, 4 heads of 128:
 // 24 -> 8 us, and no kernel that merges splits behind it where there is one; 8 sequences of 4,000 tokens 666 -> 46 us.
 #include <float.h>
 #include <type_traits>

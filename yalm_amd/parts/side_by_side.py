@@ -109,6 +109,7 @@ class SideBySide(Part):
             if self.late_bias is not None:
                 raise ValueError("a mixer whose last product has a bias writes its result (forward_to); it does not add to the stream")
             return self._joint(h, x, ctx, line, writes_cache, kernels.EPI_ADD_F32)
+        # both results whole: a second float32 [T, dim] beside the first (64 MB for 4,096 tokens of width 4,096), added in one pass
         y, y2 = (ctx.ws.get(name, (T, self.dim), torch.float32) for name in ("side.y", "side.y2"))
         self.left.forward_to(h, y, ctx, (line, "left"), writes_cache)
         self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache)
