@@ -53,6 +53,31 @@ def test_greedy_generation_matches_the_plain_implementation(folders, name):
     assert not engine.cache.slots.held
 
 
+# float32, contexts of up to 256 tokens: a request's logits have the same bits whatever the requests beside it (heads of the matrix
+# cores' attention kernel and of the general one; a head on 8,192 rows and more over short and over long sums)
+@pytest.mark.parametrize("dim,head_dim,vocab", [(256, 64, 8224), (96, 32, 311), (2112, 64, 8224)])
+def test_float32_logits_do_not_depend_on_the_batch(tmp_path, dim, head_dim, vocab):
+    from yalm_amd import Engine, Model
+    cfg = dict(tiny_configs.TINY_LLAMA, hidden_size=dim, intermediate_size=320, num_hidden_layers=1, num_attention_heads=dim // head_dim,
+               num_key_value_heads=1, head_dim=head_dim, vocab_size=vocab, max_position_embeddings=512)
+    engine = Engine(Model.from_folder(helpers.make_folder(tmp_path, "m", cfg, seed=7), dtype=torch.float32, device="cuda:0"),
+                    max_tokens=33 * 256)
+    lens = [1 + (i * 97) % 250 for i in range(33)]
+    prompts = list(helpers.random_requests(cfg, lens, seed=3).values())
+
+    def two_steps(which):
+        slots = [engine.start(1)[0] for _ in which]
+        for s, i in zip(slots, which):
+            engine.step([s], [prompts[i]])
+        got = [engine.step(slots, [[(11 * i + k) % vocab] for i in which]).clone() for k in range(2)]
+        engine.release(slots)
+        return torch.stack(got, 1)
+
+    whole = two_steps(range(33))
+    for which in [range(n) for n in (1, 2, 4, 5, 16, 17, 32)] + [[20, 3, 31]]:
+        assert torch.equal(two_steps(which), whole[list(which)]), which
+
+
 def test_temperature_sampling_with_a_fixed_seed(folders):
     """The tiny Mistral workload: prompts of 2, 30, 9, 23 tokens, 20 steps past the window at
     temperature 0.8.  A request's tokens depend on the seed and its id, not on its batch,

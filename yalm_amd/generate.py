@@ -78,7 +78,8 @@ def generate(engine, prompts, max_new_tokens=256, temperature=0.0, seed=0, stop_
     (default: if the engine has step_from and the sampler has draw).  A request that has ended
     leaves the batch a step later then, so a step may run with another number of rows and take other
     kernels: in float32 the tokens are the same either way (a row's sums do not depend on the rows beside it, up to 64 of
-    them; but the attention of contexts beyond 256 tokens is cut by their number, which moves its last bits), in bfloat16
+    them; but where a context of the step is beyond 256 tokens, or 64 at head sizes that are no multiple of 16, the rows'
+    number and the longest context decide into how many pieces the attention is cut, which moves its last bits), in bfloat16
     up to choices between logits that lie within rounding of each other."""
     from .sampling import Sampler
     sampler = sampler or Sampler(seed)
