@@ -378,6 +378,82 @@ def test_gemm_float32_every_gated_tile(M, N, Kd, choice):
     assert float((got - want).abs().max()) <= 1e-4
 
 
+# The larger tiles of float32 products, which only sums of less than 512 still take: 15 k tiles, so that each ring turns and sums
+# are folded in a whole and a broken run
+@pytest.mark.parametrize("M,N,choice", [(161, 16401, 224), (161, 12001, 233), (513, 5130, 234), (321, 20001, 244)])
+def test_gemm_float32_short_sums_on_the_larger_tiles(M, N, choice):
+    from yalm_amd.ops import library
+    k, Kd = K(), 480
+    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 0) == choice and library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) == -1
+    a, w = rnd((M, Kd), 111).to(DEV), rnd((N, Kd), 112).to(DEV)
+    want = a.double() @ w.double().t()
+    out = k.gemm(a, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double()
+    assert bool(((out - want).abs() <= (2.0 * Kd + 2.0) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())).all())
+    assert float((out - want).norm() / want.norm()) <= 1e-6
+
+
+# Every tile of the products by bfloat16 terms, with edges of 1 to 200 rows and columns, an even number of k tiles (16), odd ones (17
+# and 37: the two groups of a workgroup have unlike numbers, folds are broken)
+@pytest.mark.parametrize("Kd", [512, 544, 1184])
+@pytest.mark.parametrize("M,N,tile", [(97, 5130, 0), (161, 8201, 1), (161, 12001, 2), (513, 5131, 3), (513, 8201, 4), (321, 20001, 5)])
+def test_gemm_float32_by_terms(M, N, tile, Kd):
+    from yalm_amd.ops import library
+    k = K()
+    assert library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) == tile
+    a, w, x = rnd((M, Kd), 113).to(DEV), rnd((N, Kd), 114).to(DEV), rnd((M, N), 115).to(DEV)
+    want = a.double() @ w.double().t()
+    # as for the float32 products: six products of terms an element, the three left out together below 2^-25 of the product
+    bound = (2.0 * Kd + 2.0) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t() + x.double().abs())
+    out = k.gemm(a, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double()
+    assert bool(((out - want).abs() <= bound).all()) and float((out - want).norm() / want.norm()) <= 1e-6
+    got = k.gemm(a, w, x.clone(), k.EPI_ADD_F32).double() - x.double()
+    assert bool(((got - want).abs() <= bound).all()) and float((got - want).norm() / want.norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("M,N,tile", [(97, 5152, 0), (161, 8224, 1), (513, 5152, 3), (513, 8224, 4), (321, 20000, 5)])
+@pytest.mark.parametrize("act", ACTS)
+def test_gemm_float32_by_terms_gated(M, N, tile, act):
+    from yalm_amd.ops import library
+    k, Kd = K(), 544
+    assert library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 1) == tile
+    act_fn, epi = gate(act)
+    H = N // 2 - 3
+    a, w = rnd((M, Kd), 116).to(DEV), rnd((N, Kd), 117, scale=Kd ** -0.5).to(DEV)
+    p = (a.double() @ w.double().t()).view(M, -1, 2, 16)
+    gate_, up = p[:, :, 0].reshape(M, -1)[:, :H], p[:, :, 1].reshape(M, -1)[:, :H]
+    want = act_fn(gate_.cpu()).to(DEV) * up
+    got = k.gemm(a, w, torch.full((M, H), 7.0, device=DEV), epi, hidden=H).double()
+    assert float((got - want).norm() / want.norm()) <= 4e-6            # as for the gated float32 products above
+    assert float((got - want).abs().max()) <= 1e-4
+
+
+# Products by terms of what no bfloat16 holds: infinities, NaN, numbers that round to infinity, numbers whose last terms
+# vanish.  The sums are those of float32 products: not finite where a factor is not, the others untouched
+@pytest.mark.parametrize("M,N,Kd", [(161, 8201, 544), (321, 20001, 512)])
+def test_gemm_float32_by_terms_of_extreme_numbers(M, N, Kd):
+    from yalm_amd.ops import library
+    k = K()
+    assert library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) >= 0
+    a, w = rnd((M, Kd), 118), rnd((N, Kd), 119, scale=0.01)
+    a[3, 17], a[40, 500], a[41, 5], a[M - 1, 0] = math.inf, -math.inf, math.nan, 3.4028234e38
+    a[70] *= 1e-30
+    a[71] *= 2.0 ** -100
+    w[N - 2, 9] = math.inf
+    w[5] *= 1e-6
+    want = a.double() @ w.double().t()
+    got = k.gemm(a.to(DEV), w.to(DEV), torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double().cpu()
+    size = a.double().abs() @ w.double().abs().t()
+    over = size >= 3.4e38                                               # whose sums may pass float32's largest on the way
+    assert torch.equal(got.isnan() & ~over, want.isnan() & ~over)
+    assert torch.equal(got.isinf() & ~over, want.isinf() & ~over)
+    ok = size < 3.4e38
+    assert int(ok.sum()) > (M - 4) * (N - 1) - 1
+    assert bool(((got - want).abs()[ok] <= ((2.0 * Kd + 2.0) * 2.0 ** -24 * size + Kd * 2.0 ** -126)[ok]).all())
+    assert float((got[71] - want[71])[:N - 2].norm() / want[71][:N - 2].norm()) <= 1e-6
+    inf_row = want[3].isinf()
+    assert bool((got[3][inf_row] == want[3][inf_row]).all())
+
+
 # float32 on the matrix cores: the edges of the smallest tiles and of the rules (16 | 17 and 32 | 33 rows, 4,096 and 8,192
 # columns), of one k tile and a few, K short of one round of the waves, operands 4 bytes off
 @pytest.mark.parametrize("M,N,Kd,off", [

@@ -1,6 +1,8 @@
 // C = epilogue(A[M,K] * W[N,K]^T) in float32 on the matrix cores (v_mfma_f32_16x16x4_f32: products and sums in
 // float32, as a chain of fused multiply-adds): the products of the true 32-bit path.
 //
+// More than 64 rows and K 512 and more go to gemm_split.hip where that is sooner (all but small products).
+//
 // gemm_f32_kernel, from some 64 rows on bound by the matrix cores (157 TFLOP/s: the vector units' own rate, but an operand
 // register serves 16 products where gemm_simple_kernel reads LDS for every eight).  A workgroup of four waves owns a
 // tile of 32 FA x 32 FB; a wave FA x FB products of 16 x 16.  k tiles of 32 floats go straight into LDS (128-byte rows,
@@ -17,6 +19,7 @@
 // error of 3.0e-7 at 701 rows and K 8,192, where gemm_simple_kernel's was 1.6e-6; at most 64 rows 0.6e-7 at K 32 to 1.3e-7 at K
 // 3,072 and 1.6e-7 at K 14,336, gemm_rows_f32_kernel's 0.6e-7, 1.4e-7 and 2.8e-7).
 #include "common.h"
+#include "gemm_split.h"
 #include "yalm_hip.h"
 
 namespace {
@@ -393,6 +396,14 @@ Choice choose(int M, int N, int K, bool gate) {
   return M <= 64 && (N < 8192 || K <= 2048) ? choose_few(M, N, gate) : choose_tile(M, N, K, gate);
 }
 
+// The tile of gemm_split.hip that is sooner by the estimates than the tile chosen here, or -1 (5,120 x 3,072: 65 rows 42 us here, 47
+// there; 128 rows 61 and 47).  tile_time compares tiles with each other and leaves out a launch's start and end, some 5 us, and a
+// tenth that broken rounds take longer (up to 40 % just above one round: 65 rows, 3,072 x 8,192 69 us for 98 measured).
+int split_tile(int M, int N, int K, bool gate) {
+  const Choice c = choose(M, N, K, gate);
+  return c.kernel == Choice::COARSE ? yalm_gemm_split_choose(M, N, K, gate, 5.0 + 1.1 * tile_time(M, N, K, c.a, c.b)) : -1;
+}
+
 template <int EPI>
 int launch(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
   const Choice c = choose(M, N, K, gated(EPI));
@@ -423,7 +434,14 @@ int launch(const float* A, const float* W, float* C, int M, int N, int K, GateOu
 
 }  // namespace
 
-// Which kernel and tile a product takes: 100 kernel (0 gemm_few_f32_kernel, 1 FINE tiles, 2 tiles) + 10 a + b
+// Which tile of gemm_split.hip a product takes, or -1: it stays here
+extern "C" int yalm_gemm_f32_split_choice(int M, int N, int K, int gate) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0) return -1;
+  return split_tile(M, N, K, gate != 0);
+}
+
+// Which kernel and tile of this file a product takes (that gemm_split.hip does not): 100 kernel (0 gemm_few_f32_kernel, 1 FINE tiles,
+// 2 tiles) + 10 a + b
 extern "C" int yalm_gemm_f32_choice(int M, int N, int K, int gate) {
   if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0) return -1;
   const Choice c = choose(M, N, K, gate != 0);
@@ -435,6 +453,7 @@ int yalm_gemm_f32_mfma(const void* A, const void* W, void* C, int M, int N, int 
   if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15)) return YALM_ERR_ARG;
   const float *a = (const float*)A, *w = (const float*)W;
   float* c = (float*)C;
+  if (const int tile = split_tile(M, N, K, gated(epilogue)); tile >= 0) return yalm_gemm_split(tile, a, w, c, M, N, K, epilogue, H, stream);
   switch (epilogue) {
     case 0:
     case 1: return launch<0>(a, w, c, M, N, K, H, stream);

@@ -42,9 +42,12 @@ int yalm_gemm(const void* A, const void* W, void* C, float* workspace, long work
               int dtype, int epilogue, int H, float gate_limit, float gate_alpha, float up_shift, int force_simple,
               hipStream_t stream);
 
-// Which matrix-core kernel and tile yalm_gemm gives a float32 product with K a multiple of 32 and aligned operands (-1: none):
-// 100 kernel (0: a workgroup's waves share K, 1: tiles with finely cut sums, 2: tiles) + 10 a + b, for tests of each.
+// Which float32 matrix-core kernel and tile yalm_gemm gives a float32 product with K a multiple of 32 and aligned operands (-1:
+// none) that no kernel by bfloat16 terms takes: 100 kernel (0: a workgroup's waves share K, 1: tiles with finely cut sums, 2: tiles) +
+// 10 a + b, for tests of each.
 int yalm_gemm_f32_choice(int M, int N, int K, int gate);
+// The tile (0 to 5) of the kernel by bfloat16 terms that takes the product, or -1: none does.
+int yalm_gemm_f32_split_choice(int M, int N, int K, int gate);
 
 // Floats of workspace with which the tiled bfloat16 kernel for more than 64 rows splits K (0: it does
 // not; the output's tiles fill the chip).

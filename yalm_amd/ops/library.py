@@ -25,6 +25,7 @@ _SIGNATURES = {
     "yalm_gemm_chain": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P]),
     "yalm_gemm_chain_parts": (_I, [_I]),
     "yalm_gemm_f32_choice": (_I, [_I, _I, _I, _I]),
+    "yalm_gemm_f32_split_choice": (_I, [_I, _I, _I, _I]),
     "yalm_gemm_chain_qkv_rope": (_I, [_P, _P, _I, _F, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "yalm_rope_kv_write": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "yalm_gemm_partial": (_I, [_P, _P, _P, ctypes.c_long, _I, _I, _I, _P, _P]),
@@ -101,7 +102,7 @@ _SIGNATURES = {
     "yalm_probe_mfma": (_I, [_I, _I, _I, _P, _P, _P]),
 }
 
-ABI_VERSION = 40
+ABI_VERSION = 41
 
 
 class KernelError(RuntimeError):
