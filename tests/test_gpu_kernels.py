@@ -1597,6 +1597,67 @@ def test_gemm_norm_qkv_rope(n_heads, n_kv, hd, rd, D):
     assert (vp.float().abs().sum(dim=(1, 2)) > 0).equal(touched)
 
 
+# Rows in turn over eight waves, K of fewer k tiles than waves and of many; the sum of squares over one wave (to 1,024), over four
+# by 16 bytes (to 8,192) and element by element (beyond); one and two column tiles a workgroup
+@pytest.mark.parametrize("M,N,Kd", [(1, 40, 32), (16, 100, 96), (3, 512, 256), (9, 4100, 1024), (13, 33, 1056), (16, 4112, 4096), (2, 50, 8192),
+                                    (5, 16, 8224), (8, 17000, 2048)])
+def test_gemm_norm_float32(M, N, Kd):
+    """The norm folded into a float32 product has the bits of the norm's own kernel and the product behind it."""
+    from yalm_amd.parts.swiglu import interleave_gate_up
+    k = K()
+    x, nw = rnd((M, Kd), 120, scale=3.0).to(DEV), (1 + 0.1 * rnd((Kd,), 121)).to(DEV)
+    w = rnd((N, Kd), 122, scale=Kd ** -0.5).to(DEV)
+    assert k.can_fuse_norm(M, Kd, torch.float32, N)
+    h = k.rmsnorm(x, nw, torch.empty_like(x), 1e-5)
+    got = k.gemm_norm(x, nw, 1e-5, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32)
+    assert torch.equal(got, k.gemm(h, w, torch.empty_like(got), k.EPI_STORE_F32))
+    H = N // 2 - 3
+    gu = interleave_gate_up(w[:H], w[H:2 * H])
+    if not k.can_fuse_norm(M, Kd, torch.float32, gu.shape[0], gate=True):
+        return
+    for epi in k.GATED:
+        got = k.gemm_norm(x, nw, 1e-5, gu, torch.full((M, H), 7.0, device=DEV), epi, hidden=H)
+        assert torch.equal(got, k.gemm(h, gu, torch.empty_like(got), epi, hidden=H))
+
+
+def test_gemm_norm_float32_refuses_what_it_does_not_take():
+    k = K()
+    for M, N, Kd in ((17, 64, 64), (4, 8192, 4096), (4, 64, 48)):
+        assert not k.can_fuse_norm(M, Kd, torch.float32, N)
+        with pytest.raises(Exception):
+            k.gemm_norm(torch.zeros((M, Kd), device=DEV), torch.ones(Kd, device=DEV), 1e-5, torch.zeros((N, Kd), device=DEV),
+                        torch.empty((M, N), device=DEV), k.EPI_STORE_F32)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,rd,D", [(4, 2, 16, 16, 64), (3, 1, 48, 32, 96), (6, 3, 32, 0, 96), (32, 8, 128, 128, 256)])
+@pytest.mark.parametrize("M", [5, 11])
+def test_gemm_norm_qkv_rope_float32(n_heads, n_kv, hd, rd, D, M):
+    """norm + q/k/v + rotation + cache write of a float32 decode step in one kernel: the bits of the kernels one by one (of the
+    rotated elements up to the rounding of a fused multiply-add)."""
+    k = K()
+    pos = ([0, 63, 64, 130, 7] + list(range(190, 196)))[:M]
+    slots = ([3, 0, -1, 2, 1] + list(range(4, 10)))[:M]                    # row 2 is a padding row
+    Q, KV = n_heads * hd, n_kv * hd
+    x, nw = rnd((M, D), 57, scale=2.0).to(DEV), (1 + 0.1 * rnd((D,), 58)).to(DEV)
+    w = rnd((Q + 2 * KV, D), 59, scale=1 / math.sqrt(D)).to(DEV)
+    table = make_table(200, hd, rd, 10000.0).to(DEV) if rd else None
+    ring, n_pages = 4, 44
+    bt = torch.arange(11 * ring, dtype=torch.int32, device=DEV).reshape(11, ring)
+    pages = [torch.zeros((2, n_pages, n_kv) + s, device=DEV) for s in ((k.PAGE, hd), (hd, k.PAGE))]
+    q = torch.zeros((2, M, Q), device=DEV)
+    assert k.can_fuse_norm(M, D, torch.float32, Q + 2 * KV)
+    k.gemm_norm_qkv_rope(x, nw, 1e-5, w, q[0], pages[0][0], pages[1][0], bt, ring, i32(pos), i32(slots), table, n_heads, n_kv, hd, rd)
+    h = k.rmsnorm(x, nw, torch.empty_like(x), 1e-5)
+    qkv = k.gemm(h, w, torch.empty((M, Q + 2 * KV), device=DEV), k.EPI_STORE_F32)
+    k.rope_kv_write(qkv, q[1], None, None, None, pages[0][1], pages[1][1], bt, ring, i32(list(range(M))), i32(pos), i32(slots),
+                    i32([p + 1 for p in pos]), table, n_heads, n_kv, hd, rd)
+    assert torch.equal(pages[1][0], pages[1][1])
+    # a rotated element is x0 c - x1 s with one of its two products rounded by itself, or none: 2 roundings of at most 2^-24 of it
+    bound = 2 * 2.0 ** -24 * 2 * float(qkv.abs().max())
+    assert float((q[0] - q[1]).abs().max()) <= bound and float((pages[0][0] - pages[0][1]).abs().max()) <= bound
+    assert torch.equal(q[0] != 0, q[1] != 0) and torch.equal(pages[0][0] != 0, pages[0][1] != 0)
+
+
 @pytest.mark.parametrize("M", [1, 5, 16])
 @pytest.mark.parametrize("n_heads,n_kv,hd,rd,D", [(4, 2, 16, 16, 64), (3, 1, 48, 48, 80), (6, 3, 32, 16, 192),
                                                    (32, 8, 128, 128, 128), (24, 8, 128, 128, 64), (10, 5, 64, 64, 256)])

@@ -20,6 +20,7 @@
 // 3,072 and 1.6e-7 at K 14,336, gemm_rows_f32_kernel's 0.6e-7, 1.4e-7 and 2.8e-7).
 #include "common.h"
 #include "gemm_split.h"
+#include "rms_row.h"
 #include "yalm_hip.h"
 
 namespace {
@@ -227,14 +228,63 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
 // lines), a block's eight products are joined in a tree, and the waves' sums in a tree in LDS: at K 32 NWV, chains of 4 + 3 + 3
 // additions.  Weights and A go from memory straight into registers, the next block's while one is multiplied (two blocks ahead
 // measured the same).
+//
+// NORM (a decode step of up to 16 rows): A is the residual stream and its norm is applied on the way: the rows' sums of squares
+// first, by every workgroup (a wave a row, in the order of the norm's own kernel, so that its bits come out), then x * scale * weight
+// in front of every product.  EPI 4: the q/k/v product of a decode step, rotated and written to the pages of the cache as
+// rope_kv_write_kernel does.  A launch less each, seven of a small model's 24 a step (3 requests on two layers of 256, 16 tokens each:
+// 2,066 -> 2,016 us, which the host bounds; 12 of up to 300 and 30 tokens each 4,125 -> 3,930; a step of four 7B layers at one row
+// 922 -> 906 us, at 16 rows 1,132 -> 1,124; of 3B layers at 8 rows 929 -> 917).
 // ---------------------------------------------------------------------------
 constexpr int NWV = 8;
+constexpr int EPI_QKV = 4;
 
-template <int EPI, int MB, int NB>
+struct NormIn {
+  const float* w;                                // [K]
+  float eps;
+};
+struct QkvOut {
+  float *q_out, *k_pages, *v_pages;
+  const int *block_table, *tok_pos, *seq_slot;
+  const float2* cos_sin;
+  int table_stride, ring_pages, n_positions, n_heads, n_kv_heads, hd, rotary_dim, n_pages, page_layout;
+};
+
+// 1 / rms of row x[K], by one wave: the sum of squares as rms_row.h forms it over one or four waves
+__device__ __forceinline__ float row_scale(const float* x, int K, bool vec, float eps, int lane) {
+  float ss = 0.f;
+  if (K <= 1024) {
+    ss = wave_sum(rms_part(x, K, lane, WAVE));
+  } else {
+    float part[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int tid = p * WAVE + lane;
+      if (vec) {
+        part[p] = 0.f;
+#pragma unroll
+        for (int u = 0; u < RMS_VEC_MAX; ++u) {
+          const int i = tid + u * 256;
+          part[p] = rms_add4(part[p], i < K / 4 ? reinterpret_cast<const float4*>(x)[i] : make_float4(0.f, 0.f, 0.f, 0.f));
+        }
+      } else {
+        part[p] = rms_part(x, K, tid, 256);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) ss += wave_sum(part[p]);
+  }
+  return 1.0f / sqrtf(ss / (float)K + eps);
+}
+
+template <int EPI, int MB, int NB, bool NORM>
 __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                                    float* __restrict__ C, int M, int N, int K, GateOut H) {
+                                                                    float* __restrict__ C, int M, int N, int K, GateOut H, NormIn norm,
+                                                                    QkvOut out) {
   static_assert(!gated(EPI) || NB == 2, "a block of gate rows and its up rows");
+  static_assert((!NORM && EPI != EPI_QKV) || MB == 1, "up to 16 rows");
   __shared__ f32x4 sums[NWV][MB * NB][WAVE];
+  __shared__ float scales[16];
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int l16 = lane % 16, lq = lane / 16;
@@ -255,11 +305,13 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
     for (int b = 0; b < NB; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   const int blocks = K / TK, mine = (blocks - wave + NWV - 1) / NWV;     // this wave's: wave, wave + NWV, ...
-  f32x4 w[2][NB][2], x[2][MB][2];
+  f32x4 w[2][NB][2], x[2][MB][2], nw[2][2];
+  float scale = 1.f;
   auto load = [&](int buf, int i) {                // block i of this wave
     const size_t k = (size_t)(i * NWV + wave) * TK;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      if (NORM) nw[buf][h] = *(const f32x4*)(norm.w + k + h * 16 + lq * 4);
 #pragma unroll
       for (int b = 0; b < NB; ++b) w[buf][b][h] = __builtin_nontemporal_load((const f32x4*)(wp[b] + k + h * 16));
 #pragma unroll
@@ -267,14 +319,28 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
     }
   };
   auto multiply = [&](int buf) {
+    if (NORM)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[buf][0][h][e] = x[buf][0][h][e] * scale * nw[buf][h][e];
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
       for (int b = 0; b < NB; ++b)
         acc[a][b] += sum_of_products(x[buf][a][0], w[buf][b][0]) + sum_of_products(x[buf][a][1], w[buf][b][1]);
   };
+  if (mine > 0) load(0, 0);
+  if (NORM) {                                      // while the first weights are on their way
+    const bool vec = K <= 256 * 4 * RMS_VEC_MAX;   // (rms_row_vec: A lies on 16 bytes)
+    for (int m = wave; m < M; m += NWV) {
+      const float s = row_scale(A + (size_t)m * K, K, vec, norm.eps, lane);
+      if (lane == 0) scales[m] = s;
+    }
+    lds_barrier();
+    scale = scales[min(l16, M - 1)];
+  }
   if (mine > 0) {
-    load(0, 0);
     int i = 0;
     for (; i + 2 < mine; i += 2) {
       load(1, i + 1);
@@ -308,6 +374,34 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
         const int m = unit * 16 + row + r;
         if (m < M && hcol < H) C[(size_t)m * H + hcol] = gate_unit<EPI>(gt[r], up[r], H);
       }
+    } else if constexpr (EPI == EPI_QKV) {
+      const f32x4 v = total(unit);
+      const int n = n0 + unit * 16 + col, Q = out.n_heads * out.hd, KV = out.n_kv_heads * out.hd;
+      const int region = n < Q ? 0 : n < Q + KV ? 1 : 2, within = n - (region == 0 ? 0 : region == 1 ? Q : Q + KV);
+      const int head = within / out.hd, i = within % out.hd, pair = i >> 1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = row + r;
+        const float other = __shfl_xor(v[r], 1, WAVE);                       // the pair's other element, in the next lane
+        if (m >= M || n >= N) continue;
+        const int pos = out.tok_pos[m];
+        float y = v[r];
+        if (region < 2 && out.cos_sin != nullptr && pair < out.rotary_dim / 2 && pos >= 0 && pos < out.n_positions) {
+          const float2 c = out.cos_sin[(size_t)pos * (out.rotary_dim / 2) + pair];
+          y = (i & 1) ? other * c.y + v[r] * c.x : v[r] * c.x - other * c.y;
+        }
+        if (region == 0) {
+          out.q_out[(size_t)m * Q + n] = y;
+          continue;
+        }
+        const int slot = out.seq_slot[m];
+        if (slot < 0 || pos < 0) continue;
+        const int phys = out.block_table[(size_t)slot * out.table_stride + (pos / PAGE) % out.ring_pages];
+        if (phys < 0 || phys >= out.n_pages) continue;
+        const size_t base = ((size_t)phys * out.n_kv_heads + head) * PAGE * out.hd;
+        if (region == 1) out.k_pages[base + page_k_offset(out.page_layout, pos & (PAGE - 1), i, out.hd)] = y;
+        else out.v_pages[base + page_v_offset(out.page_layout, pos & (PAGE - 1), i, out.hd)] = y;
+      }
     } else {
       const f32x4 v = total(unit);
       const int n = n0 + (unit % NB) * 16 + col;
@@ -323,9 +417,11 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
   }
 }
 
-template <int EPI, int MB, int NB>
-int launch_few(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
-  gemm_few_f32_kernel<EPI, MB, NB><<<dim3(ceil_div(N, 16 * NB), ceil_div(M, 16 * MB)), NWV * WAVE, 0, stream>>>(A, W, C, M, N, K, H);
+template <int EPI, int MB, int NB, bool NORM = false>
+int launch_few(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream, NormIn norm = {},
+               QkvOut out = {}) {
+  gemm_few_f32_kernel<EPI, MB, NB, NORM>
+      <<<dim3(ceil_div(N, 16 * NB), ceil_div(M, 16 * MB)), NWV * WAVE, 0, stream>>>(A, W, C, M, N, K, H, norm, out);
   return launch_status();
 }
 
@@ -404,6 +500,17 @@ int split_tile(int M, int N, int K, bool gate) {
   return c.kernel == Choice::COARSE ? yalm_gemm_split_choose(M, N, K, gate, 5.0 + 1.1 * tile_time(M, N, K, c.a, c.b)) : -1;
 }
 
+// A norm is folded into the products of gemm_few_f32_kernel of up to 16 rows
+bool takes_norm(int M, int N, int K, bool gate) {
+  return M >= 1 && M <= 16 && N > 0 && K > 0 && K % TK == 0 && choose(M, N, K, gate).kernel == Choice::FEW;
+}
+template <int EPI>
+int launch_norm(const float* x, const float* W, float* C, int M, int N, int K, GateOut H, NormIn norm, QkvOut out, hipStream_t stream) {
+  if constexpr (gated(EPI)) return launch_few<EPI, 1, 2, true>(x, W, C, M, N, K, H, stream, norm, out);
+  else if (choose(M, N, K, false).b == 2) return launch_few<EPI, 1, 2, true>(x, W, C, M, N, K, H, stream, norm, out);
+  else return launch_few<EPI, 1, 1, true>(x, W, C, M, N, K, H, stream, norm, out);
+}
+
 template <int EPI>
 int launch(const float* A, const float* W, float* C, int M, int N, int K, GateOut H, hipStream_t stream) {
   const Choice c = choose(M, N, K, gated(EPI));
@@ -446,6 +553,44 @@ extern "C" int yalm_gemm_f32_choice(int M, int N, int K, int gate) {
   if (M <= 0 || N <= 0 || K <= 0 || K % TK != 0) return -1;
   const Choice c = choose(M, N, K, gate != 0);
   return 100 * c.kernel + 10 * c.a + c.b;
+}
+
+// Whether yalm_gemm_norm_f32 (and the q/k/v form) takes the product
+extern "C" int yalm_gemm_norm_f32_takes(int M, int N, int K, int gate) { return takes_norm(M, N, K, gate != 0); }
+
+static bool norm_operands_ok(const float* x, const float* norm_w, const float* W) {
+  return x != nullptr && norm_w != nullptr && W != nullptr && !((uintptr_t)x & 15) && !((uintptr_t)norm_w & 15) && !((uintptr_t)W & 15);
+}
+
+// yalm_gemm_norm with float32 weights and results: C = epilogue(rmsnorm(x, norm_w, eps) W^T), epilogue 0 or a gated one
+extern "C" int yalm_gemm_norm_f32(const float* x, const float* norm_w, float eps, const float* W, float* C, int M, int N, int K, int epilogue,
+                                  int hidden, hipStream_t stream) {
+  if (!takes_norm(M, N, K, gated(epilogue)) || !norm_operands_ok(x, norm_w, W) || C == nullptr) return YALM_ERR_ARG;
+  const GateOut H(hidden);
+  const NormIn norm = {norm_w, eps};
+  if (gated(epilogue) && (hidden <= 0 || N != 32 * ((hidden + 15) / 16))) return YALM_ERR_ARG;
+  switch (epilogue) {
+    case 0: return launch_norm<0>(x, W, C, M, N, K, H, norm, QkvOut{}, stream);
+    case 3: return launch_norm<3>(x, W, C, M, N, K, H, norm, QkvOut{}, stream);
+    case 5: return launch_norm<5>(x, W, C, M, N, K, H, norm, QkvOut{}, stream);
+  }
+  return YALM_ERR_ARG;
+}
+
+// yalm_gemm_norm_qkv_rope with everything in float32
+extern "C" int yalm_gemm_norm_qkv_rope_f32(const float* x, const float* norm_w, float eps, const float* Wqkv, float* q_out, float* k_pages,
+                                           float* v_pages, const int* block_table, int table_stride, int ring_pages, const int* tok_pos,
+                                           const int* seq_slot, const float* cos_sin, int n_positions, int M, int K, int n_heads,
+                                           int n_kv_heads, int head_dim, int rotary_dim, int n_pages, int page_layout, hipStream_t stream) {
+  const int N = (n_heads + 2 * n_kv_heads) * head_dim;
+  if (head_dim <= 0 || head_dim % 16 != 0 || rotary_dim < 0 || (rotary_dim & 1) || rotary_dim > head_dim || n_heads <= 0 || n_kv_heads <= 0 ||
+      ring_pages <= 0 || n_pages <= 0 || !page_layout_ok(page_layout, head_dim) || block_table == nullptr || tok_pos == nullptr ||
+      seq_slot == nullptr || q_out == nullptr || k_pages == nullptr || v_pages == nullptr)
+    return YALM_ERR_ARG;
+  if (!takes_norm(M, N, K, false) || !norm_operands_ok(x, norm_w, Wqkv)) return YALM_ERR_ARG;
+  const QkvOut out = {q_out, k_pages, v_pages, block_table, tok_pos, seq_slot, (const float2*)cos_sin, table_stride, ring_pages, n_positions,
+                      n_heads, n_kv_heads, head_dim, rotary_dim, n_pages, page_layout};
+  return launch_norm<EPI_QKV>(x, Wqkv, nullptr, M, N, K, GateOut(0), NormIn{norm_w, eps}, out, stream);
 }
 
 // K a multiple of 32 and 16-byte aligned operands; YALM_ERR_ARG: not taken.

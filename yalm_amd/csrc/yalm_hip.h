@@ -67,6 +67,16 @@ int yalm_gemm_norm_qkv_rope(const float* x, const float* norm_w, float eps, cons
                             int K, int n_heads, int n_kv_heads, int head_dim, int rotary_dim, int n_pages,
                             int page_layout, hipStream_t stream);
 
+// The same two with float32 weights and results, M <= 16 rows and K a multiple of 32, where yalm_gemm_norm_f32_takes the product
+// (narrow ones: N below 8,192 or K up to 2,048).  The bits are those of yalm_rmsnorm and yalm_gemm.
+int yalm_gemm_norm_f32_takes(int M, int N, int K, int gate);
+int yalm_gemm_norm_f32(const float* x, const float* norm_w, float eps, const float* W, float* C, int M, int N, int K, int epilogue,
+                       int H, hipStream_t stream);
+int yalm_gemm_norm_qkv_rope_f32(const float* x, const float* norm_w, float eps, const float* Wqkv, float* q_out, float* k_pages,
+                                float* v_pages, const int* block_table, int table_stride, int ring_pages, const int* tok_pos,
+                                const int* seq_slot, const float* cos_sin, int n_positions, int M, int K, int n_heads,
+                                int n_kv_heads, int head_dim, int rotary_dim, int n_pages, int page_layout, hipStream_t stream);
+
 // The K slices of A[M,K] * W[N,K]^T for 17..64 rows, or more with K a multiple of 64 (bfloat16), left unadded:
 // workspace [*slices][M][N] float32, for a consumer that adds them itself (yalm_rope_kv_write).  Needs at least
 // M * N floats; refuses (YALM_ERR_ARG) other shapes.

@@ -188,31 +188,36 @@ def gemm(a, w, out, epilogue, hidden=0, workspace=None, scale_from=None, unit=No
 FUSED_NORM_MAX_ROWS = 8
 
 
-def can_fuse_norm(M, K, dtype):
-    """Whether gemm_norm / gemm_norm_qkv_rope take this shape (else: rmsnorm, then gemm)."""
+def can_fuse_norm(M, K, dtype, N, gate=False):
+    """Whether gemm_norm / gemm_norm_qkv_rope take this shape (else: rmsnorm, then gemm); N: the weight's rows, gate: whether the
+    epilogue is a gated one."""
+    if dtype == torch.float32:
+        return not FORCE_SIMPLE and bool(library.lib().yalm_gemm_norm_f32_takes(int(M), int(N), int(K), 1 if gate else 0))
     return dtype == torch.bfloat16 and 1 <= M <= FUSED_NORM_MAX_ROWS and K % 8 == 0 and \
         M * (K + 8) * 2 <= 72 * 1024 and not FORCE_SIMPLE
 
 
 def gemm_norm(x, norm_w, eps, w, out, epilogue, hidden=0):
     """out = epilogue(rmsnorm(x, norm_w, eps) @ w^T) for at most 16 rows of the float32
-    residual stream x; w bfloat16 [N, K], norm_w float32 [K]; EPI_STORE_F32, EPI_GATED or EPI_GATED_GELU.
+    residual stream x; w bfloat16 or float32 [N, K], norm_w float32 [K]; EPI_STORE_F32, EPI_GATED or EPI_GATED_GELU (out in w's dtype).
     (Shapes: see can_fuse_norm.)"""
     M, K = x.shape
     N = w.shape[0]
+    if w.dtype not in (torch.bfloat16, torch.float32):
+        raise TypeError("gemm_norm: weights in %s" % (w.dtype,))
     p_x = _need(x, "x", torch.float32, (M, K))
     p_n = _need(norm_w, "norm_w", torch.float32, (K,))
-    p_w = _need(w, "w", torch.bfloat16, (N, K))
+    p_w = _need(w, "w", w.dtype, (N, K))
     if epilogue in GATED:
         if hidden <= 0 or N != 32 * ((hidden + 15) // 16):
             raise ValueError("gated gemm: weight rows %d do not match hidden %d" % (N, hidden))
-        p_o = _need(out, "out", torch.bfloat16, (M, hidden))
+        p_o = _need(out, "out", w.dtype, (M, hidden))
     elif epilogue == EPI_STORE_F32:
         p_o = _need(out, "out", torch.float32, (M, N))
     else:
         raise ValueError("gemm_norm: epilogue %r is not offered" % (epilogue,))
-    library.check(library.lib().yalm_gemm_norm(p_x, p_n, float(eps), p_w, p_o, M, N, K, epilogue, hidden, _stream()),
-                  "gemm_norm")
+    entry = library.lib().yalm_gemm_norm_f32 if w.dtype == torch.float32 else library.lib().yalm_gemm_norm
+    library.check(entry(p_x, p_n, float(eps), p_w, p_o, M, N, K, epilogue, hidden, _stream()), "gemm_norm")
     return out
 
 
@@ -238,7 +243,7 @@ def _layout(layout, head_dim):
 def gemm_norm_qkv_rope(x, norm_w, eps, wqkv, q_out, k_pages, v_pages, block_table, ring_pages, tok_pos, seq_slot,
                        cos_sin, n_heads, n_kv_heads, head_dim, rotary_dim, layout=None):
     """A decode step's rmsnorm + q/k/v projection + rotation + cache write in one kernel
-    (row m is sequence m; see rope_kv_write for the operands)."""
+    (row m is sequence m; see rope_kv_write for the operands), in wqkv's dtype."""
     _check_heads(n_heads, n_kv_heads, head_dim)
     if head_dim % 16:
         raise ValueError("gemm_norm_qkv_rope needs a head_dim that is a multiple of 16")
@@ -246,11 +251,14 @@ def gemm_norm_qkv_rope(x, norm_w, eps, wqkv, q_out, k_pages, v_pages, block_tabl
     Q, KV = n_heads * head_dim, n_kv_heads * head_dim
     p_x = _need(x, "x", torch.float32, (M, K))
     p_n = _need(norm_w, "norm_w", torch.float32, (K,))
-    p_w = _need(wqkv, "wqkv", torch.bfloat16, (Q + 2 * KV, K))
-    p_q = _need(q_out, "q_out", torch.bfloat16, (M, Q))
+    dt = wqkv.dtype
+    if dt not in (torch.bfloat16, torch.float32):
+        raise TypeError("gemm_norm_qkv_rope: weights in %s" % (dt,))
+    p_w = _need(wqkv, "wqkv", dt, (Q + 2 * KV, K))
+    p_q = _need(q_out, "q_out", dt, (M, Q))
     n_pages = k_pages.shape[0]
-    p_kp = _need(k_pages, "k_pages", torch.bfloat16, (n_pages, n_kv_heads, PAGE, head_dim))
-    p_vp = _need(v_pages, "v_pages", torch.bfloat16, (n_pages, n_kv_heads, head_dim, PAGE))
+    p_kp = _need(k_pages, "k_pages", dt, (n_pages, n_kv_heads, PAGE, head_dim))
+    p_vp = _need(v_pages, "v_pages", dt, (n_pages, n_kv_heads, head_dim, PAGE))
     p_bt = _need(block_table, "block_table", torch.int32, (None, None))
     stride = block_table.shape[1]
     if ring_pages <= 0 or ring_pages > stride:
@@ -263,7 +271,8 @@ def gemm_norm_qkv_rope(x, norm_w, eps, wqkv, q_out, k_pages, v_pages, block_tabl
         p_cs = _need(cos_sin, "cos_sin", torch.float32, (n_pos, rotary_dim // 2, 2))
     else:
         rotary_dim = 0
-    library.check(library.lib().yalm_gemm_norm_qkv_rope(
+    entry = library.lib().yalm_gemm_norm_qkv_rope_f32 if dt == torch.float32 else library.lib().yalm_gemm_norm_qkv_rope
+    library.check(entry(
         p_x, p_n, float(eps), p_w, p_q, p_kp, p_vp, p_bt, stride, ring_pages, p_tp, p_ss, p_cs, n_pos, M, K, n_heads,
         n_kv_heads, head_dim, rotary_dim, n_pages, _layout(layout, head_dim), _stream()), "gemm_norm_qkv_rope")
 

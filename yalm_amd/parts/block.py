@@ -84,8 +84,9 @@ class PreNormResidualBlock(Part):
                 plain_end = True
         # sublayers that fold no norm into their products leave nothing for whoever reads the stream next: in a decode
         # step the layer then ends with that norm as a kernel of its own, so that the head's product (or the next
-        # layer's first) takes its output as it is instead of norming the rows again for every tile of its weights
-        if plain_end and ctx.mode == "decode" and next_norm is not None and hasattr(next_norm, "fused") \
+        # layer's first) takes its output as it is instead of norming the rows again for every tile of its weights (in float32
+        # a consumer that cannot fold the norm in runs it itself, and one that can saves the launch)
+        if plain_end and ctx.mode == "decode" and ctx.act_dtype != x.dtype and next_norm is not None and hasattr(next_norm, "fused") \
                 and id(next_norm) not in ctx.normed:
             ahead = ctx.ws.get("block.ahead", (x.shape[0], self.dim), ctx.act_dtype)
             next_norm.forward(x, ahead, ctx)
