@@ -130,6 +130,33 @@ def test_middle_of_a_gated_feed_forward_with_biases(T, F, D, kind, dtype):
     assert torch.allclose(out2.float().cpu().to(F64), act0 * z.to(F64)[:, F:], rtol=tol, atol=tol)
 
 
+# The same with the middle in the first product's epilogue: one to 16 rows (K a multiple of 64 and not), to 128, tiles of 128 rows,
+# larger tiles, K in slices and whole; hidden values that end inside a block; streams narrower and wider than what one
+# element a thread covers; and the general kernels
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,F,D,Kd", [(1, 16, 16, 64), (5, 112, 48, 72), (16, 4096, 1024, 64), (9, 48, 48, 192), (17, 112, 16, 256), (33, 272, 80, 1024),
+                                      (64, 64, 64, 72), (100, 320, 208, 128), (130, 256, 96, 512), (200, 3584, 1024, 64), (300, 208, 112, 1024),
+                                      (257, 64, 32, 40), (3, 64, 32, 30), (2, 40, 1000, 64),
+                                      (16, 24, 4099, 128), (70, 33, 51, 192), (161, 1000, 72, 576)])
+def test_middle_of_a_gated_feed_forward_in_its_product(T, F, D, Kd, dtype):
+    from yalm_amd.ops import kernels
+    from yalm_amd.parts.swiglu import interleave_gate_up
+    h = randn(T, Kd, seed=1).to(dtype)
+    w = [randn(F, Kd, seed=s, scale=Kd ** -0.5).to(dtype) for s in (2, 3)]
+    b = [randn(F, seed=s) for s in (4, 5)]
+    x, xb = randn(T, D, seed=6), randn(D, seed=7)
+    out, xg = torch.full((T, F), float("nan"), dtype=dtype, device=DEV), x.to(DEV)
+    wg, bg = interleave_gate_up(*w).to(DEV), interleave_gate_up(b[0][:, None], b[1][:, None]).reshape(-1).contiguous().to(DEV)
+    n = kernels.gemm_workspace_floats(T, 2 * F, Kd) if dtype == torch.bfloat16 else 0
+    kernels.gemm_gated_bias(h.to(DEV), wg, bg, out, xg, xb.to(DEV), workspace=torch.empty(n, device=DEV) if n else None)
+    g, u = (h.to(F64) @ v.to(F64).t() + c.to(F64) for v, c in zip(w, b))
+    want = P.gelu_tanh(g) * u
+    # sums of products of size one: 2^-24 sqrt(K) and less, times slopes and factors of up to 6; the result's rounding
+    tol = 2e-5 if dtype == torch.float32 else 1e-2
+    assert torch.allclose(out.float().cpu().to(F64), want, rtol=tol, atol=tol)
+    assert torch.equal(xg.cpu(), x + xb)                              # every element of the stream once
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,H,dv,pad", [(1, 1, 4, 16), (6, 3, 20, 32), (3, 8, 64, 64), (2, 40, 100, 112)])
 def test_sigmoid_gate_on_the_heads(T, H, dv, pad, dtype):

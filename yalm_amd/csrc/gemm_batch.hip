@@ -82,7 +82,7 @@ __device__ __forceinline__ void store_tile(void* Cv, const f32x4& v, const f32x4
     int m = m_base + r;
     if (m >= M) continue;
     if (gated(EPI)) {
-      if (hcol < H) ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_unit<EPI>(v[r], u[r], H));
+      if (hcol < H) ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(v[r], u[r], H, gate_bias<EPI>(H, hcol)));
     } else if (n < N) {
       size_t o = (size_t)m * N + n;
       if (EPI == 0) ((float*)Cv)[o] = v[r];
@@ -403,7 +403,7 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ partial, void* __
     const float gv[4] = {g.x, g.y, g.z, g.w}, uv[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (c4 + e < H) C[c4 + e] = static_cast<bf16>(gate_unit<EPI>(gv[e], uv[e], H));
+      if (c4 + e < H) C[c4 + e] = static_cast<bf16>(gate_value<EPI>(gv[e], uv[e], H, gate_bias<EPI>(H, c4 + e)));
   } else {
     float v[4] = {0.f, 0.f, 0.f, 0.f};
     const float* p = partial + (size_t)m * N + c4;
@@ -779,6 +779,7 @@ static int gemm_batch_scaled(const void* A, const void* W, void* C, float* works
     case 2: return dispatch<2>(a, w, C, workspace, workspace_floats, M, N, K, H, rs, stream);
     case 3: return dispatch<3>(a, w, C, workspace, workspace_floats, M, N, K, H, rs, stream);
     case 5: return dispatch<5>(a, w, C, workspace, workspace_floats, M, N, K, H, rs, stream);
+    case 6: return dispatch<6>(a, w, C, workspace, workspace_floats, M, N, K, H, rs, stream);
   }
   return YALM_ERR_ARG;
 }
@@ -794,7 +795,7 @@ extern "C" int yalm_gemm_scaled(const void* A, const void* W, void* C, float* wo
                                 int N, int K, int epilogue, int hidden, const float* ss, int n_parts, float eps,
                                 hipStream_t stream) {
   const GateOut H(hidden);
-  if (ss == nullptr) return YALM_ERR_ARG;
+  if (ss == nullptr || epilogue == EPI_GATED_BIAS) return YALM_ERR_ARG;
   if (gated(epilogue) && (H <= 0 || N != 32 * ((H + 15) / 16))) return YALM_ERR_ARG;
   return gemm_batch_scaled(A, W, C, workspace, workspace_floats, M, N, K, epilogue, H, ss, n_parts, eps, stream);
 }
@@ -891,6 +892,7 @@ int yalm_splitk_reduce(const float* partial, void* C, int M, int N, GateOut H, i
     case 2: splitk_reduce_kernel<2><<<blocks, 256, 0, stream>>>(partial, C, M, N, H, slices); break;
     case 3: splitk_reduce_kernel<3><<<blocks, 256, 0, stream>>>(partial, C, M, N, H, slices); break;
     case 5: splitk_reduce_kernel<5><<<blocks, 256, 0, stream>>>(partial, C, M, N, H, slices); break;
+    case 6: splitk_reduce_kernel<6><<<blocks, 256, 0, stream>>>(partial, C, M, N, H, slices); break;
     default: return YALM_ERR_ARG;
   }
   return launch_status();

@@ -168,6 +168,10 @@ __global__ __launch_bounds__(NWM * NWN * WAVE, MINW) void gemm_dma_kernel(const 
       }
     return;
   }
+GateBias gb[FB / 2 + 1];
+  if (EPI == EPI_GATED_BIAS)
+#pragma unroll
+    for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN + pp * 64) / 2 + li);
 #pragma unroll
   for (int a = 0; a < FA; ++a) {
 #pragma unroll
@@ -179,7 +183,7 @@ __global__ __launch_bounds__(NWM * NWN * WAVE, MINW) void gemm_dma_kernel(const 
         for (int pp = 0; pp < FB / 2; ++pp) {
           const int hcol = (n0 + wn * WN + pp * 64) / 2 + li;
           if (hcol < H)
-            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_unit<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H));
+            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H, gb[pp]));
         }
       } else {
 #pragma unroll
@@ -427,6 +431,10 @@ __global__ __launch_bounds__(512, 1) void gemm_ring_kernel(const bf16* __restric
       }
     return;
   }
+GateBias gb[FB / 2 + 1];
+  if (EPI == EPI_GATED_BIAS)
+#pragma unroll
+    for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN + pp * 64) / 2 + li);
 #pragma unroll
   for (int a = 0; a < FA; ++a) {
 #pragma unroll
@@ -438,7 +446,7 @@ __global__ __launch_bounds__(512, 1) void gemm_ring_kernel(const bf16* __restric
         for (int pp = 0; pp < FB / 2; ++pp) {
           const int hcol = (n0 + wn * WN + pp * 64) / 2 + li;
           if (hcol < H)
-            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_unit<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H));
+            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H, gb[pp]));
         }
       } else {
 #pragma unroll
@@ -651,6 +659,10 @@ __global__ __launch_bounds__(512, 1) void gemm_ring16_kernel(const bf16* __restr
       }
     return;
   }
+GateBias gb[FB / 2 + 1];
+  if (EPI == EPI_GATED_BIAS)
+#pragma unroll
+    for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN) / 2 + pp * 16 + l16);
 #pragma unroll
   for (int a = 0; a < FA; ++a) {
 #pragma unroll
@@ -662,7 +674,7 @@ __global__ __launch_bounds__(512, 1) void gemm_ring16_kernel(const bf16* __restr
         for (int pp = 0; pp < FB / 2; ++pp) {
           const int hcol = (n0 + wn * WN) / 2 + pp * 16 + l16;
           if (hcol < H)
-            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_unit<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H));
+            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H, gb[pp]));
         }
       } else {
 #pragma unroll
@@ -865,6 +877,7 @@ int yalm_gemm_bf16_dma(const void* A, const void* W, void* C, float* workspace, 
     case 2: return launch<2>(a, w, C, workspace, workspace_floats, M, N, K, H, stream);
     case 3: return launch<3>(a, w, C, workspace, workspace_floats, M, N, K, H, stream);
     case 5: return launch<5>(a, w, C, workspace, workspace_floats, M, N, K, H, stream);
+    case 6: return launch<6>(a, w, C, workspace, workspace_floats, M, N, K, H, stream);
   }
   return YALM_ERR_ARG;
 }

@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
 #pragma unroll
         for (int p = 0; p < FB / 2; ++p) {
           const int hcol = (n0 + wn * (TN / 2)) / 2 + p * 16 + l16;
-          if (hcol < H) C[(size_t)m * H + hcol] = gate_unit<EPI>(total[a][2 * p][r], total[a][2 * p + 1][r], H);
+          if (hcol < H) C[(size_t)m * H + hcol] = gate_value<EPI>(total[a][2 * p][r], total[a][2 * p + 1][r], H, gate_bias<EPI>(H, hcol));
         }
       } else {
 #pragma unroll
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = unit * 16 + row + r;
-        if (m < M && hcol < H) C[(size_t)m * H + hcol] = gate_unit<EPI>(gt[r], up[r], H);
+        if (m < M && hcol < H) C[(size_t)m * H + hcol] = gate_value<EPI>(gt[r], up[r], H, gate_bias<EPI>(H, hcol));
       }
     } else if constexpr (EPI == EPI_QKV) {
       const f32x4 v = total(unit);
@@ -605,6 +605,7 @@ int yalm_gemm_f32_mfma(const void* A, const void* W, void* C, int M, int N, int 
     case 2: return launch<2>(a, w, c, M, N, K, H, stream);
     case 3: return launch<3>(a, w, c, M, N, K, H, stream);
     case 5: return launch<5>(a, w, c, M, N, K, H, stream);
+    case 6: return launch<6>(a, w, c, M, N, K, H, stream);
   }
   return YALM_ERR_ARG;
 }

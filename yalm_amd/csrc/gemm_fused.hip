@@ -237,7 +237,7 @@ extern "C" int yalm_gemm_norm(const float* x, const float* norm_w, float eps, co
   if (!shape_ok(x, norm_w, W, M, N, K)) return YALM_ERR_ARG;
   RopeArgs ra = {};
   if (epilogue == EPI_F32) return launch_norm<EPI_F32>(x, norm_w, eps, (const bf16*)W, C, M, N, K, H, ra, stream);
-  if (gated(epilogue)) {
+  if (gated(epilogue) && epilogue != EPI_GATED_BIAS) {
     if (H <= 0 || N != 32 * ((H + 15) / 16)) return YALM_ERR_ARG;
     if (epilogue == EPI_GATED_GELU)
       return launch_norm<EPI_GATED_GELU>(x, norm_w, eps, (const bf16*)W, C, M, N, K, H, ra, stream);
@@ -304,7 +304,7 @@ extern "C" int yalm_gemm_chain(const void* X, const void* W, void* C, int M, int
   }
   if (emit_nw != nullptr) return YALM_ERR_ARG;
   if (epilogue == EPI_F32) return skinny::launch<EPI_F32>(x, w, C, M, N, K, H, ca, stream);
-  if (gated(epilogue)) {
+  if (gated(epilogue) && epilogue != EPI_GATED_BIAS) {
     if (H <= 0 || N != 32 * ((H + 15) / 16)) return YALM_ERR_ARG;
     if (epilogue == EPI_GATED_GELU) return skinny::launch<EPI_GATED_GELU>(x, w, C, M, N, K, H, ca, stream);
     return skinny::launch<EPI_GATED>(x, w, C, M, N, K, H, ca, stream);

@@ -151,7 +151,7 @@ __global__ __launch_bounds__(NWM * NWN * WAVE, MINW) void gemm_tiled_kernel(cons
           int hcol = (n0 + wn * WN + pp * 64) / 2 + li;
           if (hcol < H)
             ((bf16*)Cv)[(size_t)m * H + hcol] =
-                static_cast<bf16>(gate_unit<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H));
+                static_cast<bf16>(gate_value<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H, gate_bias<EPI>(H, hcol)));
         }
       } else {
 #pragma unroll
@@ -208,6 +208,7 @@ int yalm_gemm_bf16_mfma(const void* A, const void* W, void* C, float* workspace,
       case 2: return skinny_dispatch<2>(a, w, C, M, N, K, H, stream);
       case 3: return skinny_dispatch<3>(a, w, C, M, N, K, H, stream);
       case 5: return skinny_dispatch<5>(a, w, C, M, N, K, H, stream);
+      case 6: return skinny_dispatch<6>(a, w, C, M, N, K, H, stream);
     }
     return YALM_ERR_ARG;
   }
@@ -221,6 +222,7 @@ int yalm_gemm_bf16_mfma(const void* A, const void* W, void* C, float* workspace,
     case 2: return tiled_launch<2>(a, w, C, M, N, K, H, stream);
     case 3: return tiled_launch<3>(a, w, C, M, N, K, H, stream);
     case 5: return tiled_launch<5>(a, w, C, M, N, K, H, stream);
+    case 6: return tiled_launch<6>(a, w, C, M, N, K, H, stream);
   }
   return YALM_ERR_ARG;
 }

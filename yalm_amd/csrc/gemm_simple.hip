@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(const T* __restrict__ 
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         int hcol = (n0 / 32 + jj) * 16 + tx;
-        if (hcol < H) C[(size_t)m * H + hcol] = from_f32<T>(gate_unit<EPI>(acc[i][2 * jj], acc[i][2 * jj + 1], H));
+        if (hcol < H) C[(size_t)m * H + hcol] = from_f32<T>(gate_value<EPI>(acc[i][2 * jj], acc[i][2 * jj + 1], H, gate_bias<EPI>(H, hcol)));
       }
     } else {
 #pragma unroll
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(gated(EPI) ? 512 : 256) void gemm_rows_f32_kernel(c
     for (int e = tid; e < 16 * MB; e += NWV * WAVE) {
       const int j = e % 16, m = e / 16, hcol = base + j;
       if (m < M && hcol < H)
-        ((float*)Cv)[(size_t)m * H + hcol] = gate_unit<EPI>(sums[j][m], sums[16 + j][m], H);
+        ((float*)Cv)[(size_t)m * H + hcol] = gate_value<EPI>(sums[j][m], sums[16 + j][m], H, gate_bias<EPI>(H, hcol));
     }
   } else {
     const int nb = blockIdx.x * NWV * 4;
@@ -197,6 +197,7 @@ int launch_rows_f32(const float* A, const float* W, void* C, int M, int N, int K
     case 2: gemm_rows_f32_kernel<MB, 2><<<ceil_div(N, 16), 256, 0, stream>>>(A, W, C, M, N, K, H); break;
     case 3: gemm_rows_f32_kernel<MB, 3><<<ceil_div(N, 32), 512, 0, stream>>>(A, W, C, M, N, K, H); break;
     case 5: gemm_rows_f32_kernel<MB, 5><<<ceil_div(N, 32), 512, 0, stream>>>(A, W, C, M, N, K, H); break;
+    case 6: gemm_rows_f32_kernel<MB, 6><<<ceil_div(N, 32), 512, 0, stream>>>(A, W, C, M, N, K, H); break;
     default: return YALM_ERR_ARG;
   }
   return launch_status();
@@ -221,6 +222,21 @@ int gemm_rows_f32(const void* A, const void* W, void* C, int M, int N, int K, in
   return YALM_OK;
 }
 
+// x[m, :] += b (dim a multiple of 4 and both on 16 bytes: four elements a thread)
+__global__ __launch_bounds__(256) void row_bias_kernel(float* __restrict__ x, const float* __restrict__ b, long n, int dim) {
+  const long stride = (long)gridDim.x * 256, first = (long)blockIdx.x * 256 + threadIdx.x;
+  if (dim % 4 == 0) {
+    for (long i = first; i < n / 4; i += stride) {
+      float4 v = reinterpret_cast<float4*>(x)[i];
+      const float4 w = reinterpret_cast<const float4*>(b)[i % (dim / 4)];
+      v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
+      reinterpret_cast<float4*>(x)[i] = v;
+    }
+  } else {
+    for (long i = first; i < n; i += stride) x[i] += b[i % dim];
+  }
+}
+
 template <typename T>
 int gemm_simple(const void* A, const void* W, void* C, int M, int N, int K, int epilogue, GateOut H, hipStream_t stream) {
   dim3 grid(ceil_div(N, BN), ceil_div(M, BM));
@@ -232,18 +248,17 @@ int gemm_simple(const void* A, const void* W, void* C, int M, int N, int K, int 
     case 2: gemm_simple_kernel<T, 2><<<grid, 256, 0, stream>>>(a, w, C, M, N, K, H); break;
     case 3: gemm_simple_kernel<T, 3><<<grid, 256, 0, stream>>>(a, w, C, M, N, K, H); break;
     case 5: gemm_simple_kernel<T, 5><<<grid, 256, 0, stream>>>(a, w, C, M, N, K, H); break;
+    case 6: gemm_simple_kernel<T, 6><<<grid, 256, 0, stream>>>(a, w, C, M, N, K, H); break;
     default: return YALM_ERR_ARG;
   }
   return launch_status();
 }
 }  // namespace
 
-extern "C" int yalm_gemm(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N,
-                         int K, int dtype, int epilogue, int hidden, float gate_limit, float gate_alpha, float up_shift,
-                         int force_simple, hipStream_t stream) {
-  const GateOut H(hidden, gate_limit, gate_alpha, up_shift);
+static int gemm_any(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N, int K, int dtype,
+                    int epilogue, const GateOut& H, int force_simple, hipStream_t stream) {
   if (M <= 0) return YALM_OK;
-  if (N <= 0 || K <= 0 || epilogue < 0 || (epilogue > 3 && epilogue != EPI_GATED_GELU)) return YALM_ERR_ARG;
+  if (N <= 0 || K <= 0) return YALM_ERR_ARG;
   if (gated(epilogue) && (H <= 0 || N != 32 * ((H + 15) / 16))) return YALM_ERR_ARG;
   if (dtype == YALM_F32) {
     if (!force_simple) {
@@ -260,4 +275,35 @@ extern "C" int yalm_gemm(const void* A, const void* W, void* C, float* workspace
     if (rc != YALM_ERR_ARG) return rc;
   }
   return gemm_simple<bf16>(A, W, C, M, N, K, epilogue, H, stream);
+}
+
+extern "C" int yalm_gemm(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N,
+                         int K, int dtype, int epilogue, int hidden, float gate_limit, float gate_alpha, float up_shift,
+                         int force_simple, hipStream_t stream) {
+  if (epilogue < 0 || (epilogue > 3 && epilogue != EPI_GATED_GELU)) return M <= 0 ? YALM_OK : YALM_ERR_ARG;
+  return gemm_any(A, W, C, workspace, workspace_floats, M, N, K, dtype, epilogue, GateOut(hidden, gate_limit, gate_alpha, up_shift),
+                  force_simple, stream);
+}
+
+// The gated product with biases: C = gelu(gate + bias) (up + bias), and x += x_bias
+extern "C" int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N, int K,
+                                    int dtype, int hidden, const float* bias, float* x, const float* x_bias, int dim, int force_simple,
+                                    hipStream_t stream) {
+  if (bias == nullptr || x == nullptr || x_bias == nullptr || dim <= 0 || hidden <= 0 || ((uintptr_t)x & 15) || ((uintptr_t)x_bias & 15))
+    return YALM_ERR_ARG;
+  if (M <= 0) return YALM_OK;
+  GateOut H(hidden);
+  H.bias = bias;
+  // A decode step's kernel (gemm_skinny_kernel) adds the stream's bias; with more rows a launch of its own is worth less than what
+  // the tiles' epilogues would take longer (1,909 rows, 4,096 of 14,336 columns: 74 us more for 12).
+  if (dtype == YALM_BF16 && M <= 16 && K % 8 == 0 && !force_simple && !((uintptr_t)A & 15) && !((uintptr_t)W & 15)) {
+    H.x = x;
+    H.x_bias = x_bias;
+    H.dim = dim;
+  } else {
+    const long n = (long)M * dim;
+    row_bias_kernel<<<(int)min((n + 1023) / 1024, 65535L), 256, 0, stream>>>(x, x_bias, n, dim);
+    if (int rc = launch_status(); rc != YALM_OK) return rc;
+  }
+  return gemm_any(A, W, C, workspace, workspace_floats, M, N, K, dtype, EPI_GATED_BIAS, H, force_simple, stream);
 }

@@ -272,7 +272,7 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
 #pragma unroll
         for (int p = 0; p < FB / 2; ++p) {
           const int hcol = (n0 + wn * 16 * FB) / 2 + p * 16 + l16;
-          if (hcol < H) C[(size_t)m * H + hcol] = gate_unit<EPI>(total[a][2 * p][r], total[a][2 * p + 1][r], H);
+          if (hcol < H) C[(size_t)m * H + hcol] = gate_value<EPI>(total[a][2 * p][r], total[a][2 * p + 1][r], H, gate_bias<EPI>(H, hcol));
         }
       } else {
 #pragma unroll
@@ -354,6 +354,7 @@ int yalm_gemm_split(int tile, const float* A, const float* W, float* C, int M, i
     case 2: return launch<2>(tile, A, W, C, M, N, K, H, stream);
     case 3: return launch<3>(tile, A, W, C, M, N, K, H, stream);
     case 5: return launch<5>(tile, A, W, C, M, N, K, H, stream);
+    case 6: return launch<6>(tile, A, W, C, M, N, K, H, stream);
   }
   return YALM_ERR_ARG;
 }

@@ -150,6 +150,19 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
     }
   }
 
+  // so are the first gated tile's biases, and the elements of the stream that this thread adds a bias to (EPI_GATED_BIAS)
+  GateBias gb = {0.f, 0.f};
+  float stream = 0.f, stream_bias = 0.f;
+  const long stream_n = EPI == EPI_GATED_BIAS && H.x != nullptr ? (long)M * H.dim : 0;
+  const long stream_at = (long)blockIdx.x * (NWAVES * WAVE) + threadIdx.x, stream_step = (long)gridDim.x * (NWAVES * WAVE);
+  if (EPI == EPI_GATED_BIAS) {
+    if (wave < MT * (NT / 2)) gb = gate_bias<EPI>(H, (n0 / 32 + wave % (NT / 2)) * 16 + j);
+    if (stream_n > 0) {
+      stream = H.x[stream_at < stream_n ? stream_at : 0];
+      stream_bias = H.x_bias[stream_at < stream_n ? stream_at % H.dim : 0];
+    }
+  }
+
   // The rotation's and the cache's addresses hang on a chain of loads: positions and slots are asked for now, the angles and
   // pages (rope_ahead) before the waves' sums meet (a step's q/k/v of 7B sizes at 8 rows 12.7 -> 11.6 us).  Of the epilogue's first
   // tile, as c_old; rows and columns past the edges repeat the last ones and are never stored.
@@ -337,6 +350,10 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
   }
 
   if (AHEAD && wave < MT * RT) rope_ahead(wave);
+  if (EPI == EPI_GATED_BIAS && stream_at < stream_n) {
+    H.x[stream_at] = stream + stream_bias;
+    for (long e = stream_at + stream_step; e < stream_n; e += stream_step) H.x[e] += H.x_bias[e % H.dim];
+  }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -361,11 +378,12 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
       const f32x4 g = tile_sum(mt, 2 * tp), u = tile_sum(mt, 2 * tp + 1);
       int hcol = (n0 / 32 + tp) * 16 + j;
       bf16* C = (bf16*)Cv;
+      if (idx != wave) gb = gate_bias<EPI>(H, hcol);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         int m = mt * 16 + 4 * q + r;
         if (m < M && hcol < H)
-          C[(size_t)m * H + hcol] = static_cast<bf16>(gate_unit<EPI>(g[r] * scale[r], u[r] * scale[r], H));
+          C[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(g[r] * scale[r], u[r] * scale[r], H, gb));
       }
       continue;
     }

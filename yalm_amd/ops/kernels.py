@@ -185,6 +185,30 @@ def gemm(a, w, out, epilogue, hidden=0, workspace=None, scale_from=None, unit=No
     return out
 
 
+def can_gemm_gated_bias(kind):
+    """Whether gemm_gated_bias takes a feed-forward of this activation (ACTIVATIONS)."""
+    return kind == "gelu_tanh"
+
+
+def gemm_gated_bias(a, w, bias, out, x, x_bias, workspace=None):
+    """out[M, hidden] (a's dtype) = gelu(a @ gate^T + bias) * (a @ up^T + bias), the gelu in its tanh form, with w and bias (float32)
+    holding gate and up interleaved in blocks of 16, and x (float32 [M, dim]) += x_bias on the way.
+    workspace: as for gemm."""
+    M, K = a.shape
+    N, hidden = w.shape[0], out.shape[1]
+    if hidden <= 0 or N != 32 * ((hidden + 15) // 16):
+        raise ValueError("gated gemm: weight rows %d do not match hidden %d" % (N, hidden))
+    p_a, p_w = _need(a, "a", a.dtype, (M, K)), _need(w, "w", a.dtype, (N, K))
+    p_b, p_o = _need(bias, "bias", torch.float32, (N,)), _need(out, "out", a.dtype, (M, hidden))
+    p_x, p_xb = _need(x, "x", torch.float32, (M, None)), _need(x_bias, "x_bias", torch.float32, (x.shape[1],))
+    p_ws, n_ws = None, 0
+    if workspace is not None:
+        p_ws, n_ws = _need(workspace, "workspace", torch.float32), workspace.numel()
+    library.check(library.lib().yalm_gemm_gated_bias(p_a, p_w, p_o, p_ws, n_ws, M, N, K, dtype_code(a.dtype), hidden, p_b, p_x, p_xb,
+                                                     x.shape[1], 1 if FORCE_SIMPLE else 0, _stream()), "gemm_gated_bias")
+    return out
+
+
 FUSED_NORM_MAX_ROWS = 8
 
 

@@ -141,12 +141,14 @@ class Part:
     def _gemm(ctx, a, w, out, epilogue, hidden=0, scale_from=None, unit=None):
         """kernels.gemm with the scratch that lets small batches split K."""
         from ..ops import kernels
+        return kernels.gemm(a, w, out, epilogue, hidden=hidden, workspace=Part._gemm_scratch(ctx, a, w), scale_from=scale_from, unit=unit)
+
+    @staticmethod
+    def _gemm_scratch(ctx, a, w):
+        from ..ops import kernels
         import torch
-        ws = None
         n = kernels.gemm_workspace_floats(a.shape[0], w.shape[0], a.shape[1]) if a.dtype == torch.bfloat16 else 0
-        if n and ctx is not None:
-            ws = ctx.ws.get("gemm.partial", (n,), torch.float32)
-        return kernels.gemm(a, w, out, epilogue, hidden=hidden, workspace=ws, scale_from=scale_from, unit=unit)
+        return ctx.ws.get("gemm.partial", (n,), torch.float32) if n and ctx is not None else None
 
     def _emit_args(self, emit_for, ctx, T, width):
         """Operands for a residual-add GEMM that also prepares the activations of the norm

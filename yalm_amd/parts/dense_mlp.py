@@ -4,12 +4,13 @@ stay float32 until the activation has been applied; its result is rounded to the
 product, whose epilogue adds to the float32 residual stream.  With `gated` there is a third matrix and the middle is
 act(gate h) * (up h) (gate and up are one product); with `biases` every product has a bias (tensors "<name>.b" unless
 named otherwise): those of the first products are added before the activation, the last one's goes to the stream
-with the kernel of the middle."""
+with the kernel of the middle, or with the first product where its epilogue does the middle (gated, tanh gelu)."""
 import torch
 
 from ..ops import kernels
 from ..weights.loader import ParamSpec, place
 from .base import Part, part
+from .swiglu import interleave_gate_up
 
 
 @part("feed_forward", "dense_mlp")
@@ -26,6 +27,8 @@ class DenseMLP(Part):
         self.names.update(spec.params.get("tensors") or {})
         for k in ("up", "down", "gate"):
             self.names.setdefault(k + "_bias", self.names[k] + ".b")
+        # the first product's epilogue does the middle; its rows are then gate and up in turn
+        self.one_kernel = self.gated and self.biases and kernels.can_gemm_gated_bias(self.activation)
         self.w_up = self.w_down = self.b_up = self.b_down = None
 
     def _first(self):
@@ -41,11 +44,12 @@ class DenseMLP(Part):
         return out
 
     def load(self, get, compute_dtype, device):
-        self.w_up = place(torch.cat([get(self.prefix + self.names[k]) for k in self._first()], dim=0), compute_dtype, device)
+        join = (lambda rows: interleave_gate_up(*rows)) if self.one_kernel else (lambda rows: torch.cat(rows, dim=0))
+        self.w_up = place(join([get(self.prefix + self.names[k]) for k in self._first()]), compute_dtype, device)
         self.w_down = place(get(self.prefix + self.names["down"]), compute_dtype, device)
         if self.biases:
-            self.b_up = torch.cat([get(self.prefix + self.names[k + "_bias"]).to(torch.float32).reshape(-1)
-                                   for k in self._first()]).to(device).contiguous()
+            self.b_up = join([get(self.prefix + self.names[k + "_bias"]).to(torch.float32).reshape(-1, 1)
+                              for k in self._first()]).reshape(-1).to(device).contiguous()
             self.b_down = get(self.prefix + self.names["down_bias"]).to(torch.float32).reshape(-1).to(device).contiguous()
 
     def weight_bytes(self):
@@ -60,6 +64,9 @@ class DenseMLP(Part):
     def _hidden(self, h, ctx, x=None):
         """The middle of the layer in the compute dtype; with x, the last product's bias is added to x on the way."""
         T = h.shape[0]
+        if self.one_kernel:
+            mid = ctx.ws.get("mlp.mid", (T, self.hidden), h.dtype)
+            return kernels.gemm_gated_bias(h, self.w_up, self.b_up, mid, x, self.b_down, workspace=self._gemm_scratch(ctx, h, self.w_up))
         z = ctx.ws.get("mlp.z", (T, self.w_up.shape[0]), torch.float32)
         self._gemm(ctx, h, self.w_up, z, kernels.EPI_STORE_F32)
         mid = ctx.ws.get("mlp.mid", (T, self.hidden), h.dtype)
