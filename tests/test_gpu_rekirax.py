@@ -130,6 +130,31 @@ def test_middle_of_a_gated_feed_forward_with_biases(T, F, D, kind, dtype):
     assert torch.allclose(out2.float().cpu().to(F64), act0 * z.to(F64)[:, F:], rtol=tol, atol=tol)
 
 
+# Few tokens are dealt to several workgroups each (20 rows), many take a wave each (40): the results agree, and every element is there.
+# Rows of 1,024 and of 256 threads, more key heads than query heads' share, heads that end inside a round
+@pytest.mark.parametrize("H,G,d,dv,head_norm", [(32, 8, 128, 128, False), (32, 8, 128, 64, True), (6, 2, 64, 48, False), (3, 3, 20, 28, False),
+                                                (44, 44, 32, 16, True)])
+def test_packing_kernel_of_few_tokens(H, G, d, dv, head_norm):
+    from yalm_amd.ops import kernels
+    T, ring, pad = 40, 2, (max(d, dv) + 15) // 16 * 16
+    raw = randn(T, H * d + G * (d + dv), seed=H + d).to(DEV)
+    wq, wk = (1 + randn(n, seed=s, scale=0.2) for s, n in ((1, d if head_norm else H * d), (2, d if head_norm else G * d)))
+    first, lam = randn(T, G * dv, seed=3).to(DEV), torch.tensor([0.3], device=DEV)
+    table = torch.arange(T * ring, dtype=torch.int32, device=DEV).reshape(T, ring)
+    pos = [(5 * t) % 128 for t in range(T)]
+    out = []
+    for cut in ([(0, 40)], [(0, 20), (20, 40)]):
+        q = torch.full((T, H * pad), float("nan"), device=DEV)
+        kp, vp = torch.zeros(T * ring, G, 64, pad, device=DEV), torch.zeros(T * ring, G, pad, 64, device=DEV)
+        for lo, hi in cut:
+            kernels.qkv_pack(raw[lo:hi], None, wq.to(DEV), wk.to(DEV), 1e-5, (0.1, 16), 1.7, first[lo:hi].clone(), 2, lam, q[lo:hi], None, None,
+                             None, kp, vp, table, ring, i32(np.arange(hi - lo)), i32(pos[lo:hi]), i32(np.arange(lo, hi)),
+                             i32([p + 1 for p in pos[lo:hi]]), H, G, d, dv, pad, head_norm=head_norm)
+        out.append((q, kp, vp))
+    for a, b in zip(*out):                            # the norms' sums in another order: a few roundings of 2^-24
+        assert torch.allclose(a, b, rtol=2e-6, atol=2e-6) and torch.equal(a != 0, b != 0)
+
+
 # The same with the middle in the first product's epilogue: one to 16 rows (K a multiple of 64 and not), to 128, tiles of 128 rows,
 # larger tiles, K in slices and whole; hidden values that end inside a block; streams narrower and wider than what one
 # element a thread covers; and the general kernels
