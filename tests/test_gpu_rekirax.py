@@ -212,6 +212,42 @@ def test_way_into_looped_layers(T, D, dtype):
     assert torch.allclose(xg.cpu().to(F64), want, rtol=tol, atol=tol)
 
 
+# A step of one token a sequence keeps a head's state in one workgroup (d and dv multiples of 4 to 128); it walks what it is given, so
+# two tokens of one sequence and none of the next are the same walk
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,d,dv", [(2, 128, 128), (3, 36, 124), (1, 124, 68), (32, 128, 128), (1, 4, 128)])
+def test_recurrence_of_single_tokens(H, d, dv, dtype):
+    from yalm_amd.ops import kernels
+    B, n_slots = 5, 7
+    w = {"m.f": torch.eye(H * d, dtype=F64), "m.f.b": randn(H * d, seed=1, scale=0.5).to(F64), "m.lower": randn(H * d, seed=2).abs().clamp(0, 1).to(F64),
+         "m.norm": (1 + randn(dv, seed=3, scale=0.2)).to(F64)}
+    N = 2 * H * d + H * dv
+    wide = randn(B, N + 12, seed=4, scale=1.5).to(DEV)                # the projections are columns of wider rows
+    proj = wide[:, 4:4 + N]
+    slots, cu = [3, -1, 0, 6, 2], [0, 1, 2, 4, 4, 5]
+    start = randn(n_slots, H * dv * d, seed=5)
+    state, out = start.clone().to(DEV), torch.full((B, H * dv), float("nan"), dtype=dtype, device=DEV)
+    kernels.hgrn2(proj, f32(w["m.f.b"]), f32(w["m.lower"]), f32(w["m.norm"]), state, torch.empty(B, H * dv, device=DEV), i32(cu), i32(slots), out,
+                  H, d, dv, 1e-5)
+    pr = proj.cpu().to(F64)
+    q, f = P.silu(pr[:, :H * d]).reshape(B, H, d), P.forget_gates(pr[:, H * d:2 * H * d], w, "m.").reshape(B, H, d)
+    v = pr[:, 2 * H * d:].reshape(B, H, dv)
+    tol = 2e-5 if dtype == torch.float32 else 2e-2
+    for b, slot in enumerate(slots):
+        rows = slice(cu[b], cu[b + 1])
+        if slot < 0:
+            assert float(out[rows].float().abs().sum()) == 0.0
+            continue
+        S0 = start[slot].reshape(H, dv, d).transpose(1, 2).to(F64).contiguous()
+        o, S = P.hgrn2_recurrence(q[rows], f[rows], v[rows], S0)
+        assert torch.allclose(state[slot].cpu().reshape(H, dv, d).transpose(1, 2).to(F64), S, rtol=2e-5, atol=2e-5)
+        if cu[b + 1] > cu[b]:
+            want = (P.rms_div(o, 1e-5) * w["m.norm"]).reshape(-1, H * dv)
+            assert torch.allclose(out[rows].float().cpu().to(F64), want, rtol=tol, atol=tol)
+    for slot in set(range(n_slots)) - set(slots):
+        assert torch.equal(state[slot].cpu(), start[slot])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n_first", [3, 40])
 @pytest.mark.parametrize("H,d,dv", [(1, 4, 4), (4, 32, 64), (3, 5, 9), (2, 64, 40), (1, 128, 70), (1, 200, 33), (2, 16, 200), (5, 36, 31)])

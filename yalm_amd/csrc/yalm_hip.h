@@ -473,7 +473,7 @@ int yalm_loop_pack(float* x, const float* x0, const float* start, void* both, in
 // out (`out_dtype` [T, H dv]) = o over its root mean square a head, times w_norm (float32 [dv]).  state float32 [n_slots, H,
 // dv, d] (a head's S column by column), read and left advanced; raw float32 [T, H dv] scratch; the tokens of sequence b are
 // cu_seqlens[b] .. cu_seqlens[b + 1] - 1, in order; a sequence with slot -1 touches no state and gives zeros.  d <= 256.
-int yalm_hgrn2(const float* proj, const float* f_bias, const float* lower, const float* w_norm, float* state, float* raw,
+int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state, float* raw,
                const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads, int d, int dv, float eps,
                int out_dtype, hipStream_t stream);
 

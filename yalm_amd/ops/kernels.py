@@ -1372,7 +1372,7 @@ def hgrn2_state_elements(n_heads, d, dv):
 
 
 def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_heads, d, dv, eps):
-    """The HGRN2 recurrence over a step's tokens.  proj float32 [T, 2 H d + H dv] = z_q | z_f | v; q = silu(z_q), f = lower
+    """The HGRN2 recurrence over a step's tokens.  proj float32 [T, 2 H d + H dv] (rows may be parts of wider ones) = z_q | z_f | v; q = silu(z_q), f = lower
     + (1 - lower) sigmoid(z_f + f_bias); per head S <- diag(f) S + (1 - f) v^T, o = S^T q; out [T, H dv] = o over its root
     mean square a head, times w_norm [dv].  state float32 [slots, H dv d] (a head's S column by column) is read and left
     advanced; raw float32 [T, H dv] is scratch.  Sequence b's tokens are cu_seqlens[b] .. cu_seqlens[b + 1] - 1."""
@@ -1381,8 +1381,10 @@ def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_
     N = 2 * n_heads * d + n_heads * dv
     if not 0 < d <= HGRN2_MAX_KEY_DIM:
         raise ValueError("hgrn2: key heads of %d (at most %d)" % (d, HGRN2_MAX_KEY_DIM))
+    if proj.dtype != torch.float32 or proj.dim() != 2 or proj.shape[1] != N or proj.stride(1) != 1 or not proj.is_cuda:
+        raise ValueError("hgrn2: the projections are float32 [%d, %d] on the device, rows contiguous" % (T, N))
     library.check(library.lib().yalm_hgrn2(
-        _need(proj, "proj", torch.float32, (T, N)), _need(f_bias, "f_bias", torch.float32, (n_heads * d,)),
+        proj.data_ptr(), int(proj.stride(0)), _need(f_bias, "f_bias", torch.float32, (n_heads * d,)),
         _need(lower, "lower", torch.float32, (n_heads * d,)), _need(w_norm, "w_norm", torch.float32, (dv,)),
         _need(state, "state", torch.float32, (None, n_heads * d * dv)), _need(raw, "raw", torch.float32, (T, n_heads * dv)),
         _need(cu_seqlens, "cu_seqlens", torch.int32, (B + 1,)), _need(seq_slot, "seq_slot", torch.int32, (B,)),

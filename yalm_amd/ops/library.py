@@ -92,7 +92,7 @@ _SIGNATURES = {
     "yalm_gated_bias_act": (_I, [_P, _P, _P, _I, _I, _I, _I, _P, _P, _I, _P]),
     "yalm_sigmoid_gate": (_I, [_P, _P, ctypes.c_long, _I, _I, _I, _I, _I, _P]),
     "yalm_loop_pack": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
-    "yalm_hgrn2": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P]),
+    "yalm_hgrn2": (_I, [_P, ctypes.c_long, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P]),
     "yalm_head_gate": (_I, [_P, _P, ctypes.c_long, _F, _P, ctypes.c_long, _I, _I, _I, _I, _P]),
     "yalm_softcap": (_I, [_P, ctypes.c_long, _F, _P]),
     "yalm_squash": (_I, [_P, _P, _P, _F, _P, _F, _P, _P, _P, _I, _F, _P, _P, _I, _I, _P]),
@@ -106,7 +106,7 @@ _SIGNATURES = {
     "yalm_probe_mfma": (_I, [_I, _I, _I, _P, _P, _P]),
 }
 
-ABI_VERSION = 43
+ABI_VERSION = 44
 
 
 class KernelError(RuntimeError):
