@@ -1597,6 +1597,29 @@ def test_gemm_norm_qkv_rope(n_heads, n_kv, hd, rd, D):
     assert (vp.float().abs().sum(dim=(1, 2)) > 0).equal(touched)
 
 
+# Workgroups of 96 weight rows, which take what 64 rows would leave to a second round of compute units: the fewest and the most rows, a
+# last workgroup of one row, sums of one, two and seven stages of K
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,Kd", [(16385, 128), (24576, 64), (22113, 448)])
+def test_decode_gemm_of_96_rows(M, N, Kd):
+    from yalm_amd.parts.swiglu import interleave_gate_up
+    k = K()
+    x, w = rnd((M, Kd), 130, torch.bfloat16).to(DEV), rnd((N, Kd), 131, torch.bfloat16, scale=Kd ** -0.5).to(DEV)
+    want = x.double() @ w.double().t()
+    # float32 sums of exact products: K roundings of the sum of magnitudes
+    bound = 2.0 ** -23 * Kd * (x.double().abs() @ w.double().abs().t())
+    got = k.gemm(x, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double()
+    assert bool(((got - want).abs() <= bound).all())
+    old = rnd((M, N), 132).to(DEV)
+    got = k.gemm(x, w, old.clone(), k.EPI_ADD_F32).double()
+    assert bool(((got - want - old.double()).abs() <= bound + 2.0 ** -23 * (want.abs() + old.double().abs())).all())
+    H = N // 2
+    wg = interleave_gate_up(w[:H], w[H:2 * H])
+    out = k.gemm(x, wg, torch.full((M, H), 7.0, dtype=torch.bfloat16, device=DEV), k.EPI_GATED, hidden=H)
+    g, u = want[:, :H], want[:, H:2 * H]
+    close(out, (g / (1 + torch.exp(-g)) * u).cpu(), torch.bfloat16, "gated")
+
+
 # Rows in turn over eight waves, K of fewer k tiles than waves and of many; the sum of squares over one wave (to 1,024), over four
 # by 16 bytes (to 8,192) and element by element (beyond); one and two column tiles a workgroup
 @pytest.mark.parametrize("M,N,Kd", [(1, 40, 32), (16, 100, 96), (3, 512, 256), (9, 4100, 1024), (13, 33, 1056), (16, 4112, 4096), (2, 50, 8192),

@@ -211,6 +211,7 @@ class JoinableMixer(Part):
     says `joinable`: it then makes one product of their first ones and one of their last ones, hands them their columns of
     the wider rows, and they load no matrices of their own."""
     joinable = False
+    front_shared = False              # whether the product in front is part of a wider one that somebody else makes (proj)
 
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
@@ -222,12 +223,13 @@ class JoinableMixer(Part):
     def load(self, get, compute_dtype, device):
         from ..weights.loader import place
         if not self.joined:
-            self.w_in = place(self.in_rows(get), compute_dtype, device)
+            if not self.front_shared:
+                self.w_in = place(self.in_rows(get), compute_dtype, device)
             self.wo = place(self.out_columns(get), compute_dtype, device)
         self.load_rest(get, compute_dtype, device, self.share)
 
     def weight_bytes(self):
-        return 0 if self.joined else (self.w_in.numel() + self.wo.numel()) * self.w_in.element_size()
+        return sum(w.numel() * w.element_size() for w in (self.w_in, self.wo) if w is not None)
 
     def forward(self, h, x, ctx, line, writes_cache=True):
         """Adds the mixer's result to the stream x."""
@@ -236,19 +238,21 @@ class JoinableMixer(Part):
             raise ValueError("a mixer whose last product has a bias writes its result (forward_to); it does not add to the stream")
         return self._run(h, x, ctx, line, writes_cache, kernels.EPI_ADD_F32)
 
-    def forward_to(self, h, y, ctx, line, writes_cache=True, late_bias_taken=False):
-        """Writes the mixer's result to y (float32 [T, dim]), without its late_bias."""
+    def forward_to(self, h, y, ctx, line, writes_cache=True, late_bias_taken=False, proj=None):
+        """Writes the mixer's result to y (float32 [T, dim]), without its late_bias; proj: the product in front where it is shared
+        (float32 [T, n_in], maybe columns of wider rows)."""
         from ..ops import kernels
         if self.late_bias is not None and not late_bias_taken:
             raise ValueError("this mixer's result lacks a bias that nobody adds")
-        return self._run(h, y, ctx, line, writes_cache, kernels.EPI_STORE_F32)
+        return self._run(h, y, ctx, line, writes_cache, kernels.EPI_STORE_F32, proj)
 
-    def _run(self, h, x, ctx, line, writes_cache, epilogue):
+    def _run(self, h, x, ctx, line, writes_cache, epilogue, proj=None):
         import torch
         from ..ops import kernels
         T = h.shape[0]
-        proj = ctx.ws.get("joinable.proj", (T, self.n_in), torch.float32)
-        self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
+        if proj is None:
+            proj = ctx.ws.get("joinable.proj", (T, self.n_in), torch.float32)
+            self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
         o = ctx.ws.get("joinable.o", (T, self.n_out), h.dtype)
         self.between(h, proj, o, ctx, line, writes_cache)
         self._gemm(ctx, o, self.wo, x, epilogue)

@@ -20,6 +20,8 @@ NAMES = {"q": "q", "f": "f", "f_bias": "f.b", "lower": "lower", "v": "v", "norm"
 
 @part("mixer", "hgrn2")
 class HGRN2(Part):
+    front_shared = False              # whether somebody else makes the product in front (as JoinableMixer has it)
+
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
         p = spec.params
@@ -46,21 +48,29 @@ class HGRN2(Part):
                 ParamSpec(self._n("v"), (self.vv, D), fan_in=D), ParamSpec(self._n("norm"), (self.value_dim,), init="norm"),
                 ParamSpec(self._n("out"), (D, self.vv), fan_in=self.vv)]
 
+    @property
+    def n_in(self):
+        return 2 * self.qk + self.vv
+
+    def in_rows(self, get):
+        return torch.cat([get(self._n(k)) for k in ("q", "f", "v")], dim=0)
+
     def load(self, get, compute_dtype, device):
         def f32(key):
             return get(self._n(key)).to(torch.float32).reshape(-1).to(device).contiguous()
-        self.w_in = place(torch.cat([get(self._n(k)) for k in ("q", "f", "v")], dim=0), compute_dtype, device)
+        if not self.front_shared:
+            self.w_in = place(self.in_rows(get), compute_dtype, device)
         self.wo = place(get(self._n("out")), compute_dtype, device)
         self.f_bias, self.lower, self.w_norm = f32("f_bias"), f32("lower"), f32("norm")
 
     def weight_bytes(self):
-        return (self.w_in.numel() + self.wo.numel()) * self.w_in.element_size()
+        return sum(w.numel() * w.element_size() for w in (self.w_in, self.wo) if w is not None)
 
     def cache_request(self):
         return StateRequest((kernels.hgrn2_state_elements(self.n_heads, self.key_dim, self.value_dim),), torch.float32)
 
     def row_elements(self):
-        return 2 * self.qk + self.vv
+        return self.n_in
 
     def describe(self, compute_dtype):
         return "HGRN2, %d heads of %d x %d: a state column in the registers of eight lanes, float32" % (
@@ -70,15 +80,16 @@ class HGRN2(Part):
         """Adds the mixer's result to the stream x."""
         return self._run(h, x, ctx, line, kernels.EPI_ADD_F32)
 
-    def forward_to(self, h, y, ctx, line, writes_cache=True):
-        """Writes the mixer's result to y (float32 [T, dim])."""
-        return self._run(h, y, ctx, line, kernels.EPI_STORE_F32)
+    def forward_to(self, h, y, ctx, line, writes_cache=True, proj=None):
+        """Writes the mixer's result to y (float32 [T, dim]); proj: as JoinableMixer.forward_to."""
+        return self._run(h, y, ctx, line, kernels.EPI_STORE_F32, proj)
 
-    def _run(self, h, x, ctx, line, epilogue):
+    def _run(self, h, x, ctx, line, epilogue, proj=None):
         T = h.shape[0]
         ws = ctx.ws
-        proj = ws.get("hgrn2.proj", (T, 2 * self.qk + self.vv), torch.float32)
-        self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
+        if proj is None:
+            proj = ws.get("hgrn2.proj", (T, self.n_in), torch.float32)
+            self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
         raw = ws.get("hgrn2.raw", (T, self.vv), torch.float32)
         o = ws.get("hgrn2.o", (T, self.vv), h.dtype)
         state = ctx.cache.group_of(line).line_state(line)

@@ -90,7 +90,8 @@ class ShapedAttention(JoinableMixer):
             raise ValueError("heads of %d are not supported (at most %d)" % (self.pad, kernels.MAX_HEAD_DIM))
         self.q_dim, self.k_dim, self.v_dim = self.n_heads * self.key_dim, self.n_kv_heads * self.key_dim, self.n_kv_heads * self.value_dim
         self.n_proj = self.q_dim + self.k_dim + (0 if self.values_from_keys else self.v_dim)      # what the packing kernel reads of a token's row
-        self.gate_rows = (self.n_heads + 3) // 4 * 4 if self.gate == "heads" else 0               # behind it, zero rows up to whole fours
+        # behind it the gate's rows (a number a head: zero rows up to whole fours)
+        self.gate_rows = {"heads": (self.n_heads + 3) // 4 * 4, "elements": self.n_heads * self.value_dim}.get(self.gate, 0)
         self.joinable = self.gate == "heads"      # the gate's kernel brings the result to its place in a wider row
         if (self.q_dim + self.k_dim + self.v_dim) * 4 > 64 * 1024:
             raise ValueError("a token's queries, keys and values (%d numbers) are more than the packing kernel holds"
@@ -101,7 +102,7 @@ class ShapedAttention(JoinableMixer):
         self.rot_dims = int(getattr(self.position, "rotary_dim", 0) or 0)
         if self.rot_dims > self.key_dim:
             raise ValueError("%d turned elements do not fit key heads of %d" % (self.rot_dims, self.key_dim))
-        self.bias = self.w_qn = self.w_kn = self.sink = self.lam = self.wg = self.log_ab = None
+        self.bias = self.w_qn = self.w_kn = self.sink = self.lam = self.log_ab = None
 
     def children(self):
         return [self.position] if self.position is not None else []
@@ -158,6 +159,8 @@ class ShapedAttention(JoinableMixer):
         if self.gate == "heads":
             g = get(self._n("gate"))
             rows += [g, g.new_zeros((self.gate_rows - self.n_heads, self.dim))]
+        elif self.gate == "elements":
+            rows.append(get(self._n("gate")))
         return torch.cat(rows, dim=0)
 
     def out_columns(self, get):
@@ -173,7 +176,6 @@ class ShapedAttention(JoinableMixer):
 
         def f32(key):
             return get(self._n(key)).to(torch.float32).reshape(-1).to(device).contiguous()
-        self.wg = place(get(self._n("gate")), compute_dtype, device) if self.gate == "elements" else None
         self.late_bias = f32("out_bias") * scale if self.has_out_bias else None
         self.bias = None
         if self.biases:
@@ -191,9 +193,6 @@ class ShapedAttention(JoinableMixer):
         self.log_ab = (f32("log_a"), f32("log_b")) if self.has_log_distance else None
         self.sink = f32("sink") if self.has_sink else None
         self.lam = f32("blend") if self.value_blend == "later" else None
-
-    def weight_bytes(self):
-        return super().weight_bytes() + (self.wg.numel() * self.wg.element_size() if self.wg is not None else 0)
 
     def cache_request(self):
         # a query inside a block sees fewer than `block` keys back: the ring of a window of that width holds them
@@ -281,6 +280,4 @@ class ShapedAttention(JoinableMixer):
         if self.gate == "heads":
             kernels.head_gate(o, proj[:, self.n_proj:self.n_proj + H], H, scale, joint)
         elif self.gate == "elements":
-            gates = ws.get("attn.gate", (T, H * self.value_dim), torch.float32)
-            self._gemm(ctx, h, self.wg, gates, kernels.EPI_STORE_F32)
-            kernels.sigmoid_gate(o, gates, H, self.value_dim, P)
+            kernels.sigmoid_gate(o, proj[:, self.n_proj:], H, self.value_dim, P)

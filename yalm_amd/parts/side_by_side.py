@@ -3,7 +3,8 @@
 (left, right) the results are not normed: the mixer's result is left * (the left one's) + right * (the right one's).  The two
 (JoinableMixer, both joinable) then share one product in front and one behind: their first matrices stand one below the other,
 their last ones side by side, and a side's scale rides on what it puts in front of the last product (in float32, before that is
-rounded to the compute dtype).
+rounded to the compute dtype).  Normed ones share the product in front where both can (a product of 10,240 weight rows and one of
+12,288 are one of 22,528: a launch less, and rows that deal evenly to the compute units).
 
 The two are any registered mixers that offer forward_to (which writes a result instead of adding it); each keeps what
 it keeps (keys and values in pages, a fixed-size state) under a cache line of its own: this mixer's cache request is
@@ -36,6 +37,10 @@ class SideBySide(Part):
         self.w_left = self.w_right = None
         self.scales = tuple(float(s) for s in p["scales"]) if p.get("scales") else None
         self.w_in = self.wo = None
+        self.shares_front = self.scales is None and all(hasattr(m, "front_shared") for m in (self.left, self.right))
+        if self.shares_front:
+            for m in (self.left, self.right):
+                m.front_shared = True
         if self.scales is not None:
             for m, scale in zip((self.left, self.right), self.scales):
                 if not isinstance(m, JoinableMixer) or not m.joinable:
@@ -61,8 +66,9 @@ class SideBySide(Part):
         return [ParamSpec(self.left_norm, (self.dim,), init="norm"), ParamSpec(self.right_norm, (self.dim,), init="norm")]
 
     def load(self, get, compute_dtype, device):
-        if self.scales is not None:
+        if self.scales is not None or self.shares_front:
             self.w_in = place(torch.cat([m.in_rows(get) for m in (self.left, self.right)], dim=0), compute_dtype, device)
+        if self.scales is not None:
             self.wo = place(torch.cat([m.out_columns(get) for m in (self.left, self.right)], dim=1), compute_dtype, device)
             return                        # the members load the rest themselves
         # the share of each side rides on its norm's weight (exact for a power of two)
@@ -72,7 +78,7 @@ class SideBySide(Part):
     def weight_bytes(self):
         if self.scales is not None:
             return (self.w_in.numel() + self.wo.numel()) * self.w_in.element_size()
-        return 2 * self.dim * 4
+        return 2 * self.dim * 4 + (self.w_in.numel() * self.w_in.element_size() if self.w_in is not None else 0)
 
     def cache_request(self):
         return {"left": self.left.cache_request(), "right": self.right.cache_request()}
@@ -80,10 +86,14 @@ class SideBySide(Part):
     def describe(self, compute_dtype):
         if self.scales is not None:
             return "two mixers side by side, one product in front of both and one behind", False
+        if self.shares_front:
+            return "two mixers side by side, one product in front of both, each result normed over the width", False
         return "two mixers side by side, each normed over the width", False
 
     def row_elements(self):
-        return max(self.left.n_in + self.right.n_in, self.left.n_out + self.right.n_out) if self.scales is not None else self.dim
+        if self.scales is not None:
+            return max(self.left.n_in + self.right.n_in, self.left.n_out + self.right.n_out)
+        return max(self.dim, self.left.n_in + self.right.n_in) if self.shares_front else self.dim
 
     def forward_to(self, h, y, ctx, line, writes_cache=True, late_bias_taken=False):
         """Writes the mixer's result to y (float32 [T, dim]), without its late_bias."""
@@ -111,8 +121,14 @@ class SideBySide(Part):
             return self._joint(h, x, ctx, line, writes_cache, kernels.EPI_ADD_F32)
         # both results whole: a second float32 [T, dim] beside the first (64 MB for 4,096 tokens of width 4,096), added in one pass
         y, y2 = (ctx.ws.get(name, (T, self.dim), torch.float32) for name in ("side.y", "side.y2"))
-        self.left.forward_to(h, y, ctx, (line, "left"), writes_cache)
-        self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache)
+        front = ({}, {})
+        if self.shares_front:
+            n = self.left.n_in
+            proj = ctx.ws.get("side.proj", (T, n + self.right.n_in), torch.float32)
+            self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
+            front = ({"proj": proj[:, :n]}, {"proj": proj[:, n:]})
+        self.left.forward_to(h, y, ctx, (line, "left"), writes_cache, **front[0])
+        self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache, **front[1])
         if emit_for is None or not hasattr(emit_for, "fused"):
             kernels.norm_add_pair(y, self.w_left, y2, self.w_right, self.eps, x)
             return
