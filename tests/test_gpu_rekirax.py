@@ -212,6 +212,25 @@ def test_way_into_looped_layers(T, D, dtype):
     assert torch.allclose(xg.cpu().to(F64), want, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("d,dv", [(72, 36), (128, 64), (100, 33)])
+def test_recurrence_of_many_workgroups(d, dv):
+    """Beyond three workgroups a compute unit a lane group takes two columns: the bits are those of one."""
+    from yalm_amd.ops import kernels
+    H, lens = 300, [19, 1, 34]
+    T, cu = sum(lens), np.concatenate([[0], np.cumsum(lens)])
+    assert 2 * H * 3 > 3 * torch.cuda.get_device_properties(0).multi_processor_count >= 2 * H
+    proj = randn(T, 2 * H * d + H * dv, seed=1, scale=1.5).to(DEV)
+    bias, lower, w = randn(H * d, seed=2).to(DEV), randn(H * d, seed=3).abs().clamp(0, 1).to(DEV), (1 + randn(dv, seed=4, scale=0.2)).to(DEV)
+    start = randn(3, H * dv * d, seed=5)
+    state, out, raw = start.clone().to(DEV), torch.empty(T, H * dv, device=DEV), torch.empty(T, H * dv, device=DEV)
+    kernels.hgrn2(proj, bias, lower, w, state, raw, i32(cu), i32([0, 1, 2]), out, H, d, dv, 1e-5)
+    for b in (0, 2):
+        one, rows = torch.empty(lens[b], H * dv, device=DEV), slice(cu[b], cu[b + 1])
+        alone = start[b:b + 1].clone().to(DEV)
+        kernels.hgrn2(proj[rows].contiguous(), bias, lower, w, alone, raw[:lens[b]], i32([0, lens[b]]), i32([0]), one, H, d, dv, 1e-5)
+        assert torch.equal(one, out[rows]) and torch.equal(alone[0], state[b])
+
+
 # A step of one token a sequence keeps a head's state in one workgroup (d and dv multiples of 4 to 128); it walks what it is given, so
 # two tokens of one sequence and none of the next are the same walk
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

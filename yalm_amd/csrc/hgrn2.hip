@@ -142,6 +142,10 @@ extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias,
   rc = diag_scan_launch<Hgrn2Op, NR_, LANES_, NC_, TOK_>(op, state, raw, cu_seqlens, seq_slot, B, n_heads, d, dv, 0, stream)
   if (d <= 32) SCAN(4, 8, 1, 16);
   else if (d <= 64) SCAN(8, 8, 1, 16);
+  // Two columns a lane group halve the reads of the operands from LDS, and pay where more than three workgroups of 32 columns share a
+  // compute unit (nine prompts of 700 tokens, 32 heads of 128 x 128: 617 -> 527 us, twenty of 64 126 -> 100); with few the walk waits for itself, and
+  // longer with two (2,048 tokens 534 -> 780; 640 workgroups 239 and 238).  The sums are the same.
+  else if (d <= 128 && (long)B * n_heads * ceil_div(dv, 32) > 3L * compute_units()) SCAN(16, 8, 2, 16);
   else if (d <= 128) SCAN(16, 8, 1, 16);
   else SCAN(32, 8, 1, 16);
 #undef SCAN
