@@ -122,7 +122,7 @@ KERNEL_FACES = ("embed", "rmsnorm", "gemm", "gemm_norm", "gemm_norm_qkv_rope", "
                 "attn_decode", "sink_store", "attn_sink_mix", "argmax", "cast", "norm_add", "polynorm", "head_matmul",
                 "latent_pack", "moe_route", "moe_select", "moe_pair_gate_up", "moe_pair_down", "moe_grouped", "embed_sinusoid",
                 "qkv_pack", "v_tiles", "mlstm_scan", "mlstm_chunks", "gated_delta", "embed_learned", "activate", "gated_add",
-                "time_conv", "gated_bias_act", "sigmoid_gate", "loop_pack", "hgrn2", "norm_add_pair", "layer_norm", "layer_norm_sum", "embed_pairs",
+                "time_conv", "gated_bias_act", "gemm_gated_bias", "sigmoid_gate", "loop_pack", "hgrn2", "norm_add_pair", "layer_norm", "layer_norm_sum", "embed_pairs",
                 "latent_norm", "moe_select_groups", "gla", "gla_tiles", "squash", "squash_add", "rms_gate", "head_gate", "softcap",
                 "lightning", "lightning_tiles", "lru", "lru_step")
 FP32_FACES = ("mlstm_scan", "mlstm_chunks", "gated_delta", "hgrn2", "gla", "gla_tiles", "lightning", "lightning_tiles")     # kernels of float32 multiply-adds whatever the model's dtype: priced against that peak
@@ -249,9 +249,9 @@ def kernel_cost(name, a, kw, kv_tokens, torch):
         proj, raw, seq_slot, out = a[0], a[5], a[7], a[8]
         H, d, dv = a[9], a[10], a[11]
         T, B = proj.shape[0], seq_slot.shape[0]
-        # per token and head: the gate's blend and the read-out, each over the d x dv state; the read-outs pass through
+        # per token and head: the gate's blend and the read-out, each over the d x dv state; the read-outs of a prompt pass through
         # memory twice (recurrence -> heads' norm), the state once each way
-        return "hgrn2 %d tokens" % T, nbytes(proj, out) + 2 * nbytes(raw) + 2 * B * H * d * dv * 4, 4.0 * T * H * d * dv
+        return "hgrn2 %d tokens" % T, nbytes(proj, out) + (0 if T == B else 2 * nbytes(raw)) + 2 * B * H * d * dv * 4, 4.0 * T * H * d * dv
     if name == "gla_tiles":
         proj, raw, seq_slot, n_tiles, out = a[0], a[5], a[7], a[9], a[10]
         H, d, dv = a[11], a[12], a[13]
@@ -295,6 +295,10 @@ def kernel_cost(name, a, kw, kv_tokens, torch):
         return "softcap %dx%d" % tuple(a[0].shape), 2 * nbytes(a[0]), 0.0
     if name == "time_conv":
         return "time_conv %dx%d" % tuple(a[0].shape), nbytes(a[0], a[3]), 0.0
+    if name == "gemm_gated_bias":
+        x, w, out, stream = a[0], a[1], a[3], a[4]
+        return "gemm_gated_bias %dx%dx%d" % (x.shape[0], w.shape[0], x.shape[1]), nbytes(x, w, out) + 2 * nbytes(stream), \
+            2.0 * x.shape[0] * w.numel()
     if name == "gated_bias_act":
         return "gated_bias_act %dx%d" % tuple(a[0].shape), nbytes(a[0], a[2]) + (2 * nbytes(a[4]) if len(a) > 4 and a[4] is not None else 0), 0.0
     if name == "sigmoid_gate":
