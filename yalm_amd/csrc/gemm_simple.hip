@@ -296,14 +296,15 @@ extern "C" int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float
   H.bias = bias;
   // A decode step's kernel (gemm_skinny_kernel) adds the stream's bias; with more rows a launch of its own is worth less than what
   // the tiles' epilogues would take longer (1,909 rows, 4,096 of 14,336 columns: 74 us more for 12).
-  if (dtype == YALM_BF16 && M <= 16 && K % 8 == 0 && !force_simple && !((uintptr_t)A & 15) && !((uintptr_t)W & 15)) {
+  const bool inside = dtype == YALM_BF16 && M <= 16 && K % 8 == 0 && !force_simple && !((uintptr_t)A & 15) && !((uintptr_t)W & 15);
+  if (inside) {
     H.x = x;
     H.x_bias = x_bias;
     H.dim = dim;
-  } else {
-    const long n = (long)M * dim;
-    row_bias_kernel<<<(int)min((n + 1023) / 1024, 65535L), 256, 0, stream>>>(x, x_bias, n, dim);
-    if (int rc = launch_status(); rc != YALM_OK) return rc;
   }
-  return gemm_any(A, W, C, workspace, workspace_floats, M, N, K, dtype, EPI_GATED_BIAS, H, force_simple, stream);
+  const int rc = gemm_any(A, W, C, workspace, workspace_floats, M, N, K, dtype, EPI_GATED_BIAS, H, force_simple, stream);
+  if (rc != YALM_OK || inside) return rc;
+  const long n = (long)M * dim;
+  row_bias_kernel<<<(int)min((n + 1023) / 1024, 65535L), 256, 0, stream>>>(x, x_bias, n, dim);
+  return launch_status();
 }
