@@ -454,6 +454,25 @@ def test_gemm_float32_by_terms_of_extreme_numbers(M, N, Kd):
     assert bool((got[3][inf_row] == want[3][inf_row]).all())
 
 
+# Operands at the lower end of float32, whose last terms would fall off bfloat16's: every row (or weight row) at another power of
+# two from 2^-100 into the subnormal numbers, the other operand large, so that the sums are ordinary numbers; a workgroup of one group
+# and of two
+@pytest.mark.parametrize("small", ["a", "w"])
+@pytest.mark.parametrize("M,N,tile", [(97, 5130, 0), (513, 5131, 3)])
+def test_gemm_float32_by_terms_of_small_numbers(M, N, tile, small):
+    from yalm_amd.ops import library
+    k, Kd = K(), 512
+    assert library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) == tile
+    scale = lambda n: torch.tensor([2.0 ** -(100 + i % 46) for i in range(n)], dtype=torch.float64)[:, None]
+    a, w = (rnd((n, Kd), s, torch.float64) * (scale(n) if name == small else 2.0 ** 80) for n, s, name in ((M, 141, "a"), (N, 142, "w")))
+    a, w = a.float(), w.float()
+    want = a.double().to(DEV) @ w.double().to(DEV).t()
+    got = k.gemm(a.to(DEV), w.to(DEV), torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double()
+    axis = 1 if small == "a" else 0
+    # as for ordinary numbers, row by row (column by column)
+    assert float(((got - want).norm(dim=axis) / want.norm(dim=axis)).max()) <= 1e-6
+
+
 # float32 on the matrix cores: the edges of the smallest tiles and of the rules (16 | 17 and 32 | 33 rows, 4,096 and 8,192
 # columns), of one k tile and a few, K short of one round of the waves, operands 4 bytes off
 @pytest.mark.parametrize("M,N,Kd,off", [

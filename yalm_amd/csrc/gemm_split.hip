@@ -1,8 +1,14 @@
 // C = epilogue(A[M,K] * W[N,K]^T) in float32, more than 64 rows, on the matrix cores' bfloat16 products: a float is the sum
-// of three bfloat16 numbers (8 + 8 + 8 significant bits; exact from 2^-108 up, below that to 2^-134), and of the nine products of
-// two such sums the six largest are made and added in float32, the smallest first.  The three left out are below 2^-25 of
-// the product, under the rounding of one addition.  v_mfma_f32_16x16x32_bf16 takes 32 products in the time in which
-// v_mfma_f32_16x16x4_f32 takes 2, so six of them still leave a factor of 2.7 over gemm_f32.hip's tiles.
+// of three bfloat16 numbers (8 + 8 + 8 significant bits), and of the nine products of two such sums the six largest are made and
+// added in float32, the smallest first (the way of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations", 2019).  The three left out are below 2^-25 of the product, under the rounding of one
+// addition.  v_mfma_f32_16x16x32_bf16 takes 32 products in the time in which v_mfma_f32_16x16x4_f32 takes 2, so six of them still
+// leave a factor of 2.7 over gemm_f32.hip's tiles.
+//
+// A bfloat16 number has float32's exponents, so the last terms of a float below 2^-108 would fall off their end (an operand of 2^-120
+// kept 14 bits).  Both operands are therefore split at 2^41 times their size, where every float, a subnormal one too, is the sum of its
+// terms exactly, and a fold's sums come back by 2^-82 as they join the total.  What that leaves no room for (an operand from about 2^87
+// on, a fold's sum from 2^46 on) comes out as no finite number, and is made again with float32 products like an infinity.
 //
 // The error against 64 bits is smaller than gemm_f32_kernel's, whose sums are chains of four products at a time: relative, K 512
 // 1.6e-7 (2.9e-7), 3,072 1.7 to 1.8e-7 (2.95e-7), 8,192 1.9 to 2.1e-7 (3.05e-7), 14,336 2.1 to 2.5e-7 (3.2e-7).  The instruction drops the
@@ -33,6 +39,8 @@ constexpr int ROWB = TK * 2;                     // bytes of a row in one of the
 constexpr int TERMS = 3;
 constexpr int GROUP = 4;                         // tile columns that an XCD walks together
 constexpr int FOLD = 4;                          // k tiles whose sums join before they are added to the total (8: the errors 1.4 times these, 2 % sooner)
+
+constexpr float UP = 0x1p41f, DOWN = 0x1p-82f;   // the operands' scale on the way into terms, and the sums' on the way back
 
 struct Terms { u32x4 t[TERMS]; };
 
@@ -96,16 +104,15 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
 #pragma unroll
       for (int h = 0; h < 2; ++h) raw[i][h] = *reinterpret_cast<const f32x4*>(from[i] + (size_t)kt * TK + h * 4);
   };
-  unsigned flip = 0;                               // what turns A's signs in the tile that is stored
+  float a_scale = UP;                              // A's scale in the tile that is stored, with the sign that it takes there
   auto store = [&](int buf, int i) {
     if ((i + 1) * NT > ROWS * 4 && (wave + i * NW) * WAVE >= ROWS * 4) return;    // a last share that only some waves have
-    if (i * NT < TM * 4) {                         // rows of A among them (whole waves')
-      const unsigned by = (i + 1) * NT <= TM * 4 || (wave + i * NW) * WAVE < TM * 4 ? flip : 0u;
+    // rows of A or of W (whole waves')
+    const float by = i * NT < TM * 4 && ((i + 1) * NT <= TM * 4 || (wave + i * NW) * WAVE < TM * 4) ? a_scale : UP;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) raw[i][h][e] = __uint_as_float(__float_as_uint(raw[i][h][e]) ^ by);
-    }
+      for (int e = 0; e < 4; ++e) raw[i][h][e] *= by;
     Terms s;
     split4(s, 0, raw[i][0]);
     split4(s, 1, raw[i][1]);
@@ -133,9 +140,9 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
 
   const int nk = K / TK, mine = (nk - grp + KG - 1) / KG, most = (nk + KG - 1) / KG;     // this group's k tiles: grp, grp + KG, ...
   auto tile_of = [&](int i) { return min(grp + i * KG, nk - 1); };               // (behind the last one: read again, not used)
-  auto sign_of = [&](int i) { return (unsigned)(((i / FOLD + grp) & 1) << 31); };
+  auto turned = [&](int i) { return ((i / FOLD + grp) & 1) != 0; };               // whether tile i's fold takes A with its signs turned
   load(tile_of(0));
-  flip = sign_of(0);
+  a_scale = turned(0) ? -UP : UP;
 #pragma unroll
   for (int i = 0; i < U; ++i) store(0, i);
   load(tile_of(1));
@@ -147,7 +154,7 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
   // The barrier stands in front of the last column's products: by then nobody reads `buf` any more, the next tile is whole, and
   // its first fragments are read among these products.
   auto one_tile = [&](int i, int buf) {
-    flip = sign_of(i + 1);
+    a_scale = turned(i + 1) ? -UP : UP;
 #pragma unroll
     for (int b = 0; b < FB - 1; ++b) {
       bf16x8 next[TERMS];
@@ -189,14 +196,14 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
   for (int k0 = 0; k0 < mine; k0 += FOLD) {
     const int k1 = min(k0 + FOLD, mine);
     for (int i = k0; i < k1; ++i) one_tile(i, i & 1);
-    const float sign = sign_of(k0) != 0 ? -1.f : 1.f;
+    const float back = turned(k0) ? -DOWN : DOWN;
 #pragma unroll
     for (int a = 0; a < FA; ++a)
 #pragma unroll
       for (int b = 0; b < FB; ++b) {
         asm volatile("" : "+v"(acc[a][b]));        // added here, not in every turn of the loop
 #pragma unroll
-        for (int r = 0; r < 4; ++r) total[a][b][r] = fmaf(acc[a][b][r], sign, total[a][b][r]);
+        for (int r = 0; r < 4; ++r) total[a][b][r] = fmaf(acc[a][b][r], back, total[a][b][r]);
         acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
       }
   }
@@ -218,8 +225,8 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
       for (int b = 0; b < FB; ++b) total[a][b] += other[(a * FB + b) * NT + tid];
   }
 
-  // An infinity, a NaN, or a number that rounds to infinity as bfloat16 (from 3.39e38) makes every sum that it enters a NaN
-  // (infinity less infinity in its terms).  A wave that holds a sum that is no finite number makes all of its sums again with
+  // An infinity, a NaN, or a number that is infinite at 2^41 times its size makes every sum that it enters a NaN (infinity less
+  // infinity in its terms), and a fold's sum that has no room is infinite.  A wave that holds a sum that is no finite number makes all of its sums again with
   // float32 products, chains as in gemm_f32_kernel.
   bool bad = false;
 #pragma unroll
