@@ -450,8 +450,24 @@ def test_gemm_float32_by_terms_of_extreme_numbers(M, N, Kd):
     assert int(ok.sum()) > (M - 4) * (N - 1) - 1
     assert bool(((got - want).abs()[ok] <= ((2.0 * Kd + 2.0) * 2.0 ** -24 * size + Kd * 2.0 ** -126)[ok]).all())
     assert float((got[71] - want[71])[:N - 2].norm() / want[71][:N - 2].norm()) <= 1e-6
-    inf_row = want[3].isinf()
-    assert bool((got[3][inf_row] == want[3][inf_row]).all())
+
+
+# Sums that are not finite are made again; the sums beside them, of the same wave too, keep the bits that they have without such a
+# neighbour: one row and one weight row of infinities and NaN, the last ones (which the rows behind the edge repeat) among them
+@pytest.mark.parametrize("M,N,tile", [(97, 5130, 0), (161, 8201, 1), (513, 5131, 3), (321, 20001, 5)])
+def test_gemm_float32_by_terms_beside_numbers_that_are_not_finite(M, N, tile):
+    from yalm_amd.ops import library
+    k, Kd = K(), 512
+    assert library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) == tile
+    a, w = rnd((M, Kd), 143).to(DEV), rnd((N, Kd), 144).to(DEV)
+    plain = k.gemm(a, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32)
+    rows, cols = [5, 40, M - 1], [3, 77, N - 1]
+    for r, c, v in zip(rows, cols, (math.inf, math.nan, -math.inf)):
+        a[r, 9], w[c, 100] = v, v
+    got = k.gemm(a, w, torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32)
+    assert not bool(got[rows].isfinite().any()) and not bool(got[:, cols].isfinite().any())
+    keep_m, keep_n = [m for m in range(M) if m not in rows], [n for n in range(N) if n not in cols]
+    assert torch.equal(got[keep_m][:, keep_n], plain[keep_m][:, keep_n])
 
 
 # Operands at the lower end of float32, whose last terms would fall off bfloat16's: every row (or weight row) at another power of

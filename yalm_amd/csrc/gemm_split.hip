@@ -226,46 +226,44 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
   }
 
   // An infinity, a NaN, or a number that is infinite at 2^41 times its size makes every sum that it enters a NaN (infinity less
-  // infinity in its terms), and a fold's sum that has no room is infinite.  A wave that holds a sum that is no finite number makes all of its sums again with
-  // float32 products, chains as in gemm_f32_kernel.
-  bool bad = false;
+  // infinity in its terms), and a fold's sum that has no room is infinite.  Sums that are no finite numbers are made again with float32
+  // products, chains as in gemm_f32_kernel, 16 rows at a time; the sums beside them stay as they are.
+  auto finite = [](float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; };
 #pragma unroll
-  for (int a = 0; a < FA; ++a)
+  for (int a = 0; a < FA; ++a) {
+    bool all = true;
 #pragma unroll
     for (int b = 0; b < FB; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bad |= (__float_as_uint(total[a][b][r]) & 0x7f800000u) == 0x7f800000u;
-  if (__any(bad)) {
-    const float *ra[FA], *rw[FB];
+      for (int r = 0; r < 4; ++r) all &= finite(total[a][b][r]);
+    if (__all(all)) continue;
+    const float *ra = A + (size_t)min(m0 + (wm * FA + a) * 16 + l16, M - 1) * K + lq * 4, *rw[FB];
+    f32x4 again[FB], fold[FB];
 #pragma unroll
-    for (int a = 0; a < FA; ++a) ra[a] = A + (size_t)min(m0 + (wm * FA + a) * 16 + l16, M - 1) * K + lq * 4;
-#pragma unroll
-    for (int b = 0; b < FB; ++b) rw[b] = W + (size_t)min(n0 + (wn * FB + b) * 16 + l16, N - 1) * K + lq * 4;
-#pragma unroll
-    for (int a = 0; a < FA; ++a)
-#pragma unroll
-      for (int b = 0; b < FB; ++b) total[a][b] = acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < FB; ++b) {
+      rw[b] = W + (size_t)min(n0 + (wn * FB + b) * 16 + l16, N - 1) * K + lq * 4;
+      again[b] = fold[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
     for (int k = 0; k < K; k += 16) {
-      f32x4 va[FA], vw[FB];
-#pragma unroll
-      for (int a = 0; a < FA; ++a) va[a] = *reinterpret_cast<const f32x4*>(ra[a] + k);
+      const f32x4 va = *reinterpret_cast<const f32x4*>(ra + k);
+      f32x4 vw[FB];
 #pragma unroll
       for (int b = 0; b < FB; ++b) vw[b] = *reinterpret_cast<const f32x4*>(rw[b] + k);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int a = 0; a < FA; ++a)
-#pragma unroll
-          for (int b = 0; b < FB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[a][e], vw[b][e], acc[a][b], 0, 0, 0);
+        for (int b = 0; b < FB; ++b) fold[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[e], vw[b][e], fold[b], 0, 0, 0);
       if ((k + 16) % (FOLD * TK) == 0 || k + 16 == K)
 #pragma unroll
-        for (int a = 0; a < FA; ++a)
-#pragma unroll
-          for (int b = 0; b < FB; ++b) {
-            total[a][b] += acc[a][b];
-            acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-          }
+        for (int b = 0; b < FB; ++b) {
+          again[b] += fold[b];
+          fold[b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
     }
+#pragma unroll
+    for (int b = 0; b < FB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) total[a][b][r] = finite(total[a][b][r]) ? total[a][b][r] : again[b][r];
   }
 
   // lane (lq, l16) holds rows 4 lq .. 4 lq + 3 of column l16 of every 16 x 16
