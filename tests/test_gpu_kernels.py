@@ -443,9 +443,12 @@ def test_gemm_float32_by_terms_of_extreme_numbers(M, N, Kd):
     want = a.double() @ w.double().t()
     got = k.gemm(a.to(DEV), w.to(DEV), torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double().cpu()
     size = a.double().abs() @ w.double().abs().t()
-    over = size >= 3.4e38                                               # whose sums may pass float32's largest on the way
+    over = size.isfinite() & (size >= 3.4e38)                           # whose sums may pass float32's largest on the way
+    inf = want.isinf()
+    assert int(inf.sum()) > M + 2 * N - 6 and int((inf & over).sum()) == 0
     assert torch.equal(got.isnan() & ~over, want.isnan() & ~over)
-    assert torch.equal(got.isinf() & ~over, want.isinf() & ~over)
+    assert torch.equal(got.isinf() & ~over, inf & ~over)
+    assert torch.equal(got[inf], want[inf])                             # of the same sign
     ok = size < 3.4e38
     assert int(ok.sum()) > (M - 4) * (N - 1) - 1
     assert bool(((got - want).abs()[ok] <= ((2.0 * Kd + 2.0) * 2.0 ** -24 * size + Kd * 2.0 ** -126)[ok]).all())
