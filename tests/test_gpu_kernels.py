@@ -1693,8 +1693,8 @@ def test_gemm_norm_float32_refuses_what_it_does_not_take():
 @pytest.mark.parametrize("n_heads,n_kv,hd,rd,D", [(4, 2, 16, 16, 64), (3, 1, 48, 32, 96), (6, 3, 32, 0, 96), (32, 8, 128, 128, 256)])
 @pytest.mark.parametrize("M", [5, 11])
 def test_gemm_norm_qkv_rope_float32(n_heads, n_kv, hd, rd, D, M):
-    """norm + q/k/v + rotation + cache write of a float32 decode step in one kernel: the bits of the kernels one by one (of the
-    rotated elements up to the rounding of a fused multiply-add)."""
+    """norm + q/k/v + rotation + cache write of a float32 decode step in one kernel: the bits of the kernels one by one, which a step
+    of 17 rows takes."""
     k = K()
     pos = ([0, 63, 64, 130, 7] + list(range(190, 196)))[:M]
     slots = ([3, 0, -1, 2, 1] + list(range(4, 10)))[:M]                    # row 2 is a padding row
@@ -1712,11 +1712,9 @@ def test_gemm_norm_qkv_rope_float32(n_heads, n_kv, hd, rd, D, M):
     qkv = k.gemm(h, w, torch.empty((M, Q + 2 * KV), device=DEV), k.EPI_STORE_F32)
     k.rope_kv_write(qkv, q[1], None, None, None, pages[0][1], pages[1][1], bt, ring, i32(list(range(M))), i32(pos), i32(slots),
                     i32([p + 1 for p in pos]), table, n_heads, n_kv, hd, rd)
-    assert torch.equal(pages[1][0], pages[1][1])
-    # a rotated element is x0 c - x1 s with one of its two products rounded by itself, or none: 2 roundings of at most 2^-24 of it
-    bound = 2 * 2.0 ** -24 * 2 * float(qkv.abs().max())
-    assert float((q[0] - q[1]).abs().max()) <= bound and float((pages[0][0] - pages[0][1]).abs().max()) <= bound
-    assert torch.equal(q[0] != 0, q[1] != 0) and torch.equal(pages[0][0] != 0, pages[0][1] != 0)
+    assert torch.equal(q[0], q[1])
+    for p in pages:
+        assert torch.equal(p[0], p[1]) and bool((p[0] != 0).any())
 
 
 @pytest.mark.parametrize("M", [1, 5, 16])

@@ -110,6 +110,13 @@ __device__ __forceinline__ float gate_value(float g, float u, const GateOut& out
   return gate_unit<EPI>(g, u, out);
 }
 
+// An element of a pair of neighbours, turned by the angle whose cosine and sine are c; `other` the pair's other element, `odd` whether
+// this is the second one.  The other element's product is rounded by itself: which of the two is would be the compiler's choice in
+// each kernel, and a row of a float32 step is to have the same bits in the kernels of its different numbers of rows.
+__device__ __forceinline__ float rotate_one(float x, float other, bool odd, float2 c) {
+  return fmaf(x, c.x, odd ? other * c.y : -(other * c.y));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);

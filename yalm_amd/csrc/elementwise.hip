@@ -238,8 +238,8 @@ __global__ __launch_bounds__(ROPE_JOBS * WAVE) void rope_kv_write_kernel(const f
       float x0 = x.x, x1 = x.y;
       if (rotate && p < half_rot) {
         float2 c = cs[p];
-        float y0 = x0 * c.x - x1 * c.y;
-        float y1 = x0 * c.y + x1 * c.x;
+        float y0 = rotate_one(x0, x1, false, c);
+        float y1 = rotate_one(x1, x0, true, c);
         x0 = y0;
         x1 = y1;
       }
@@ -289,8 +289,8 @@ __global__ __launch_bounds__(ROPE_JOBS * WAVE) void rope_kv_write_kernel(const f
       float x0 = x.x, x1 = x.y;
       if (rotate && p < half_rot) {
         float2 c = cs[p];
-        float y0 = x0 * c.x - x1 * c.y;
-        float y1 = x0 * c.y + x1 * c.x;
+        float y0 = rotate_one(x0, x1, false, c);
+        float y1 = rotate_one(x1, x0, true, c);
         x0 = y0;
         x1 = y1;
       }
@@ -407,8 +407,8 @@ __global__ __launch_bounds__(256) void rope_kv_tiles_kernel(
       if (cos_sin != nullptr && p + u < half_rot && pos < n_positions) {
         const float2 c = cos_sin[(size_t)pos * half_rot + p + u];
         const float a = v[2 * u], b2 = v[2 * u + 1];
-        v[2 * u] = a * c.x - b2 * c.y;
-        v[2 * u + 1] = a * c.y + b2 * c.x;
+        v[2 * u] = rotate_one(a, b2, false, c);
+        v[2 * u + 1] = rotate_one(b2, a, true, c);
       }
     }
   };

@@ -388,7 +388,7 @@ __global__ __launch_bounds__(NWV * WAVE, 2) void gemm_few_f32_kernel(const float
         float y = v[r];
         if (region < 2 && out.cos_sin != nullptr && pair < out.rotary_dim / 2 && pos >= 0 && pos < out.n_positions) {
           const float2 c = out.cos_sin[(size_t)pos * (out.rotary_dim / 2) + pair];
-          y = (i & 1) ? other * c.y + v[r] * c.x : v[r] * c.x - other * c.y;
+          y = rotate_one(v[r], other, (i & 1) != 0, c);
         }
         if (region == 0) {
           out.q_out[(size_t)m * Q + n] = y;
