@@ -1690,6 +1690,27 @@ def test_gemm_norm_float32_refuses_what_it_does_not_take():
                         torch.empty((M, N), device=DEV), k.EPI_STORE_F32)
 
 
+# Either side of the lines up to which a float32 step folds a norm into the product behind it: what follows from them is asked of the
+# parts (whose weights' shapes are all that they look at)
+@pytest.mark.parametrize("part,M,N,D,folded", [
+    ("head", 1, 128256, 2048, False), ("head", 16, 128256, 1024, False), ("head", 3, 512, 256, True), ("head", 16, 8192, 1024, True),
+    ("head", 1, 8193, 1024, False), ("head", 1, 4096, 1056, False), ("head", 17, 512, 256, False),
+    ("mlp", 16, 8192, 1024, True), ("mlp", 1, 8224, 1024, False), ("mlp", 4, 2048, 2048, False),
+    ("attention", 16, 6144, 4096, True), ("attention", 1, 8192, 1024, True), ("attention", 1, 12288, 2048, False)])
+def test_float32_steps_fold_a_norm_where_it_pays(part, M, N, D, folded):
+    from types import SimpleNamespace as NS
+    from yalm_amd.parts.attention import GQAttention
+    from yalm_amd.parts.embedding import LMHead
+    from yalm_amd.parts.swiglu import SwiGLU
+    w = torch.empty((N, D), device="meta")
+    kind, fields = {"head": (LMHead, dict(weight=w)), "mlp": (SwiGLU, dict(w_gate_up=w, w_down=w, unit=None)),
+                    "attention": (GQAttention, dict(wo=w, head_dim=64, q_dim=N // 2, kv_dim=N // 4))}[part]
+    one = kind.__new__(kind)
+    vars(one).update(fields, dim=D)
+    ctx, norm = NS(mode="decode", normed={}), NS(fused=lambda: None)
+    assert one.fuses_norm(norm, torch.empty((M, D), device="meta"), ctx) == folded
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,rd,D", [(4, 2, 16, 16, 64), (3, 1, 48, 32, 96), (6, 3, 32, 0, 96), (32, 8, 128, 128, 256)])
 @pytest.mark.parametrize("M", [5, 11])
 def test_gemm_norm_qkv_rope_float32(n_heads, n_kv, hd, rd, D, M):

@@ -504,6 +504,16 @@ int split_tile(int M, int N, int K, bool gate) {
 bool takes_norm(int M, int N, int K, bool gate) {
   return M >= 1 && M <= 16 && N > 0 && K > 0 && K % TK == 0 && choose(M, N, K, gate).kernel == Choice::FEW;
 }
+// Whether a step is sooner with it than with the norm's kernel in front (and the rotation's behind, `qkv`): every workgroup forms the
+// rows' sums of squares anew, which pays while there are at most two of them a CU, one in the wide form, and without the rotation's launch
+// while a wave takes a row at once (K to 1,024).  us folded and apart, one row and 16: 4,096 x 1,024 8.4 and 10.7, 11.3 and 12.2; 8,192
+// x 1,024 12.7 and 13.9, 15.3 and 16.0; gated 12.9 and 14.4, 15.6 and 16.3.  More weight rows: 10,240 x 512 11.0 and 9.9, gated 13.2 and
+// 11.4; 128,256 x 2,048 246 and 191, 287 and 237.  Longer rows: 4,096 x 1,056 8.1 and 8.1, 11.4 and 10.1; 2,048 x 2,048 10.5 and
+// 10.1, 15.2 and 13.0.  q/k/v: 6,144 x 1,024 12.6 and 16.3, 17.3 and 18.8; 6,144 x 4,096 33.1 and 35.2, 39.2 and 38.5 (a step of four
+// 7B layers 955 and 974, 1,137 and 1,152); 12,288 x 2,048 32.8 and 29.0, 44.7 and 38.6.
+bool norm_pays(int M, int N, int K, bool gate, bool qkv) {
+  return takes_norm(M, N, K, gate) && N <= 32L * compute_units() && (qkv || K <= 1024);
+}
 template <int EPI>
 int launch_norm(const float* x, const float* W, float* C, int M, int N, int K, GateOut H, NormIn norm, QkvOut out, hipStream_t stream) {
   if constexpr (gated(EPI)) return launch_few<EPI, 1, 2, true>(x, W, C, M, N, K, H, stream, norm, out);
@@ -557,6 +567,9 @@ extern "C" int yalm_gemm_f32_choice(int M, int N, int K, int gate) {
 
 // Whether yalm_gemm_norm_f32 (and the q/k/v form) takes the product
 extern "C" int yalm_gemm_norm_f32_takes(int M, int N, int K, int gate) { return takes_norm(M, N, K, gate != 0); }
+
+// Whether it is sooner than the kernels one by one; what: 0 a plain product, 1 a gated one, 2 q/k/v
+extern "C" int yalm_gemm_norm_f32_pays(int M, int N, int K, int what) { return norm_pays(M, N, K, what == 1, what == 2); }
 
 static bool norm_operands_ok(const float* x, const float* norm_w, const float* W) {
   return x != nullptr && norm_w != nullptr && W != nullptr && !((uintptr_t)x & 15) && !((uintptr_t)norm_w & 15) && !((uintptr_t)W & 15);

@@ -75,8 +75,10 @@ int yalm_gemm_norm_qkv_rope(const float* x, const float* norm_w, float eps, cons
                             int page_layout, hipStream_t stream);
 
 // The same two with float32 weights and results, M <= 16 rows and K a multiple of 32, where yalm_gemm_norm_f32_takes the product
-// (narrow ones: N below 8,192 or K up to 2,048).  The bits are those of yalm_rmsnorm and yalm_gemm.
+// (narrow ones: N below 8,192 or K up to 2,048).  The bits are those of yalm_rmsnorm and yalm_gemm (and yalm_rope_kv_write).
 int yalm_gemm_norm_f32_takes(int M, int N, int K, int gate);
+// Whether it takes the product and is sooner than those kernels; what: 0 a plain product, 1 a gated one, 2 q/k/v
+int yalm_gemm_norm_f32_pays(int M, int N, int K, int what);
 int yalm_gemm_norm_f32(const float* x, const float* norm_w, float eps, const float* W, float* C, int M, int N, int K, int epilogue,
                        int H, hipStream_t stream);
 int yalm_gemm_norm_qkv_rope_f32(const float* x, const float* norm_w, float eps, const float* Wqkv, float* q_out, float* k_pages,

@@ -221,6 +221,13 @@ def can_fuse_norm(M, K, dtype, N, gate=False):
         M * (K + 8) * 2 <= 72 * 1024 and not FORCE_SIMPLE
 
 
+def fuse_norm_pays(M, K, dtype, N, gate=False, qkv=False):
+    """Whether gemm_norm (qkv: gemm_norm_qkv_rope) takes this shape and is sooner than the kernels one by one."""
+    if dtype == torch.float32:
+        return not FORCE_SIMPLE and bool(library.lib().yalm_gemm_norm_f32_pays(int(M), int(N), int(K), 2 if qkv else 1 if gate else 0))
+    return can_fuse_norm(M, K, dtype, N, gate)
+
+
 def gemm_norm(x, norm_w, eps, w, out, epilogue, hidden=0):
     """out = epilogue(rmsnorm(x, norm_w, eps) @ w^T) for at most 16 rows of the float32
     residual stream x; w bfloat16 or float32 [N, K], norm_w float32 [K]; EPI_STORE_F32, EPI_GATED or EPI_GATED_GELU (out in w's dtype).

@@ -161,7 +161,7 @@ class GQAttention(Part):
         if ctx.mode != "decode":
             return False
         if self.wo.dtype == torch.float32:
-            return kernels.can_fuse_norm(T, self.dim, torch.float32, self.q_dim + 2 * self.kv_dim)
+            return kernels.fuse_norm_pays(T, self.dim, torch.float32, self.q_dim + 2 * self.kv_dim, qkv=True)
         return kernels.can_chain(T, self.dim, self.wo.dtype) or kernels.can_add_norm(T, self.dim, self.wo.dtype)
 
     def forward_prenorm(self, x, norm, ctx, line, writes_cache=True, emit_for=None):
@@ -195,7 +195,7 @@ class GQAttention(Part):
             kernels.gemm_chain_qkv_rope(xn, (ss, eps), self.wqkv, q, k_pages, v_pages, group.table, group.ring_pages,
                                         ctx.tok_pos, ctx.seq_slot, pos.table, self.n_heads, self.n_kv_heads,
                                         self.head_dim, pos.rotary_dim)
-        elif src is None and kernels.can_fuse_norm(T, self.dim, self.wo.dtype, self.q_dim + 2 * self.kv_dim):
+        elif src is None and kernels.fuse_norm_pays(T, self.dim, self.wo.dtype, self.q_dim + 2 * self.kv_dim, qkv=True):
             nw, eps = norm.fused()
             kernels.gemm_norm_qkv_rope(x, nw, eps, self.wqkv, q, k_pages, v_pages, group.table, group.ring_pages,
                                        ctx.tok_pos, ctx.seq_slot, pos.table, self.n_heads, self.n_kv_heads,

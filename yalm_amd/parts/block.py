@@ -85,7 +85,7 @@ class PreNormResidualBlock(Part):
         # sublayers that fold no norm into their products leave nothing for whoever reads the stream next: in a decode
         # step the layer then ends with that norm as a kernel of its own, so that the head's product (or the next
         # layer's first) takes its output as it is instead of norming the rows again for every tile of its weights (in float32
-        # a consumer that cannot fold the norm in runs it itself, and one that can saves the launch)
+        # a consumer that does not fold the norm in runs it itself, and one that does saves the launch)
         if plain_end and ctx.mode == "decode" and ctx.act_dtype != x.dtype and next_norm is not None and hasattr(next_norm, "fused") \
                 and id(next_norm) not in ctx.normed:
             ahead = ctx.ws.get("block.ahead", (x.shape[0], self.dim), ctx.act_dtype)

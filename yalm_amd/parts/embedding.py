@@ -135,7 +135,7 @@ class LMHead(Part):
             return True                                   # whoever prepared it checked the shape
         if not hasattr(norm, "fused"):
             return False
-        return kernels.can_fuse_norm(x.shape[0], self.dim, self.weight.dtype, self.weight.shape[0])
+        return kernels.fuse_norm_pays(x.shape[0], self.dim, self.weight.dtype, self.weight.shape[0])
 
     def forward_prenorm(self, x, norm, logits, ctx):
         """logits for every row of x (no row selection)."""

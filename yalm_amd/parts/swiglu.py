@@ -74,7 +74,7 @@ class SwiGLU(Part):
         if ctx.mode == "prefill":             # takes the norm's output where the product before has left it
             return kernels.can_add_norm(T, self.dim, self.w_down.dtype)
         if self.w_down.dtype == torch.float32:
-            return kernels.can_fuse_norm(T, self.dim, torch.float32, self.w_gate_up.shape[0], gate=True)
+            return kernels.fuse_norm_pays(T, self.dim, torch.float32, self.w_gate_up.shape[0], gate=True)
         return kernels.can_chain(T, self.dim, self.w_down.dtype) or kernels.can_add_norm(T, self.dim, self.w_down.dtype)
 
     def forward_prenorm(self, x, norm, ctx, emit_for=None):
@@ -89,7 +89,7 @@ class SwiGLU(Part):
             self._gemm(ctx, xn, self.w_gate_up, mid, self.gated, hidden=self.hidden, scale_from=(ss, eps))
         elif src is not None:                     # the norm's output is ready
             self._gemm(ctx, src[0], self.w_gate_up, mid, self.gated, hidden=self.hidden)
-        elif kernels.can_fuse_norm(T, self.dim, self.w_down.dtype, self.w_gate_up.shape[0], gate=True):
+        elif kernels.fuse_norm_pays(T, self.dim, self.w_down.dtype, self.w_gate_up.shape[0], gate=True):
             nw, eps = norm.fused()
             kernels.gemm_norm(x, nw, eps, self.w_gate_up, mid, self.gated, hidden=self.hidden)
         else:
