@@ -735,3 +735,10 @@ def test_decode_metadata_orders_a_ragged_batch_by_length():
         ls = [int(x) for x in rng.integers(1, 5000, size=B)]
         Engine._fill_decode_meta(host, Bk, [0] * B, [n - 1 for n in ls], list(range(B)), ls, ragged=True)
         assert sorted(host[6 * Bk + 2:7 * Bk + 2]) == list(range(Bk))
+
+
+def test_whether_a_norm_can_be_folded_in_is_asked_without_the_weights_rows():
+    """The three-argument form, which float32 (whose answer hangs on the weight's rows) answers with no."""
+    from yalm_amd.ops import kernels
+    assert kernels.can_fuse_norm(8, 4096, torch.bfloat16) and not kernels.can_fuse_norm(9, 4096, torch.bfloat16)
+    assert not kernels.can_fuse_norm(8, 4096, torch.float32)

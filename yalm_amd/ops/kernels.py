@@ -212,11 +212,11 @@ def gemm_gated_bias(a, w, bias, out, x, x_bias, workspace=None):
 FUSED_NORM_MAX_ROWS = 8
 
 
-def can_fuse_norm(M, K, dtype, N, gate=False):
-    """Whether gemm_norm / gemm_norm_qkv_rope take this shape (else: rmsnorm, then gemm); N: the weight's rows, gate: whether the
-    epilogue is a gated one."""
+def can_fuse_norm(M, K, dtype, N=None, gate=False):
+    """Whether gemm_norm / gemm_norm_qkv_rope take this shape (else: rmsnorm, then gemm); N: the weight's rows (which float32 asks
+    for), gate: whether the epilogue is a gated one."""
     if dtype == torch.float32:
-        return not FORCE_SIMPLE and bool(library.lib().yalm_gemm_norm_f32_takes(int(M), int(N), int(K), 1 if gate else 0))
+        return N is not None and not FORCE_SIMPLE and bool(library.lib().yalm_gemm_norm_f32_takes(int(M), int(N), int(K), 1 if gate else 0))
     return dtype == torch.bfloat16 and 1 <= M <= FUSED_NORM_MAX_ROWS and K % 8 == 0 and \
         M * (K + 8) * 2 <= 72 * 1024 and not FORCE_SIMPLE
 
