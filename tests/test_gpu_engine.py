@@ -389,3 +389,28 @@ def test_a_decode_batch_of_very_unequal_lengths(tmp_path_factory, dtype):
     for rid, toks in requests.items():
         want = helpers.plain_logits(folder, tuple(toks), dtype)
         helpers.check_logits(got[rid][first[rid] - 1:], want[first[rid] - 1:], dtype, "ragged batch %s request %s" % (dtype, rid))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_weights_that_lie_between_16_bytes(folders, dtype):
+    """A model loaded from parts of larger device buffers, 4 bytes off, computes what the one from its folder does."""
+    from yalm_amd.config import config_from_folder
+    from yalm_amd.engine import Engine, Model
+    from yalm_amd.weights import TensorSource
+    source = TensorSource(folders["tiny_llama"])
+
+    def get(name):
+        t = source.get(name)
+        out = torch.empty(t.numel() + 4, dtype=torch.float32, device="cuda:0")[1:t.numel() + 1].view(t.shape)
+        assert out.data_ptr() % 16 == 4
+        return out.copy_(t)
+
+    cfg = config_from_folder(folders["tiny_llama"])
+    logits = []
+    for model in (Model.from_folder(folders["tiny_llama"], dtype=helpers.torch_dtype(dtype), device="cuda:0"),
+                  Model(cfg.to_spec(), cfg).load(get, helpers.torch_dtype(dtype), "cuda:0")):
+        engine = Engine(model, max_tokens=1024)
+        slots = engine.start(3)
+        engine.step(slots, [[5, 17, 3], [7], [9, 11]])
+        logits += [engine.step(slots, [[4], [6], [8]]).clone(), engine.step(slots[:1], [[2]]).clone()]
+    assert torch.equal(logits[0], logits[2]) and torch.equal(logits[1], logits[3])

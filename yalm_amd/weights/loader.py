@@ -120,5 +120,7 @@ def device_dtype(stored_dtype, ndim, compute_dtype):
 
 
 def place(t, compute_dtype, device):
-    """Copies a CPU tensor to the device in the dtype `device_dtype` gives it."""
-    return t.to(device=device, dtype=device_dtype(t.dtype, t.dim(), compute_dtype)).contiguous()
+    """A tensor on the device in the dtype `device_dtype` gives it, on 16 bytes: one that is there already, as part of a larger
+    buffer, may lie between them, and the kernels that fold a norm in refuse such weights."""
+    t = t.to(device=device, dtype=device_dtype(t.dtype, t.dim(), compute_dtype)).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
