@@ -183,6 +183,22 @@ def test_middle_of_a_gated_feed_forward_in_its_product(T, F, D, Kd, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [5, 40, 130])
+@pytest.mark.parametrize("off", [(1, 0), (0, 1), (3, 2)])
+def test_middle_of_a_gated_feed_forward_in_its_product_off_16_bytes(T, off, dtype):
+    """The stream and its bias may lie at any float."""
+    from yalm_amd.ops import kernels
+    from yalm_amd.parts.swiglu import interleave_gate_up
+    F, D, Kd = 64, 48, 64
+    h, w = randn(T, Kd, seed=1).to(dtype).to(DEV), [randn(F, Kd, seed=s, scale=Kd ** -0.5).to(dtype) for s in (2, 3)]
+    wg, bg = interleave_gate_up(*w).to(DEV), randn(2 * F, seed=4).to(DEV)
+    x, xb = randn(T, D, seed=6), randn(D, seed=7)
+    xg, xbg = (torch.empty(t.numel() + 4, device=DEV)[o:o + t.numel()].view(t.shape).copy_(t) for t, o in zip((x, xb), off))
+    kernels.gemm_gated_bias(h, wg, bg, torch.empty(T, F, dtype=dtype, device=DEV), xg, xbg)
+    assert torch.equal(xg.cpu(), x + xb)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,H,dv,pad", [(1, 1, 4, 16), (6, 3, 20, 32), (3, 8, 64, 64), (2, 40, 100, 112)])
 def test_sigmoid_gate_on_the_heads(T, H, dv, pad, dtype):
     from yalm_amd.ops import kernels

@@ -222,10 +222,10 @@ int gemm_rows_f32(const void* A, const void* W, void* C, int M, int N, int K, in
   return YALM_OK;
 }
 
-// x[m, :] += b (dim a multiple of 4 and both on 16 bytes: four elements a thread)
-__global__ __launch_bounds__(256) void row_bias_kernel(float* __restrict__ x, const float* __restrict__ b, long n, int dim) {
+// x[m, :] += b (fours: dim a multiple of 4 and both on 16 bytes, four elements a thread)
+__global__ __launch_bounds__(256) void row_bias_kernel(float* __restrict__ x, const float* __restrict__ b, long n, int dim, bool fours) {
   const long stride = (long)gridDim.x * 256, first = (long)blockIdx.x * 256 + threadIdx.x;
-  if (dim % 4 == 0) {
+  if (fours) {
     for (long i = first; i < n / 4; i += stride) {
       float4 v = reinterpret_cast<float4*>(x)[i];
       const float4 w = reinterpret_cast<const float4*>(b)[i % (dim / 4)];
@@ -289,8 +289,7 @@ extern "C" int yalm_gemm(const void* A, const void* W, void* C, float* workspace
 extern "C" int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N, int K,
                                     int dtype, int hidden, const float* bias, float* x, const float* x_bias, int dim, int force_simple,
                                     hipStream_t stream) {
-  if (bias == nullptr || x == nullptr || x_bias == nullptr || dim <= 0 || hidden <= 0 || ((uintptr_t)x & 15) || ((uintptr_t)x_bias & 15))
-    return YALM_ERR_ARG;
+  if (bias == nullptr || x == nullptr || x_bias == nullptr || dim <= 0 || hidden <= 0) return YALM_ERR_ARG;
   if (M <= 0) return YALM_OK;
   GateOut H(hidden);
   H.bias = bias;
@@ -305,6 +304,7 @@ extern "C" int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float
   const int rc = gemm_any(A, W, C, workspace, workspace_floats, M, N, K, dtype, EPI_GATED_BIAS, H, force_simple, stream);
   if (rc != YALM_OK || inside) return rc;
   const long n = (long)M * dim;
-  row_bias_kernel<<<(int)min((n + 1023) / 1024, 65535L), 256, 0, stream>>>(x, x_bias, n, dim);
+  row_bias_kernel<<<(int)min((n + 1023) / 1024, 65535L), 256, 0, stream>>>(x, x_bias, n, dim,
+                                                                              dim % 4 == 0 && !(((uintptr_t)x | (uintptr_t)x_bias) & 15));
   return launch_status();
 }

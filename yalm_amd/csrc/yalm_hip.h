@@ -44,7 +44,7 @@ int yalm_gemm(const void* A, const void* W, void* C, float* workspace, long work
 
 // yalm_gemm's gated product with biases: C = gelu(gate + bias) (up + bias) (tanh form, sqrt(2 / pi) to float32's precision), bias
 // float32 [N] laid out as the weight's rows, and the bias x_bias[dim] of the product behind goes to the stream, x float32 [M, dim]
-// += x_bias, both on 16 bytes.
+// += x_bias.
 int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N, int K,
                          int dtype, int hidden, const float* bias, float* x, const float* x_bias, int dim, int force_simple,
                          hipStream_t stream);
