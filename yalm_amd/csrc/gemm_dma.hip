@@ -168,7 +168,7 @@ __global__ __launch_bounds__(NWM * NWN * WAVE, MINW) void gemm_dma_kernel(const 
       }
     return;
   }
-GateBias gb[FB / 2 + 1];
+  GateBias gb[FB / 2 + 1];
   if (EPI == EPI_GATED_BIAS)
 #pragma unroll
     for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN + pp * 64) / 2 + li);
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(512, 1) void gemm_ring_kernel(const bf16* __restric
       }
     return;
   }
-GateBias gb[FB / 2 + 1];
+  GateBias gb[FB / 2 + 1];
   if (EPI == EPI_GATED_BIAS)
 #pragma unroll
     for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN + pp * 64) / 2 + li);
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(512, 1) void gemm_ring16_kernel(const bf16* __restr
       }
     return;
   }
-GateBias gb[FB / 2 + 1];
+  GateBias gb[FB / 2 + 1];
   if (EPI == EPI_GATED_BIAS)
 #pragma unroll
     for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN) / 2 + pp * 16 + l16);

@@ -509,9 +509,9 @@ int launch_mt(const bf16* X, const bf16* W, void* C, int M, int N, int K, GateOu
         if (N >= 200 * 128)                        // workgroups of 128 weight rows while they still fill the chip
           return few ? launch_dma<8, 8, EPI, 2, 3, 8>(X, W, C, M, N, K, H, ca, stream)
                      : launch_dma<8, 8, EPI, 2, 2, 16>(X, W, C, M, N, K, H, ca, stream);
-        // workgroups of 96 rows where 64 would leave a few to a second round (8 rows, 22,528 x 4,096 38.0 -> 31.0
+        // workgroups of 96 rows where 64 would leave a few to a second round of compute units (8 rows, 22,528 x 4,096 38.0 -> 31.0
         // us, 18,000 x 4,096 36.0 -> 27.0, gated 22,016 x 4,096 41.2 -> 32.2; 16 rows 39.6 -> 35.8)
-        if (ceil_div(N, 64) > 256 && ceil_div(N, 96) <= 256)
+        if (ceil_div(N, 64) > compute_units() && ceil_div(N, 96) <= compute_units())
           return few ? launch_dma<6, 12, EPI, 1, 3, 8>(X, W, C, M, N, K, H, ca, stream)
                      : launch_dma<6, 12, EPI, 1, 2, 16>(X, W, C, M, N, K, H, ca, stream);
         if (N >= 200 * 64)                         // (9..16 rows: a wave with two row tiles stages the activations once
@@ -520,7 +520,7 @@ int launch_mt(const bf16* X, const bf16* W, void* C, int M, int N, int K, GateOu
         if constexpr (!gated(EPI)) {
           // workgroups of 24 rows where they are at most one a compute unit (6,144 rows: 256 workgroups instead of
           // 192 of 32 rows, which leave a quarter of the chip idle)
-          if (ceil_div(N, 24) <= 256)
+          if (ceil_div(N, 24) <= compute_units())
             return few ? launch_dma<2, 16, EPI, 1, 2, 8, 24>(X, W, C, M, N, K, H, ca, stream)
                        : launch_dma<2, 16, EPI, 1, 2, 16, 24>(X, W, C, M, N, K, H, ca, stream);
         }
