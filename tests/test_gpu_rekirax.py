@@ -180,6 +180,22 @@ def test_middle_of_a_gated_feed_forward_in_its_product(T, F, D, Kd, dtype):
     tol = 2e-5 if dtype == torch.float32 else 1e-2
     assert torch.allclose(out.float().cpu().to(F64), want, rtol=tol, atol=tol)
     assert torch.equal(xg.cpu(), x + xb)                              # every element of the stream once
+    # the same with the middle in a kernel behind: the same float32 numbers
+    behind, xg = torch.full((T, F), float("nan"), dtype=dtype, device=DEV), x.to(DEV)
+    kernels.gemm_gated_bias(h.to(DEV), wg, bg, behind, xg, xb.to(DEV), workspace=torch.empty(n, device=DEV) if n else None,
+                            z=torch.full((T * wg.shape[0],), float("nan"), device=DEV))
+    assert torch.allclose(behind.float().cpu().to(F64), want, rtol=tol, atol=tol) and torch.equal(xg.cpu(), x + xb)
+    if dtype == torch.float32:
+        assert torch.equal(behind, out)
+
+
+@pytest.mark.parametrize("M,F,Kd,dtype,inside", [
+    (16, 64, 64, torch.bfloat16, True), (17, 1024, 512, torch.bfloat16, False), (128, 4096, 1024, torch.bfloat16, False),
+    (146, 4096, 1024, torch.bfloat16, False), (147, 4096, 1024, torch.bfloat16, True), (16, 64, 36, torch.bfloat16, False), (1, 14336, 4096, torch.float32, False),
+    (200, 14336, 4096, torch.float32, True)])
+def test_where_the_middle_rides_in_the_product(M, F, Kd, dtype, inside):
+    from yalm_amd.ops import kernels
+    assert kernels.gated_bias_scratch_floats(M, F, Kd, dtype) == (0 if inside else M * 2 * F)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

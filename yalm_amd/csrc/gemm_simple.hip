@@ -237,6 +237,19 @@ __global__ __launch_bounds__(256) void row_bias_kernel(float* __restrict__ x, co
   }
 }
 
+// The middle of a gated feed-forward with biases behind a product with float32 results z [M][N] (16 gate columns, 16 up columns, ...), the
+// numbers of the epilogue that does it: out[m, h], and x[m, :] += x_bias
+template <typename T>
+__global__ __launch_bounds__(256) void gated_bias_rows_kernel(const float* __restrict__ z, T* __restrict__ out, GateOut H, int N) {
+  const int m = blockIdx.x, first = blockIdx.y * 256 + threadIdx.x, stride = gridDim.y * 256;
+  const float* row = z + (size_t)m * N;
+  for (int h = first; h < H; h += stride) {
+    const int at = (h / 16) * 32 + h % 16;
+    out[(size_t)m * H + h] = from_f32<T>(gate_value<EPI_GATED_BIAS>(row[at], row[at + 16], H, gate_bias<EPI_GATED_BIAS>(H, h)));
+  }
+  for (int i = first; i < H.dim; i += stride) H.x[(size_t)m * H.dim + i] += H.x_bias[i];
+}
+
 template <typename T>
 int gemm_simple(const void* A, const void* W, void* C, int M, int N, int K, int epilogue, GateOut H, hipStream_t stream) {
   dim3 grid(ceil_div(N, BN), ceil_div(M, BM));
@@ -285,14 +298,37 @@ extern "C" int yalm_gemm(const void* A, const void* W, void* C, float* workspace
                   force_simple, stream);
 }
 
-// The gated product with biases: C = gelu(gate + bias) (up + bias), and x += x_bias
-extern "C" int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N, int K,
-                                    int dtype, int hidden, const float* bias, float* x, const float* x_bias, int dim, int force_simple,
-                                    hipStream_t stream) {
+// Whether the product's epilogue does the middle of a gated feed-forward with biases sooner than a kernel behind it.  The epilogue's gelus
+// run in as few waves as the product has, one a SIMD, each waiting for itself, where the kernel spreads them over the chip; so it pays in
+// a decode step's kernel and for many hidden values.  us in the epilogue and behind, rows of hidden x K, bfloat16: 16 of 1,024 x 512 6.8
+// and 7.4, 17 11.2 and 10.0, 128 19.0 and 12.5, 500 15.7 and 16.8; 128 of 4,096 x 1,024 24.7 and 20.4, 200 22.0 and 25.6, 129 of 4,096
+// x 256 13.7 and 12.3; 17 of 7,168 x 2,048 18.9 and 17.9, 129 34.3 and 37.2; 17 of 14,336 x 4,096 43.2 and 43.3, 64 46.1 and 48.6.  float32: 8 of 1,024 x 512 10.0 and 8.4, 1,000
+// 24.6 and 31.2; one of 14,336 x 4,096 94.2 and 92.1, 200 298 and 513 (most of it gemm_split.hip's).
+extern "C" int yalm_gemm_gated_bias_inside(int M, int hidden, int K, int dtype) {
+  return (dtype == YALM_BF16 && M <= 16 && K % 8 == 0) || (long)M * hidden > 600000;
+}
+
+// The gated product with biases: C = gelu(gate + bias) (up + bias), and x += x_bias.  z (float32 [M, N]) not null: the product goes
+// there, and a kernel behind it does the rest.
+extern "C" int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* z, float* workspace, long workspace_floats, int M, int N,
+                                    int K, int dtype, int hidden, const float* bias, float* x, const float* x_bias, int dim,
+                                    int force_simple, hipStream_t stream) {
   if (bias == nullptr || x == nullptr || x_bias == nullptr || dim <= 0 || hidden <= 0) return YALM_ERR_ARG;
   if (M <= 0) return YALM_OK;
   GateOut H(hidden);
   H.bias = bias;
+  if (z != nullptr) {
+    if (N != 32 * ceil_div(hidden, 16) || (dtype != YALM_F32 && dtype != YALM_BF16)) return YALM_ERR_ARG;
+    const int rc = gemm_any(A, W, z, workspace, workspace_floats, M, N, K, dtype, 0, GateOut(0), force_simple, stream);
+    if (rc != YALM_OK) return rc;
+    H.x = x;
+    H.x_bias = x_bias;
+    H.dim = dim;
+    const dim3 grid(M, min(M >= 512 ? 1 : ceil_div(512, M), ceil_div(hidden, 256)));      // few rows still fill the chip
+    if (dtype == YALM_F32) gated_bias_rows_kernel<float><<<grid, 256, 0, stream>>>(z, (float*)C, H, N);
+    else gated_bias_rows_kernel<bf16><<<grid, 256, 0, stream>>>(z, (bf16*)C, H, N);
+    return launch_status();
+  }
   // A decode step's kernel (gemm_skinny_kernel) adds the stream's bias; with more rows a launch of its own is worth less than what
   // the tiles' epilogues would take longer (1,909 rows, 4,096 of 14,336 columns: 74 us more for 12).
   const bool inside = dtype == YALM_BF16 && M <= 16 && K % 8 == 0 && !force_simple && !((uintptr_t)A & 15) && !((uintptr_t)W & 15);

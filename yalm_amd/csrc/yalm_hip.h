@@ -44,10 +44,12 @@ int yalm_gemm(const void* A, const void* W, void* C, float* workspace, long work
 
 // yalm_gemm's gated product with biases: C = gelu(gate + bias) (up + bias) (tanh form, sqrt(2 / pi) to float32's precision), bias
 // float32 [N] laid out as the weight's rows, and the bias x_bias[dim] of the product behind goes to the stream, x float32 [M, dim]
-// += x_bias.
-int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N, int K,
+// += x_bias.  With z (float32 scratch [M, N]) the product goes there and a kernel behind it does the rest; null: the product's
+// epilogue does it, which yalm_gemm_gated_bias_inside says is the sooner way.  The same numbers in float32 either way.
+int yalm_gemm_gated_bias(const void* A, const void* W, void* C, float* z, float* workspace, long workspace_floats, int M, int N, int K,
                          int dtype, int hidden, const float* bias, float* x, const float* x_bias, int dim, int force_simple,
                          hipStream_t stream);
+int yalm_gemm_gated_bias_inside(int M, int hidden, int K, int dtype);
 
 // Which float32 matrix-core kernel and tile yalm_gemm gives a float32 product with K a multiple of 32 and aligned operands (-1:
 // none) that no kernel by bfloat16 terms takes: 100 kernel (0: a workgroup's waves share K, 1: tiles with finely cut sums, 2: tiles) +

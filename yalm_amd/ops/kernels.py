@@ -190,10 +190,17 @@ def can_gemm_gated_bias(kind):
     return kind == "gelu_tanh"
 
 
-def gemm_gated_bias(a, w, bias, out, x, x_bias, workspace=None):
+def gated_bias_scratch_floats(M, hidden, K, dtype):
+    """Floats of `z` with which gemm_gated_bias is sooner (0: without one)."""
+    inside = library.lib().yalm_gemm_gated_bias_inside(int(M), int(hidden), int(K), dtype_code(dtype))
+    return 0 if inside else M * 32 * ((hidden + 15) // 16)
+
+
+def gemm_gated_bias(a, w, bias, out, x, x_bias, workspace=None, z=None):
     """out[M, hidden] (a's dtype) = gelu(a @ gate^T + bias) * (a @ up^T + bias), the gelu in its tanh form, with w and bias (float32)
     holding gate and up interleaved in blocks of 16, and x (float32 [M, dim]) += x_bias on the way.
-    workspace: as for gemm."""
+    workspace: as for gemm.  z (float32, M N elements of scratch): the product goes there and a kernel behind it does the rest
+    (gated_bias_scratch_floats)."""
     M, K = a.shape
     N, hidden = w.shape[0], out.shape[1]
     if hidden <= 0 or N != 32 * ((hidden + 15) // 16):
@@ -204,7 +211,9 @@ def gemm_gated_bias(a, w, bias, out, x, x_bias, workspace=None):
     p_ws, n_ws = None, 0
     if workspace is not None:
         p_ws, n_ws = _need(workspace, "workspace", torch.float32), workspace.numel()
-    library.check(library.lib().yalm_gemm_gated_bias(p_a, p_w, p_o, p_ws, n_ws, M, N, K, dtype_code(a.dtype), hidden, p_b, p_x, p_xb,
+    if z is not None and z.numel() < M * N:
+        raise ValueError("gemm_gated_bias: z holds %d of %d numbers" % (z.numel(), M * N))
+    library.check(library.lib().yalm_gemm_gated_bias(p_a, p_w, p_o, _opt(z, "z", torch.float32, None), p_ws, n_ws, M, N, K, dtype_code(a.dtype), hidden, p_b, p_x, p_xb,
                                                      x.shape[1], 1 if FORCE_SIMPLE else 0, _stream()), "gemm_gated_bias")
     return out
 

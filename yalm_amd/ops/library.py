@@ -26,7 +26,8 @@ _SIGNATURES = {
     "yalm_gemm_norm_qkv_rope_f32": (_I, [_P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "yalm_gemm_norm_f32_takes": (_I, [_I, _I, _I, _I]),
     "yalm_gemm_norm_f32_pays": (_I, [_I, _I, _I, _I]),
-    "yalm_gemm_gated_bias": (_I, [_P, _P, _P, _P, ctypes.c_long, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P]),
+    "yalm_gemm_gated_bias_inside": (_I, [_I, _I, _I, _I]),
+    "yalm_gemm_gated_bias": (_I, [_P, _P, _P, _P, _P, ctypes.c_long, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P]),
     "yalm_gemm_chain": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P]),
     "yalm_gemm_chain_parts": (_I, [_I]),
     "yalm_gemm_f32_choice": (_I, [_I, _I, _I, _I]),
@@ -107,7 +108,7 @@ _SIGNATURES = {
     "yalm_probe_mfma": (_I, [_I, _I, _I, _P, _P, _P]),
 }
 
-ABI_VERSION = 45
+ABI_VERSION = 46
 
 
 class KernelError(RuntimeError):

@@ -4,7 +4,7 @@ stay float32 until the activation has been applied; its result is rounded to the
 product, whose epilogue adds to the float32 residual stream.  With `gated` there is a third matrix and the middle is
 act(gate h) * (up h) (gate and up are one product); with `biases` every product has a bias (tensors "<name>.b" unless
 named otherwise): those of the first products are added before the activation, the last one's goes to the stream
-with the kernel of the middle, or with the first product where its epilogue does the middle (gated, tanh gelu)."""
+with the kernel of the middle, or with the first product where its epilogue may do the middle (gated, tanh gelu)."""
 import torch
 
 from ..ops import kernels
@@ -27,7 +27,7 @@ class DenseMLP(Part):
         self.names.update(spec.params.get("tensors") or {})
         for k in ("up", "down", "gate"):
             self.names.setdefault(k + "_bias", self.names[k] + ".b")
-        # the first product's epilogue does the middle; its rows are then gate and up in turn
+        # the first product's epilogue does the middle where that is sooner; its rows are gate and up in turn
         self.one_kernel = self.gated and self.biases and kernels.can_gemm_gated_bias(self.activation)
         self.w_up = self.w_down = self.b_up = self.b_down = None
 
@@ -66,7 +66,9 @@ class DenseMLP(Part):
         T = h.shape[0]
         if self.one_kernel:
             mid = ctx.ws.get("mlp.mid", (T, self.hidden), h.dtype)
-            return kernels.gemm_gated_bias(h, self.w_up, self.b_up, mid, x, self.b_down, workspace=self._gemm_scratch(ctx, h, self.w_up))
+            n = kernels.gated_bias_scratch_floats(T, self.hidden, self.dim, h.dtype)
+            return kernels.gemm_gated_bias(h, self.w_up, self.b_up, mid, x, self.b_down, workspace=self._gemm_scratch(ctx, h, self.w_up),
+                                           z=ctx.ws.get("mlp.z", (n,), torch.float32) if n else None)
         z = ctx.ws.get("mlp.z", (T, self.w_up.shape[0]), torch.float32)
         self._gemm(ctx, h, self.w_up, z, kernels.EPI_STORE_F32)
         mid = ctx.ws.get("mlp.mid", (T, self.hidden), h.dtype)
