@@ -266,7 +266,8 @@ def test_recurrence_of_many_workgroups(d, dv):
 # A step of one token a sequence keeps a head's state in one workgroup (d and dv multiples of 4 to 128); it walks what it is given, so
 # two tokens of one sequence and none of the next are the same walk
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,d,dv", [(2, 128, 128), (3, 36, 124), (1, 124, 68), (32, 128, 128), (1, 4, 128)])
+@pytest.mark.parametrize("H,d,dv", [(2, 128, 128), (3, 36, 124), (1, 124, 68), (32, 128, 128), (1, 4, 128), (3, 128, 64), (2, 40, 36), (5, 128, 32),
+                                    (3, 4, 4), (2, 16, 28)])
 def test_recurrence_of_single_tokens(H, d, dv, dtype):
     from yalm_amd.ops import kernels
     B, n_slots = 5, 7

@@ -5,6 +5,7 @@
 // and each head's o is divided by its root mean square over dv and multiplied by a weight shared by the heads.
 // Everything behind the projections z_q | z_f | v (float32) is float32; the walk over the tokens is diag_scan.h's, but in a step of
 // one token a sequence (hgrn2_step_kernel).
+#include <climits>
 #include "diag_scan.h"
 #include "yalm_hip.h"
 
@@ -15,8 +16,7 @@ struct Hgrn2Op {
   const float* proj;
   const float* f_bias;
   const float* lower;
-  long N;                                         // from one token's projections to the next one's
-  int Hd, d, dv;                                  // Hd: heads * d
+  int Hd, N, d, dv;                               // heads * d; from one token's projections to the next one's
   __device__ Row begin(int h, int r, bool ok) const {
     return {ok ? f_bias[h * d + r] : 0.f, ok ? lower[h * d + r] : 0.f};
   }
@@ -38,14 +38,16 @@ struct Hgrn2Op {
 // column, so that the head's norm needs no launch of its own.  Bound by one trip of the state from memory and back behind one of
 // the slot's number: the operands of the token are asked for beside the state.  d and dv multiples of 4 to 128.
 // Eight rows (five live), 32 heads of 128 x 128, 6.3 us (21 MB of state); diag_scan_kernel and heads_norm_kernel
-// took 12.2 and 4.7.
-constexpr int HS_THREADS = 512, HS_MAX = 128;
+// took 12.2 and 4.7.  Two columns a lane group: 512 threads for 128 columns, 128 for 32, so that many small heads share a compute unit
+// (800 sequences of 8 heads of 16 x 16 9.3 us, with 512 threads each 23.3, those two kernels 13.8).
+constexpr int HS_MAX = 128;
 
-template <typename T>
-__global__ __launch_bounds__(HS_THREADS) void hgrn2_step_kernel(Hgrn2Op op, float* __restrict__ state, const float* __restrict__ w_norm,
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS) void hgrn2_step_kernel(Hgrn2Op op, float* __restrict__ state, const float* __restrict__ w_norm,
                                                                 T* __restrict__ out, const int* __restrict__ cu_seqlens,
                                                                 const int* __restrict__ seq_slot, int n_heads, int d, int dv, float eps) {
-  constexpr int LANES = 8, GROUPS = HS_THREADS / LANES, NC = HS_MAX / GROUPS, NV = HS_MAX / (4 * LANES);
+  constexpr int LANES = 8, GROUPS = THREADS / LANES, NC = 2, NV = HS_MAX / (4 * LANES);
+  constexpr int VALUES = THREADS > HS_MAX ? HS_MAX : 0;       // the first of the threads that fetch a token's values
   __shared__ __attribute__((aligned(16))) float s_q[HS_MAX], s_f[HS_MAX], s_v[HS_MAX], s_o[HS_MAX];
   const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, group = tid / LANES, rl = tid % LANES;
   const int slot = seq_slot[b], t0 = cu_seqlens[b], t1 = cu_seqlens[b + 1], HV = n_heads * dv;
@@ -72,9 +74,8 @@ __global__ __launch_bounds__(HS_THREADS) void hgrn2_step_kernel(Hgrn2Op op, floa
       op.form(mine, z, nullptr, q, f, k);
       s_q[tid] = tid < d ? q : 0.f;
       s_f[tid] = tid < d ? f : 0.f;
-    } else if (tid < 2 * HS_MAX) {
-      s_v[tid - HS_MAX] = op.value(t, h, min(tid - HS_MAX, dv - 1));
     }
+    if (tid >= VALUES && tid < VALUES + HS_MAX) s_v[tid - VALUES] = op.value(t, h, min(tid - VALUES, dv - 1));
     lds_barrier();
     float sum[NC];
 #pragma unroll
@@ -126,15 +127,19 @@ extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias,
   if (T <= 0 || B <= 0) return YALM_OK;
   if (n_heads <= 0 || d <= 0 || d > 256 || dv <= 0) return YALM_ERR_ARG;
   if (out_dtype != YALM_F32 && out_dtype != YALM_BF16) return YALM_ERR_DTYPE;
-  if (proj_row < 2 * n_heads * d + n_heads * dv) return YALM_ERR_ARG;
-  const Hgrn2Op op = {proj, f_bias, lower, proj_row, n_heads * d, d, dv};
+  if (proj_row < 2 * n_heads * d + n_heads * dv || proj_row > INT_MAX) return YALM_ERR_ARG;
+  const Hgrn2Op op = {proj, f_bias, lower, n_heads * d, (int)proj_row, d, dv};
   // one token a sequence, as the numbers say (the kernel walks whatever cu_seqlens holds)
   if (T == B && n_heads <= 65535 && B <= 65535 && d <= HS_MAX && dv <= HS_MAX && d % 4 == 0 && dv % 4 == 0 && ((uintptr_t)state & 15) == 0) {
     const dim3 grid(n_heads, B);
-    if (out_dtype == YALM_F32)
-      hgrn2_step_kernel<float><<<grid, HS_THREADS, 0, stream>>>(op, state, w_norm, (float*)out, cu_seqlens, seq_slot, n_heads, d, dv, eps);
-    else
-      hgrn2_step_kernel<bf16><<<grid, HS_THREADS, 0, stream>>>(op, state, w_norm, (bf16*)out, cu_seqlens, seq_slot, n_heads, d, dv, eps);
+#define STEP(T_, THREADS_) \
+  hgrn2_step_kernel<T_, THREADS_><<<grid, THREADS_, 0, stream>>>(op, state, w_norm, (T_*)out, cu_seqlens, seq_slot, n_heads, d, dv, eps)
+#define STEP_OF(T_) \
+  if (dv <= 32) STEP(T_, 128); else if (dv <= 64) STEP(T_, 256); else STEP(T_, 512)
+    if (out_dtype == YALM_F32) { STEP_OF(float); }
+    else { STEP_OF(bf16); }
+#undef STEP_OF
+#undef STEP
     return launch_status();
   }
   int rc;
