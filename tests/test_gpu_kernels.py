@@ -1638,7 +1638,7 @@ def test_gemm_norm_qkv_rope(n_heads, n_kv, hd, rd, D):
 # Workgroups of 96 weight rows, which take what 64 rows would leave to a second round of compute units: the fewest and the most rows, a
 # last workgroup of one row, sums of one, two and seven stages of K
 @pytest.mark.parametrize("M", [1, 8, 9, 16])
-@pytest.mark.parametrize("N,Kd", [(16385, 128), (24576, 64), (22113, 448)])
+@pytest.mark.parametrize("N,Kd", [(16385, 128), (16417, 128), (24576, 64), (22113, 448)])
 def test_decode_gemm_of_96_rows(M, N, Kd):
     from yalm_amd.parts.swiglu import interleave_gate_up
     k = K()

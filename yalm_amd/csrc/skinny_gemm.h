@@ -510,8 +510,9 @@ int launch_mt(const bf16* X, const bf16* W, void* C, int M, int N, int K, GateOu
           return few ? launch_dma<8, 8, EPI, 2, 3, 8>(X, W, C, M, N, K, H, ca, stream)
                      : launch_dma<8, 8, EPI, 2, 2, 16>(X, W, C, M, N, K, H, ca, stream);
         // workgroups of 96 rows where 64 would leave a few to a second round of compute units (8 rows, 22,528 x 4,096 38.0 -> 31.0
-        // us, 18,000 x 4,096 36.0 -> 27.0, gated 22,016 x 4,096 41.2 -> 32.2; 16 rows 39.6 -> 35.8)
-        if (ceil_div(N, 64) > compute_units() && ceil_div(N, 96) <= compute_units())
+        // us, 18,000 x 4,096 36.0 -> 27.0, gated 22,016 x 4,096 41.2 -> 32.2; 16 rows 39.6 -> 35.8); more than 8 rows not where that
+        // is half a workgroup (16 rows, 16,400 x 7,168 47.3 with 64 and 54.2 with 96, 16,448 x 7,168 55.7 and 54.3)
+        if (N > 64L * compute_units() + (few ? 0 : 32) && ceil_div(N, 96) <= compute_units())
           return few ? launch_dma<6, 12, EPI, 1, 3, 8>(X, W, C, M, N, K, H, ca, stream)
                      : launch_dma<6, 12, EPI, 1, 2, 16>(X, W, C, M, N, K, H, ca, stream);
         if (N >= 200 * 64)                         // (9..16 rows: a wave with two row tiles stages the activations once
