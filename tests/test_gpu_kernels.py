@@ -337,16 +337,17 @@ def test_gemm_float32_rows_do_not_depend_on_their_number(N, Kd, epi):
 
 
 # Every kernel and tile of the float32 products on the matrix cores (yalm_gemm_f32_choice), with edges of 1 to 31 rows and columns
-# and K of 37 or 69 k tiles: each ring of two to four stages turns many times, and sums are folded in whole and broken runs
+# and K of 37 or 69 k tiles: each ring of two to four stages turns many times, and sums are folded in whole and broken runs.  More than 64
+# rows of 512 k and more go by bfloat16 terms but for few tiles' worth, so most tiles there have K of 15 k tiles
 @pytest.mark.parametrize("M,N,Kd,choice", [
     (1, 40, 1184, 11), (9, 4100, 1184, 12), (17, 3000, 1184, 21), (33, 4100, 1184, 22), (47, 2001, 1184, 41),
     (3, 8200, 2208, 111), (1, 20001, 2208, 112), (33, 11999, 2208, 121), (47, 40001, 2208, 122),
-    (70, 41, 1184, 211), (129, 4001, 1184, 212), (97, 5130, 1184, 221), (161, 8201, 1184, 222), (161, 16401, 1184, 224),
-    (161, 12001, 1184, 233), (513, 5131, 1184, 234), (321, 20001, 1184, 244)])
+    (70, 41, 1184, 211), (129, 6144, 1184, 212), (129, 4001, 480, 212), (97, 5130, 480, 221), (161, 8201, 480, 222), (161, 16401, 480, 224),
+    (161, 12001, 480, 233), (513, 5131, 480, 234), (321, 20001, 480, 244)])
 def test_gemm_float32_every_tile(M, N, Kd, choice):
     from yalm_amd.ops import library
     k = K()
-    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 0) == choice
+    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 0) == choice and library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) == -1
     a, w, x = rnd((M, Kd), 101).to(DEV), rnd((N, Kd), 102).to(DEV), rnd((M, N), 103).to(DEV)
     want = a.double() @ w.double().t()
     # K products and K additions in any order, the residual's addition once more (as below)
@@ -361,12 +362,12 @@ def test_gemm_float32_every_tile(M, N, Kd, choice):
 
 
 @pytest.mark.parametrize("M,N,Kd,choice", [
-    (1, 64, 1184, 12), (33, 3008, 1184, 22), (3, 8224, 2208, 112), (47, 40000, 2208, 122), (65, 64, 1184, 212), (161, 8224, 1184, 222),
-    (161, 16416, 1184, 224), (513, 5152, 1184, 234), (321, 20000, 1184, 244)])
+    (1, 64, 1184, 12), (33, 3008, 1184, 22), (3, 8224, 2208, 112), (47, 40000, 2208, 122), (65, 64, 1184, 212), (161, 8224, 480, 222),
+    (161, 16416, 480, 224), (513, 5152, 480, 234), (321, 20000, 480, 244)])
 def test_gemm_float32_every_gated_tile(M, N, Kd, choice):
     from yalm_amd.ops import library
     k = K()
-    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 1) == choice
+    assert library.lib().yalm_gemm_f32_choice(M, N, Kd, 1) == choice and library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 1) == -1
     H = N // 2 - 3
     a, w = rnd((M, Kd), 104).to(DEV), rnd((N, Kd), 105, scale=Kd ** -0.5).to(DEV)
     p = (a.double() @ w.double().t()).view(M, -1, 2, 16)
