@@ -232,9 +232,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
 // NORM (a decode step of up to 16 rows): A is the residual stream and its norm is applied on the way: the rows' sums of squares
 // first, by every workgroup (a wave a row, in the order of the norm's own kernel, so that its bits come out), then x * scale * weight
 // in front of every product.  EPI 4: the q/k/v product of a decode step, rotated and written to the pages of the cache as
-// rope_kv_write_kernel does.  A launch less each, seven of a small model's 24 a step (3 requests on two layers of 256, 16 tokens each:
-// 2,066 -> 2,016 us, which the host bounds; 12 of up to 300 and 30 tokens each 4,125 -> 3,930; a step of four 7B layers at one row
-// 922 -> 906 us, at 16 rows 1,132 -> 1,124; of 3B layers at 8 rows 929 -> 917).
+// rope_kv_write_kernel does.  A launch less each, seven of a small model's 24 a step (two layers of 256, steps queued: one row 82 -> 70
+// us, three 92 -> 80, sixteen 99 -> 88; a step of four 7B layers at one row 974 -> 955 us, at 16 rows 1,152 -> 1,137; of 3B layers at
+// 8 rows 857 -> 846).  norm_pays says where.
 // ---------------------------------------------------------------------------
 constexpr int NWV = 8;
 constexpr int EPI_QKV = 4;
@@ -492,9 +492,10 @@ Choice choose(int M, int N, int K, bool gate) {
   return M <= 64 && (N < 8192 || K <= 2048) ? choose_few(M, N, gate) : choose_tile(M, N, K, gate);
 }
 
-// The tile of gemm_split.hip that is sooner by the estimates than the tile chosen here, or -1 (5,120 x 3,072: 65 rows 42 us here, 47
-// there; 128 rows 61 and 47).  tile_time compares tiles with each other and leaves out a launch's start and end, some 5 us, and a
-// tenth that broken rounds take longer (up to 40 % just above one round: 65 rows, 3,072 x 8,192 69 us for 98 measured).
+// The tile of gemm_split.hip that is sooner by the estimates than the tile chosen here, or -1 (5,120 x 3,072: 65 rows 41 us here, 47
+// there; 128 rows 59 and 53; of 398 sizes that it takes there four are up to 5 % slower than here).  tile_time compares tiles with
+// each other and leaves out a launch's start and end, some 5 us, and a tenth that broken rounds take longer (up to 40 % just above one
+// round: 65 rows, 3,072 x 8,192 69 us for 98 measured).
 int split_tile(int M, int N, int K, bool gate) {
   const Choice c = choose(M, N, K, gate);
   return c.kernel == Choice::COARSE ? yalm_gemm_split_choose(M, N, K, gate, 5.0 + 1.1 * tile_time(M, N, K, c.a, c.b)) : -1;

@@ -15,14 +15,19 @@
 // bits that it shifts out of a sum's addends towards minus infinity: all results of a product would lie low by 2e-8 (K 512) to 1.2e-7
 // (K 14,336) of their size, and what every number of a stream is off by alike does not average out in the layers behind it
 // (probabilities of a scored text 5.5e-7 off, with gemm_f32_kernel 4.6e-7).  So every second fold of k tiles is summed with A's signs
-// turned and subtracted: the means are 1e-10 of a size then.
+// turned and subtracted: the means are 1e-10 of a size then.  Operands of one sign, of exponents spread over 2^+-24 and with a few numbers a
+// thousand times the others are no further off than there either; rows of one number that is not zero are (3.5e-8, 4.3e-8 here), and
+// rows of eight (5.1 to 6.1e-8, 6.2 to 7.0e-8), whose sums have hardly any rounding but the products' own.
+//
+// A row's sums hang on how many rows stand beside it, by which tile they choose: gemm_f32_kernel's, one of one group of waves and
+// one of two add in three orders.
 //
 // Bound by the power that the matrix cores may draw (full rounds of 128 x 256: 1.45 PFLOP/s of bfloat16 products) and by
 // rounds of tiles that do not come out even.  Every element is split once a workgroup, on its way from registers into LDS
 // (the next k tile's, a vector instruction or two behind every matrix product): split by each wave that multiplies it, straight
 // from fragments of float32, the vector instructions take as long as the products (701 rows, 16,384 x 3,072 415 us against 365).
-// 701 rows against gemm_f32_kernel, us: 16,384 x 3,072 571 -> 371, 128,256 x 3,072 4,120 -> 2,780, 5,120 x 3,072 192 -> 130, 3,072 x 8,192
-// 297 -> 216, 3,072 x 3,072 114 -> 85.
+// 701 rows against gemm_f32_kernel, us: 16,384 x 3,072 573 -> 372, 128,256 x 3,072 4,130 -> 2,753, 5,120 x 3,072 195 -> 137, 3,072 x 8,192
+// 304 -> 222, 3,072 x 3,072 117 -> 85 (1 to 2 % of it the scale of W's elements).
 #include "common.h"
 #include "gemm_split.h"
 

@@ -129,7 +129,8 @@ extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias,
   if (out_dtype != YALM_F32 && out_dtype != YALM_BF16) return YALM_ERR_DTYPE;
   if (proj_row < 2 * n_heads * d + n_heads * dv || proj_row > INT_MAX) return YALM_ERR_ARG;
   const Hgrn2Op op = {proj, f_bias, lower, n_heads * d, (int)proj_row, d, dv};
-  // one token a sequence, as the numbers say (the kernel walks whatever cu_seqlens holds)
+  // one token a sequence, as the numbers say (the kernel walks whatever cu_seqlens holds; eight tokens of one sequence and none of seven
+  // others, which no step of the engine is, take it 12 us and diag_scan_kernel 6)
   if (T == B && n_heads <= 65535 && B <= 65535 && d <= HS_MAX && dv <= HS_MAX && d % 4 == 0 && dv % 4 == 0 && ((uintptr_t)state & 15) == 0) {
     const dim3 grid(n_heads, B);
 #define STEP(T_, THREADS_) \

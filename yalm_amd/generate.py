@@ -80,7 +80,9 @@ def generate(engine, prompts, max_new_tokens=256, temperature=0.0, seed=0, stop_
     kernels: in float32 the tokens are the same either way (a row's sums do not depend on the rows beside it, up to 64 of
     them; but where a context of the step is beyond 256 tokens, or 64 at head sizes that are no multiple of 16, the rows'
     number and the longest context decide into how many pieces the attention is cut, which moves its last bits), in bfloat16
-    up to choices between logits that lie within rounding of each other."""
+    up to choices between logits that lie within rounding of each other.  A prompt step of more than 64 tokens in all is another
+    matter: its products take the tiles that its number of tokens asks for, which add in different orders, so that a request's
+    prompt logits move in their last bits with the prompts that start beside it, in float32 too."""
     from .sampling import Sampler
     sampler = sampler or Sampler(seed)
     stats = stats if stats is not None else GenerationStats()
