@@ -493,6 +493,21 @@ def test_gemm_float32_by_terms_of_small_numbers(M, N, tile, small):
     assert float(((got - want).norm(dim=axis) / want.norm(dim=axis)).max()) <= 1e-6
 
 
+# And at the upper end: sums beyond 2^80, operands beyond 2^104, and rows of both kinds beside ordinary ones
+@pytest.mark.parametrize("up_a,up_w", [(70, 30), (110, -60), (-60, 115), (79, 0)])
+@pytest.mark.parametrize("M,N,tile", [(97, 5130, 0), (513, 5131, 3)])
+def test_gemm_float32_by_terms_of_large_numbers(M, N, tile, up_a, up_w):
+    from yalm_amd.ops import library
+    k, Kd = K(), 512
+    assert library.lib().yalm_gemm_f32_split_choice(M, N, Kd, 0) == tile
+    a, w = (rnd((n, Kd), s, torch.float64) * 2.0 ** up for n, s, up in ((M, 145, up_a), (N, 146, up_w)))
+    a[::3] *= 2.0 ** -up_a
+    a, w = a.float(), w.float()
+    want = a.double().to(DEV) @ w.double().to(DEV).t()
+    got = k.gemm(a.to(DEV), w.to(DEV), torch.full((M, N), 7.0, device=DEV), k.EPI_STORE_F32).double()
+    assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) <= 1e-6
+
+
 # float32 on the matrix cores: the edges of the smallest tiles and of the rules (16 | 17 and 32 | 33 rows, 4,096 and 8,192
 # columns), of one k tile and a few, K short of one round of the waves, operands 4 bytes off
 @pytest.mark.parametrize("M,N,Kd,off", [

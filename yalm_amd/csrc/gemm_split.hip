@@ -6,9 +6,10 @@
 // leave a factor of 2.7 over gemm_f32.hip's tiles.
 //
 // A bfloat16 number has float32's exponents, so the last terms of a float below 2^-108 would fall off their end (an operand of 2^-120
-// kept 14 bits).  Both operands are therefore split at 2^41 times their size, where every float, a subnormal one too, is the sum of its
-// terms exactly, and a fold's sums come back by 2^-82 as they join the total.  What that leaves no room for (an operand from about 2^87
-// on, a fold's sum from 2^46 on) comes out as no finite number, and is made again with float32 products like an infinity.
+// kept 14 bits).  Both operands are therefore split at 2^24 times their size, where every float, a subnormal one too, is the sum of its
+// terms exactly (no bit of a float is below 2^-149, none there below 2^-125), and a fold's sums come back by 2^-48 as they join the
+// total.  What that leaves no room for (an operand from about 2^104 on, a fold's sum from 2^80 on) comes out as no finite number, and
+// is made again with float32 products like an infinity (a product of nothing else: 366 us where gemm_f32_kernel takes 117).
 //
 // The error against 64 bits is smaller than gemm_f32_kernel's, whose sums are chains of four products at a time: relative, K 512
 // 1.6e-7 (2.9e-7), 3,072 1.7 to 1.8e-7 (2.95e-7), 8,192 1.9 to 2.1e-7 (3.05e-7), 14,336 2.1 to 2.5e-7 (3.2e-7).  The instruction drops the
@@ -45,7 +46,7 @@ constexpr int TERMS = 3;
 constexpr int GROUP = 4;                         // tile columns that an XCD walks together
 constexpr int FOLD = 4;                          // k tiles whose sums join before they are added to the total (8: the errors 1.4 times these, 2 % sooner)
 
-constexpr float UP = 0x1p41f, DOWN = 0x1p-82f;   // the operands' scale on the way into terms, and the sums' on the way back
+constexpr float UP = 0x1p24f, DOWN = 0x1p-48f;   // the operands' scale on the way into terms, and the sums' on the way back
 
 struct Terms { u32x4 t[TERMS]; };
 
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(WM * WN * KG * WAVE, 2) void gemm_split_kernel(cons
       for (int b = 0; b < FB; ++b) total[a][b] += other[(a * FB + b) * NT + tid];
   }
 
-  // An infinity, a NaN, or a number that is infinite at 2^41 times its size makes every sum that it enters a NaN (infinity less
+  // An infinity, a NaN, or a number that is infinite at 2^24 times its size makes every sum that it enters a NaN (infinity less
   // infinity in its terms), and a fold's sum that has no room is infinite.  Sums that are no finite numbers are made again with float32
   // products, chains as in gemm_f32_kernel, 16 rows at a time; the sums beside them stay as they are.
   auto finite = [](float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; };
