@@ -1806,6 +1806,25 @@ def test_gemm_chain_qkv_rope(n_heads, n_kv, hd, rd, D, M):
     assert (vp.float().abs().sum(dim=(1, 2)) > 0).equal(touched)
 
 
+@pytest.mark.parametrize("M", [1, 7, 9, 16, 33])
+@pytest.mark.parametrize("parts", [1, 63, 65, 256, 257, 600])
+def test_gemm_chain_scales_of_any_number_of_parts(M, parts):
+    """A chained consumer adds a row's partial sums of squares four times 64 at a time: every remainder, one and two rows a
+    wave, K with fewer stages than waves.  Float32 sums of exact products: 2 sqrt(K) roundings of half a unit, and three of the scale."""
+    k = K()
+    for Kd, N in ((64, 70), (1024, 4112)):
+        x = rnd((M, Kd), 70, torch.bfloat16)
+        w = rnd((N, Kd), 71, torch.bfloat16, scale=1 / math.sqrt(Kd))
+        ss = rnd((M, parts), 72).abs() * Kd / parts + 0.01
+        out = torch.full((M + 1, N), 7.0, device=DEV)
+        k.gemm_chain(x.to(DEV), w.to(DEV), out[:M], k.EPI_STORE_F32, scale_from=(ss.to(DEV).contiguous(), 1e-5))
+        want = x.double() @ w.double().T / torch.sqrt(ss.double().sum(1, keepdim=True) / Kd + 1e-5)
+        size = x.double().abs() @ w.double().abs().T / torch.sqrt(ss.double().sum(1, keepdim=True) / Kd + 1e-5)
+        off = ((out[:M].double().cpu() - want).abs() / size).max().item()
+        assert off <= (2 * math.sqrt(Kd) + 3) * 2.0 ** -24, "M %d, %d parts, K %d: %g" % (M, parts, Kd, off)
+        assert bool((out[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,N,Kd", [(1, 64, 256), (8, 4096, 1000), (33, 80, 96), (64, 4096, 264), (5, 16400, 64),
                                     (11, 192, 192), (16, 4096, 128), (9, 1024, 64), (8, 3072, 128), (3, 3000, 64),
                                     (20, 3072, 64)])

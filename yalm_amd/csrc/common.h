@@ -117,15 +117,34 @@ __device__ __forceinline__ float rotate_one(float x, float other, bool odd, floa
   return fmaf(x, c.x, odd ? other * c.y : -(other * c.y));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+// A value of all 64 lanes folded with itself 32, 16, 8, 4, 2 and 1 lanes on, in that order, in the registers: the halves and the
+// quarters by exchanges of rows, the rest by rotations inside rows of 16 lanes, which by then hold a value again every 8, 4 and 2
+// lanes, so that lane + 8 (4, 2) stands for lane ^ 8 (4, 2).  The same sums, to the bit, as six permutes through LDS, one waiting for
+// the other.  All lanes of the wave take part.
+template <int CTRL>
+__device__ __forceinline__ float dpp_of(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <class F>
+__device__ __forceinline__ float wave_fold(float v, F f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((ext_vector_type(2))) unsigned both;
+  both x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(x[0]), __uint_as_float(x[1]));
+  x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(x[0]), __uint_as_float(x[1]));
+  v = f(v, dpp_of<0x128>(v));                    // row_ror:8
+  v = f(v, dpp_of<0x124>(v));                    // row_ror:4
+  v = f(v, dpp_of<0x122>(v));                    // row_ror:2
+  v = f(v, dpp_of<0x121>(v));                    // row_ror:1
+#endif
   return v;
 }
+__device__ __forceinline__ float wave_sum(float v) {
+  return wave_fold(v, [](float a, float b) { return a + b; });
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-  return v;
+  return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a block of NW waves; every thread gets the result.  `red` holds NW floats.

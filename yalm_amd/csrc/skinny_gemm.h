@@ -102,7 +102,7 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
                 "a last tile of 8 rows: one tile a wave, the DMA path, no gated pairs");
   __shared__ f32x4 red[NWAVES][MT * TW][WAVE];
   __shared__ float sm_scale[MT * 16];
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int q = lane / 16, j = lane % 16;
   const int n0 = blockIdx.x * RW;
 
@@ -150,7 +150,11 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
     }
   }
 
-  // so are the first gated tile's biases, and the elements of the stream that this thread adds a bias to (EPI_GATED_BIAS)
+  // so is the weight of the next norm with which the first tile's activations are emitted,
+  float nw_first = 0.f;
+  if (EPI == EPI_ADD && ca.emit_nw != nullptr && wave < MT * NT) nw_first = ca.emit_nw[min(n0 + (wave % NT) * 16 + j, N - 1)];
+
+  // the first gated tile's biases, and the elements of the stream that this thread adds a bias to (EPI_GATED_BIAS)
   GateBias gb = {0.f, 0.f};
   float stream = 0.f, stream_bias = 0.f;
   const long stream_n = EPI == EPI_GATED_BIAS && H.x != nullptr ? (long)M * H.dim : 0;
@@ -206,12 +210,43 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
       for (int mt = 0; mt < MT; ++mt) x[mt][s] = zero_unless(load8_always(xrow[mt] + kk), ok);
     }
   };
-  auto row_scales = [&]() {   // from the producer's partial sums of squares (a wave per row, lanes over the parts)
+  // Row scales from the producer's partial sums of squares: a wave a row (rows wave, wave + NWAVES, ...), its lanes over the parts,
+  // four of a lane at a time.  With one batch tile the first 256 parts of the wave's rows are asked for in front of the weights
+  // and added when its products are done: the epilogue is the first that wants them.  (A part a trip to memory, added behind the first
+  // weights, held the waves up four times at 256 parts and eight at more than 8 rows: steps of 32 layers of 7B sizes
+  // at one row 2.810 ms and now 2.765, at 8 rows 3.330 and 3.280, of 28 layers of 3B sizes at 13 rows 2.744 and 2.685.)
+  constexpr int SR = (MT * 16 + NWAVES - 1) / NWAVES, SP = 4;
+  constexpr bool ASK = MT == 1;
+  float ss[ASK ? SR : 1][SP];
+  // (what lies behind the last row or part is read again and counts nothing)
+  auto part_of = [&](int m, int p) { return ca.ss_in[(size_t)min(m, M - 1) * ca.n_parts_in + min(p, ca.n_parts_in - 1)]; };
+  if (ASK && ca.ss_in != nullptr) {
+#pragma unroll
+    for (int i = 0; i < SR; ++i)
+#pragma unroll
+      for (int u = 0; u < SP; ++u) ss[i][u] = part_of(wave + i * NWAVES, lane + u * WAVE);
+  }
+  auto row_scales = [&]() {
     if (ca.ss_in == nullptr) return;
-    for (int m = wave; m < MT * 16; m += NWAVES) {
+#pragma unroll
+    for (int i = 0; i < SR; ++i) {
+      const int m = wave + i * NWAVES;
+      if (m >= M) break;
       float s = 0.f;
-      if (m < M)
-        for (int p = lane; p < ca.n_parts_in; p += WAVE) s += ca.ss_in[(size_t)m * ca.n_parts_in + p];
+      if constexpr (ASK) {
+#pragma unroll
+        for (int u = 0; u < SP; ++u) {
+          asm volatile("" : "+v"(ss[i][u]));     // waited for here, not where it is asked for
+          s += lane + u * WAVE < ca.n_parts_in ? ss[i][u] : 0.f;
+        }
+      }
+      for (int p0 = ASK ? SP * WAVE : 0; p0 < ca.n_parts_in; p0 += SP * WAVE) {
+        float v[SP];
+#pragma unroll
+        for (int u = 0; u < SP; ++u) v[u] = part_of(m, p0 + lane + u * WAVE);
+#pragma unroll
+        for (int u = 0; u < SP; ++u) s += p0 + lane + u * WAVE < ca.n_parts_in ? v[u] : 0.f;
+      }
       s = wave_sum(s);
       if (lane == 0) sm_scale[m] = 1.0f / sqrtf(s / (float)K + ca.eps);
     }
@@ -258,7 +293,6 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
     for (int i = 0; i < DMA_S - 1; ++i)
       if (i < mine) issue(i, i);
     if (AHEAD && wave < MT * RT) rope_where(wave);
-    row_scales();
     // fragment reads: lane (q, j) of step s wants chunk 4 s + q of row j, which lies at (4 s + q) ^ (j & 7)
     const int rd_w = j * 128, rd_x = (16 * TW + (j % XR)) * 128, swz = j & 7;
     int buf = 0;
@@ -306,11 +340,8 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
     if (!PREFETCH) {
       // few, large chunks: all loads of a chunk are in flight at once and the products
       // start as the first arrive (K <= 512 * NWAVES is one round trip to memory)
-      bool first = true;
       for (int c = kw; c < n_chunks; c += KW) {
         load_chunk(c, wv, xv);
-        if (first) row_scales();
-        first = false;
   #pragma unroll
         for (int s = 0; s < KS; ++s)
   #pragma unroll
@@ -319,11 +350,9 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
             for (int t = 0; t < TW; ++t)
               acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[mt][s], wv[t][s], acc[mt][t], 0, 0, 0);
       }
-      if (first) row_scales();
     } else {
       int c = kw;
       if (c < n_chunks) load_chunk(c, wv, xv);
-      row_scales();
       for (; c < n_chunks; c += KW) {
         bf16x8 wn[TW][KS], xn[MT][KS];
         const bool more = c + KW < n_chunks;
@@ -350,6 +379,7 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
   }
 
   if (AHEAD && wave < MT * RT) rope_ahead(wave);
+  row_scales();
   if (EPI == EPI_GATED_BIAS && stream_at < stream_n) {
     H.x[stream_at] = stream + stream_bias;
     for (long e = stream_at + stream_step; e < stream_n; e += stream_step) H.x[e] += H.x_bias[e % H.dim];
@@ -403,7 +433,7 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
       }
     } else if (EPI == EPI_ADD) {
       const bool emit = ca.emit_nw != nullptr;   // NT == 1 then (the launcher sees to it)
-      const float nw = (emit && n < N) ? ca.emit_nw[n] : 0.f;
+      const float nw = !emit || n >= N ? 0.f : idx == wave ? nw_first : ca.emit_nw[n];
       float sq[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
