@@ -742,3 +742,39 @@ def test_whether_a_norm_can_be_folded_in_is_asked_without_the_weights_rows():
     from yalm_amd.ops import kernels
     assert kernels.can_fuse_norm(8, 4096, torch.bfloat16) and not kernels.can_fuse_norm(9, 4096, torch.bfloat16)
     assert not kernels.can_fuse_norm(8, 4096, torch.float32)
+
+
+def test_decode_splits_over_rows_pages_and_heads():
+    """Into how many pieces a decode step's attention cuts its sequences: at least one, never more than a page each; float32, whose
+    sums hang on the pieces, keeps four pages a piece (one piece up to 256 tokens); bfloat16 never cuts less than float32 where few rows run
+    and never more workgroups than the chip takes in one round, but for unequal sequences and the quarters of a nearly empty second round."""
+    from yalm_amd.ops import kernels
+    from yalm_amd.parts.attention import decode_order, decode_splits
+
+    class Step:
+        seq_order = "the order"
+    for heads, kv, hd in ((32, 8, 128), (24, 8, 128), (8, 2, 64), (16, 1, 128), (40, 1, 256), (32, 32, 80), (3, 3, 16)):
+        for B in (1, 2, 4, 5, 8, 16, 17, 31, 32, 64, 96, 128, 192, 260, 1024):
+            per = B * kv * ((heads // kv + 15) // 16)
+            for pages in (1, 2, 3, 4, 5, 8, 9, 16, 17, 33, 64, 65, 256, 512):
+                for ragged in (False, True):
+                    quarters = min((pages + 3) // 4, 4)
+                    even = max(1, min((pages + 3) // 4, 256 // per))
+                    f32 = decode_splits(heads, kv, hd, B, pages, ragged, own=True)
+                    assert f32 == (quarters if per > 512 else max(even, quarters) if ragged and per <= 256 else even)
+                    n = decode_splits(heads, kv, hd, B, pages, ragged)
+                    assert 1 <= n <= max(1, pages)
+                    assert n * per <= max(per, 256) or ragged or per > 512
+                    if pages <= 4:
+                        assert n == 1
+                    if per > 512:
+                        assert n == (quarters if per < 768 else 1)
+                    elif ragged and (per <= 128 or (per <= 256 and pages > 16)):
+                        assert n == max(quarters, decode_splits(heads, kv, hd, B, pages))
+                    elif per > 64:
+                        assert n == even
+                    elif pages <= 32:
+                        assert n >= even
+                    assert decode_order(Step, B, heads, kv, n, own=True) == Step.seq_order
+                    assert decode_order(Step, B, heads, kv, n) == (None if n > 1 and 128 < per <= 512 else Step.seq_order)
+    assert 128 in kernels.MFMA_HEAD_DIMS and 256 in kernels.MFMA_WIDE_HEAD_DIMS

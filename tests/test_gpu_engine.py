@@ -139,6 +139,25 @@ def test_a_batch_of_more_than_256_rows(tmp_path_factory, dtype):
     assert checked >= 25
 
 
+def test_rows_just_above_a_round_of_workgroups(tmp_path_factory):
+    """260 unequal sequences without graphs, so that 520 workgroups stand for them: eight more than the chip holds at once, the
+    decode attention in four splits, most of them empty for the short sequences.  Some requests against the plain implementation."""
+    from yalm_amd.engine import Engine, Model
+    folder = helpers.make_folder(tmp_path_factory.mktemp("many_rows_eager"), "many_rows", MANY_ROWS, seed=10)
+    rng = np.random.default_rng(17)
+    lengths = [int(x) for x in rng.integers(3, 700, size=260)]
+    requests = helpers.random_requests(MANY_ROWS, lengths, seed=18)
+    first = {rid: len(t) - 2 for rid, t in requests.items()}
+    steps = schedules.batches(requests, [list(requests)], first)
+    model = Model.from_folder(folder, dtype=helpers.torch_dtype("bfloat16"), device="cuda:0")
+    engine = Engine(model, max_tokens=schedules.max_tokens_needed(steps), max_batch=260, use_graphs=False)
+    assert model.blocks[0].mixer.decode_splits(260, 16) == 4
+    got = schedules.per_request(steps, schedules.replay_in_process(engine, steps), requests)
+    for rid in list(requests)[::20]:
+        want = helpers.plain_logits(folder, tuple(requests[rid]), "bfloat16")
+        helpers.check_logits(got[rid][first[rid] - 1:], want[first[rid] - 1:], "bfloat16", "520 workgroups, request " + rid)
+
+
 def test_warmup_captures_ahead_and_leaves_live_sequences_alone(folders):
     """Graphs are captured on padding rows: in the middle of a request, for the bucket the request
     is in, and nothing the request holds changes; afterwards no live step captures."""

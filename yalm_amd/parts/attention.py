@@ -18,6 +18,8 @@ i - (window + sinks - 1) when it is read.
 The three projections are one matrix [q; k; v] (the reference fuses them by
 pointer, src/infer.cu:290-337); q/k rows are re-ordered at load if the folder
 keeps them half-split (convert.py:145-158)."""
+import math
+
 import torch
 
 from ..cache.manager import KVRequest
@@ -48,24 +50,47 @@ def kv_tiles(n_tok):
 kv_tiles.name = "kv_tiles"
 
 
-def decode_splits(n_heads, n_kv_heads, head_dim, B, max_pages, ragged=False, shaped=False):
+def decode_splits(n_heads, n_kv_heads, head_dim, B, max_pages, ragged=False, shaped=False, own=False):
     """Into how many pieces a decode step's attention cuts every sequence, so that about TARGET_WORKGROUPS
-    workgroups run.  shaped: the scores have a shape (a bias, a cap, ...), which the wide heads' kernels do not take."""
+    workgroups run.  shaped: the scores have a shape (a bias, a cap, ...), which the wide heads' kernels do not take.
+    own: float32, whose kernel cuts every sequence by its own length: four pages and more a piece, whoever stands beside it.
+    us below: bfloat16, 32 heads of 128 in 8 groups, all caches cold."""
     mfma = (head_dim in kernels.MFMA_HEAD_DIMS or (head_dim in kernels.MFMA_WIDE_HEAD_DIMS and not shaped)) \
         and not kernels.FORCE_SIMPLE
     if mfma:         # a workgroup of 4 waves per (split, KV head and up to 16 of its query heads, sequence), a page per wave at a time
         per = max(1, B * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16))
         quarters = max(1, min((max_pages + 3) // 4, 4))
-        if per > RESIDENT_WORKGROUPS:         # more than run at once: in quarters the last round is short
-            return quarters
-        even = max(1, min((max_pages + 3) // 4, TARGET_WORKGROUPS // per))
+        # More workgroups than run at once: in quarters the last round is short, which pays while it is nearly empty; from half
+        # a round on a split more is only another merge (96 rows of 1,000 tokens 70.2 in one, 82.1 in four; 80 of 3,000 158 and 169;
+        # 128 of 300 31.4, in two 43.2; of 200 to 1,000 tokens 96 rows 48.0 and 65.9).
+        if per > RESIDENT_WORKGROUPS:
+            return quarters if own or 2 * per < 3 * RESIDENT_WORKGROUPS else 1
+        if own or per > 64 or max_pages <= 4:
+            even = max(1, min((max_pages + 3) // 4, TARGET_WORKGROUPS // per))
+        else:
+            # Few rows: a wave's pages come one behind the other, 2.3 us each, and a split more costs the merge 0.15 us, which is
+            # least at the root of 3.8 pages; three pages of eight a split at the least (one row of 500 tokens in two splits 8.5, in three 7.5,
+            # of 1,000 in four 8.4, in six 7.5; three rows of 1,000 9.4 and 8.2; eight of 500 in two 9.2, in three 8.8).
+            # A workgroup on three quarters of the units reads as fast as one on each (one row of 28,000: 24 splits 23.6, 32 24.9).
+            most = TARGET_WORKGROUPS // per if per > 8 else TARGET_WORKGROUPS * 3 // 4 // per
+            even = max(1, min((3 * max_pages + 7) // 8, math.isqrt(19 * max_pages // 5), most))
         # Sequences of very unequal lengths.  Where the workgroups stand two to a compute unit anyway, one split and
         # the rows in the order that pairs a long sequence with a short one; else splits of the longest sequence's
-        # split size (the kernel cuts them so), enough of them that the long sequences' work spreads over the chip.
-        if ragged and per <= TARGET_WORKGROUPS:
+        # split size (the kernel cuts them so), enough of them that the long sequences' work spreads over the chip.  With a workgroup on more than
+        # half of the units and up to 16 pages the longest one's rounds are few, and one split is sooner (32 rows of 200 to 1,000
+        # tokens 19.1 in one, 25.7 in four; 17 of them 15.1 and 22.1; of 800 to 4,000 tokens 61 and 67 to 71, 17 of them 46 and 42).
+        if ragged and per <= TARGET_WORKGROUPS and (own or 2 * per <= TARGET_WORKGROUPS or max_pages > 16):
             return max(even, quarters)
         return even
     return max(1, min(max_pages, TARGET_WORKGROUPS // max(1, B * n_heads)))
+
+
+def decode_order(ctx, B, n_heads, n_kv_heads, n_splits, own=False):
+    """The order in which a decode step's attention takes the rows, or None.  It pairs a long sequence's workgroup with a short one's, which
+    holds where a row has one workgroup a KV head, or the workgroups of all its splits are few; with several splits of many rows the
+    plain order spreads them better (24 rows of 50 to 4,000 tokens in four splits 49.5 us in this order, 44.9 in the plain one; 9 rows 21.1 and 29.0)."""
+    per = B * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
+    return ctx.seq_order if own or n_splits == 1 or 2 * per <= TARGET_WORKGROUPS or per > RESIDENT_WORKGROUPS else None
 
 
 def decode_counters(ctx, B, n_heads, n_kv_heads, n_splits):
@@ -150,7 +175,8 @@ class GQAttention(Part):
                       "of 16 to 256 in steps of 16, to 128 with a score bias, not %d): correct, many times slower" % self.head_dim, True
 
     def decode_splits(self, B, max_pages, ragged=False):
-        return decode_splits(self.n_heads, self.n_kv_heads, self.head_dim, B, max_pages, ragged, shaped=hasattr(self.position, "score_bias"))
+        return decode_splits(self.n_heads, self.n_kv_heads, self.head_dim, B, max_pages, ragged, shaped=hasattr(self.position, "score_bias"),
+                             own=self.wo is not None and self.wo.dtype == torch.float32)
 
     def fuses_norm(self, norm, x, ctx):
         if not hasattr(norm, "fused") or self.head_dim % 16:
@@ -253,7 +279,8 @@ class GQAttention(Part):
             sinks = (sink_k, sink_v, self.position.table, self.position.rotary_dim, writes_cache)
         kernels.attn_decode(q, k_pages, v_pages, group.table, group.ring_pages, ctx.seq_slot, ctx.seq_len, o, partial,
                             self.n_heads, self.n_kv_heads, self.head_dim, self.window, n_splits, sinks=sinks,
-                            step_max_len=ctx.step_max_len, seq_order=ctx.seq_order, score_bias=self.score_bias,
+                            step_max_len=ctx.step_max_len, seq_order=decode_order(ctx, T, self.n_heads, self.n_kv_heads, n_splits, q.dtype == torch.float32),
+                            score_bias=self.score_bias,
                             counters=decode_counters(ctx, T, self.n_heads, self.n_kv_heads, n_splits))
 
     def forward(self, h, x, ctx, line, writes_cache=True, emit_for=None):

@@ -31,7 +31,7 @@ import torch
 from ..cache.manager import KVRequest
 from ..ops import kernels
 from ..weights.loader import ParamSpec, place
-from .attention import ROPE_TILES_MIN_TOKENS, decode_counters, decode_splits, kv_tiles
+from .attention import ROPE_TILES_MIN_TOKENS, decode_counters, decode_order, decode_splits, kv_tiles
 from .base import Part, build_part, part
 from .rope import interleave_rows
 
@@ -211,10 +211,10 @@ class LatentAttention(Part):
             kernels.attn_prefill(q, kst, vst, o, ctx.cu_seqlens, seq_tile0, ctx.tok_seq, ctx.tok_pos, H, 1, P,
                                  self.window, tiles.get("tile_order"))
         else:
-            n_splits = decode_splits(H, 1, P, T, min(group.ring_pages, ctx.pages_bucket), ctx.ragged)
+            n_splits = decode_splits(H, 1, P, T, min(group.ring_pages, ctx.pages_bucket), ctx.ragged, own=act == torch.float32)
             partial = ws.get("attn.partial", (kernels.attn_decode_workspace_floats(T, H, P, n_splits),), torch.float32)
             kernels.attn_decode(q, k_pages, v_pages, group.table, group.ring_pages, ctx.seq_slot, ctx.seq_len, o, partial,
-                                H, 1, P, self.window, n_splits, step_max_len=ctx.step_max_len, seq_order=ctx.seq_order,
+                                H, 1, P, self.window, n_splits, step_max_len=ctx.step_max_len, seq_order=decode_order(ctx, T, H, 1, n_splits, act == torch.float32),
                                 counters=decode_counters(ctx, T, H, 1, n_splits))
         # 4. the heads' values from their latent results, the gate, the output projection
         values = ws.get("latent.values", (T, H * self.v_dim), act)

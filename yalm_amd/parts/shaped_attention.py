@@ -30,7 +30,7 @@ import torch
 from ..cache.manager import KVRequest
 from ..ops import kernels
 from ..weights.loader import ParamSpec, place
-from .attention import decode_counters, decode_splits, kv_tiles
+from .attention import decode_counters, decode_order, decode_splits, kv_tiles
 from .base import JoinableMixer, build_part, part
 
 # A prompt step of at least this many tokens leaves its values row by row and transposes them a tile of 64 tokens at a
@@ -270,10 +270,10 @@ class ShapedAttention(JoinableMixer):
                                  tiles.get("tile_order"), score_bias=self.score_bias, softcap=self.softcap,
                                  sink_logit=self.sink, slopes=self.slopes, block=self.block, log_distance=self.log_ab)
         else:
-            n_splits = decode_splits(H, G, P, T, min(group.ring_pages, ctx.pages_bucket), ctx.ragged, shaped=self.shaped_scores)
+            n_splits = decode_splits(H, G, P, T, min(group.ring_pages, ctx.pages_bucket), ctx.ragged, shaped=self.shaped_scores, own=act == torch.float32)
             partial = ws.get("attn.partial", (kernels.attn_decode_workspace_floats(T, H, P, n_splits),), torch.float32)
             kernels.attn_decode(q, k_pages, v_pages, group.table, group.ring_pages, ctx.seq_slot, ctx.seq_len, o, partial,
-                                H, G, P, self.window, n_splits, step_max_len=ctx.step_max_len, seq_order=ctx.seq_order,
+                                H, G, P, self.window, n_splits, step_max_len=ctx.step_max_len, seq_order=decode_order(ctx, T, H, G, n_splits, act == torch.float32),
                                 counters=decode_counters(ctx, T, H, G, n_splits),
                                 score_bias=self.score_bias, softcap=self.softcap, sink_logit=self.sink, slopes=self.slopes,
                                 block=self.block, log_distance=self.log_ab)
