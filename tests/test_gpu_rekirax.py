@@ -355,6 +355,61 @@ def test_recurrence_kernel(dtype, H, d, dv, n_first):
     assert bool(torch.isnan(state[1]).all()) and float(state[3].abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("gates", ["ordinary", "strong", "weak", "zero and one"])
+@pytest.mark.parametrize("H,d,dv", [(1, 4, 4), (3, 32, 33), (2, 33, 16), (2, 64, 40), (1, 65, 130), (8, 128, 128), (16, 100, 64)])
+def test_recurrence_by_tiles(H, d, dv, gates):
+    """Prompts a tile of 64 tokens at a time: every remainder of a quarter, a half and a block of a tile, several tiles, states that
+    hold something, projections that are columns of wider rows, one and two column groups a workgroup, padded heads; against the
+    plain recurrence in float64 and held to what the walk is held to."""
+    from yalm_amd.ops import kernels
+    lens = [1, 3, 4, 6, 9, 17, 63, 64, 65, 131, 200] if H < 8 else [40] * 14 + [200]
+    g = gen(H * 1000 + d + dv)
+    rn = lambda *s, sc=1.0: torch.randn(*s, generator=g, dtype=F64) * sc
+    N, T = 2 * H * d + H * dv, sum(lens)
+    wide = f32(rn(T, N + 7, sc=1.5))
+    proj = wide[:, 5:5 + N]
+    lower = torch.rand(H * d, generator=g, dtype=F64)
+    bias = rn(H * d, sc=0.5)
+    if gates == "strong":
+        lower, bias = lower * 0.0, bias - 4.0
+    elif gates == "weak":
+        lower = 1.0 - 0.02 * lower
+    elif gates == "zero and one":
+        lower, bias = (lower > 0.7).to(F64), torch.where(lower < 0.3, -300.0, torch.where(lower < 0.5, 300.0, bias))
+    w = {"m.f": torch.eye(H * d, dtype=F64), "m.f.b": f32(bias).cpu().to(F64), "m.lower": f32(lower).cpu().to(F64), "m.norm": f32(1 + rn(dv, sc=0.2)).cpu().to(F64)}
+    slots = list(range(len(lens) + 1))[::-1][:len(lens)]
+    state = f32(rn(len(lens) + 2, H * dv * d, sc=0.5))
+    state[0].fill_(float("nan"))
+    before = state.clone()
+    out = torch.full((T, H * dv), float("nan"), device=DEV)
+    raw = torch.full((T, H * dv), float("nan"), device=DEV)
+    cu = [0] + list(np.cumsum(lens))
+    tile0 = [0] + list(np.cumsum([(n + 63) // 64 for n in lens]))
+    scratch = lambda name, shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device=DEV)
+    kernels.hgrn2_tiles(proj, f32(w["m.f.b"]), f32(w["m.lower"]), f32(w["m.norm"]), state, raw, i32(cu), i32(slots), i32(tile0), int(tile0[-1]),
+                        out, H, d, dv, 1e-5, scratch)
+    for b, n in enumerate(lens):
+        pr = proj[cu[b]:cu[b + 1]].cpu().to(F64)
+        q = P.silu(pr[:, :H * d]).reshape(n, H, d)
+        f = P.forget_gates(pr[:, H * d:2 * H * d], w, "m.").reshape(n, H, d)
+        S0 = before[slots[b]].cpu().to(F64).reshape(H, dv, d).transpose(1, 2)
+        o, S = P.hgrn2_recurrence(q, f, pr[:, 2 * H * d:].reshape(n, H, dv), S0)
+        want = (P.rms_div(o, 1e-5) * w["m.norm"]).reshape(n, H * dv)
+        assert torch.allclose(out[cu[b]:cu[b + 1]].cpu().to(F64), want, rtol=2e-5, atol=2e-5), (b, n)
+        got = state[slots[b]].cpu().to(F64).reshape(H, dv, d).transpose(1, 2)
+        assert torch.allclose(got, S, rtol=1e-5, atol=1e-5), (b, n)
+    assert bool(torch.isnan(state[0]).all()) and torch.equal(state[-1], before[-1])
+
+
+def test_when_the_recurrence_goes_by_tiles():
+    """Few workgroups of the walk and prompts long enough; never key heads that the tiles do not take."""
+    from yalm_amd.ops import kernels
+    pay = kernels.hgrn2_tiles_pay
+    assert pay(96, 1, 32, 128, 128) and not pay(95, 1, 32, 128, 128) and pay(1909, 5, 32, 128, 128) and not pay(2340, 9, 32, 128, 128)
+    assert pay(384, 1, 4, 64, 64) and not pay(383, 1, 4, 64, 64) and not pay(3000, 4, 64, 64, 64)
+    assert not pay(5000, 1, 1, 129, 16) and pay(5000, 1, 1, 128, 4000) and kernels.hgrn2_tiles_fit(128) == 128 and kernels.hgrn2_tiles_fit(129) == 0
+
+
 def test_recurrent_state_is_carried_in_32_bits():
     """A thousand tokens under gates close to one, token by token in steps of 1 to 50: the state stays within 2e-5 of its
     scale of the float64 recurrence."""
@@ -620,6 +675,15 @@ def test_unequal_batches_with_reuse(folders, name, dtype):
     if len(plan) > 1:
         steps = schedules.interleaved(reqs, plan, firsts, [0] + [3 * i for i in range(1, len(plan))])
         compare(folders, name, dtype, steps, reqs, engine_for(folders, name, dtype), "overlapping batches")
+
+
+@pytest.mark.parametrize("name", sorted(GROUPS))
+def test_unequal_batches_whose_recurrence_goes_by_tiles(folders, monkeypatch, name):
+    from yalm_amd.ops import kernels
+    taken = []
+    monkeypatch.setattr(kernels, "hgrn2_tiles_pay", lambda T, B, n_heads, d, dv: taken.append(T) or kernels.hgrn2_tiles_fit(d) > 0)
+    test_unequal_batches_with_reuse(folders, name, "bfloat16")
+    assert taken or not any("right" in layer["mixer"] for layer in KC.ALL[name]["layers"])
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -5,8 +5,18 @@
 // and each head's o is divided by its root mean square over dv and multiplied by a weight shared by the heads.
 // Everything behind the projections z_q | z_f | v (float32) is float32; the walk over the tokens is diag_scan.h's, but in a step of
 // one token a sequence (hgrn2_step_kernel).
+//
+// Prompts go a tile of 64 tokens at a time on the matrix cores, in float32 (v_mfma_f32_16x16x4_f32).  With F(s, t) the product of the
+// gates of the tokens behind s up to and including t (a number a channel),
+//     o_t = (q_t F(start, t)) S_0 + sum over s <= t of (sum over channels of q_t F(s, t) (1 - f_s)) v_s,
+//     S_64 = diag(F(start, 63)) S_0 + sum over s of (F(s, 63) (1 - f_s)) v_s^T.
+// Every F is a product of gates, formed factor by factor: no quotient, no logarithm, so that gates of 0 and of 1 and runs of small ones
+// are exact where the walk is.  hgrn2_tiles_kernel (every tile and head at once) makes the scaled operands and the second sum of o;
+// tile_scan.h's walk over the tiles the products with S_0 and the state.  Between two tokens of different blocks F is cut at the blocks'
+// borders into factors of the one, of the blocks between and of the other, which makes the sum over channels a matrix product: blocks of 16
+// tokens, halves of one and quarters of one; inside four tokens every pair's product is carried on from token to token.
 #include <climits>
-#include "diag_scan.h"
+#include "tile_scan.h"
 #include "yalm_hip.h"
 
 namespace {
@@ -16,7 +26,7 @@ struct Hgrn2Op {
   const float* proj;
   const float* f_bias;
   const float* lower;
-  int Hd, N, d, dv;                               // heads * d; from one token's projections to the next one's
+  int Hd, N, d, dv, Hv;                           // heads * d; from one token's projections to the next one's; heads * dv
   __device__ Row begin(int h, int r, bool ok) const {
     return {ok ? f_bias[h * d + r] : 0.f, ok ? lower[h * d + r] : 0.f};
   }
@@ -121,6 +131,288 @@ __global__ __launch_bounds__(THREADS) void hgrn2_step_kernel(Hgrn2Op op, float* 
 }
 }  // namespace
 
+namespace {
+constexpr int HT_HALF = 8, HT_QUAD = 4;          // tokens of half a block, of a quarter
+
+size_t hgrn2_tiles_lds(int dp) { return ((size_t)4 * GT * (dp + 4) + GNB * dp + (size_t)GT * GA_ROW) * sizeof(float); }
+
+// 1 / (1 + e^-z) to about an ulp of it: e^x by the exponential instruction with the rounding of x log2(e) put back, the reciprocal
+// instruction with one step of Newton's; behind -80, where the result is 1.8e-35, it stays there.  (expf and a division are three times
+// as many instructions, 2,048 of which a wave issues a tile.)
+__device__ __forceinline__ float tile_sigmoid(float z) {
+  const float x = fminf(-z, 80.f), t = x * 1.4426950408889634f;
+  const float lost = fmaf(x, 1.4426950408889634f, -t) + x * 1.925963033500601e-8f;      // log2(e) in two floats
+  const float e = __builtin_amdgcn_exp2f(t), den = 1.0f + fmaf(e, lost * 0.6931471805599453f, e), r = __builtin_amdgcn_rcpf(den);
+  return r * (2.0f - den * r);
+}
+
+// qd [tile][head][64][DP], kd [tile][head][DP][64] and gd [tile][head][DP] as tile_scan.h wants them; raw = the second sum of o.
+// A thread owns one channel of one block of 16 tokens.  LDS (155 KB at DP 128: a workgroup of eight waves a compute unit): four rows
+// a token, first q, 1 - f and f; then q F(block's start, t), (1 - f) F(t, block's end) and, for the halves of a block, q F(half's start, t)
+// in the second and (1 - f) F(t, half's end) in the first, and the same for the quarters of a half.
+// Bound by its phases one behind the other, 15 us a workgroup: the operands' way in 3, their gates 2, the scaled rows through LDS 4, the
+// products 2, the rest barriers and the way out (five prompts of 255 to 509 tokens, 32 heads of 128 x 128, 992 workgroups: 67 us, the
+// walk over the tiles behind it 83, the heads' norm 9; token by token 212 and 16).  Errors against 64 bits, relative, of
+// the normed heads: ordinary gates 9.2e-8 (token by token 8.6e-8), gates close to one 4.7e-7 (8.3e-7), small ones 7.0e-8 (7.1e-8); the state's
+// 1.1e-7 (1.4e-7), 1.6e-6 (2.8e-6), 3.3e-8 (2.7e-8).
+template <int DP>
+__global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float* __restrict__ raw, float* __restrict__ qd,
+                                                               float* __restrict__ kd, float* __restrict__ gd,
+                                                               const int* __restrict__ cu_seqlens, const int* __restrict__ seq_tile0,
+                                                               int B, int n_heads) {
+  constexpr int ROW = DP + 4, NWAVES = GNB * DP / WAVE, CH = DP / 16, CV = CH < 4 ? CH : 4;      // channels a lane of the pairs inside four tokens, and a load
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* s_q = lds;                               // [64][ROW]
+  float* s_k = s_q + GT * ROW;                    // [64][ROW]
+  float* s_f = s_k + GT * ROW;                    // [64][ROW]
+  float* s_e = s_f + GT * ROW;                    // [64][ROW]
+  float* s_tot = s_e + GT * ROW;                  // [4][DP]  the product of a block's gates
+  float* s_a = s_tot + GNB * DP;                  // [64][GA_ROW] scores
+  auto load_v = [](float* to, const float* from) {
+    typedef __attribute__((ext_vector_type(CV))) float vec;
+    const vec x = *reinterpret_cast<const vec*>(from);
+#pragma unroll
+    for (int u = 0; u < CV; ++u) to[u] = x[u];
+  };
+  const int gt = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int b = seq_of_tile(seq_tile0, B, gt);
+  const int p0 = (gt - seq_tile0[b]) * GT, first = cu_seqlens[b] + p0, n = min(GT, cu_seqlens[b + 1] - first);
+  if (n <= 0) return;
+  const int ch = tid % DP, sb = tid / DP, lane = tid % WAVE, li = lane % 16, lq = lane / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int d = op.d, dv = op.dv;
+  const bool ch_ok = ch < d;
+  // the values of the wave's first columns, in the order of the last product's operand: asked for first, needed last
+  const int n_cols = (dv + 15) / 16;
+  float vb[GT / 4];
+  auto load_values = [&](int col) {
+    const int j = min(col * 16 + li, dv - 1);
+#pragma unroll
+    for (int i = 0; i < GT / 4; ++i) {
+      const int s = 16 * (i / 4) + 4 * lq + i % 4;
+      vb[i] = op.value(first + min(s, n - 1), h, j);           // behind the text the score is zero
+    }
+  };
+  float q[GB], k[GB], f[GB];
+  {
+    float z[GB][2];
+#pragma unroll
+    for (int u = 0; u < GB; ++u) op.fetch(first + min(sb * GB + u, n - 1), h, min(ch, d - 1), z[u]);
+    if (wave < n_cols) load_values(wave);
+    const Hgrn2Op::Row mine = op.begin(h, ch, ch_ok);
+#pragma unroll
+    for (int u = 0; u < GB; ++u) {
+      const float qq = z[u][0] * tile_sigmoid(z[u][0]), ff = fmaf(1.0f - mine.lower, tile_sigmoid(z[u][1] + mine.bias), mine.lower);
+      const bool ok = ch_ok && sb * GB + u < n;    // what lies behind the text or the head adds nothing and forgets nothing
+      q[u] = ok ? qq : 0.f;
+      f[u] = ok ? ff : 1.f;
+      k[u] = ok ? 1.0f - ff : 0.f;
+    }
+  }
+  float total = 1.f;
+#pragma unroll
+  for (int u = 0; u < GB; ++u) {
+    const int at = (sb * GB + u) * ROW + ch;
+    s_q[at] = q[u], s_k[at] = k[u], s_f[at] = f[u];
+    total *= f[u];
+  }
+  s_tot[sb * DP + ch] = total;
+  lds_barrier();
+  float before = 1.f, after = 1.f, whole = 1.f;    // the gates of the blocks before and behind this thread's, of all
+#pragma unroll
+  for (int i = 0; i < GNB; ++i) {
+    const float t = s_tot[i * DP + ch];
+    if (i < sb) before *= t;
+    if (i > sb) after *= t;
+    whole *= t;
+  }
+  {
+    const size_t at = (size_t)gt * n_heads + h;
+    float* qo = qd + (at * GT + sb * GB) * DP + ch;
+    float* ko = kd + (at * DP + ch) * GT + sb * GB;
+    float c = before;
+#pragma unroll
+    for (int u = 0; u < GB; ++u) {
+      c *= f[u];
+      qo[(size_t)u * DP] = q[u] * c;
+    }
+    float e = after;
+#pragma unroll
+    for (int u = GB - 4; u >= 0; u -= 4) {
+      float4 o;
+      o.w = k[u + 3] * e, e *= f[u + 3];
+      o.z = k[u + 2] * e, e *= f[u + 2];
+      o.y = k[u + 1] * e, e *= f[u + 1];
+      o.x = k[u] * e, e *= f[u];
+      *reinterpret_cast<float4*>(ko + u) = o;
+    }
+    if (sb == 0) gd[at * DP + ch] = whole;
+  }
+  // Scores inside four tokens: a lane a token s and CH channels, whose product it carries on to the tokens s, s + 1, ...; the sixteen
+  // lanes of a token are four apart.
+  for (int quad = wave; quad < GT / HT_QUAD; quad += NWAVES) {
+    const int s = lane % HT_QUAD, e0 = lane / HT_QUAD * CH, row0 = quad * HT_QUAD;
+    float p[CH], sum[HT_QUAD];
+#pragma unroll
+    for (int i = 0; i < CH; i += CV) load_v(p + i, s_k + (row0 + s) * ROW + e0 + i);
+#pragma unroll
+    for (int step = 0; step < HT_QUAD; ++step) {
+      const int at = (row0 + min(s + step, HT_QUAD - 1)) * ROW + e0;
+      float acc[2] = {0.f, 0.f}, a[CH], g[CH];
+#pragma unroll
+      for (int i = 0; i < CH; i += CV) {
+        load_v(a + i, s_q + at + i);
+        if (step > 0) load_v(g + i, s_f + at + i);
+      }
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        if (step > 0) p[i] *= g[i];
+        acc[i & 1] = fmaf(a[i], p[i], acc[i & 1]);
+      }
+      sum[step] = acc[0] + acc[1];
+    }
+#pragma unroll
+    for (int step = 0; step < HT_QUAD; ++step) {
+#pragma unroll
+      for (int o = HT_QUAD; o < WAVE; o *= 2) sum[step] += __shfl_xor(sum[step], o, WAVE);
+    }
+    // the lanes of a token share its four results: one a lane, and the zeros of the tokens that do not see it
+    const int mine = lane / HT_QUAD;
+    const float r = mine == 0 ? sum[0] : mine == 1 ? sum[1] : mine == 2 ? sum[2] : sum[3];
+    const int t = s + mine;
+    if (mine < HT_QUAD) s_a[(row0 + t % HT_QUAD) * GA_ROW + row0 + s] = t < HT_QUAD ? r : 0.f;
+  }
+  lds_barrier();
+  {
+    float c = 1.f, c8 = 1.f, c4 = 1.f, e = 1.f, e8 = 1.f, e4 = 1.f;
+#pragma unroll
+    for (int u = 0; u < GB; ++u) {
+      const int at = (sb * GB + u) * ROW + ch;
+      c *= f[u];
+      s_q[at] = q[u] * c;
+      if (u & HT_HALF) {
+        c8 *= f[u];
+        s_f[at] = q[u] * c8;
+      }
+      if (u & HT_QUAD) {
+        c4 = (u & (HT_QUAD - 1)) == 0 ? f[u] : c4 * f[u];
+        s_e[at] = q[u] * c4;
+      }
+    }
+#pragma unroll
+    for (int u = GB - 1; u >= 0; --u) {
+      const int at = (sb * GB + u) * ROW + ch;
+      s_k[at] = k[u] * e;
+      e *= f[u];
+      if (!(u & HT_HALF)) {
+        s_f[at] = k[u] * e8;
+        e8 *= f[u];
+      }
+      if (!(u & HT_QUAD)) {
+        if ((u & (HT_QUAD - 1)) == HT_QUAD - 1) e4 = 1.f;
+        s_e[at] = k[u] * e4;
+        e4 *= f[u];
+      }
+    }
+  }
+  lds_barrier();
+  // scores between the blocks i > j (jobs 0 .. 5), between the halves of block i (6 .. 9) and between the quarters of its halves (the others);
+  // the rows of the last two are both operands: the later part's the queries, the earlier part's the keys
+  constexpr int PAIRS = GNB * (GNB - 1) / 2;
+  for (int job = wave; job < PAIRS + 2 * GNB; job += NWAVES) {
+    const int part = job < PAIRS ? 0 : job < PAIRS + GNB ? HT_HALF : HT_QUAD;      // tokens of a part
+    const int i = part ? (job - PAIRS) % GNB : job < 1 ? 1 : job < 3 ? 2 : 3, j = part ? i : job - i * (i - 1) / 2;
+    const float* pa = (part == 0 ? s_q : part == HT_HALF ? s_f : s_e) + (i * GB + li) * ROW + 4 * lq;
+    const float* px = part == 0 ? s_k + (j * GB + li) * ROW + 4 * lq : pa;
+    gf32x4 acc[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = (gf32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int m = 0; m < DP / 16; ++m) {
+      float4 a = *reinterpret_cast<const float4*>(pa + 16 * m);
+      const float4 x = *reinterpret_cast<const float4*>(px + 16 * m);
+      for (int g = j + 1; g < i; ++g) {            // the blocks between
+        const float4 t = *reinterpret_cast<const float4*>(s_tot + g * DP + 16 * m + 4 * lq);
+        a.x *= t.x, a.y *= t.y, a.z *= t.z, a.w *= t.w;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = mfma4(el(a, r), el(x, r), acc[r]);
+    }
+    const gf32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 4 * lq + r, s = li;
+      float* to = s_a + (i * GB + t) * GA_ROW + j * GB + s;
+      if (part == 0) {
+        *to = sum[r];
+      } else if (t / (2 * part) == s / (2 * part)) {
+        if ((t & part) && !(s & part)) *to = sum[r];
+        else if (!(t & part) && (s & part)) *to = 0.f;           // the earlier part does not see the later one
+      }
+    }
+  }
+  lds_barrier();
+  for (int col = wave; col < n_cols; col += NWAVES) {
+    if (col != wave) load_values(col);
+    const int j = col * 16 + li;
+#pragma unroll
+    for (int i = 0; i < GNB; ++i) {
+      gf32x4 acc[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = (gf32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m <= i; ++m) {
+        const float4 a = *reinterpret_cast<const float4*>(s_a + (i * GB + li) * GA_ROW + 16 * m + 4 * lq);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = mfma4(el(a, r), vb[4 * m + r], acc[r]);
+      }
+      const gf32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = i * GB + 4 * lq + r;
+        if (t < n && j < dv) raw[(size_t)(first + t) * op.Hv + h * dv + j] = sum[r];
+      }
+    }
+  }
+}
+
+int hgrn2_padded_dim(int d) { return d <= 0 ? 0 : d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 0; }
+
+template <int DP>
+int hgrn2_tiles_launch(const Hgrn2Op& op, float* state, float* raw, float* qd, float* kd, float* gd, const int* cu_seqlens,
+                       const int* seq_slot, const int* seq_tile0, int n_tiles, int B, int n_heads, hipStream_t stream) {
+  static LdsAllowance allowance;
+  const size_t lds = hgrn2_tiles_lds(DP);
+  int rc = allow_dynamic_lds(allowance, reinterpret_cast<const void*>(hgrn2_tiles_kernel<DP>), (int)lds);
+  if (rc != YALM_OK) return rc;
+  hgrn2_tiles_kernel<DP><<<dim3(n_tiles, n_heads), GNB * DP, lds, stream>>>(op, raw, qd, kd, gd, cu_seqlens, seq_tile0, B, n_heads);
+  rc = launch_status();
+  if (rc != YALM_OK) return rc;
+  return scan_carry_launch<DP>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, B, n_heads, stream);
+}
+}  // namespace
+
+extern "C" int yalm_hgrn2_tiles_fit(int d) { return hgrn2_padded_dim(d); }
+
+extern "C" int yalm_hgrn2_tiles(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm,
+                                float* state, float* raw, float* qd, float* kd, float* gd, const int* cu_seqlens, const int* seq_slot,
+                                const int* seq_tile0, int n_tiles, void* out, int T, int B, int n_heads, int d, int dv, float eps,
+                                int out_dtype, hipStream_t stream) {
+  if (T <= 0 || B <= 0 || n_tiles <= 0) return YALM_OK;
+  const int dp = hgrn2_padded_dim(d);
+  if (n_heads <= 0 || n_heads > 65535 || B > 65535 || dp == 0 || dv <= 0 || ceil_div(dv, 16) > 65535 ||
+      ((((uintptr_t)qd) | ((uintptr_t)kd) | ((uintptr_t)gd)) & 15))
+    return YALM_ERR_ARG;
+  if (out_dtype != YALM_F32 && out_dtype != YALM_BF16) return YALM_ERR_DTYPE;
+  if (proj_row < 2 * n_heads * d + n_heads * dv || proj_row > INT_MAX) return YALM_ERR_ARG;
+  const Hgrn2Op op = {proj, f_bias, lower, n_heads * d, (int)proj_row, d, dv, n_heads * dv};
+  const int rc = dp == 32   ? hgrn2_tiles_launch<32>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, n_tiles, B, n_heads, stream)
+                 : dp == 64 ? hgrn2_tiles_launch<64>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, n_tiles, B, n_heads, stream)
+                            : hgrn2_tiles_launch<128>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, n_tiles, B, n_heads, stream);
+  if (rc != YALM_OK) return rc;
+  return heads_norm_launch(raw, w_norm, nullptr, 0, out, T, n_heads, dv, eps, out_dtype, stream);
+}
+
 extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state,
                           float* raw, const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads,
                           int d, int dv, float eps, int out_dtype, hipStream_t stream) {
@@ -128,7 +420,7 @@ extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias,
   if (n_heads <= 0 || d <= 0 || d > 256 || dv <= 0) return YALM_ERR_ARG;
   if (out_dtype != YALM_F32 && out_dtype != YALM_BF16) return YALM_ERR_DTYPE;
   if (proj_row < 2 * n_heads * d + n_heads * dv || proj_row > INT_MAX) return YALM_ERR_ARG;
-  const Hgrn2Op op = {proj, f_bias, lower, n_heads * d, (int)proj_row, d, dv};
+  const Hgrn2Op op = {proj, f_bias, lower, n_heads * d, (int)proj_row, d, dv, n_heads * dv};
   // one token a sequence, as the numbers say (the kernel walks whatever cu_seqlens holds; eight tokens of one sequence and none of seven
   // others, which no step of the engine is, take it 12 us and diag_scan_kernel 6)
   if (T == B && n_heads <= 65535 && B <= 65535 && d <= HS_MAX && dv <= HS_MAX && d % 4 == 0 && dv % 4 == 0 && ((uintptr_t)state & 15) == 0) {

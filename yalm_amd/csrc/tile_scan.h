@@ -32,10 +32,10 @@ __device__ __forceinline__ int seq_of_tile(const int* __restrict__ seq_tile0, in
   return lo;
 }
 
-// The state over the tiles of a sequence, and its share of o added to raw.  NW waves, wave w the rows 32 w .. 32 w + 31.
-// WHOLE: dv is a multiple of 16, so that every tile but a sequence's last one is stored without a branch (behind a branch
-// the compiler would wait for the operands that are still on their way).
-template <class Op, int NW, bool WHOLE>
+// The state over the tiles of a sequence, and its share of o added to raw.  NW waves, wave w the rows 32 w .. 32 w + 31, of NC times 16
+// columns.  WHOLE: dv is a multiple of the workgroup's columns, so that every tile but a sequence's last one is stored without a branch (behind
+// a branch the compiler would wait for the operands that are still on their way).
+template <class Op, int NW, int NC, bool WHOLE>
 __global__ __launch_bounds__(NW * WAVE) void scan_carry_kernel(Op op, float* __restrict__ state, float* __restrict__ raw,
                                                                const float* __restrict__ qd, const float* __restrict__ kd,
                                                               const float* __restrict__ gd, const int* __restrict__ cu_seqlens,
@@ -43,27 +43,30 @@ __global__ __launch_bounds__(NW * WAVE) void scan_carry_kernel(Op op, float* __r
                                                               int n_heads) {
   constexpr int DP = 32 * NW, TB = GNB / NW > 0 ? GNB / NW : 1;      // row blocks of o a wave adds up
   static_assert(GNB % NW == 0, "");
-  __shared__ gf32x4 s_o[2][NW][GNB][WAVE];
+  __shared__ gf32x4 s_o[2][NW][NC][GNB][WAVE];
   // heads run fastest: with a number of heads that is a multiple of the chip's eight parts, the workgroups of one head (which
   // read the same scaled queries and keys) share a second-level cache
   const int b = blockIdx.z, h = blockIdx.x, tid = threadIdx.x, lane = tid % WAVE, li = lane % 16, lq = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int j = blockIdx.y * 16 + li, d = op.d, dv = op.dv;
+  const int j0 = blockIdx.y * (16 * NC) + li, d = op.d, dv = op.dv;
   const int slot = seq_slot[b], start = cu_seqlens[b], len = cu_seqlens[b + 1] - start, tile0 = seq_tile0[b];
   const int n_tiles = (len + GT - 1) / GT;
-  const bool col_ok = j < dv;
-  float* sp = state + (((size_t)max(slot, 0) * n_heads + h) * dv + min(j, dv - 1)) * d;
-  gf32x4 S[2];
+  auto column = [&](int c) { return min(j0 + 16 * c, dv - 1); };
+  auto col_ok = [&](int c) { return j0 + 16 * c < dv; };
+  float* sp = state + ((size_t)max(slot, 0) * n_heads + h) * dv * d;
+  gf32x4 S[NC][2];
 #pragma unroll
-  for (int R = 0; R < 2; ++R)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int e = 32 * wave + 16 * R + 4 * lq + r;
-      S[R][r] = slot >= 0 && col_ok && e < d ? sp[e] : 0.f;
-    }
+    for (int R = 0; R < 2; ++R)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = 32 * wave + 16 * R + 4 * lq + r;
+        S[c][R][r] = slot >= 0 && col_ok(c) && e < d ? sp[(size_t)column(c) * d + e] : 0.f;
+      }
   struct Operands {
     float4 q[GNB][2], k[2][GNB], g[2];
-    float v[GT / 4], o[TB][4];
+    float v[NC][GT / 4], o[NC][TB][4];
   };
   auto load = [&](int tile, Operands& x) {
     const size_t at = (size_t)(tile0 + tile) * n_heads + h;
@@ -80,51 +83,65 @@ __global__ __launch_bounds__(NW * WAVE) void scan_carry_kernel(Op op, float* __r
       }
     }
 #pragma unroll
-    for (int i = 0; i < GT / 4; ++i) {
-      const int s = 16 * (i / 4) + 4 * lq + i % 4;
-      x.v[i] = op.value(first + min(s, n - 1), h, min(j, dv - 1));       // behind the text k is zero
-    }
+    for (int c = 0; c < NC; ++c) {
 #pragma unroll
-    for (int i = 0; i < TB; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = (wave * TB + i) * GB + 4 * lq + r;
-        x.o[i][r] = raw[(size_t)(first + min(t, n - 1)) * op.Hv + h * dv + min(j, dv - 1)];
+      for (int i = 0; i < GT / 4; ++i) {
+        const int s = 16 * (i / 4) + 4 * lq + i % 4;
+        x.v[c][i] = op.value(first + min(s, n - 1), h, column(c));       // behind the text k is zero
       }
+#pragma unroll
+      for (int i = 0; i < TB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = (wave * TB + i) * GB + 4 * lq + r;
+          x.o[c][i][r] = raw[(size_t)(first + min(t, n - 1)) * op.Hv + h * dv + column(c)];
+        }
+    }
   };
   auto work = [&](int tile, const Operands& x, auto whole) {
     const int first = start + tile * GT, n = min(GT, len - tile * GT), buf = tile & 1;
-    gf32x4 acc[GNB];
 #pragma unroll
-    for (int i = 0; i < GNB; ++i) acc[i] = (gf32x4){0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NC; ++c) {
+      gf32x4 acc[GNB];
 #pragma unroll
-    for (int R = 0; R < 2; ++R)
+      for (int i = 0; i < GNB; ++i) acc[i] = (gf32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int R = 0; R < 2; ++R)
 #pragma unroll
-        for (int i = 0; i < GNB; ++i) acc[i] = mfma4(el(x.q[i][R], r), S[R][r], acc[i]);
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int R = 0; R < 2; ++R)
+          for (int i = 0; i < GNB; ++i) acc[i] = mfma4(el(x.q[i][R], r), S[c][R][r], acc[i]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[R][r] *= el(x.g[R], r);
+      for (int i = 0; i < GNB; ++i) s_o[buf][wave][c][i][lane] = acc[i];
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+#pragma unroll
+      for (int R = 0; R < 2; ++R)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[c][R][r] *= el(x.g[R], r);
+    }
 #pragma unroll
     for (int i = 0; i < GT / 4; ++i)
 #pragma unroll
-      for (int R = 0; R < 2; ++R) S[R] = mfma4(el(x.k[R][i / 4], i % 4), Op::act(x.v[i]), S[R]);
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int i = 0; i < GNB; ++i) s_o[buf][wave][i][lane] = acc[i];
+        for (int R = 0; R < 2; ++R) S[c][R] = mfma4(el(x.k[R][i / 4], i % 4), Op::act(x.v[c][i]), S[c][R]);
     lds_barrier();                                // the next tile's operands stay in flight
 #pragma unroll
-    for (int i = 0; i < TB; ++i) {
-      gf32x4 sum = s_o[buf][0][wave * TB + i][lane];
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int w = 1; w < NW; ++w) sum += s_o[buf][w][wave * TB + i][lane];
+      for (int i = 0; i < TB; ++i) {
+        gf32x4 sum = s_o[buf][0][c][wave * TB + i][lane];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = (wave * TB + i) * GB + 4 * lq + r;
-        if (decltype(whole)::value || (t < n && col_ok)) raw[(size_t)(first + t) * op.Hv + h * dv + j] = x.o[i][r] + sum[r];
+        for (int w = 1; w < NW; ++w) sum += s_o[buf][w][c][wave * TB + i][lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = (wave * TB + i) * GB + 4 * lq + r;
+          if (decltype(whole)::value || (t < n && col_ok(c)))
+            raw[(size_t)(first + t) * op.Hv + h * dv + j0 + 16 * c] = x.o[c][i][r] + sum[r];
+        }
       }
-    }
   };
   Operands even, odd;                             // the next tile's operands are asked for before this tile's products
   if (n_tiles <= 0) return;
@@ -146,26 +163,40 @@ __global__ __launch_bounds__(NW * WAVE) void scan_carry_kernel(Op op, float* __r
   } else {
     work(tile, even, std::false_type{});
   }
-  if (slot < 0 || !col_ok) return;
+  if (slot < 0) return;
 #pragma unroll
-  for (int R = 0; R < 2; ++R)
+  for (int c = 0; c < NC; ++c) {
+    if (!col_ok(c)) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int e = 32 * wave + 16 * R + 4 * lq + r;
-      if (e < d) sp[e] = S[R][r];
-    }
+    for (int R = 0; R < 2; ++R)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = 32 * wave + 16 * R + 4 * lq + r;
+        if (e < d) sp[(size_t)column(c) * d + e] = S[c][R][r];
+      }
+  }
 }
 
+template <int DP, int NC, class Op>
+int scan_carry_columns(const Op& op, float* state, float* raw, const float* qd, const float* kd, const float* gd, const int* cu_seqlens,
+                       const int* seq_slot, const int* seq_tile0, int B, int n_heads, hipStream_t stream) {
+  const dim3 grid(n_heads, ceil_div(op.dv, 16 * NC), B);
+  if (op.dv % (16 * NC) == 0)
+    scan_carry_kernel<Op, DP / 32, NC, true><<<grid, DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
+                                                                             seq_tile0, n_heads);
+  else
+    scan_carry_kernel<Op, DP / 32, NC, false><<<grid, DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
+                                                                              seq_tile0, n_heads);
+  return launch_status();
+}
+
+// Every workgroup of a head reads the head's scaled queries and keys whole: with 32 columns half as often as with 16, which pays where
+// that still leaves a workgroup and a half for each compute unit (HGRN2, five prompts of 255 to 509 tokens, 32 heads of 128 x 128: 102 -> 83 us).  The sums are the same.
 template <int DP, class Op>
 int scan_carry_launch(const Op& op, float* state, float* raw, const float* qd, const float* kd, const float* gd, const int* cu_seqlens,
                       const int* seq_slot, const int* seq_tile0, int B, int n_heads, hipStream_t stream) {
-  const dim3 grid(n_heads, ceil_div(op.dv, 16), B);
-  if (op.dv % 16 == 0)
-    scan_carry_kernel<Op, DP / 32, true><<<grid, DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
-                                                                         seq_tile0, n_heads);
-  else
-    scan_carry_kernel<Op, DP / 32, false><<<grid, DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
-                                                                          seq_tile0, n_heads);
-  return launch_status();
+  if (2L * n_heads * ceil_div(op.dv, 32) * B >= 3L * compute_units())
+    return scan_carry_columns<DP, 2>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, B, n_heads, stream);
+  return scan_carry_columns<DP, 1>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, B, n_heads, stream);
 }
 }  // namespace

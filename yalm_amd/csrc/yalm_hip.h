@@ -480,6 +480,12 @@ int yalm_loop_pack(float* x, const float* x0, const float* start, void* both, in
 int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state, float* raw,
                const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads, int d, int dv, float eps,
                int out_dtype, hipStream_t stream);
+// The same for steps of prompts, a tile of 64 tokens at a time (seq_tile0, n_tiles and scratch as for yalm_gla_tiles, DP =
+// yalm_hgrn2_tiles_fit(d); 0: key heads of d are not taken).
+int yalm_hgrn2_tiles_fit(int d);
+int yalm_hgrn2_tiles(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state, float* raw,
+                     float* qd, float* kd, float* gd, const int* cu_seqlens, const int* seq_slot, const int* seq_tile0, int n_tiles,
+                     void* out, int T, int B, int n_heads, int d, int dv, float eps, int out_dtype, hipStream_t stream);
 
 // Gated linear attention (gla.hip): proj float32 [T, 2 H d + 2 H dv + rank] = q | k | v | g | low of every token; a decay per
 // head and key channel f = sigmoid(w2 low + bias)^inv_tau (w2 float32 [H d, rank rounded up to a multiple of 4], zeros behind

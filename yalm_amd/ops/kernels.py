@@ -1408,6 +1408,48 @@ def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_
     return out
 
 
+def hgrn2_tiles_pay(T, B, n_heads, d, dv):
+    """Whether a step of prompts goes tile by tile (hgrn2_tiles) instead of token by token (hgrn2).  The walk takes 0.26 us a token (heads of
+    128 x 128; 0.16 of 64 x 64) while its workgroups, 32 columns of a sequence and head each, are not much more than two a compute
+    unit, and more in proportion behind that; the tiles take 13 to 16 us for every 256 of them and 3 us for each of a sequence's, and all
+    operands pass through memory.  Measured, us, walk and tiles: 32 heads of 128 x 128: one prompt of 64 tokens 22 and 24,
+    100 34 and 28, 2,048 529 and 181; five of 255 to 509 228 and 167; nine of 260 187 and 236, nine of 700 500 and 532; 64 of 33 170
+    and 428; 8 heads, 700 tokens 181 and 57.  Heads of 64 x 64: 4 of them, 100 tokens 21 and 22, 700 112 and 40; eight prompts of 100, 16 heads
+    25 and 32; four of 300, 16 heads of 32 x 64 38 and 40; 4 of 16 x 16, 500 tokens 52 and 33."""
+    groups = B * n_heads * ((dv + 31) // 32)
+    if d <= 64:
+        return hgrn2_tiles_fit(d) > 0 and T >= 384 * B and groups <= 256
+    return hgrn2_tiles_fit(d) > 0 and T >= 96 * B and groups <= 640
+
+
+def hgrn2_tiles_fit(d):
+    """The padded key size with which hgrn2_tiles takes key heads of d, or 0: it does not."""
+    return library.lib().yalm_hgrn2_tiles_fit(int(d))
+
+
+def hgrn2_tiles(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, seq_tile0, n_tiles, out, n_heads, d, dv, eps, scratch):
+    """hgrn2 for a step of prompts, a tile of 64 tokens at a time on the matrix cores in float32; seq_tile0 and scratch as for
+    gla_tiles."""
+    T, B = proj.shape[0], seq_slot.shape[0]
+    N = 2 * n_heads * d + n_heads * dv
+    dp = hgrn2_tiles_fit(d)
+    if not dp:
+        raise ValueError("hgrn2_tiles: key heads of %d are not taken" % d)
+    if proj.dtype != torch.float32 or proj.dim() != 2 or proj.shape[1] != N or proj.stride(1) != 1 or not proj.is_cuda:
+        raise ValueError("hgrn2_tiles: the projections are float32 [%d, %d] on the device, rows contiguous" % (T, N))
+    qd = scratch("scan.qd", (n_tiles, n_heads, PAGE, dp), torch.float32)
+    kd = scratch("scan.kd", (n_tiles, n_heads, dp, PAGE), torch.float32)
+    gd = scratch("scan.gd", (n_tiles, n_heads, dp), torch.float32)
+    library.check(library.lib().yalm_hgrn2_tiles(
+        proj.data_ptr(), int(proj.stride(0)), _need(f_bias, "f_bias", torch.float32, (n_heads * d,)),
+        _need(lower, "lower", torch.float32, (n_heads * d,)), _need(w_norm, "w_norm", torch.float32, (dv,)),
+        _need(state, "state", torch.float32, (None, n_heads * d * dv)), _need(raw, "raw", torch.float32, (T, n_heads * dv)),
+        qd.data_ptr(), kd.data_ptr(), gd.data_ptr(), _need(cu_seqlens, "cu_seqlens", torch.int32, (B + 1,)),
+        _need(seq_slot, "seq_slot", torch.int32, (B,)), _need(seq_tile0, "seq_tile0", torch.int32, (B + 1,)), n_tiles,
+        _need(out, "out", None, (T, n_heads * dv)), T, B, n_heads, d, dv, float(eps), dtype_code(out.dtype), _stream()), "hgrn2_tiles")
+    return out
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # gated linear attention
 GLA_MAX_KEY_DIM = 256             # rows of a state column over a workgroup's lanes

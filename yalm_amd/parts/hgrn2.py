@@ -13,6 +13,7 @@ import torch
 from ..cache.manager import StateRequest
 from ..ops import kernels
 from ..weights.loader import ParamSpec, place
+from .attention import kv_tiles
 from .base import Part, part
 
 NAMES = {"q": "q", "f": "f", "f_bias": "f.b", "lower": "lower", "v": "v", "norm": "norm", "out": "o"}
@@ -20,6 +21,7 @@ NAMES = {"q": "q", "f": "f", "f_bias": "f.b", "lower": "lower", "v": "v", "norm"
 
 @part("mixer", "hgrn2")
 class HGRN2(Part):
+    prompt_tables = (kv_tiles,)
     front_shared = False              # whether somebody else makes the product in front (as JoinableMixer has it)
 
     def __init__(self, spec, dim, prefix):
@@ -93,6 +95,16 @@ class HGRN2(Part):
         raw = ws.get("hgrn2.raw", (T, self.vv), torch.float32)
         o = ws.get("hgrn2.o", (T, self.vv), h.dtype)
         state = ctx.cache.group_of(line).line_state(line)
+        B = ctx.seq_slot.shape[0]
+        if ctx.mode == "prefill" and h.dtype == torch.bfloat16 and not kernels.FORCE_SIMPLE \
+                and kernels.hgrn2_tiles_pay(T, B, self.n_heads, self.key_dim, self.value_dim):
+            tiles = ctx.tables["kv_tiles"]
+            kernels.hgrn2_tiles(proj, self.f_bias, self.lower, self.w_norm, state, raw, ctx.cu_seqlens, ctx.seq_slot, tiles["seq_tile0"],
+                                tiles["n_tiles"], o, self.n_heads, self.key_dim, self.value_dim, self.eps, ws.get)
+        else:                 # float32 as the compute dtype: prompts go token by token too, so that their bits stay what they were
+            self._walk(proj, state, raw, o, ctx)
+        self._gemm(ctx, o, self.wo, x, epilogue)
+
+    def _walk(self, proj, state, raw, o, ctx):
         kernels.hgrn2(proj, self.f_bias, self.lower, self.w_norm, state, raw, ctx.cu_seqlens, ctx.seq_slot, o, self.n_heads,
                       self.key_dim, self.value_dim, self.eps)
-        self._gemm(ctx, o, self.wo, x, epilogue)
