@@ -198,6 +198,33 @@ def test_where_the_middle_rides_in_the_product(M, F, Kd, dtype, inside):
     assert kernels.gated_bias_scratch_floats(M, F, Kd, dtype) == (0 if inside else M * 2 * F)
 
 
+@pytest.mark.parametrize("residual", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,D,taps", [(1, 1028, 4), (7, 2048, 3), (3, 4096, 4), (40, 4100, 2), (5, 4096, 1), (2, 8192, 4), (260, 1536, 4)])
+def test_norm_and_convolution_of_single_tokens(T, D, taps, dtype, residual):
+    """One launch has the bits of the two: the results and the carried inputs, with rows of padding among the tokens."""
+    from yalm_amd.ops import kernels
+    x, nw, w = randn(T, D, seed=1, scale=3.0).to(DEV), (1.0 + 0.2 * randn(D, seed=2)).to(DEV), randn(taps, D, seed=3).to(DEV)
+    slots = i32([-1 if t % 5 == 3 else T - 1 - t for t in range(T)])
+    held = [randn(T, taps - 1, D, seed=4).to(DEV) if taps > 1 else None for _ in range(2)]
+    h, want, got = (torch.full((T, D), float("nan"), dtype=dtype, device=DEV) for _ in range(3))
+    assert kernels.norm_conv_fits(x, taps, nw, w)
+    kernels.rmsnorm(x, nw, h, 1e-5)
+    kernels.time_conv(h, w, held[0], want, i32(range(T)), i32(range(T + 1)), slots, residual, one_token_each=True)
+    kernels.norm_conv(x, nw, 1e-5, w, held[1], got, slots, residual)
+    assert bool(torch.isfinite(want).all()) and torch.equal(got, want)
+    assert taps == 1 or torch.equal(held[0], held[1])
+
+
+def test_norm_and_convolution_what_is_taken():
+    from yalm_amd.ops import kernels
+    flat = torch.zeros(8192 * 2 + 4, device=DEV)
+    rows = lambda D, at=0: flat[at:at + D].view(1, D)
+    assert [kernels.norm_conv_fits(rows(D), 4) for D in (1024, 1026, 1028, 8192, 8196)] == [False, False, True, True, False]
+    assert [kernels.norm_conv_fits(rows(2048), t) for t in (0, 1, 4, 5)] == [False, True, True, False]
+    assert not kernels.norm_conv_fits(rows(2048, 1), 4) and not kernels.norm_conv_fits(rows(2048), 4, flat[2:10])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T", [5, 40, 130])
 @pytest.mark.parametrize("off", [(1, 0), (0, 1), (3, 2)])
@@ -684,6 +711,26 @@ def test_unequal_batches_whose_recurrence_goes_by_tiles(folders, monkeypatch, na
     monkeypatch.setattr(kernels, "hgrn2_tiles_pay", lambda T, B, n_heads, d, dv: taken.append(T) or kernels.hgrn2_tiles_fit(d) > 0)
     test_unequal_batches_with_reuse(folders, name, "bfloat16")
     assert taken or not any("right" in layer["mixer"] for layer in KC.ALL[name]["layers"])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_unequal_batches_whose_norm_rides_on_the_convolution(folders, monkeypatch, dtype):
+    """The way of the wide models through a layer, at a small width: the two kernels stand in for the one."""
+    from yalm_amd.ops import kernels
+    taken = []
+
+    def both(x, nw, eps, w, carried, out, seq_slot, residual=True):
+        taken.append(x.shape[0])
+        T = x.shape[0]
+        h = kernels.rmsnorm(x, nw, torch.empty(out.shape, dtype=out.dtype, device=x.device), eps)
+        rows = torch.arange(T + 1, dtype=torch.int32, device=x.device)
+        return kernels.time_conv(h, w, carried, out, rows[:T], rows, seq_slot, residual, one_token_each=True)
+    monkeypatch.setattr(kernels, "norm_conv_fits", lambda x, taps, *others: True)
+    monkeypatch.setattr(kernels, "norm_conv", both)
+    requests = requests_for(KC.MIXED, [90, 20, 3], seed=7)
+    steps = schedules.batches(requests, [list(requests)], {"r0": 50, "r1": 3, "r2": 1})
+    compare(folders, "mixed", dtype, steps, requests, engine_for(folders, "mixed", dtype, use_graphs=False), "norm in the convolution")
+    assert taken
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

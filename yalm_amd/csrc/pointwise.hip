@@ -5,6 +5,7 @@
 // gate on an attention's heads (a number an element, or a number a head), the way into a walk of looped layers, and the cap
 // on logits.
 #include "common.h"
+#include "rms_row.h"
 #include "yalm_hip.h"
 
 namespace {
@@ -220,6 +221,65 @@ __global__ void time_conv_vec_kernel(const E* __restrict__ h, long h_row, const 
   }
 }
 
+// A step of one token a sequence from the residual stream: out = (residual ? h : 0) + conv(h) with h = rmsnorm(x, nw) rounded to the
+// compute dtype, the carried inputs left advanced, bit for bit what the norm's kernel and time_conv_vec_kernel leave.  Such a step is
+// latency: two launches, and the carried rows and taps asked for only behind the norm's sum.  Here they are on their way while the row is
+// summed.  The workgroups of a row (blockIdx.y, 1,024 channels each) all form the row's sum and take their channels.  At most
+// NORM_CONV_MAX_TAPS taps, whose carried rows wait in registers.  Rows of 4,096 with 4 taps, two launches and this one: 8 tokens 6.0 and
+// 2.8 us, 64 tokens 6.7 and 3.3, 256 tokens 9.6 and 6.2, 512 tokens 15.0 and 10.3 (24 MB: 2.4 TB/s, the row read once a workgroup).
+constexpr int NORM_CONV_MAX_TAPS = 4;
+template <typename TO, int VEC>
+__global__ __launch_bounds__(256) void norm_conv_step_kernel(
+    const float* __restrict__ x, const float* __restrict__ nw, float eps, const float* __restrict__ w, float* __restrict__ carried,
+    TO* __restrict__ out, const int* __restrict__ seq_slot, int D, int taps, int residual) {
+  __shared__ float red[4];
+  const int t = blockIdx.x, n4 = D / 4, own4 = blockIdx.y * 256 + threadIdx.x, keep = taps - 1;
+  const int c4 = min(own4, n4 - 1);               // (threads behind the row load its end and store nothing)
+  const float4* xr = reinterpret_cast<const float4*>(x + (size_t)t * D);
+  const int slot = seq_slot[t];
+  float4 v[VEC];
+#pragma unroll
+  for (int u = 0; u < VEC; ++u) {
+    const int i = threadIdx.x + u * 256;
+    v[u] = i < n4 ? xr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const float4 mine = xr[c4], nw4 = reinterpret_cast<const float4*>(nw)[c4];
+  float4 wj[NORM_CONV_MAX_TAPS], prev[NORM_CONV_MAX_TAPS - 1];
+#pragma unroll
+  for (int j = 0; j < NORM_CONV_MAX_TAPS; ++j)
+    wj[j] = j < taps ? reinterpret_cast<const float4*>(w + (size_t)j * D)[c4] : make_float4(0.f, 0.f, 0.f, 0.f);
+  float4* held = slot >= 0 && keep > 0 ? reinterpret_cast<float4*>(carried + (size_t)slot * keep * D) : nullptr;
+#pragma unroll
+  for (int j = 0; j < NORM_CONV_MAX_TAPS - 1; ++j)
+    prev[j] = held != nullptr && j < keep ? held[(size_t)j * n4 + c4] : make_float4(0.f, 0.f, 0.f, 0.f);
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < VEC; ++u) ss = rms_add4(ss, v[u]);
+  ss = block_sum<4>(ss, red);
+  const float scale = 1.0f / sqrtf(ss / (float)D + eps);
+  if (own4 >= n4) return;
+  auto as_read = [](float a) { return to_f32(from_f32<TO>(a)); };      // the norm's output as the convolution reads it
+  const float4 own = make_float4(as_read(mine.x * scale * nw4.x), as_read(mine.y * scale * nw4.y), as_read(mine.z * scale * nw4.z),
+                                 as_read(mine.w * scale * nw4.w));
+  float4 acc = residual ? own : make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [&](float4 f, float4 in) {
+    acc.x = fmaf(f.x, in.x, acc.x), acc.y = fmaf(f.y, in.y, acc.y), acc.z = fmaf(f.z, in.z, acc.z), acc.w = fmaf(f.w, in.w, acc.w);
+  };
+#pragma unroll
+  for (int j = 0; j < NORM_CONV_MAX_TAPS; ++j) {
+    if (j < keep && j < NORM_CONV_MAX_TAPS - 1) add(wj[j], prev[j]);
+    else if (j == keep) add(wj[j], own);
+  }
+  if (held != nullptr) {                          // every row moves one place towards the oldest; the token itself is the newest
+#pragma unroll
+    for (int j = 1; j < NORM_CONV_MAX_TAPS - 1; ++j)
+      if (j < keep) held[(size_t)(j - 1) * n4 + c4] = prev[j];
+    held[(size_t)(keep - 1) * n4 + c4] = own;
+  }
+  TO* o = out + (size_t)t * D + 4 * (size_t)c4;
+  o[0] = from_f32<TO>(acc.x), o[1] = from_f32<TO>(acc.y), o[2] = from_f32<TO>(acc.z), o[3] = from_f32<TO>(acc.w);
+}
+
 // carried[slot] <- the last taps - 1 inputs of each sequence after this step's tokens; a thread a (sequence, channel)
 // reads what it needs of the old rows before it writes the new ones
 template <typename T, int MAX_TAPS>
@@ -423,6 +483,34 @@ extern "C" int yalm_time_conv(const void* h, long h_row, const float* in_bias, c
   } else {
     return YALM_ERR_DTYPE;
   }
+  return launch_status();
+}
+
+// whether yalm_norm_conv takes the shape (its memory lies on 16 bytes)
+extern "C" int yalm_norm_conv_fits(int D, int taps) {
+  return D > 1024 && D % 4 == 0 && D <= 256 * 4 * RMS_VEC_MAX && taps > 0 && taps <= NORM_CONV_MAX_TAPS;
+}
+
+extern "C" int yalm_norm_conv(const float* x, const float* nw, float eps, const float* w, float* carried, void* out, const int* seq_slot,
+                              int T, int D, int taps, int residual, int dtype, hipStream_t stream) {
+  if (T <= 0) return YALM_OK;
+  if (!yalm_norm_conv_fits(D, taps) || (taps > 1 && carried == nullptr) || !rms_row_vec(x, out, D) ||
+      (((uintptr_t)nw | (uintptr_t)w | (uintptr_t)carried) & 15) != 0)
+    return YALM_ERR_ARG;
+  const dim3 grid(T, ceil_div(D, 1024));
+#define YALM_NORM_CONV(TYPE, VEC) \
+  norm_conv_step_kernel<TYPE, VEC><<<grid, 256, 0, stream>>>(x, nw, eps, w, carried, (TYPE*)out, seq_slot, D, taps, residual)
+#define YALM_NORM_CONV_N(TYPE) \
+  if (D <= 4096) YALM_NORM_CONV(TYPE, 4); else YALM_NORM_CONV(TYPE, RMS_VEC_MAX)
+  if (dtype == YALM_F32) {
+    YALM_NORM_CONV_N(float);
+  } else if (dtype == YALM_BF16) {
+    YALM_NORM_CONV_N(bf16);
+  } else {
+    return YALM_ERR_DTYPE;
+  }
+#undef YALM_NORM_CONV_N
+#undef YALM_NORM_CONV
   return launch_status();
 }
 

@@ -463,6 +463,12 @@ int yalm_gated_add(const float* y, const void* h, const void* w, int dtype, floa
 // are h_row apart; in_bias (float32 [D], may be null) is added to every input (the carried ones hold it), out_bias to every sum.
 int yalm_time_conv(const void* h, long h_row, const float* in_bias, const float* out_bias, const float* w, float* carried, void* out, const int* tok_seq, const int* cu_seqlens,
                    const int* seq_slot, int T, int B, int D, int taps, int residual, int one_each, int dtype, hipStream_t stream);
+// yalm_rmsnorm of the stream x (float32 [T, D], weights nw float32 [D]) and yalm_time_conv of its result with one_each, in one launch and
+// with their bits; out [T, D] of `dtype`.  _fits: whether the shape is taken (D over 1,024 to 8,192, a multiple of 4; up to 4 taps; every
+// pointer on 16 bytes), else YALM_ERR_ARG.
+int yalm_norm_conv_fits(int D, int taps);
+int yalm_norm_conv(const float* x, const float* nw, float eps, const float* w, float* carried, void* out, const int* seq_slot, int T, int D,
+                   int taps, int residual, int dtype, hipStream_t stream);
 // out[t, i] = act(z[t, i] + bias[i]) * (z[t, F + i] + bias[F + i]), i < F: z float32 [T, 2 F] (gate | up), bias float32
 // [2 F] or null, out of `out_dtype`, kind as yalm_activate; with x_bias (float32 [D]) also x[t, :] += x_bias (x float32 [T, D]).
 int yalm_gated_bias_act(const float* z, const float* bias, void* out, int T, int F, int kind, int out_dtype, float* x,

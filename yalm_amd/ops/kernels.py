@@ -1321,6 +1321,25 @@ def time_conv(h, w, carried, out, tok_seq, cu_seqlens, seq_slot, residual=True, 
     return out
 
 
+def norm_conv_fits(x, taps, *others):
+    """Whether norm_conv takes the stream x [T, D] and that many taps (others: the tensors it is given, which lie on 16 bytes as x does)."""
+    return not FORCE_SIMPLE and bool(library.lib().yalm_norm_conv_fits(int(x.shape[1]), int(taps))) and \
+        all(t.data_ptr() % 16 == 0 for t in (x,) + others)
+
+
+def norm_conv(x, norm_w, eps, w, carried, out, seq_slot, residual=True):
+    """rmsnorm (x float32 [T, D], norm_w float32 [D]) and time_conv of its result in out's dtype, for a step of one token a sequence: one
+    launch, the same bits.  The other arguments are time_conv's.  (Shapes: see norm_conv_fits.)"""
+    T, D = x.shape
+    taps = w.shape[0]
+    p_c = _need(carried, "carried", torch.float32, (None, taps - 1, D)) if taps > 1 else None
+    library.check(library.lib().yalm_norm_conv(
+        _need(x, "x", torch.float32), _need(norm_w, "norm_w", torch.float32, (D,)), float(eps), _need(w, "w", torch.float32, (taps, D)), p_c,
+        _need(out, "out", None, (T, D)), _need(seq_slot, "seq_slot", torch.int32, (T,)), T, D, taps, 1 if residual else 0,
+        dtype_code(out.dtype), _stream()), "norm_conv")
+    return out
+
+
 def gated_bias_act(z, bias, out, kind, x=None, x_bias=None):
     """out[t, i] = act(z[t, i] + bias[i]) * (z[t, F + i] + bias[F + i]): z float32 [T, 2 F] (gate | up), bias float32
     [2 F] or None, out [T, F] of its own dtype; kind as in activate.  With x (float32 [T, D]) and x_bias (float32 [D])

@@ -91,6 +91,8 @@ _SIGNATURES = {
     "yalm_activate": (_I, [_P, _P, ctypes.c_long, _I, _I, _P]),
     "yalm_gated_add": (_I, [_P, _P, _P, _I, _P, _I, _I, _I, _P]),
     "yalm_time_conv": (_I, [_P, ctypes.c_long, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]),
+    "yalm_norm_conv_fits": (_I, [_I, _I]),
+    "yalm_norm_conv": (_I, [_P, _P, _F, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "yalm_gated_bias_act": (_I, [_P, _P, _P, _I, _I, _I, _I, _P, _P, _I, _P]),
     "yalm_sigmoid_gate": (_I, [_P, _P, ctypes.c_long, _I, _I, _I, _I, _I, _P]),
     "yalm_loop_pack": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),

@@ -22,6 +22,7 @@ class PreNormResidualBlock(Part):
         self.mixer_input = None
         if layer_spec.part("mixer_input") is not None:
             self.mixer_input = build_part("input_filter", layer_spec.mixer_input, dim, p)
+            self.mixer_norm.taken_by = self.mixer_input
 
     def children(self):
         return [c for c in (self.mixer_norm, self.mixer_input, self.mixer, self.feed_forward_norm, self.feed_forward)
@@ -49,13 +50,15 @@ class PreNormResidualBlock(Part):
         plain_end = False                 # whether the layer's last sublayer ran behind a norm kernel of its own
         if self.mixer_input is not None:
             left = ctx.normed.pop(id(self.mixer_norm), None)
+            filtered = ctx.ws.get("block.filtered", (x.shape[0], self.dim), ctx.act_dtype)
             if left is not None and left[1] is None:      # the layer before has left this norm's output
-                h = left[0]
+                self.mixer_input.forward(left[0], filtered, ctx, (line, "input"))
+            elif self.mixer_input.fuses_norm(self.mixer_norm, x, ctx):
+                self.mixer_input.forward_prenorm(x, self.mixer_norm, filtered, ctx, (line, "input"))
             else:
                 h = ctx.ws.get("block.h", (x.shape[0], self.dim), ctx.act_dtype)
                 self.mixer_norm.forward(x, h, ctx)
-            filtered = ctx.ws.get("block.filtered", (x.shape[0], self.dim), ctx.act_dtype)
-            self.mixer_input.forward(h, filtered, ctx, (line, "input"))
+                self.mixer_input.forward(h, filtered, ctx, (line, "input"))
             self._mix(filtered, x, ctx, (line, "mixer"), writes_cache)
             plain_end = self.feed_forward is None
         elif self.mixer.fuses_norm(self.mixer_norm, x, ctx):
@@ -85,7 +88,11 @@ class PreNormResidualBlock(Part):
         # sublayers that fold no norm into their products leave nothing for whoever reads the stream next: in a decode
         # step the layer then ends with that norm as a kernel of its own, so that the head's product (or the next
         # layer's first) takes its output as it is instead of norming the rows again for every tile of its weights (in float32
-        # a consumer that does not fold the norm in runs it itself, and one that does saves the launch)
+        # a consumer that does not fold the norm in runs it itself, and one that does saves the launch; nor for a filter in front of
+        # the next mixer that takes the norm in)
+        taker = getattr(next_norm, "taken_by", None)
+        if taker is not None and taker.fuses_norm(next_norm, x, ctx):
+            return
         if plain_end and ctx.mode == "decode" and ctx.act_dtype != x.dtype and next_norm is not None and hasattr(next_norm, "fused") \
                 and id(next_norm) not in ctx.normed:
             ahead = ctx.ws.get("block.ahead", (x.shape[0], self.dim), ctx.act_dtype)

@@ -33,6 +33,17 @@ class TimeConv(Part):
     def cache_request(self):
         return StateRequest((self.taps - 1, self.dim), torch.float32) if self.taps > 1 else None
 
+    def fuses_norm(self, norm, x, ctx):
+        """Whether forward_prenorm takes the norm of the stream x in front of the convolution in this step."""
+        return ctx.mode == "decode" and hasattr(norm, "fused") and ctx.seq_slot.shape[0] == x.shape[0] \
+            and kernels.norm_conv_fits(x, self.taps, self.w, norm.fused()[0])
+
+    def forward_prenorm(self, x, norm, out, ctx, line):
+        """forward for the norm's output of the stream x, a token a sequence."""
+        carried = ctx.cache.group_of(line).line_state(line) if self.taps > 1 else None
+        nw, eps = norm.fused()
+        return kernels.norm_conv(x, nw, eps, self.w, carried, out, ctx.seq_slot, self.residual)
+
     def forward(self, h, out, ctx, line):
         """out = h (+) conv(h) over the step's tokens, from the inputs that the line's state holds, which it leaves advanced."""
         carried = ctx.cache.group_of(line).line_state(line) if self.taps > 1 else None
