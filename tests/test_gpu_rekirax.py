@@ -256,6 +256,26 @@ def test_sigmoid_gate_on_the_heads(T, H, dv, pad, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,H,dv,pad,shift", [(1, 1, 8, 16, 0), (6, 3, 24, 32, 0), (3, 32, 128, 128, 0), (2, 37, 40, 48, 0), (2, 32, 64, 64, 1), (2, 3, 20, 32, 0)])
+def test_sigmoid_gate_of_whole_chunks(T, H, dv, pad, shift, dtype):
+    """Against 64 bits where 16 bytes go at once, and where the gates' place or the heads' size keeps the elements one by one; numbers
+    whose exponential overflows; nothing behind a head's elements changes."""
+    from yalm_amd.ops import kernels
+    o = randn(T, H * pad, seed=1).to(dtype)
+    wide = randn(T, H * dv + 16, seed=2, scale=2.0)
+    wide[:, shift], wide[:, shift + 1] = 200.0, -200.0
+    wide = wide.to(DEV)
+    g = wide[:, shift:shift + H * dv]
+    got = o.clone().to(DEV)
+    kernels.sigmoid_gate(got, g, H, dv, pad)
+    want = o.to(F64).reshape(T, H, pad).clone()
+    want[:, :, :dv] *= torch.sigmoid(g.cpu().to(F64)).reshape(T, H, dv)
+    tol = 1e-6 if dtype == torch.float32 else 2.0 ** -8           # a rounding of the result is half of that
+    assert torch.allclose(got.float().cpu().to(F64).reshape(T, H, pad), want, rtol=tol, atol=1e-30)
+    assert torch.equal(got.cpu().reshape(T, H, pad)[:, :, dv:], o.reshape(T, H, pad)[:, :, dv:])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,D", [(1, 5), (7, 72), (3, 2100)])
 def test_way_into_looped_layers(T, D, dtype):
     """The packing kernel and the product behind it give W [x; x0] + start, as the plain function does."""
