@@ -113,6 +113,28 @@ def test_embed(dtype):
     assert torch.equal(out.cpu().double(), want)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("D,T", [(1028, 1), (2052, 5), (4096, 7), (8192, 3), (1536, 300)])
+def test_embed_and_norm_in_one(D, T, dtype):
+    """The bits of the two kernels, in both outputs; tokens outside the table give zeros."""
+    V = 37
+    table, w = rnd((V, D), 1, dtype).to(DEV), (1 + 0.1 * rnd((D,), 3)).to(DEV)
+    tokens = i32([(5 * t) % V if t % 4 != 1 else (-1, V)[t % 8 == 1] for t in range(T)])
+    raw, want, x, kept, alone = (torch.full((T, D), 7.0, device=DEV) for _ in range(5))
+    assert K().embed_norm_fits(table, w, x, kept)
+    K().embed(table, tokens, raw)
+    K().rmsnorm(raw, w, want, 1e-3)
+    K().embed_norm(table, tokens, w, 1e-3, x, kept)
+    K().embed_norm(table, tokens, w, 1e-3, alone)
+    assert torch.equal(x, want) and torch.equal(kept, want) and torch.equal(alone, want)
+
+
+def test_embed_and_norm_what_is_taken():
+    flat = torch.zeros(8200, device=DEV)
+    fits = lambda D, at=0: K().embed_norm_fits(flat, flat, flat[at:at + D].view(1, D))
+    assert [fits(D) for D in (1024, 1026, 1028, 8192, 8196)] == [False, False, True, True, False] and not fits(2048, 1)
+
+
 @pytest.mark.parametrize("out_dtype", DTYPES)
 @pytest.mark.parametrize("w_dtype", DTYPES)
 @pytest.mark.parametrize("D", [50, 1000, 4100, 4096, 8192, 8196, 2050])

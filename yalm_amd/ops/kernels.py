@@ -95,6 +95,23 @@ def embed(table, tokens, out):
     return out
 
 
+def embed_norm_fits(table, norm_w, x, kept=None):
+    """Whether embed_norm takes these (rows of more than 1,024 to 8,192 elements, a multiple of 4, on 16 bytes)."""
+    D = x.shape[1]
+    return not FORCE_SIMPLE and 1024 < D <= 8192 and D % 4 == 0 and all(t.data_ptr() % 16 == 0 for t in (table, norm_w, x, kept) if t is not None)
+
+
+def embed_norm(table, tokens, norm_w, eps, x, kept=None):
+    """x[t] = rmsnorm(float(table[tokens[t]])) with the weights norm_w (float32 [D]), and the same into kept (x, kept float32 [T, D]);
+    a negative token gives zeros.  One launch, the bits of embed and rmsnorm.  (Shapes: see embed_norm_fits.)"""
+    V, D = table.shape
+    T = tokens.shape[0]
+    library.check(library.lib().yalm_embed_norm(
+        _need(table, "table"), dtype_code(table.dtype), _need(tokens, "tokens", torch.int32, (T,)), _need(norm_w, "norm_w", torch.float32, (D,)),
+        float(eps), _need(x, "x", torch.float32, (T, D)), _opt(kept, "kept", torch.float32, (T, D)), T, D, V, _stream()), "embed_norm")
+    return x
+
+
 def embed_sinusoid(table, tokens, positions, freq, scale, out):
     """out[t] = float(table[tokens[t]]) * scale + (freq given) the sinusoidal vector of positions[t]: entry 2i is
     sin(p freq[i]), entry 2i + 1 the cosine; freq float64 [ceil(D / 2)] on the device.  A negative token gives zeros."""

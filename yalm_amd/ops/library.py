@@ -17,6 +17,7 @@ _F = ctypes.c_float
 _SIGNATURES = {
     "yalm_abi_version": (ctypes.c_int, []),
     "yalm_error_string": (ctypes.c_char_p, [_I]),
+    "yalm_embed_norm": (_I, [_P, _I, _P, _P, _F, _P, _P, _I, _I, _I, _P]),
     "yalm_embed": (_I, [_P, _I, _P, _P, _I, _I, _I, _P]),
     "yalm_rmsnorm": (_I, [_P, _P, _I, _P, _I, _P, _I, _I, _F, _P]),
     "yalm_gemm": (_I, [_P, _P, _P, _P, ctypes.c_long, _I, _I, _I, _I, _I, _I, _F, _F, _F, _I, _P]),

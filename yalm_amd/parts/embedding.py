@@ -78,6 +78,10 @@ class TokenEmbedding(Part):
             if kept is not None:
                 self._rows(tokens, kept, ctx)
             return x
+        if self.positions is None and self.pair_table is None and self.freq is None and self.scale == 1.0 and hasattr(self.norm, "fused"):
+            w, eps = self.norm.fused()
+            if kernels.embed_norm_fits(self.table, w, x, kept):
+                return kernels.embed_norm(self.table, tokens, w, eps, x, kept)
         raw = ctx.ws.get("embed.raw", tuple(x.shape), torch.float32)
         self._rows(tokens, raw, ctx)
         self.norm.forward(raw, x, ctx)
