@@ -129,6 +129,33 @@ def test_embed_and_norm_in_one(D, T, dtype):
     assert torch.equal(x, want) and torch.equal(kept, want) and torch.equal(alone, want)
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,Kd", [(16, 64), (40, 128), (1000, 576), (4096, 4096), (1024, 14336)])
+def test_two_products_in_one_launch(M, N, Kd):
+    """The bits of each product alone (up to 4,096 weight rows one kernel serves both), against 64 bits too: K products of bfloat16 are
+    exact in float32, and a sum of K of them in any order is off by at most K units in the last place of the sum of their sizes."""
+    a, a2, w, w2 = (rnd((r, Kd), s, torch.bfloat16) for r, s in ((M, 1), (M, 2), (N, 3), (N, 4)))
+    dev = [t.to(DEV) for t in (a, w, a2, w2)]
+    out, out2, alone, alone2 = (torch.full((M, N), float("nan"), device=DEV) for _ in range(4))
+    assert K().gemm_pair_fits(*dev)
+    K().gemm_pair(dev[0], dev[1], out, dev[2], dev[3], out2)
+    K().gemm(dev[0], dev[1], alone, K().EPI_STORE_F32)
+    K().gemm(dev[2], dev[3], alone2, K().EPI_STORE_F32)
+    assert torch.equal(out, alone) and torch.equal(out2, alone2)
+    for got, x, y in ((out, a, w), (out2, a2, w2)):
+        x, y = x.double(), y.double()
+        assert bool(((got.cpu().double() - x @ y.t()).abs() <= Kd * 2.0 ** -24 * (x.abs() @ y.abs().t())).all())
+
+
+def test_two_products_what_is_taken():
+    t = lambda r, c, dt=torch.bfloat16: torch.zeros(r, c, dtype=dt, device=DEV)
+    fits = lambda M, N, Kd, dt=torch.bfloat16: K().gemm_pair_fits(t(M, Kd, dt), t(N, Kd, dt), t(M, Kd, dt), t(N, Kd, dt))
+    assert fits(16, 4096, 64) and not fits(17, 64, 64) and not fits(1, 4097, 64) and not fits(1, 64, 72) and not fits(1, 64, 64, torch.float32)
+    assert not K().gemm_pair_fits(t(1, 64), t(32, 64), t(1, 64), t(16, 64))
+    off = torch.zeros(64 * 16 + 8, dtype=torch.bfloat16, device=DEV)[1:1 + 64 * 16].view(16, 64)
+    assert not K().gemm_pair_fits(t(1, 64), off, t(1, 64), t(16, 64))
+
+
 def test_embed_and_norm_what_is_taken():
     flat = torch.zeros(8200, device=DEV)
     fits = lambda D, at=0: K().embed_norm_fits(flat, flat, flat[at:at + D].view(1, D))

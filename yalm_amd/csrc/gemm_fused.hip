@@ -349,4 +349,18 @@ extern "C" int yalm_gemm_chain_qkv_rope(const void* X, const float* ss_in, int n
   return skinny::launch<EPI_ROPE>((const bf16*)X, (const bf16*)Wqkv, nullptr, M, N, K, GateOut(0), ca, stream);
 }
 
+extern "C" int yalm_gemm_pair_fits(int M, int N, int K) {
+  return M >= 1 && M <= 16 && N >= 1 && N <= 4096 && K >= 64 && K % 64 == 0;
+}
+
+extern "C" int yalm_gemm_pair(const void* X, const void* W, float* C, const void* X2, const void* W2, float* C2, int M, int N, int K,
+                              hipStream_t stream) {
+  if (!yalm_gemm_pair_fits(M, N, K) || C == C2 ||
+      (((uintptr_t)X | (uintptr_t)W | (uintptr_t)X2 | (uintptr_t)W2) & 15))
+    return YALM_ERR_ARG;
+  ChainArgs ca = {};
+  ca.pair = {(const bf16*)X2, (const bf16*)W2, C2};
+  return skinny::launch_pair((const bf16*)X, (const bf16*)W, C, M, N, K, ca, stream);
+}
+
 extern "C" int yalm_gemm_chain_parts(int N) { return skinny::parts_of(N); }

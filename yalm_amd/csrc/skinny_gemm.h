@@ -53,6 +53,12 @@ struct RopeArgs {                                // epilogue of the fused q/k/v 
   int table_stride, ring_pages, n_positions, n_heads, n_kv_heads, hd, rotary_dim, n_pages, page_layout;
 };
 
+struct PairArgs {                                // the second of two products of one shape (PAIR)
+  const bf16* X;
+  const bf16* W;
+  void* C;
+};
+
 struct ChainArgs {
   const float* ss_in;                            // [M][n_parts_in] partial sums of squares, or null: no row scale
   int n_parts_in;
@@ -61,6 +67,7 @@ struct ChainArgs {
   bf16* emit_xn;                                 // [M][N] = bfloat16(x_new * emit_nw)
   float* emit_ss;                                // [M][gridDim.x] sums of squares of this workgroup's columns
   RopeArgs ra;
+  PairArgs pair;
 };
 
 // MFMA 16x16x32: operand A = activations (row i = batch row, 8 k per lane), operand
@@ -88,8 +95,10 @@ struct ChainArgs {
 // 16 (the waves of that tile ask for one instruction of weights a stage instead of two, and the tile's other columns,
 // which hold whatever was in LDS, are never stored).  6,144 rows are 256 workgroups of 24, one for every compute unit,
 // where 192 of 32 left a quarter of the units idle.
+//
+// PAIR: two products of one shape, neither reading what the other writes, the second in the workgroups with blockIdx.y = 1.
 template <int MT, int NT, int NWAVES, int EPI, int KS, bool PREFETCH = true, int TW = NT, int DMA_S = 0, int XR = 16,
-          int RW = 16 * NT>
+          int RW = 16 * NT, bool PAIR = false>
 __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* __restrict__ X,
                                                                      const bf16* __restrict__ W,
                                                                      void* __restrict__ Cv, int M, int N, int K,
@@ -102,6 +111,10 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
                 "a last tile of 8 rows: one tile a wave, the DMA path, no gated pairs");
   __shared__ f32x4 red[NWAVES][MT * TW][WAVE];
   __shared__ float sm_scale[MT * 16];
+  if constexpr (PAIR) {
+    static_assert(EPI == EPI_F32, "plain results");
+    if (blockIdx.y != 0) X = ca.pair.X, W = ca.pair.W, Cv = ca.pair.C;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int q = lane / 16, j = lane % 16;
   const int n0 = blockIdx.x * RW;
@@ -515,16 +528,27 @@ __global__ __launch_bounds__(NWAVES * WAVE) void gemm_skinny_kernel(const bf16* 
 // 512-wide chunks; the small projections 16 rows, 8 waves and prefetched 128-wide chunks.  More
 // batch rows (only when the split-K kernel refused the shape) keep 128-wide chunks for the registers.
 // the LDS-DMA variant: its ring of stages is dynamic LDS, which has to be allowed once beyond 64 KB
-template <int NT, int NWAVES, int EPI, int TW, int S, int XR, int RW = 16 * NT>
+template <int NT, int NWAVES, int EPI, int TW, int S, int XR, int RW = 16 * NT, bool PAIR = false>
 int launch_dma(const bf16* X, const bf16* W, void* C, int M, int N, int K, GateOut H, const ChainArgs& ca,
                hipStream_t stream) {
   constexpr size_t lds = (size_t)NWAVES * S * (16 * TW + XR) * 128;
   static_assert(lds + NWAVES * TW * WAVE * 16 + 1024 <= 160 * 1024, "the ring and the partial sums fit the LDS of a CU");
-  auto kernel = &gemm_skinny_kernel<1, NT, NWAVES, EPI, 1, false, TW, S, XR, RW>;
+  auto kernel = &gemm_skinny_kernel<1, NT, NWAVES, EPI, 1, false, TW, S, XR, RW, PAIR>;
   static LdsAllowance allowed;                     // once a device
   if (int rc = allow_dynamic_lds(allowed, (const void*)kernel, (int)lds); rc != YALM_OK) return rc;
-  kernel<<<ceil_div(N, RW), NWAVES * WAVE, lds, stream>>>(X, W, C, M, N, K, H, ca);
+  kernel<<<dim3(ceil_div(N, RW), PAIR ? 2 : 1), NWAVES * WAVE, lds, stream>>>(X, W, C, M, N, K, H, ca);
   return launch_status();
+}
+
+// Two products C = X W^T and ca.pair's, float32 results, at most 16 rows, K a multiple of 64, in the workgroups of 16 weight rows that
+// launch_mt gives up to 4,096 of them.  Alone, 4,096 rows are one workgroup a compute unit, and the launch ends as its own last ones
+// do; together a unit holds one of each.  Two
+// stages a ring, so that two workgroups' LDS stands in a unit (three stages: one after the other, 14.1 us for 13.0 below).  us alone and
+// together: 8 rows of 4,096 x 4,096 15.5 and 13.0 (67 MB: 5.2 TB/s), 16 rows 16.6 and 14.3, 8 of 2,048 x 2,048 9.3 and 5.6, of 4,096 x
+// 14,336 44.3 and 41.2.
+inline int launch_pair(const bf16* X, const bf16* W, void* C, int M, int N, int K, const ChainArgs& ca, hipStream_t stream) {
+  return M <= 8 ? launch_dma<1, 8, EPI_F32, 1, 2, 8, 16, true>(X, W, C, M, N, K, GateOut(0), ca, stream)
+                : launch_dma<1, 8, EPI_F32, 1, 2, 16, 16, true>(X, W, C, M, N, K, GateOut(0), ca, stream);
 }
 
 template <int MT, int EPI>

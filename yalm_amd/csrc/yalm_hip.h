@@ -127,6 +127,11 @@ int yalm_gemm_chain(const void* X, const void* W, void* C, int M, int N, int K, 
                     const float* ss_in, int n_parts_in, float eps, const float* emit_nw, void* emit_xn,
                     float* emit_ss, hipStream_t stream);
 int yalm_gemm_chain_parts(int N);
+// C = X W^T and C2 = X2 W2^T in one launch: bfloat16 X, X2 [M, K], W, W2 [N, K] on 16 bytes, float32 C, C2 [M, N].  _fits: whether the
+// shape is taken (up to 16 rows, up to 4,096 weight rows, K a multiple of 64), else YALM_ERR_ARG.
+int yalm_gemm_pair_fits(int M, int N, int K);
+int yalm_gemm_pair(const void* X, const void* W, float* C, const void* X2, const void* W2, float* C2, int M, int N, int K,
+                   hipStream_t stream);
 // The consumer form of the fused q/k/v projection with rotation and cache write (see yalm_gemm_norm_qkv_rope).
 int yalm_gemm_chain_qkv_rope(const void* X, const float* ss_in, int n_parts_in, float eps, const void* Wqkv,
                              void* q_out, void* k_pages, void* v_pages, const int* block_table, int table_stride,

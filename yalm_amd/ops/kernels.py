@@ -202,6 +202,25 @@ def gemm(a, w, out, epilogue, hidden=0, workspace=None, scale_from=None, unit=No
     return out
 
 
+def gemm_pair_fits(a, w, a2, w2):
+    """Whether gemm_pair takes two products a @ w^T and a2 @ w2^T (bfloat16, of one shape, on 16 bytes)."""
+    return not FORCE_SIMPLE and a.dtype == torch.bfloat16 and a.shape == a2.shape and w.shape == w2.shape \
+        and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 for t in (a, w, a2, w2)) \
+        and bool(library.lib().yalm_gemm_pair_fits(a.shape[0], w.shape[0], a.shape[1]))
+
+
+def gemm_pair(a, w, out, a2, w2, out2):
+    """out = a @ w^T and out2 = a2 @ w2^T in one launch: bfloat16 a, a2 [M, K], w, w2 [N, K], float32 out, out2 [M, N].  (Shapes: see
+    gemm_pair_fits.)"""
+    M, K = a.shape
+    N = w.shape[0]
+    bf, f32 = torch.bfloat16, torch.float32
+    library.check(library.lib().yalm_gemm_pair(
+        _need(a, "a", bf, (M, K)), _need(w, "w", bf, (N, K)), _need(out, "out", f32, (M, N)), _need(a2, "a2", bf, (M, K)),
+        _need(w2, "w2", bf, (N, K)), _need(out2, "out2", f32, (M, N)), M, N, K, _stream()), "gemm_pair")
+    return out, out2
+
+
 def can_gemm_gated_bias(kind):
     """Whether gemm_gated_bias takes a feed-forward of this activation (ACTIVATIONS)."""
     return kind == "gelu_tanh"

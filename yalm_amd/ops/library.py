@@ -31,6 +31,8 @@ _SIGNATURES = {
     "yalm_gemm_gated_bias": (_I, [_P, _P, _P, _P, _P, ctypes.c_long, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P]),
     "yalm_gemm_chain": (_I, [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P]),
     "yalm_gemm_chain_parts": (_I, [_I]),
+    "yalm_gemm_pair_fits": (_I, [_I, _I, _I]),
+    "yalm_gemm_pair": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "yalm_gemm_f32_choice": (_I, [_I, _I, _I, _I]),
     "yalm_gemm_f32_split_choice": (_I, [_I, _I, _I, _I]),
     "yalm_gemm_chain_qkv_rope": (_I, [_P, _P, _I, _F, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P]),

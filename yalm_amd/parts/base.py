@@ -246,13 +246,19 @@ class JoinableMixer(Part):
             raise ValueError("this mixer's result lacks a bias that nobody adds")
         return self._run(h, y, ctx, line, writes_cache, kernels.EPI_STORE_F32, proj)
 
-    def _run(self, h, x, ctx, line, writes_cache, epilogue, proj=None):
+    mixed_in = "joinable.o"           # the step's buffer in which `mixed` leaves its result, until the next mixer that uses it runs
+
+    def mixed(self, h, ctx, line, writes_cache=True, proj=None):
+        """What the last product reads."""
         import torch
         from ..ops import kernels
         T = h.shape[0]
         if proj is None:
             proj = ctx.ws.get("joinable.proj", (T, self.n_in), torch.float32)
             self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
-        o = ctx.ws.get("joinable.o", (T, self.n_out), h.dtype)
+        o = ctx.ws.get(self.mixed_in, (T, self.n_out), h.dtype)
         self.between(h, proj, o, ctx, line, writes_cache)
-        self._gemm(ctx, o, self.wo, x, epilogue)
+        return o
+
+    def _run(self, h, x, ctx, line, writes_cache, epilogue, proj=None):
+        self._gemm(ctx, self.mixed(h, ctx, line, writes_cache, proj), self.wo, x, epilogue)

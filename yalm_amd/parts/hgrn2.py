@@ -86,14 +86,17 @@ class HGRN2(Part):
         """Writes the mixer's result to y (float32 [T, dim]); proj: as JoinableMixer.forward_to."""
         return self._run(h, y, ctx, line, kernels.EPI_STORE_F32, proj)
 
-    def _run(self, h, x, ctx, line, epilogue, proj=None):
+    mixed_in = "hgrn2.o"
+
+    def mixed(self, h, ctx, line, writes_cache=True, proj=None):
+        """As JoinableMixer has it."""
         T = h.shape[0]
         ws = ctx.ws
         if proj is None:
             proj = ws.get("hgrn2.proj", (T, self.n_in), torch.float32)
             self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
         raw = ws.get("hgrn2.raw", (T, self.vv), torch.float32)
-        o = ws.get("hgrn2.o", (T, self.vv), h.dtype)
+        o = ws.get(self.mixed_in, (T, self.vv), h.dtype)
         state = ctx.cache.group_of(line).line_state(line)
         B = ctx.seq_slot.shape[0]
         if ctx.mode == "prefill" and h.dtype == torch.bfloat16 and not kernels.FORCE_SIMPLE \
@@ -103,7 +106,10 @@ class HGRN2(Part):
                                 tiles["n_tiles"], o, self.n_heads, self.key_dim, self.value_dim, self.eps, ws.get)
         else:                 # float32 as the compute dtype: prompts go token by token too, so that their bits stay what they were
             self._walk(proj, state, raw, o, ctx)
-        self._gemm(ctx, o, self.wo, x, epilogue)
+        return o
+
+    def _run(self, h, x, ctx, line, epilogue, proj=None):
+        self._gemm(ctx, self.mixed(h, ctx, line, proj=proj), self.wo, x, epilogue)
 
     def _walk(self, proj, state, raw, o, ctx):
         kernels.hgrn2(proj, self.f_bias, self.lower, self.w_norm, state, raw, ctx.cu_seqlens, ctx.seq_slot, o, self.n_heads,

@@ -41,6 +41,8 @@ class SideBySide(Part):
         if self.shares_front:
             for m in (self.left, self.right):
                 m.front_shared = True
+        # whether a step of few rows may run the two last products, of one shape, as one launch: results that wait in buffers of their own
+        self.products_together = all(hasattr(m, "mixed") for m in (self.left, self.right)) and self.left.mixed_in != self.right.mixed_in
         if self.scales is not None:
             for m, scale in zip((self.left, self.right), self.scales):
                 if not isinstance(m, JoinableMixer) or not m.joinable:
@@ -127,8 +129,16 @@ class SideBySide(Part):
             proj = ctx.ws.get("side.proj", (T, n + self.right.n_in), torch.float32)
             self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
             front = ({"proj": proj[:, :n]}, {"proj": proj[:, n:]})
-        self.left.forward_to(h, y, ctx, (line, "left"), writes_cache, **front[0])
-        self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache, **front[1])
+        if T <= kernels.CHAIN_MAX_ROWS and self.products_together and all(getattr(m, "late_bias", None) is None for m in (self.left, self.right)) \
+                and kernels.gemm_pair_fits(
+                ctx.ws.get(self.left.mixed_in, (T, self.left.wo.shape[1]), h.dtype), self.left.wo,
+                ctx.ws.get(self.right.mixed_in, (T, self.right.wo.shape[1]), h.dtype), self.right.wo):
+            o = self.left.mixed(h, ctx, (line, "left"), writes_cache, **front[0])
+            o2 = self.right.mixed(h, ctx, (line, "right"), writes_cache, **front[1])
+            kernels.gemm_pair(o, self.left.wo, y, o2, self.right.wo, y2)
+        else:
+            self.left.forward_to(h, y, ctx, (line, "left"), writes_cache, **front[0])
+            self.right.forward_to(h, y2, ctx, (line, "right"), writes_cache, **front[1])
         if emit_for is None or not hasattr(emit_for, "fused"):
             kernels.norm_add_pair(y, self.w_left, y2, self.w_right, self.eps, x)
             return
