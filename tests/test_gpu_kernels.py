@@ -273,6 +273,21 @@ def test_gemm_of_prompt_steps(M, N, Kd, epi, with_workspace):
         close(out, want + res.double(), torch.float32, "residual add")
 
 
+# Every tiling of the launcher's plan (rows x columns), with every epilogue: rows and columns that end inside a tile, fewer k tiles than
+# the ring has stages, and whole rounds of 256 x 256 tiles with a second launch of each narrower tiling behind them.  In brackets
+# what the plan takes for plain products.
+@pytest.mark.parametrize("epi", ["f32", "bf16", "add", "gated"])
+@pytest.mark.parametrize("M,N,Kd", [
+    (513, 16416, 320),      # 256 x 256 or 192
+    (256, 16416, 192), (200, 16416, 1024),                                                # 256 x 128
+    (129, 16416, 1024), (150, 4096, 2240), (192, 28640, 64), (191, 4096, 7168),           # 192 x 128, the last one in slices of K
+    (193, 8224, 192), (383, 16416, 128), (129, 4096, 2048), (640, 4128, 1024),            # 128 x 128
+    (129, 96, 448), (385, 4128, 128), (255, 160, 2048), (150, 4128, 2048), (193, 32, 64),  # 64 x 128
+    (1100, 16416, 1024), (1000, 16416, 1024), (768, 28672, 512)])                         # two launches
+def test_gemm_of_every_tiling(M, N, Kd, epi):
+    test_gemm_of_prompt_steps(M, N // 2 if epi == "gated" else N, Kd, epi, True)
+
+
 def test_gemm_of_a_prompt_step_is_the_same_with_and_without_k_slices():
     """A product in K slices agrees with the whole one within float32 rounding, and a launch repeats itself bit
     for bit."""

@@ -11,11 +11,10 @@
 // (s_waitcnt vmcnt) and use the bare s_barrier, because __syncthreads() carries a fence that
 // would wait for the loads of all stages.
 //
-// gemm_dma_kernel (128x128 tiles, two stages, two workgroups a CU) serves decode batches of 65 to 159
-// rows: with few tiles K is split over grid z as well, every slice writes its float32 partial product and
-// yalm_splitk_reduce adds them in order and applies the epilogue.  gemm_ring_kernel and gemm_ring16_kernel
-// (256-row tiles, five slots in turn, loads issued between the products; K split the same way for short
-// prompts) serve prompt steps and the biggest decode batches.
+// gemm_stages_kernel (256, 192, 128 or 64 rows x 128 columns, whole k tiles of both operands as stages, three to six of them) serves
+// the short and middle prompts and what whole rounds of large tiles leave; gemm_ring16_kernel (256 x 256 and 256 x 192, five slots in
+// turn) the long ones.  With few tiles K is split over the grid as well: every slice writes its float32 partial product, and
+// yalm_splitk_reduce (or the consumer) adds them in order and applies the epilogue.  tile_plan says which.
 //
 // Takes any M and N and K % 64 == 0; other shapes are refused (YALM_ERR_ARG) and the
 // caller runs the kernel of gemm_mfma.hip.  Sums are in a fixed order for a given shape.
@@ -29,7 +28,6 @@ int yalm_splitk_reduce(const float* partial, void* C, int M, int N, GateOut H, i
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int TK = 64;
@@ -44,188 +42,14 @@ __device__ __forceinline__ void wait_vmcnt() {   // vmcnt only: expcnt and lgkmc
   __builtin_amdgcn_s_waitcnt((N_ & 0xF) | ((N_ >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
-// MFMA 32x32x16: operand rows i/j = lane % 32, 8 k per lane at k offset 8 * (lane / 32);
-// C: lane holds column j = lane % 32 and rows 8 * (r / 4) + 4 * (lane / 32) + r % 4 for r < 16.
-template <int EPI, int TM, int TN, int S, int NWM, int NWN, int MINW>
-__global__ __launch_bounds__(NWM * NWN * WAVE, MINW) void gemm_dma_kernel(const bf16* __restrict__ A,
-                                                                         const bf16* __restrict__ W,
-                                                                         void* __restrict__ Cv, int M, int N, int K,
-                                                                         GateOut H, float* __restrict__ partial,
-                                                                         int tiles_per_slice, int n_tile0) {
-  constexpr int NW = NWM * NWN;
-  constexpr int ROWS = TM + TN;                    // A rows, then W rows
-  constexpr int STAGE_B = ROWS * ROWB;
-  constexpr int L = ROWS / (RPI * NW);             // load instructions a wave and stage
-  static_assert(ROWS % (RPI * NW) == 0, "the rows of a stage must divide over the waves");
-  static_assert((S - 2) * L < 64, "vmcnt holds 6 bits");
-  constexpr int WM = TM / NWM, WN = TN / NWN, FA = WM / 32, FB = WN / 32;
-  constexpr int KS = TK / 16;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char stages[];
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-  const int wm = wave / NWN, wn = wave % NWN;
-  const int m0 = blockIdx.y * TM, n0 = (blockIdx.x + n_tile0) * TN;   // a launch may own a range of the columns
-  const int li = lane % 32, lh = lane / 32;
-
-  // instruction i of this wave fills rows (i * NW + wave) * RPI ... of a stage; the lane's
-  // place there is (row, slot), and it asks memory for the chunk that belongs in that slot
-  const bf16* gp[L];
-#pragma unroll
-  for (int i = 0; i < L; ++i) {
-    const int row = (i * NW + wave) * RPI + lane / CPR;
-    const int chunk = (lane % CPR) ^ swizzle_of(row);
-    const bf16* base = row < TM ? A + (size_t)min(m0 + row, M - 1) * K          // rows past the edge repeat the last
-                                : W + (size_t)min(n0 + row - TM, N - 1) * K;    // one and are never stored
-    gp[i] = base + chunk * 8;
-  }
-  auto issue = [&](int kt, int stage) {
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-#if defined(__HIP_DEVICE_COMPILE__)   // the host pass drops a template that names this builtin, and its launch stub with it
-      __builtin_amdgcn_global_load_lds(gp[i] + (size_t)kt * TK, stages + stage * STAGE_B + (i * NW + wave) * 1024, 16, 0,
-                                       0);
-#endif
-    }
-  };
-
-  f32x16 acc[FA][FB];
-#pragma unroll
-  for (int a = 0; a < FA; ++a)
-#pragma unroll
-    for (int b = 0; b < FB; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-
-  // fragment rows of this lane: A rows of the wave's row tiles; W rows of its column tiles, where
-  // for the gated epilogue even tiles are the gate rows and odd tiles the up rows of two 16-row blocks
-  int a_base[FA], a_swz[FA], w_base[FB], w_swz[FB];
-#pragma unroll
-  for (int a = 0; a < FA; ++a) {
-    const int row = wm * WM + a * 32 + li;
-    a_base[a] = row * ROWB;
-    a_swz[a] = swizzle_of(row);
-  }
-#pragma unroll
-  for (int b = 0; b < FB; ++b) {
-    const int r = (gated(EPI)) ? wn * WN + (b / 2) * 64 + (li / 16) * 32 + (b % 2) * 16 + (li % 16) : wn * WN + b * 32 + li;
-    const int row = TM + r;
-    w_base[b] = row * ROWB;
-    w_swz[b] = swizzle_of(row);
-  }
-
-  // grid z: slices of K (each writes its float32 partial product; a second kernel adds them)
-  const int kt0 = blockIdx.z * tiles_per_slice;
-  const int nk = min(K / TK - kt0, tiles_per_slice);
-#pragma unroll
-  for (int i = 0; i < L; ++i) gp[i] += (size_t)kt0 * TK;
-#pragma unroll
-  for (int s = 0; s < S - 1; ++s)
-    if (s < nk) issue(s, s);
-  for (int kt = 0; kt < nk; ++kt) {
-    // stage kt has landed when at most the loads of the S - 2 stages behind it are in flight
-    if (kt + S - 2 < nk) wait_vmcnt<(S - 2) * L>(); else wait_vmcnt<0>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();                  // everyone's part of stage kt is there, and everyone has read stage kt - 1
-    asm volatile("" ::: "memory");
-    if (kt + S - 1 < nk) issue(kt + S - 1, (kt + S - 1) % S);      // into the buffer that iteration kt - 1 read
-    const unsigned char* cur = stages + (kt % S) * STAGE_B;
-    bf16x8 fa[2][FA], fw[2][FB];
-#pragma unroll
-    for (int a = 0; a < FA; ++a) fa[0][a] = *reinterpret_cast<const bf16x8*>(cur + a_base[a] + ((lh ^ a_swz[a]) << 4));
-#pragma unroll
-    for (int b = 0; b < FB; ++b) fw[0][b] = *reinterpret_cast<const bf16x8*>(cur + w_base[b] + ((lh ^ w_swz[b]) << 4));
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c = ks & 1, n = c ^ 1;
-      if (ks + 1 < KS) {                           // the next fragments are read while these are multiplied
-        const int ch = (ks + 1) * 2 + lh;
-#pragma unroll
-        for (int a = 0; a < FA; ++a) fa[n][a] = *reinterpret_cast<const bf16x8*>(cur + a_base[a] + ((ch ^ a_swz[a]) << 4));
-#pragma unroll
-        for (int b = 0; b < FB; ++b) fw[n][b] = *reinterpret_cast<const bf16x8*>(cur + w_base[b] + ((ch ^ w_swz[b]) << 4));
-      }
-#pragma unroll
-      for (int a = 0; a < FA; ++a)
-#pragma unroll
-        for (int b = 0; b < FB; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[c][a], fw[c][b], acc[a][b], 0, 0, 0);
-    }
-  }
-
-  if (gridDim.z > 1) {                             // a slice of K: the plain sums, column n = weight row n
-    float* plane = partial + (size_t)blockIdx.z * M * N;
-#pragma unroll
-    for (int a = 0; a < FA; ++a)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * WM + a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
-        if (m >= M) continue;
-#pragma unroll
-        for (int b = 0; b < FB; ++b) {
-          const int wr = (gated(EPI)) ? wn * WN + (b / 2) * 64 + (li / 16) * 32 + (b % 2) * 16 + (li % 16) : wn * WN + b * 32 + li;
-          const int n = n0 + wr;
-          if (n < N) plane[(size_t)m * N + n] = acc[a][b][r];
-        }
-      }
-    return;
-  }
-  GateBias gb[FB / 2 + 1];
-  if (EPI == EPI_GATED_BIAS)
-#pragma unroll
-    for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN + pp * 64) / 2 + li);
-#pragma unroll
-  for (int a = 0; a < FA; ++a) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = m0 + wm * WM + a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
-      if (m >= M) continue;
-      if (gated(EPI)) {
-#pragma unroll
-        for (int pp = 0; pp < FB / 2; ++pp) {
-          const int hcol = (n0 + wn * WN + pp * 64) / 2 + li;
-          if (hcol < H)
-            ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H, gb[pp]));
-        }
-      } else {
-#pragma unroll
-        for (int b = 0; b < FB; ++b) {
-          const int n = n0 + wn * WN + b * 32 + li;
-          if (n >= N) continue;
-          const size_t o = (size_t)m * N + n;
-          if (EPI == 0) ((float*)Cv)[o] = acc[a][b][r];
-          if (EPI == 1) ((bf16*)Cv)[o] = static_cast<bf16>(acc[a][b][r]);
-          if (EPI == 2) ((float*)Cv)[o] += acc[a][b][r];
-        }
-      }
-    }
-  }
-}
-
-template <int EPI, int TM, int TN, int S, int NWM, int NWN, int MINW>
-int launch_shape(const bf16* A, const bf16* W, void* C, int M, int N, int K, GateOut H, float* partial, int slices,
-                 hipStream_t stream, bool add_slices = true, int n_tile0 = 0, int n_tiles = -1) {
-  const int tiles_per_slice = ceil_div(K / TK, slices);
-  if (n_tiles < 0) n_tiles = ceil_div(N, TN) - n_tile0;     // column tiles n_tile0 ... of this launch
-  const dim3 grid(n_tiles, ceil_div(M, TM), ceil_div(K / TK, tiles_per_slice));
-  const size_t lds = (size_t)S * (TM + TN) * ROWB;
-  static LdsAllowance allowed;                     // more than 64 KB of LDS has to be asked for once a device
-  if (int rc = allow_dynamic_lds(allowed, (const void*)&gemm_dma_kernel<EPI, TM, TN, S, NWM, NWN, MINW>, (int)lds);
-      rc != YALM_OK)
-    return rc;
-  gemm_dma_kernel<EPI, TM, TN, S, NWM, NWN, MINW><<<grid, NWM * NWN * WAVE, lds, stream>>>(A, W, C, M, N, K, H, partial,
-                                                                                       tiles_per_slice, n_tile0);
-  int rc = launch_status();
-  if (rc != YALM_OK || grid.z == 1 || !add_slices) return rc;
-  return yalm_splitk_reduce(partial, C, M, N, H, (int)grid.z, EPI, stream);
-}
-
 // ---------------------------------------------------------------------------
 // The kernel for many tiles: 256 x TN tiles, 8 waves, and a ring of five 32 KB slots that holds the k tiles of
 // W and of A in turn (W0 A0 W1 A1 W2 ...; tile t has W in slot 2t mod 5 and A in slot (2t + 1) mod 5), so that
-// two and a half k tiles are in flight or in use.  What it does differently from the kernel above, each measured:
+// two and a half k tiles are in flight or in use.  What it does beside a plain double buffer, each measured:
 //  * a vector memory instruction holds its wave for tens of clocks, more while the memory system is busy; issued
 //    as a burst behind the barrier they stall every wave at once and the matrix cores idle.  Here a wave issues
 //    one DMA instruction in every few products, all through the iteration, and each has a k step or more to land;
-//  * the barrier stands between k steps 2 and 3 of a tile: the fragments of the last k step are in registers by
+//  * the barrier stands in front of a tile's last products: their fragments are in registers by
 //    then, so nobody reads the tile's slots any more and they are refilled at once, and the first fragments
 //    of the next tile are read while the last products of this one run;
 //  * the fragments of a k step are read during the products of the one before (two register sets);
@@ -244,189 +68,163 @@ __host__ __device__ constexpr int dma_place(int d, int n_dma, int n_products) {
   return at < 0 ? 0 : at;
 }
 
-template <int EPI, int TN, int MAP>
-__global__ __launch_bounds__(512, 1) void gemm_ring_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
-                                                           void* __restrict__ Cv, int M, int N, int K, GateOut H, int n_tile0,
-                                                           int n_tiles, float* __restrict__ partial,
-                                                           int tiles_per_slice) {
-  constexpr int TM = RING_TM, NW = 8, NWM = 4, NWN = 2, WM = TM / NWM, WN = TN / NWN, FA = WM / 32, FB = WN / 32;
-  constexpr int KS = TK / 16;
-  constexpr int DA = (TM / 8) / NW, DW = (TN / 8) / NW;     // DMA instructions (8 rows each) a wave and slot
-  constexpr int DA1 = DA / 2, DW1 = (DW + 1) / 2;           // of them in the first of the two k steps that issue them
-  constexpr int NMF = FA * FB;                              // products a k step
-  static_assert(TM % (8 * NW) == 0 && TN % (8 * NW) == 0 && DA % 2 == 0, "the rows of a slot must divide over the waves");
-  static_assert(FA + FB <= NMF, "a fragment read follows a product");
+// ---------------------------------------------------------------------------
+// Tiles of TM x 128 with TM 256, 192, 128 or 64: as many whole k tiles (A rows, then W rows: (TM + 128) x 128 bytes) as LDS holds, all but
+// one in flight.  A prompt of 65 to some 1,000 rows has too few tiles of 256 x 256 to fill the chip, and what bounds it is the way of
+// the operands into a CU (192 rows of 4,096 x 28,672: 60 us; without its products and fragment reads 57, without its loads 41), so the
+// tile is cut to the rows there are and the depth of the ring hides the memory's latency.  The timetable is the one above: a wave issues
+// its DMA instructions between the products of a k step, the barrier stands between the two k steps of a tile (the fragments of the
+// last one are in registers by then), and fragments are read one k step ahead.
+// us before (tiles of 128 x 128 with two stages below 160 rows, the ring of five slots above) and with this kernel, slices unadded:
+//   28,672 x 4,096 gated  150 rows 88.0 57.9   192 rows 70.9 59.5   256 rows 73.0 66.6
+//   4,096 x 14,336        150 rows 45.2 36.3   384 rows 68.6 51.2   448 rows 72.4 57.0
+//   16,384 x 3,072 gated  150 rows 42.4 36.5   256 rows 53.1 39.7   384 rows 55.0 47.6
+//   4,096 x 4,096         150 rows 19.5 15.0   256 rows 23.5 17.8   640 rows 31.5 30.6
+// ---------------------------------------------------------------------------
+template <int TM> struct StageTiling;               // waves over rows and columns, stages
+template <> struct StageTiling<256> { static constexpr int NWM = 4, NWN = 2, S = 3; };
+template <> struct StageTiling<192> { static constexpr int NWM = 4, NWN = 2, S = 4; };
+template <> struct StageTiling<128> { static constexpr int NWM = 4, NWN = 2, S = 5; };
+template <> struct StageTiling<64> { static constexpr int NWM = 2, NWN = 4, S = 6; };
+constexpr int STAGES_TN = 128, TILE_GROUP = 4;      // columns a tile; tile columns whose tiles follow each other
+
+template <int EPI, int TM>
+__global__ __launch_bounds__(512, 1) void gemm_stages_kernel(const bf16* __restrict__ A, const bf16* __restrict__ W,
+                                                             void* __restrict__ Cv, int M, int N, int K, GateOut H, int n_tile0,
+                                                             int n_tiles, float* __restrict__ partial, int tiles_per_slice) {
+  constexpr int NWM = StageTiling<TM>::NWM, NWN = StageTiling<TM>::NWN, S = StageTiling<TM>::S, TN = STAGES_TN, NW = NWM * NWN;
+  constexpr int WM = TM / NWM, WN = TN / NWN, FA = WM / 16, FB = WN / 16, NMF = FA * FB;
+  constexpr int STAGE = (TM + TN) * ROWB, L = (TM + TN) / (8 * NW);      // bytes a stage; DMA instructions (8 rows each) a wave and stage
+  static_assert(NW == 8 && (TM + TN) % (8 * NW) == 0 && TM % (8 * NW) == 0, "an instruction of all waves lies in one operand");
+  static_assert(S * STAGE <= 160 * 1024 && (S - 1) * L < 64, "the ring fits the LDS of a CU; vmcnt holds 6 bits");
+  static_assert(FA + FB <= NMF && L <= NMF, "a fragment read and a DMA instruction follow a product");
   static_assert(!gated(EPI) || FB % 2 == 0, "the gated epilogue pairs column tiles");
   extern __shared__ __attribute__((aligned(1024))) unsigned char stages[];
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int wm = wave / NWN, wn = wave % NWN;
-  const int li = lane % 32, lh = lane / 32;
-  int tile_m, tile_n;
-  if (MAP == 0) {
-    tile_m = blockIdx.y;
-    tile_n = blockIdx.x + n_tile0;
-  } else {
-    // Workgroup L runs on XCD L mod 8.  Every XCD takes a run of the tile sequence (groups of MAP tile columns;
-    // in a group the rows fastest, then the columns), so that the tiles it works on at a time share rows and
-    // columns in its second-level cache.
-    const int mt = (M + TM - 1) / TM, T = mt * n_tiles, chunk = (T + 7) / 8;
-    const int L = blockIdx.x, t = (L % 8) * chunk + L / 8;
-    if (t >= T || L / 8 >= chunk) return;
-    const int per_group = mt * MAP, g = t / per_group, r = t % per_group;
-    const int width = min(MAP, n_tiles - g * MAP);        // the last group may be narrower
-    tile_n = n_tile0 + g * MAP + r % width;
-    tile_m = r / width;
-  }
-  const int m0 = tile_m * TM, n0 = tile_n * TN;
-  // slices of K (grid z without the XCD mapping, grid y with it): each writes its float32 partial product
-  const int slice = MAP == 0 ? blockIdx.z : blockIdx.y, n_slices = MAP == 0 ? gridDim.z : gridDim.y;
-  const int kt0 = slice * tiles_per_slice;
+  const int wm = wave / NWN, wn = wave % NWN, l16 = lane % 16, lq = lane / 16;
+  // blocks of tiles for every XCD (workgroup L runs on XCD L mod 8): TILE_GROUP tile columns, all rows of one block after the other
+  const int mt = (M + TM - 1) / TM, T = mt * n_tiles, chunk = (T + 7) / 8;
+  const int Lb = blockIdx.x, t = (Lb % 8) * chunk + Lb / 8;
+  if (t >= T || Lb / 8 >= chunk) return;
+  const int per_group = mt * TILE_GROUP, g = t / per_group, rest = t % per_group, width = min(TILE_GROUP, n_tiles - g * TILE_GROUP);
+  const int m0 = (rest / width) * TM, n0 = (n_tile0 + g * TILE_GROUP + rest % width) * TN;
+  const int slice = blockIdx.y, n_slices = gridDim.y, kt0 = slice * tiles_per_slice;
   const int nk = min(K / TK - kt0, tiles_per_slice);
 
-  // DMA instruction i of a wave fills rows (i * 8 + wave) * 8 ... + 7 of a slot; a lane's place there is (row,
-  // 16-byte slot of the row), and it asks memory for the chunk that belongs there (rows past the edge repeat the
-  // last one and are never stored)
-  unsigned off_a[DA], off_w[DW];
+  // instruction i of a wave brings rows (i * NW + wave) * 8 ... + 7 of a stage; rows past the edge repeat the last one
+  constexpr int LA = TM / (8 * NW);                         // the first LA instructions bring rows of A
+  unsigned off[L];
   const char* a_base = (const char*)(A + (size_t)m0 * K + (size_t)kt0 * TK);
   const char* w_base = (const char*)(W + (size_t)n0 * K + (size_t)kt0 * TK);
 #pragma unroll
-  for (int i = 0; i < DA; ++i) {
+  for (int i = 0; i < L; ++i) {
     const int row = (i * NW + wave) * RPI + lane / CPR;
-    off_a[i] = (unsigned)(((size_t)min(row, M - 1 - m0) * K + ((lane % CPR) ^ swizzle_of(row)) * 8) * 2);
+    const int there = i < LA ? min(row, M - 1 - m0) : min(row - TM, N - 1 - n0);
+    off[i] = (unsigned)(((size_t)there * K + ((lane % CPR) ^ swizzle_of(row)) * 8) * 2);
   }
-#pragma unroll
-  for (int i = 0; i < DW; ++i) {
-    const int row = (i * NW + wave) * RPI + lane / CPR;
-    off_w[i] = (unsigned)(((size_t)min(row, N - 1 - n0) * K + ((lane % CPR) ^ swizzle_of(row)) * 8) * 2);
-  }
-  auto dma = [&](const char* base, unsigned off, int slot, int i) {
-    const unsigned lds_addr = (unsigned)(uintptr_t)(stages + slot * RING_SLOT + (i * NW + wave) * 1024);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(off), "s"(base) : "memory", "m0");
+  const unsigned lds0 = (unsigned)(uintptr_t)stages + (unsigned)(wave * 1024);
+  auto dma = [&](int kt, int slot, int i) {
+    const char* base = (i < LA ? a_base : w_base) + (size_t)kt * ROWB;
+    const unsigned at = lds0 + (unsigned)slot * STAGE;
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 : : "s"(at), "v"(off[i]), "s"(base), "s"((unsigned)(i * NW * 1024)) : "memory", "m0", "scc");
   };
 
-  f32x16 acc[FA][FB];
+  // the running sums go into the whole ones every FOLD k tiles: sums of 512 products at a time round as little as the finest slices of K
+  f32x4 acc[FA][FB], run[FA][FB];
 #pragma unroll
   for (int a = 0; a < FA; ++a)
 #pragma unroll
-    for (int b = 0; b < FB; ++b)
+    for (int b = 0; b < FB; ++b) acc[a][b] = run[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto fold = [&]() {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-
-  // fragments: A rows of the wave's row tiles; W rows of its column tiles, where for the gated epilogue even tiles
-  // are the gate rows and odd tiles the up rows of two 16-row blocks.  Address in a slot: row * 128 + ((2 ks + lh)
-  // ^ swizzle) * 16; tiles 32 (16, 64) rows apart share the swizzle.
-  const int a_row = wm * WM + li;
-  const int w_row = (gated(EPI)) ? wn * WN + (li / 16) * 32 + (li % 16) : wn * WN + li;
-  int a_at[KS], w_at[KS];
+    for (int a = 0; a < FA; ++a)
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    a_at[ks] = a_row * ROWB + (((2 * ks + lh) ^ swizzle_of(a_row)) << 4);
-    w_at[ks] = w_row * ROWB + (((2 * ks + lh) ^ swizzle_of(w_row)) << 4);
-  }
-  auto frag_a = [&](int slot, int ks, int a) {
-    return *reinterpret_cast<const bf16x8*>(stages + slot * RING_SLOT + a_at[ks] + a * 32 * ROWB);
+      for (int b = 0; b < FB; ++b) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[a][b][r] += run[a][b][r];
+        run[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
   };
-  auto frag_w = [&](int slot, int ks, int b) {
-    const int rows = (gated(EPI)) ? (b / 2) * 64 + (b % 2) * 16 : b * 32;
-    return *reinterpret_cast<const bf16x8*>(stages + slot * RING_SLOT + w_at[ks] + rows * ROWB);
-  };
-
-  // before the loop: W0 A0 W1 and the first half of A1 (what iterations -2 and -1 would have issued)
+  const int a_row = wm * WM + l16, w_row = TM + wn * WN + l16;
+  int a_at[2], w_at[2];
 #pragma unroll
-  for (int i = 0; i < DW; ++i) dma(w_base, off_w[i], 0, i);
-#pragma unroll
-  for (int i = 0; i < DA; ++i) dma(a_base, off_a[i], 1, i);
-  if (nk > 1) {
-#pragma unroll
-    for (int i = 0; i < DW; ++i) dma(w_base + ROWB, off_w[i], 2, i);
-#pragma unroll
-    for (int i = 0; i < DA1; ++i) dma(a_base + ROWB, off_a[i], 3, i);
-    wait_vmcnt<DW + DA1>();
-  } else {
-    wait_vmcnt<0>();
+  for (int s = 0; s < 2; ++s) {
+    a_at[s] = a_row * ROWB + (((4 * s + lq) ^ swizzle_of(a_row)) << 4);
+    w_at[s] = w_row * ROWB + (((4 * s + lq) ^ swizzle_of(w_row)) << 4);
   }
+  auto frag_a = [&](const unsigned char* st, int s, int a) { return *reinterpret_cast<const bf16x8*>(st + a_at[s] + a * 16 * ROWB); };
+  auto frag_w = [&](const unsigned char* st, int s, int b) { return *reinterpret_cast<const bf16x8*>(st + w_at[s] + b * 16 * ROWB); };
+
+#pragma unroll
+  for (int p = 0; p < S - 1; ++p)
+    if (p < nk)
+#pragma unroll
+      for (int i = 0; i < L; ++i) dma(p, p, i);
+  if (nk >= S - 1) wait_vmcnt<(S - 2) * L>(); else wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   bf16x8 fa[2][FA], fw[2][FB];
 #pragma unroll
-  for (int a = 0; a < FA; ++a) fa[0][a] = frag_a(1, 0, a);
+  for (int a = 0; a < FA; ++a) fa[0][a] = frag_a(stages, 0, a);
 #pragma unroll
-  for (int b = 0; b < FB; ++b) fw[0][b] = frag_w(0, 0, b);
-
-  int ws = 0, as = 1;                              // slots of the tile that is multiplied
-  for (int kt = 0; kt < nk; ++kt) {
-    const int ws1 = ws + 2 >= RING_SLOTS ? ws + 2 - RING_SLOTS : ws + 2;          // of tile kt + 1
-    const int as1 = as + 2 >= RING_SLOTS ? as + 2 - RING_SLOTS : as + 2;
-    const int ws2 = ws1 + 2 >= RING_SLOTS ? ws1 + 2 - RING_SLOTS : ws1 + 2;       // of tile kt + 2
-    const int as2 = as1 + 2 >= RING_SLOTS ? as1 + 2 - RING_SLOTS : as1 + 2;
-    const bool t1 = kt + 1 < nk, t2 = kt + 2 < nk;
-    const char* a1 = a_base + (size_t)(kt + 1) * ROWB;
-    const char* a2 = a_base + (size_t)(kt + 2) * ROWB;
-    const char* w2 = w_base + (size_t)(kt + 2) * ROWB;
+  for (int b = 0; b < FB; ++b) fw[0][b] = frag_w(stages, 0, b);
+  int slot = 0;
+  auto iteration = [&](int kt, auto more) {                 // more: k tile kt + S - 1 exists and is asked for here
+    constexpr bool MORE = decltype(more)::value;
+    const int next = slot + 1 == S ? 0 : slot + 1, last = slot == 0 ? S - 1 : slot - 1;
+    const unsigned char *cur = stages + slot * STAGE, *nx = stages + next * STAGE;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c = ks & 1, n = c ^ 1;
-      if (ks == KS - 1) {
-        // The last fragments of tile kt are in registers; this wave's share of tile kt + 1 has landed (the second
-        // half of A(kt + 1) from k step 0, and everything older; W(kt + 2) may still be on its way).  Behind the
-        // barrier that holds for all waves: tile kt + 1 can be read and the slots of tile kt written.
+    for (int s = 0; s < 2; ++s) {
+      if (s == 1) {                                         // nobody reads the tile any more, and the next one has landed
         wait_lgkmcnt0();
-        if (t2) wait_vmcnt<DW>(); else wait_vmcnt<0>();
+        if (MORE) wait_vmcnt<(S - 2) * L>(); else wait_vmcnt<0>();
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int j = 0; j < NMF; ++j) {
-        const int a = j / FB, b = j % FB;
-        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[c][a], fw[c][b], acc[a][b], 0, 0, 0);
+        const int a = j % FA, b = j / FA;
+        run[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[s][a], fw[s][b], run[a][b], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        if (ks < KS - 1) {                           // a fragment of k step ks + 1 of this tile
-          if (j < FA) fa[n][j] = frag_a(as, ks + 1, j);
-          else if (j < FA + FB) fw[n][j - FA] = frag_w(ws, ks + 1, j - FA);
-        } else {                                     // of k step 0 of the next tile (behind the last tile: read, never used)
-          if (j < FA) fa[n][j] = frag_a(as1, 0, j);
-          else if (j < FA + FB) fw[n][j - FA] = frag_w(ws1, 0, j - FA);
-        }
-        // k step 0: the second half of A(kt + 1); 1 and 2: W(kt + 2); 3, behind the barrier: the first half of A(kt + 2)
-        if (ks == 0) {
+        // (behind the last tile the next slot's fragments are read as they lie and not used)
+        if (j < FA) fa[s ^ 1][j] = s == 0 ? frag_a(cur, 1, j) : frag_a(nx, 0, j);
+        else if (j < FA + FB) fw[s ^ 1][j - FA] = s == 0 ? frag_w(cur, 1, j - FA) : frag_w(nx, 0, j - FA);
+        if (s == 0 && MORE) {                               // into the slot of tile kt - 1, free since that tile's barrier
 #pragma unroll
-          for (int d = 0; d < DA - DA1; ++d)
-            if (j == dma_place(d, DA - DA1, NMF) && t1) dma(a1, off_a[DA1 + d], as1, DA1 + d);
-        } else if (ks == 1) {
-#pragma unroll
-          for (int d = 0; d < DW1; ++d)
-            if (j == dma_place(d, DW1, NMF) && t2) dma(w2, off_w[d], ws2, d);
-        } else if (ks == 2) {
-#pragma unroll
-          for (int d = 0; d < DW - DW1; ++d)
-            if (j == dma_place(d, DW - DW1, NMF) && t2) dma(w2, off_w[DW1 + d], ws2, DW1 + d);
-        } else {
-#pragma unroll
-          for (int d = 0; d < DA1; ++d)
-            if (j == dma_place(d, DA1, NMF) && t2) dma(a2, off_a[d], as2, d);
+          for (int i = 0; i < L; ++i)
+            if (j == dma_place(i, L, NMF)) dma(kt + S - 1, last, i);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    ws = ws1;
-    as = as1;
+    slot = next;
+  };
+  constexpr int FOLD = 8;
+  int kt = 0;
+  for (; kt + S - 1 < nk; ++kt) {
+    iteration(kt, std::true_type{});
+    if (kt % FOLD == FOLD - 1) fold();
   }
+  for (; kt < nk; ++kt) iteration(kt, std::false_type{});
+  fold();
   wait_vmcnt<0>();                                 // nothing of this workgroup is on its way into LDS when it ends
 
+  // C: lane (lq, l16) holds rows 4 lq .. 4 lq + 3 of column l16 of every tile
   if (n_slices > 1) {                              // a slice of K: the plain sums, column n = weight row n
     float* plane = partial + (size_t)slice * M * N;
 #pragma unroll
     for (int a = 0; a < FA; ++a)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * WM + a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + wm * WM + a * 16 + 4 * lq + r;
         if (m >= M) continue;
 #pragma unroll
         for (int b = 0; b < FB; ++b) {
-          const int wr = (gated(EPI)) ? wn * WN + (b / 2) * 64 + (li / 16) * 32 + (b % 2) * 16 + (li % 16) : wn * WN + b * 32 + li;
-          if (n0 + wr < N) plane[(size_t)m * N + n0 + wr] = acc[a][b][r];
+          const int nn = n0 + wn * WN + b * 16 + l16;
+          if (nn < N) plane[(size_t)m * N + nn] = acc[a][b][r];
         }
       }
     return;
@@ -434,24 +232,24 @@ __global__ __launch_bounds__(512, 1) void gemm_ring_kernel(const bf16* __restric
   GateBias gb[FB / 2 + 1];
   if (EPI == EPI_GATED_BIAS)
 #pragma unroll
-    for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN + pp * 64) / 2 + li);
+    for (int pp = 0; pp < FB / 2; ++pp) gb[pp] = gate_bias<EPI>(H, (n0 + wn * WN) / 2 + pp * 16 + l16);
 #pragma unroll
   for (int a = 0; a < FA; ++a) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = m0 + wm * WM + a * 32 + 8 * (r / 4) + 4 * lh + (r % 4);
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + wm * WM + a * 16 + 4 * lq + r;
       if (m >= M) continue;
-      if (gated(EPI)) {
+      if (gated(EPI)) {                              // weight rows: 16 gate rows, 16 up rows, ...: even tiles gate, odd tiles up
 #pragma unroll
         for (int pp = 0; pp < FB / 2; ++pp) {
-          const int hcol = (n0 + wn * WN + pp * 64) / 2 + li;
+          const int hcol = (n0 + wn * WN) / 2 + pp * 16 + l16;
           if (hcol < H)
             ((bf16*)Cv)[(size_t)m * H + hcol] = static_cast<bf16>(gate_value<EPI>(acc[a][2 * pp][r], acc[a][2 * pp + 1][r], H, gb[pp]));
         }
       } else {
 #pragma unroll
         for (int b = 0; b < FB; ++b) {
-          const int nn = n0 + wn * WN + b * 32 + li;
+          const int nn = n0 + wn * WN + b * 16 + l16;
           if (nn >= N) continue;
           const size_t o = (size_t)m * N + nn;
           if (EPI == 0) ((float*)Cv)[o] = acc[a][b][r];
@@ -464,11 +262,10 @@ __global__ __launch_bounds__(512, 1) void gemm_ring_kernel(const bf16* __restric
 }
 
 // ---------------------------------------------------------------------------
-// The same ring with v_mfma_f32_16x16x32_bf16, for tiles of 256 and 192 columns.  The chip is power-bound under
+// The ring for tiles of 256 and 192 columns.  It uses v_mfma_f32_16x16x32_bf16: the chip is power-bound under
 // this loop (the shader clock falls to 1.5-1.8 GHz), and on random operands the 16x16x32 instruction does about a
 // sixth more products for the same power than 32x32x16 (2.16 against 1.83 PFLOP/s out of registers: it moves a
-// quarter of the accumulator registers per product); the whole GEMM gains 5-10 %.  (Tiles of 128 columns, 64x64 a
-// wave, are 2-9 % slower this way and stay with the kernel above.)
+// quarter of the accumulator registers per product); the whole GEMM gains 5-10 %.
 // A wave owns 64 rows x TN/2 columns: 4 x FB tiles of 16x16.  A tile's 64 k are two k steps of 32; a k step is FB
 // groups of four products that share one W fragment.  The W fragments come from LDS through a ring of four, three
 // groups ahead of their use; the A fragments of a k step are read during the one before.  The barrier stands in
@@ -500,7 +297,7 @@ __global__ __launch_bounds__(512, 1) void gemm_ring16_kernel(const bf16* __restr
   if (MAP == 0) {
     tile_m = blockIdx.y;
     tile_n = blockIdx.x + n_tile0;
-  } else {                                                  // blocks of tiles for every XCD, as in gemm_ring_kernel
+  } else {                                                  // blocks of tiles for every XCD, as in gemm_stages_kernel
     const int mt = (M + TM - 1) / TM, T = mt * n_tiles, chunk = (T + 7) / 8;
     const int L = blockIdx.x, t = (L % 8) * chunk + L / 8;
     if (t >= T || L / 8 >= chunk) return;
@@ -691,59 +488,64 @@ __global__ __launch_bounds__(512, 1) void gemm_ring16_kernel(const bf16* __restr
   }
 }
 
-// column tiles n_tile0 ... n_tile0 + n_tiles - 1 (n_tiles < 0: to the last) of a 256 x TN tiling
+// column tiles n_tile0 ... n_tile0 + n_tiles - 1 (n_tiles < 0: to the last) of a TM x TN tiling
 // (slices > 1: the slices of K go to `partial` as [slices][M][N], unadded)
-template <int EPI, int TN, int MAP>
-int launch_ring(const bf16* A, const bf16* W, void* C, int M, int N, int K, GateOut H, hipStream_t stream, int n_tile0 = 0,
-                int n_tiles = -1, float* partial = nullptr, int slices = 1) {
+template <int EPI, int TM, int TN, int MAP>
+int launch_tiles(const bf16* A, const bf16* W, void* C, int M, int N, int K, GateOut H, hipStream_t stream, int n_tile0 = 0,
+                 int n_tiles = -1, float* partial = nullptr, int slices = 1) {
   if (n_tiles < 0) n_tiles = ceil_div(N, TN) - n_tile0;
-  const int mt = ceil_div(M, RING_TM);
+  const int mt = ceil_div(M, TM);
   const int tiles_per_slice = ceil_div(K / TK, slices);
   slices = ceil_div(K / TK, tiles_per_slice);
   const dim3 grid = MAP == 0 ? dim3(n_tiles, mt, slices) : dim3(8 * ceil_div(mt * n_tiles, 8), slices, 1);
-  const size_t lds = (size_t)RING_SLOTS * RING_SLOT;
-  // tiles of 256 and 192 columns: the kernel with the 16x16x32 products; of 128: the one with 32x32x16
   void (*kernel)(const bf16*, const bf16*, void*, int, int, int, GateOut, int, int, float*, int);
-  if constexpr (TN == 128) kernel = &gemm_ring_kernel<EPI, TN, MAP>;
-  else kernel = &gemm_ring16_kernel<EPI, TN, MAP>;
+  size_t lds;
+  if constexpr (TN == STAGES_TN) {
+    static_assert(MAP == TILE_GROUP, "the kernel's own order of tiles");
+    kernel = &gemm_stages_kernel<EPI, TM>;
+    lds = (size_t)StageTiling<TM>::S * (TM + TN) * ROWB;
+  } else {
+    static_assert(TM == RING_TM, "the ring's rows");
+    kernel = &gemm_ring16_kernel<EPI, TN, MAP>;
+    lds = (size_t)RING_SLOTS * RING_SLOT;
+  }
   static LdsAllowance allowed;                     // more than 64 KB of LDS has to be asked for once a device
   if (int rc = allow_dynamic_lds(allowed, (const void*)kernel, (int)lds); rc != YALM_OK) return rc;
   kernel<<<grid, 512, lds, stream>>>(A, W, C, M, N, K, H, n_tile0, n_tiles, partial, tiles_per_slice);
   return launch_status();
 }
 
-// slices of K for the 128x128 tiles: with few rows (a big decode batch) the tiles alone leave most CUs
-// without work and the weights would stream through a few of them
-int slices_for(int M, int N, int K, long workspace_floats) {
-  const long tiles = (long)ceil_div(M, 128) * ceil_div(N, 128);
-  int slices = 1;
-  while (tiles * slices < 384 && slices * 2 <= (K / TK) / 8 && slices < 16 &&
-         (long)slices * 2 * M * N <= workspace_floats)
-    slices *= 2;
-  return slices;
-}
+// A tiling and what a launch of it takes: `start` us for a workgroup's first loads and its end; an iteration (64 k) of a round on all
+// 256 compute units `full` us, of the last round on the fraction f of them f last + (1 - f) alone (fewer units have more of the memory
+// and clock higher each); and `out` us for a million floats written.  Fitted (least squares of the relative errors, which are 6 to 10
+// %) to 2,362 launches: 12 shapes of 1,024 to 28,672 weight rows and K of 1,024 to 14,336, 129 to 8,192 rows, 1 to 12 slices of K.  What the
+// plan picks by it is 1 % slower than the fastest of them in the mean and 16 % at worst.  Those launches were short bursts.  In the long
+// products of a prompt, layer after layer, the power the chip may take sets its clock, and a narrower tile moves more operands for a product:
+// `warm` is what a product of several rounds, or of more than 1,024 rows, takes longer then (six layers of 7B sizes with 1,536 tokens whose down
+// products went one round of 192 x 128, 170 us for 175 by themselves, took 3 % longer; a step of 28 layers of 3B sizes with 3,641 tokens: q/k/v on 192 x 128
+// 103 us by itself against 116 in two launches, and the step 20,750 us against 20,000).
+struct Tiling {
+  int tm, tn;
+  double start, full, last, alone, out, warm;
+};
+constexpr Tiling TILINGS[] = {
+    {256, 256, 7.74, 1.438, 1.301, 1.069, 0.586, 1.0},   {256, 192, 6.13, 1.170, 1.157, 0.967, 0.531, 1.06},
+    {256, 128, 5.33, 0.827, 0.820, 0.648, 0.734, 1.12},  {192, 128, 4.98, 0.641, 0.656, 0.514, 0.928, 1.12},
+    {128, 128, 3.68, 0.546, 0.567, 0.391, 1.157, 1.12},  {64, 128, 4.22, 0.401, 0.435, 0.305, 0.170, 1.12}};
+constexpr int N_TILINGS = sizeof(TILINGS) / sizeof(TILINGS[0]);
 
-// Which kernel takes a shape.  160 rows and more (prompt steps, big decode batches) go to the ring kernel; fewer
-// to 128x128 tiles with K split over workgroups (a layer's four products at 160 / 256 / 383 rows: 161 / 170 /
-// 250 us against 182 / 180 / 259).
-bool takes_ring(int M) { return M >= 160; }
-
-// What a prompt step's GEMM is launched as: the tile width, the slices of K, and whether whole rounds of 256x256
-// tiles are followed by a second launch of 256x128 tiles for the remaining columns.
-struct RingPlan {
-  int tn = 256, slices = 1, nt_main = 0;         // nt_main > 0: two launches, the first over nt_main tile columns
+// What a prompt step's GEMM is launched as: the tiling, the slices of K, and whether whole rounds of 256 x 256
+// tiles are followed by a second launch of narrower tiles for the remaining columns.
+struct TilePlan {
+  int tiling = 0, slices = 1, nt_main = 0;       // nt_main > 0: two launches, the first over nt_main tile columns; `tiling` is the second's
 };
 
-// Estimated time in us of `tiles` workgroups of `iters` k tiles each.  An iteration of a 256x256 tile takes about
-// 1.47 us with all CUs at work, of a tile of 192 columns 1.30 and of 128 columns 1.00 (8,192 x 4,096 x 14,336: 329,
-// 291 and 225 us a round of 224 iterations); a last round on the fraction f of the CUs
-// costs about 0.55 + 0.45 f of a full one (the chip clocks higher with fewer CUs at work); a workgroup's first loads
-// and its epilogue take some 6 us.
-double ring_time(long tiles, int iters, int tn) {
-  const double per_iter = tn == 256 ? 1.47 : (tn == 192 ? 1.30 : 1.00);
-  const long rounds = tiles / 256, rest = tiles % 256;
-  const double f = (double)rest / 256.0;
-  return ((double)rounds + (rest ? 0.55 + 0.45 * f : 0.0)) * iters * per_iter + 6.0;
+// Estimated time in us of `tiles` workgroups of `iters` k tiles each that write `floats` numbers in all.
+double tiles_time(const Tiling& t, int M, long tiles, int iters, double floats) {
+  const long rounds = (tiles - 1) / 256;           // before the last one
+  const double f = (double)(tiles - 256 * rounds) / 256.0;
+  const double iter = (double)rounds * t.full + f * t.last + (1.0 - f) * t.alone;
+  return t.start + iters * iter * (rounds > 0 || M > 1024 ? t.warm : 1.0) + floats * 1e-6 * t.out;
 }
 
 // Splits K where the tiles alone leave most CUs without work (short prompts, narrow outputs): a second kernel then
@@ -751,76 +553,74 @@ double ring_time(long tiles, int iters, int tn) {
 // residual stream.  Unsplit, the tiles read and write that stream in their epilogue, M * N * 8 bytes that no loop
 // hides (2,048 x 4,096 x 4,096 on tiles of 128 columns: 87 us, the same tiles with the gated epilogue 65); split,
 // the kernel that adds the slices also does the norm behind them, whose own pass (M * N * 6 bytes) is saved.
-// consumer: who takes the product.  RING_PLAIN: the epilogue, or a kernel that adds the slices; RING_RESIDUAL:
-// as described above; RING_READER: a kernel that reads the product anyway adds the slices as it reads (the
+// consumer: who takes the product.  TAKES_PLAIN: the epilogue, or a kernel that adds the slices; TAKES_RESIDUAL:
+// as described above; TAKES_READER: a kernel that reads the product anyway adds the slices as it reads (the
 // rotation kernel behind q/k/v), a slice more is M * N * 4 bytes more for it to read.
-enum { RING_PLAIN = 0, RING_RESIDUAL = 1, RING_READER = 2 };
-RingPlan ring_plan(int M, int N, int K, long workspace_floats, int consumer) {
-  const bool residual = consumer == RING_RESIDUAL;
-  const int mt = ceil_div(M, 256), nk = K / TK;
-  RingPlan best;
+enum { TAKES_PLAIN = 0, TAKES_RESIDUAL = 1, TAKES_READER = 2 };
+TilePlan tile_plan(int M, int N, int K, long workspace_floats, int consumer) {
+  const bool residual = consumer == TAKES_RESIDUAL;
+  const int nk = K / TK;
+  const double MN = (double)M * N;
+  TilePlan best;
   double best_t = 1e30;
-  const double in_epilogue = residual ? (double)M * N * 8.0 / 4.0e6 : 0.0;
-  const double norm_saved = residual ? (double)M * N * 6.0 / 5.0e6 : 0.0;
-  for (int tn : {256, 192, 128}) {
-    const long tiles = (long)mt * ceil_div(N, tn);
-    for (int s = 1; s <= 8; s *= 2) {
-      if (s > 1 && (tiles * s > 256 || nk / s < 8 || (long)s * M * N > workspace_floats)) break;
-      const int iters = ceil_div(nk, s);
-      const double adding = consumer == RING_READER ? (double)(s - 1) * M * N * 4.0 / 5.0e6
-                                                    : 3.0 + (double)(s + 2) * M * N * 4.0 / 4.0e6 - norm_saved;
-      const double t = ring_time(tiles * s, iters, tn) + (s > 1 ? adding : in_epilogue);
-      if (t < best_t) { best_t = t; best.tn = tn; best.slices = s; best.nt_main = 0; }
+  const double in_epilogue = residual ? MN * 8.0 / 4.0e6 : 0.0;
+  const double norm_saved = residual ? MN * 6.0 / 5.0e6 : 0.0;
+  for (int i = 0; i < N_TILINGS; ++i) {
+    const long tiles = (long)ceil_div(M, TILINGS[i].tm) * ceil_div(N, TILINGS[i].tn);
+    for (int want : {1, 2, 3, 4, 6, 8, 12}) {
+      if (want > 1 && (tiles * want > 256 || nk / want < 6 || (long)want * M * N > workspace_floats)) break;
+      const int iters = ceil_div(nk, want), s = ceil_div(nk, iters);
+      const double adding = consumer == TAKES_READER ? (s - 1) * MN * 4.0 / 5.0e6 : 3.0 + (s + 2) * MN * 4.0 / 4.0e6 - norm_saved;
+      const double t = tiles_time(TILINGS[i], M, tiles * s, iters, MN * s) + (s > 1 ? adding : in_epilogue);
+      if (t < best_t) { best_t = t; best.tiling = i; best.slices = s; best.nt_main = 0; }
     }
   }
-  const int nt = ceil_div(N, 256);
+  const int mt = ceil_div(M, 256), nt = ceil_div(N, 256);
   const int nt_main = (int)(((long)mt * nt / 256) * 256 / mt);
-  if (nt_main > 0 && nt_main < nt) {
-    const double t = ring_time((long)mt * nt_main, nk, 256) +
-                     ring_time((long)mt * (ceil_div(N, 128) - 2 * nt_main), nk, 128) + in_epilogue;
-    if (t < best_t) { best_t = t; best.tn = 256; best.slices = 1; best.nt_main = nt_main; }
-  }
-  return best;
+  TilePlan main;
+  double main_t = 1e30;
+  if (nt_main > 0 && nt_main < nt)
+    for (int i = 2; i < N_TILINGS; ++i) {
+      const long rest = (long)ceil_div(M, TILINGS[i].tm) * (ceil_div(N, STAGES_TN) - 2 * nt_main);
+      const double t = tiles_time(TILINGS[0], M, (long)mt * nt_main, nk, 256.0 * nt_main * M) +
+                       tiles_time(TILINGS[i], M, rest, nk, MN - 256.0 * nt_main * M) + in_epilogue;
+      if (t < main_t) { main_t = t; main.tiling = i; main.nt_main = nt_main; }
+    }
+  // (a second launch waits for the first one's last tile: for a gain of 3 % and more; 6,000 rows of 4,096 x 28,672 1,054 us in one
+  // launch and 1,122 in two that the estimate has level, 2,048 rows 393 and 383 where it has 5 %)
+  return main_t < 0.97 * best_t ? main : best;
 }
 
-// partial: scratch for the slices of K (the plan was made with its size); with always_partial the product's slices
-// stay there unadded (one slice: the product itself), *slices_out says how many
 template <int EPI>
-int launch_ring_shape(const bf16* A, const bf16* W, void* C, float* partial, long partial_floats, int M, int N, int K,
-                      GateOut H, hipStream_t stream, int* slices_out = nullptr,
-                      int consumer = EPI == 2 ? RING_RESIDUAL : RING_PLAIN) {
+int launch_tiling(int tiling, const bf16* A, const bf16* W, void* C, int M, int N, int K, GateOut H, hipStream_t stream, int n_tile0 = 0,
+                  float* partial = nullptr, int slices = 1) {
+  switch (tiling) {
+    case 0: return launch_tiles<EPI, 256, 256, 4>(A, W, C, M, N, K, H, stream, n_tile0, -1, partial, slices);
+    case 1: return launch_tiles<EPI, 256, 192, 0>(A, W, C, M, N, K, H, stream, n_tile0, -1, partial, slices);
+    case 2: return launch_tiles<EPI, 256, STAGES_TN, TILE_GROUP>(A, W, C, M, N, K, H, stream, n_tile0, -1, partial, slices);
+    case 3: return launch_tiles<EPI, 192, STAGES_TN, TILE_GROUP>(A, W, C, M, N, K, H, stream, n_tile0, -1, partial, slices);
+    case 4: return launch_tiles<EPI, 128, STAGES_TN, TILE_GROUP>(A, W, C, M, N, K, H, stream, n_tile0, -1, partial, slices);
+    case 5: return launch_tiles<EPI, 64, STAGES_TN, TILE_GROUP>(A, W, C, M, N, K, H, stream, n_tile0, -1, partial, slices);
+  }
+  return YALM_ERR_ARG;
+}
+
+// partial: scratch for the slices of K (the plan was made with its size); with slices_out the product's slices
+// stay there unadded, *slices_out says how many
+template <int EPI>
+int launch(const bf16* A, const bf16* W, void* C, float* partial, long partial_floats, int M, int N, int K,
+           GateOut H, hipStream_t stream, int* slices_out = nullptr, int consumer = EPI == 2 ? TAKES_RESIDUAL : TAKES_PLAIN) {
   const bool keep = slices_out != nullptr;
-  const RingPlan p = ring_plan(M, N, K, partial != nullptr ? partial_floats : 0, consumer);
+  const TilePlan p = tile_plan(M, N, K, partial != nullptr ? partial_floats : 0, consumer);
+  if (keep) *slices_out = p.slices;
   if (p.nt_main > 0) {
-    if (keep) *slices_out = 1;
-    int rc = launch_ring<EPI, 256, 4>(A, W, C, M, N, K, H, stream, 0, p.nt_main);
+    int rc = launch_tiles<EPI, 256, 256, 4>(A, W, C, M, N, K, H, stream, 0, p.nt_main);
     if (rc != YALM_OK) return rc;
-    return launch_ring<EPI, 128, 4>(A, W, C, M, N, K, H, stream, 2 * p.nt_main);
+    return launch_tiling<EPI>(p.tiling, A, W, C, M, N, K, H, stream, 2 * p.nt_main);
   }
-  int slices = p.slices;
-  if (slices > 1) {                                // what the launch makes of it
-    const int per = ceil_div(K / TK, slices);
-    slices = ceil_div(K / TK, per);
-  }
-  if (keep) *slices_out = slices;
-  int rc;
-  if (p.tn == 192) {
-    rc = launch_ring<EPI, 192, 0>(A, W, C, M, N, K, H, stream, 0, -1, partial, slices);
-  } else if (p.tn == 128) {
-    rc = launch_ring<EPI, 128, 4>(A, W, C, M, N, K, H, stream, 0, -1, partial, slices);
-  } else {
-    rc = launch_ring<EPI, 256, 4>(A, W, C, M, N, K, H, stream, 0, -1, partial, slices);
-  }
-  if (rc != YALM_OK || slices == 1 || keep) return rc;
-  return yalm_splitk_reduce(partial, C, M, N, H, slices, EPI, stream);
-}
-
-template <int EPI>
-int launch(const bf16* A, const bf16* W, void* C, float* ws, long ws_floats, int M, int N, int K, GateOut H,
-           hipStream_t stream) {
-  if (takes_ring(M)) return launch_ring_shape<EPI>(A, W, C, ws, ws_floats, M, N, K, H, stream);
-  const int slices = ws != nullptr ? slices_for(M, N, K, ws_floats) : 1;
-  return launch_shape<EPI, 128, 128, 2, 2, 2, 2>(A, W, C, M, N, K, H, ws, slices, stream);
+  int rc = launch_tiling<EPI>(p.tiling, A, W, C, M, N, K, H, stream, 0, partial, p.slices);
+  if (rc != YALM_OK || p.slices == 1 || keep) return rc;
+  return yalm_splitk_reduce(partial, C, M, N, H, p.slices, EPI, stream);
 }
 
 }  // namespace
@@ -829,19 +629,14 @@ int launch(const bf16* A, const bf16* W, void* C, float* ws, long ws_floats, int
 // the residual stream; other products split as much or less
 long yalm_gemm_bf16_dma_workspace(int M, int N, int K) {
   if (M <= 64 || K < TK || K % TK != 0) return 0;
-  if (takes_ring(M)) {
-    const int s = max(ring_plan(M, N, K, (long)1 << 40, RING_RESIDUAL).slices,
-                      ring_plan(M, N, K, (long)1 << 40, RING_READER).slices);
-    return s > 1 ? (long)s * M * N : 0;
-  }
-  const int slices = slices_for(M, N, K, (long)1 << 40);
-  return slices > 1 ? (long)slices * M * N : 0;
+  const int s = max(tile_plan(M, N, K, (long)1 << 40, TAKES_RESIDUAL).slices, tile_plan(M, N, K, (long)1 << 40, TAKES_READER).slices);
+  return s > 1 ? (long)s * M * N : 0;
 }
 
 // The product's K slices, left unadded, as [*slices][M][N] float32 in the workspace (one slice: the product
 // itself), for a consumer that adds them.  More than 64 rows, K a multiple of 64, at least M * N floats.
 // residual: the consumer adds them to the residual stream; else it is a kernel that reads the product anyway
-// (see ring_plan).
+// (see tile_plan).
 int yalm_gemm_bf16_dma_partial(const void* A, const void* W, float* workspace, long workspace_floats, int M, int N,
                                int K, int* slices_out, int residual, hipStream_t stream) {
   if (M <= 64 || K < TK || K % TK != 0 || ((uintptr_t)A & 15) || ((uintptr_t)W & 15) || workspace == nullptr ||
@@ -849,21 +644,13 @@ int yalm_gemm_bf16_dma_partial(const void* A, const void* W, float* workspace, l
     return YALM_ERR_ARG;
   const bf16* a = (const bf16*)A;
   const bf16* w = (const bf16*)W;
-  if (takes_ring(M)) {              // one slice: the ring kernel stores the product itself, to the workspace
-    const int consumer = residual ? RING_RESIDUAL : RING_READER;
-    const RingPlan p = ring_plan(M, N, K, workspace_floats, consumer);
-    if (p.slices == 1) {
-      *slices_out = 1;
-      return launch_ring_shape<0>(a, w, workspace, nullptr, 0, M, N, K, GateOut(0), stream);
-    }
-    return launch_ring_shape<0>(a, w, nullptr, workspace, workspace_floats, M, N, K, GateOut(0), stream, slices_out,
-                                consumer);
+  const int consumer = residual ? TAKES_RESIDUAL : TAKES_READER;
+  const TilePlan p = tile_plan(M, N, K, workspace_floats, consumer);
+  if (p.slices == 1) {              // the kernel stores the product itself, to the workspace
+    *slices_out = 1;
+    return launch<0>(a, w, workspace, nullptr, 0, M, N, K, GateOut(0), stream);
   }
-  int slices = slices_for(M, N, K, workspace_floats);
-  const int tiles_per_slice = ceil_div(K / TK, slices);
-  slices = ceil_div(K / TK, tiles_per_slice);          // what the launch makes of it
-  *slices_out = slices;
-  return launch_shape<0, 128, 128, 2, 2, 2, 2>(a, w, workspace, M, N, K, GateOut(0), workspace, slices, stream, false);
+  return launch<0>(a, w, nullptr, workspace, workspace_floats, M, N, K, GateOut(0), stream, slices_out, consumer);
 }
 
 int yalm_gemm_bf16_dma(const void* A, const void* W, void* C, float* workspace, long workspace_floats, int M, int N,
