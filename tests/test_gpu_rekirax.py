@@ -448,6 +448,79 @@ def test_recurrence_by_tiles(H, d, dv, gates):
     assert bool(torch.isnan(state[0]).all()) and torch.equal(state[-1], before[-1])
 
 
+def recurrence(tiles, proj, bias, lower, w, state, lens, H, d, dv):
+    """(heads float32, sums before their norm) of one of the two ways over prompts of these lengths; state is left advanced."""
+    from yalm_amd.ops import kernels
+    cu = i32(np.concatenate([[0], np.cumsum(lens)]))
+    tile0 = np.concatenate([[0], np.cumsum([(n + 63) // 64 for n in lens])])
+    slots = i32(range(len(lens)))
+    out, raw = (torch.full((sum(lens), H * dv), float("nan"), device=DEV) for _ in range(2))
+    if tiles:
+        scratch = lambda name, shape, dtype: torch.full(shape, float("nan"), dtype=dtype, device=DEV)
+        kernels.hgrn2_tiles(proj, bias, lower, w, state, raw, cu, slots, i32(tile0), int(tile0[-1]), out, H, d, dv, 1e-5, scratch)
+    else:
+        kernels.hgrn2(proj, bias, lower, w, state, raw, cu, slots, out, H, d, dv, 1e-5)
+    return out, raw
+
+
+@pytest.mark.parametrize("d,dv", [(4, 8), (33, 16), (64, 40), (128, 128)])
+@pytest.mark.parametrize("gate", ["one", "one by a number", "zero", "zero by a number"])
+def test_recurrence_by_tiles_under_gates_of_exactly_zero_and_one(gate, d, dv):
+    """A forget gate behind an infinity, or behind a number whose exponential overflows, is the bound it tends to, whatever the state holds:
+    a gate of one keeps it and a gate of zero leaves nothing of it, as token by token."""
+    H, lens = 2, [1, 5, 64, 70, 130]
+    one = gate.startswith("one")
+    z = {"one": float("inf"), "one by a number": 3e38, "zero": -float("inf"), "zero by a number": -200.0}[gate]
+    proj = randn(sum(lens), 2 * H * d + H * dv, seed=d).to(DEV)
+    bias = torch.full((H * d,), z, device=DEV)
+    lower = torch.zeros(H * d, device=DEV)
+    start = randn(len(lens), H * dv * d, seed=2, scale=1.0 if one else 1e30).to(DEV)
+    state = start.clone()
+    out, raw = recurrence(True, proj, bias, lower, torch.ones(dv, device=DEV), state, lens, H, d, dv)
+    q = P.silu(proj[:, :H * d].cpu().to(F64)).reshape(-1, H, d)
+    v = proj[:, 2 * H * d:].cpu().to(F64).reshape(-1, H, dv)
+    at = 0
+    for b, n in enumerate(lens):
+        S0 = start[b].cpu().to(F64).reshape(H, dv, d)
+        # gates of one: the state that stood there, for every token; of zero: the token's own value in every channel
+        S = S0[None].expand(n, H, dv, d) if one else v[at:at + n, :, :, None].expand(n, H, dv, d)
+        assert torch.equal(state[b].cpu().reshape(H, dv, d), S[-1].to(torch.float32)), b
+        want = torch.einsum("thjd,thd->thj", S, q[at:at + n])
+        size = torch.einsum("thjd,thd->thj", S.abs(), q[at:at + n].abs())
+        got = raw[at:at + n].cpu().to(F64).reshape(n, H, dv)
+        # roundings: seven of q at most, one a product, one for each of d sums
+        assert bool(((got - want).abs() <= (d + 8) * 2.0 ** -24 * size).all()), b
+        at += n
+    assert bool(torch.isfinite(out).all())
+
+
+@pytest.mark.parametrize("at", [0, 5, 63, 64, 100])
+@pytest.mark.parametrize("where", ["gate", "query", "bias"])
+def test_recurrence_by_tiles_shows_what_is_not_a_number(where, at):
+    """A NaN in a token's gate, query or a gate's bias is seen where the walk from token to token shows it: in that head from the token
+    on (a query's in that token alone), in that channel of the state, and nowhere else."""
+    H, d, dv, lens = 3, 64, 32, [130]
+    h, c = 1, 7
+    proj = randn(130, 2 * H * d + H * dv, seed=3).to(DEV)
+    bias, lower = randn(H * d, seed=4).to(DEV), randn(H * d, seed=5).abs().clamp(0, 0.9).to(DEV)
+    w = torch.ones(dv, device=DEV)
+    if where == "bias":
+        bias[h * d + c] = float("nan")
+    else:
+        proj[at, (H * d if where == "gate" else 0) + h * d + c] = float("nan")
+    res = []
+    for tiles in (False, True):
+        state = randn(1, H * dv * d, seed=6).to(DEV)
+        out, raw = recurrence(tiles, proj, bias, lower, w, state, lens, H, d, dv)
+        res.append((raw.reshape(130, H, dv), out.reshape(130, H, dv), state.reshape(H, dv, d)))
+    for walk, tiled in zip(*res):
+        assert torch.equal(torch.isnan(walk), torch.isnan(tiled))
+        ok = ~torch.isnan(walk)
+        assert torch.allclose(walk[ok], tiled[ok], rtol=2e-5, atol=2e-5)
+    first = 0 if where == "bias" else at
+    assert bool(torch.isnan(res[1][0][first, h]).all()) and not bool(torch.isnan(res[1][0][:first]).any())
+
+
 def test_when_the_recurrence_goes_by_tiles():
     """Few workgroups of the walk and prompts long enough; never key heads that the tiles do not take."""
     from yalm_amd.ops import kernels

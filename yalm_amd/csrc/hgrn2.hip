@@ -136,16 +136,6 @@ constexpr int HT_HALF = 8, HT_QUAD = 4;          // tokens of half a block, of a
 
 size_t hgrn2_tiles_lds(int dp) { return ((size_t)4 * GT * (dp + 4) + GNB * dp + (size_t)GT * GA_ROW) * sizeof(float); }
 
-// 1 / (1 + e^-z) to about an ulp of it: e^x by the exponential instruction with the rounding of x log2(e) put back, the reciprocal
-// instruction with one step of Newton's; behind -80, where the result is 1.8e-35, it stays there.  (expf and a division are three times
-// as many instructions, 2,048 of which a wave issues a tile.)
-__device__ __forceinline__ float tile_sigmoid(float z) {
-  const float x = fminf(-z, 80.f), t = x * 1.4426950408889634f;
-  const float lost = fmaf(x, 1.4426950408889634f, -t) + x * 1.925963033500601e-8f;      // log2(e) in two floats
-  const float e = __builtin_amdgcn_exp2f(t), den = 1.0f + fmaf(e, lost * 0.6931471805599453f, e), r = __builtin_amdgcn_rcpf(den);
-  return r * (2.0f - den * r);
-}
-
 // qd [tile][head][64][DP], kd [tile][head][DP][64] and gd [tile][head][DP] as tile_scan.h wants them; raw = the second sum of o.
 // A thread owns one channel of one block of 16 tokens.  LDS (155 KB at DP 128: a workgroup of eight waves a compute unit): four rows
 // a token, first q, 1 - f and f; then q F(block's start, t), (1 - f) F(t, block's end) and, for the halves of a block, q F(half's start, t)
@@ -202,7 +192,8 @@ __global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float
     const Hgrn2Op::Row mine = op.begin(h, ch, ch_ok);
 #pragma unroll
     for (int u = 0; u < GB; ++u) {
-      const float qq = z[u][0] * tile_sigmoid(z[u][0]), ff = fmaf(1.0f - mine.lower, tile_sigmoid(z[u][1] + mine.bias), mine.lower);
+      float qq, ff, none;
+      op.form(mine, z[u], nullptr, qq, ff, none);
       const bool ok = ch_ok && sb * GB + u < n;    // what lies behind the text or the head adds nothing and forgets nothing
       q[u] = ok ? qq : 0.f;
       f[u] = ok ? ff : 1.f;
