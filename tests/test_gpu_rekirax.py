@@ -521,6 +521,39 @@ def test_recurrence_by_tiles_shows_what_is_not_a_number(where, at):
     assert bool(torch.isnan(res[1][0][first, h]).all()) and not bool(torch.isnan(res[1][0][:first]).any())
 
 
+@pytest.mark.parametrize("bad", [float("inf"), -float("inf"), float("nan")])
+@pytest.mark.parametrize("H,d,dv", [(2, 33, 33), (1, 100, 64), (3, 128, 128)])
+def test_a_value_that_is_not_finite_reaches_no_earlier_token(H, d, dv, bad):
+    """One element of one token's value is not finite, at every place of a block, a tile and a sequence: the tokens in front of it, the other
+    columns and the other heads stay what they are without it, its own column shows it from that token on."""
+    lens = [70] * 19 + [64, 1, 33]
+    places = [0, 1, 3, 4, 7, 8, 12, 15, 16, 17, 31, 32, 47, 62, 63, 64, 65, 68, 69, 63, 0, 32]
+    h, j = H - 1, dv - 2
+    g = gen(d)
+    rn = lambda *s, sc=1.0: torch.randn(*s, generator=g) * sc
+    proj = rn(sum(lens), 2 * H * d + H * dv).to(DEV)
+    bias, lower, w = rn(H * d).to(DEV), torch.rand(H * d, generator=g).to(DEV), torch.ones(dv, device=DEV)
+    start = rn(len(lens), H * dv * d, sc=0.5).to(DEV)
+    cu = [0] + list(np.cumsum(lens))
+    state = start.clone()
+    clean, clean_raw = recurrence(True, proj, bias, lower, w, state, lens, H, d, dv)
+    hit = proj.clone()
+    for b, t in enumerate(places):
+        hit[cu[b] + t, 2 * H * d + h * dv + j] = bad
+    state_hit = start.clone()
+    out, raw = recurrence(True, hit, bias, lower, w, state_hit, lens, H, d, dv)
+    close = lambda a, b: torch.allclose(a, b, rtol=2e-5, atol=2e-5)
+    others = [k for k in range(dv) if k != j]
+    for b, t in enumerate(places):
+        rows = slice(cu[b], cu[b + 1])
+        a, r, ra = out[rows].view(-1, H, dv), raw[rows].view(-1, H, dv), clean_raw[rows].view(-1, H, dv)
+        assert close(a[:t], clean[rows].view(-1, H, dv)[:t]), (b, t)
+        assert close(r[:t], ra[:t]) and close(r[:, :, others], ra[:, :, others]), (b, t)
+        assert torch.equal(r[:, :h], ra[:, :h]) and not bool(torch.isfinite(r[t:, h, j]).any()), (b, t)
+        s, sc = state_hit[b].view(H, dv, d), state[b].view(H, dv, d)
+        assert torch.equal(s[:, others], sc[:, others]) and torch.equal(s[:h], sc[:h]) and not bool(torch.isfinite(s[h, j]).any()), (b, t)
+
+
 def test_when_the_recurrence_goes_by_tiles():
     """Few workgroups of the walk and prompts long enough; never key heads that the tiles do not take."""
     from yalm_amd.ops import kernels

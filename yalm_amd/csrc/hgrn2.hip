@@ -15,6 +15,7 @@
 // tile_scan.h's walk over the tiles the products with S_0 and the state.  Between two tokens of different blocks F is cut at the blocks'
 // borders into factors of the one, of the blocks between and of the other, which makes the sum over channels a matrix product: blocks of 16
 // tokens, halves of one and quarters of one; inside four tokens every pair's product is carried on from token to token.
+#include <cfloat>
 #include <climits>
 #include "tile_scan.h"
 #include "yalm_hip.h"
@@ -346,6 +347,12 @@ __global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float
   for (int col = wave; col < n_cols; col += NWAVES) {
     if (col != wave) load_values(col);
     const int j = col * 16 + li;
+    // Where a value is not finite, the zeros of the tokens that do not see it would make their results NaN: the tokens of one block then
+    // meet one by one.
+    bool all_finite = true;
+#pragma unroll
+    for (int i = 0; i < GT / 4; ++i) all_finite = all_finite && fabsf(vb[i]) <= FLT_MAX;
+    const bool one_by_one = __any(!all_finite);
 #pragma unroll
     for (int i = 0; i < GNB; ++i) {
       gf32x4 acc[4];
@@ -353,11 +360,23 @@ __global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float
       for (int r = 0; r < 4; ++r) acc[r] = (gf32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m <= i; ++m) {
+        if (m == i && one_by_one) break;
         const float4 a = *reinterpret_cast<const float4*>(s_a + (i * GB + li) * GA_ROW + 16 * m + 4 * lq);
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = mfma4(el(a, r), vb[4 * m + r], acc[r]);
       }
-      const gf32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      gf32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      if (one_by_one) {
+#pragma unroll
+        for (int s = 0; s < GB; ++s) {
+          const float v = __shfl(vb[4 * i + s % 4], s / 4 * 16 + li, WAVE);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int t = 4 * lq + r;
+            if (t >= s) sum[r] = fmaf(s_a[(i * GB + t) * GA_ROW + i * GB + s], v, sum[r]);
+          }
+        }
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = i * GB + 4 * lq + r;
