@@ -554,6 +554,32 @@ def test_a_value_that_is_not_finite_reaches_no_earlier_token(H, d, dv, bad):
         assert torch.equal(s[:, others], sc[:, others]) and torch.equal(s[:h], sc[:h]) and not bool(torch.isfinite(s[h, j]).any()), (b, t)
 
 
+@pytest.mark.parametrize("H,d,dv,lens", [(8, 128, 128, [300, 64, 65, 1, 130]), (6, 64, 64, [200, 33, 129]), (6, 32, 40, [129, 7, 300])])
+def test_the_tiles_are_no_further_off_than_the_walk(H, d, dv, lens):
+    """Under gates of 0.1 to 1, the range of lower bounds and projections that models have: the relative errors (2-norm) of the heads and
+    of the state that is left, against 64 bits.  A twentieth for one draw against another."""
+    g = gen(11)
+    rn = lambda *s, sc=1.0: torch.randn(*s, generator=g) * sc
+    proj = rn(sum(lens), 2 * H * d + H * dv)
+    bias, lower = rn(H * d, sc=0.3), 0.1 + 0.8 * torch.rand(H * d, generator=g)
+    w = {"m.f": torch.eye(H * d, dtype=F64), "m.f.b": bias.to(F64), "m.lower": lower.to(F64)}
+    q, v = P.silu(proj[:, :H * d].to(F64)).reshape(-1, H, d), proj[:, 2 * H * d:].to(F64).reshape(-1, H, dv)
+    f = P.forget_gates(proj[:, H * d:2 * H * d].to(F64), w, "m.").reshape(-1, H, d)
+    want, left, at = [], [], 0
+    for n in lens:
+        o, S = P.hgrn2_recurrence(q[at:at + n], f[at:at + n], v[at:at + n], torch.zeros(H, d, dv, dtype=F64))
+        want.append((P.rms_div(o, 1e-5)).reshape(n, H * dv))
+        left.append(S.transpose(1, 2).reshape(-1))
+        at += n
+    want, left = torch.cat(want), torch.stack(left)
+    off = []
+    for tiles in (False, True):
+        state = torch.zeros(len(lens), H * dv * d, device=DEV)
+        out, _ = recurrence(tiles, proj.to(DEV), bias.to(DEV), lower.to(DEV), torch.ones(dv, device=DEV), state, lens, H, d, dv)
+        off.append([((a.cpu().to(F64) - b).norm() / b.norm()).item() for a, b in ((out, want), (state, left))])
+    assert all(tiled <= 1.05 * walk for walk, tiled in zip(*off)), off
+
+
 def test_when_the_recurrence_goes_by_tiles():
     """Few workgroups of the walk and prompts long enough; never key heads that the tiles do not take."""
     from yalm_amd.ops import kernels

@@ -35,9 +35,12 @@ struct Hgrn2Op {
     z[0] = proj[(size_t)t * N + h * d + r];
     z[1] = proj[(size_t)t * N + Hd + h * d + r];
   }
-  __device__ void form(const Row& m, const float* z, const float*, float& q, float& f, float&) const {
+  // k = 1 - f as (1 - lower) e / (1 + e), e = e^-z, where that keeps digits: of an f close to one the rounding would be most of 1 - f
+  __device__ void form(const Row& m, const float* z, const float*, float& q, float& f, float& k) const {
     q = z[0] / (1.0f + expf(-z[0]));
-    f = m.lower + (1.0f - m.lower) / (1.0f + expf(-(z[1] + m.bias)));
+    const float e = expf(-(z[1] + m.bias)), free = 1.0f - m.lower, open = free / (1.0f + e);
+    f = m.lower + open;
+    k = e > 1.0f ? free - open : open * e;
   }
   __device__ float value(int t, int h, int j) const { return proj[(size_t)t * N + 2 * Hd + h * dv + j]; }
   __device__ static float act(float v) { return v; }
@@ -144,8 +147,8 @@ size_t hgrn2_tiles_lds(int dp) { return ((size_t)4 * GT * (dp + 4) + GNB * dp + 
 // Bound by its phases one behind the other, 15 us a workgroup: the operands' way in 3, their gates 2, the scaled rows through LDS 4, the
 // products 2, the rest barriers and the way out (five prompts of 255 to 509 tokens, 32 heads of 128 x 128, 992 workgroups: 67 us, the
 // walk over the tiles behind it 83, the heads' norm 9; token by token 212 and 16).  Errors against 64 bits, relative, of
-// the normed heads: ordinary gates 9.2e-8 (token by token 8.6e-8), gates close to one 4.7e-7 (8.3e-7), small ones 7.0e-8 (7.1e-8); the state's
-// 1.1e-7 (1.4e-7), 1.6e-6 (2.8e-6), 3.3e-8 (2.7e-8).
+// the normed heads: ordinary gates 8.4e-8 (token by token 8.5e-8), gates close to one 1.0e-7 (8.2e-7), small ones 6.6e-8 (7.0e-8); of
+// the state 8.2e-8 (1.4e-7), 2.2e-7 (2.8e-6), 3.3e-8 (2.7e-8: there 1 - f is close to one and rounded, which the walk's f (S - v) + v is not).
 template <int DP>
 __global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float* __restrict__ raw, float* __restrict__ qd,
                                                                float* __restrict__ kd, float* __restrict__ gd,
@@ -193,12 +196,12 @@ __global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float
     const Hgrn2Op::Row mine = op.begin(h, ch, ch_ok);
 #pragma unroll
     for (int u = 0; u < GB; ++u) {
-      float qq, ff, none;
-      op.form(mine, z[u], nullptr, qq, ff, none);
+      float qq, ff, kk;
+      op.form(mine, z[u], nullptr, qq, ff, kk);
       const bool ok = ch_ok && sb * GB + u < n;    // what lies behind the text or the head adds nothing and forgets nothing
       q[u] = ok ? qq : 0.f;
       f[u] = ok ? ff : 1.f;
-      k[u] = ok ? 1.0f - ff : 0.f;
+      k[u] = ok ? kk : 0.f;
     }
   }
   float total = 1.f;
@@ -365,7 +368,9 @@ __global__ __launch_bounds__(GNB * DP) void hgrn2_tiles_kernel(Hgrn2Op op, float
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = mfma4(el(a, r), vb[4 * m + r], acc[r]);
       }
-      gf32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      gf32x4 sum;                                  // (in 64 bits: two roundings less, a twentieth of the heads' error)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[r] = (float)(((double)acc[0][r] + (double)acc[1][r]) + ((double)acc[2][r] + (double)acc[3][r]));
       if (one_by_one) {
 #pragma unroll
         for (int s = 0; s < GB; ++s) {
