@@ -2091,3 +2091,47 @@ def test_gemm_add_emit_and_its_consumers(M, N, Kd, N2, small_workspace):
         close(mid, act_fn(h @ wg.double().T) * (h @ wu.double().T), torch.bfloat16, "scaled gated product " + act, factor=2)
     with pytest.raises(Exception):                        # a row scale is for these batches only
         k.gemm(xn[:8].contiguous(), w2.to(DEV), out[:8].contiguous(), k.EPI_STORE_F32, scale_from=(ss[:8].contiguous(), eps))
+
+
+# ------------------------------------------------------------------ recurrences by tiles
+
+@pytest.mark.parametrize("kind", ["hgrn2", "gla", "lightning"])
+@pytest.mark.parametrize("d,dv", [(32, 32), (20, 96), (64, 64), (128, 128), (100, 32), (32, 48), (64, 33), (128, 48), (64, 16)])
+def test_recurrences_by_tiles_of_many_workgroups(kind, d, dv):
+    """From a workgroup and a half a compute unit on, whole groups of 32 columns share a workgroup of the walk over tiles: read-outs and
+    states have the bits that each sequence has alone (which goes 16 columns a workgroup)."""
+    k = K()
+    H, rank, lens = 16, 5, [1, 64, 65, 130, 17, 200] * 4
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    assert 2 * H * ((dv + 31) // 32) * len(lens) >= 3 * units > 2 * H * ((dv + 31) // 32)
+    T, Hd, Hv = sum(lens), H * d, H * dv
+    width = {"hgrn2": 2 * Hd + Hv, "gla": 2 * Hd + 2 * Hv + rank, "lightning": 2 * Hd + Hv}[kind]
+    proj, start = rnd((T, width), 1).to(DEV), rnd((len(lens), Hv * d), 2, scale=0.3).to(DEV)
+    bias, lower, w = rnd((Hd,), 3).to(DEV), rnd((Hd,), 4).abs().clamp(0, 0.9).to(DEV), (1 + 0.1 * rnd((dv,), 5)).to(DEV)
+    w2 = torch.zeros(Hd, k.gla_padded_rank(rank))
+    w2[:, :rank] = rnd((Hd, rank), 6)
+    w2 = w2.to(DEV)
+    powers = (torch.linspace(0.9, 1.0, H, dtype=torch.float64)[:, None] ** torch.arange(65)).float().contiguous().to(DEV)
+    scratch = lambda name, shape, dt: torch.full(shape, float("nan"), dtype=dt, device=DEV)
+
+    def run(rows, lens, state):
+        n = sum(lens)
+        out, raw = (torch.full((n, Hv), float("nan"), device=DEV) for _ in range(2))
+        ends = lambda sizes: [0] + torch.tensor(sizes).cumsum(0).tolist()
+        tile0 = ends([(x + 63) // 64 for x in lens])
+        places = (i32(ends(lens)), i32(list(range(len(lens)))), i32(tile0), tile0[-1])
+        if kind == "hgrn2":
+            k.hgrn2_tiles(rows, bias, lower, w, state, raw, *places, out, H, d, dv, 1e-5, scratch)
+        elif kind == "gla":
+            k.gla_tiles(rows, w2, bias, w, state, raw, *places, out, H, d, dv, rank, d ** -0.5, 16.0, 1e-5, scratch)
+        else:
+            k.lightning_tiles(rows, powers, state, raw, *places, H, d, dv, scratch)
+        return raw
+    state = start.clone()
+    raw, at = run(proj, lens, state), 0
+    assert bool(torch.isfinite(raw).all())
+    for b, n in enumerate(lens):
+        if b % 5 == 0 or n == 200:
+            alone = start[b:b + 1].clone()
+            assert torch.equal(run(proj[at:at + n].contiguous(), [n], alone), raw[at:at + n]) and torch.equal(alone[0], state[b]), b
+        at += n

@@ -14,7 +14,7 @@
 // gla_tiles_kernel (every tile and head at once): the decays and their sums, the three scaled operands above, and the
 // second sum of o.  No e^(-L) is ever formed, whatever the decays: the tile is cut into four blocks of 16 tokens;
 // between blocks the exponent is split at the blocks' borders into parts that are each <= 0, and inside a block every
-// (t, s, channel) has its own e^(L_t - L_s).  scan_carry_kernel (a workgroup 16 columns of a head, the tiles in order): the
+// (t, s, channel) has its own e^(L_t - L_s).  scan_carry_kernel (a workgroup 16 or 32 columns of a head, the tiles in order): the
 // products with S_0 and the state (tile_scan.h).
 #include "tile_scan.h"
 #include "yalm_hip.h"

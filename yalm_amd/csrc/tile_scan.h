@@ -4,7 +4,7 @@
 //     kd [DP][64]   the keys times the decays behind their token up to the tile's end (zeros behind the text),
 //     gd [DP]       the decays of the whole tile,
 // and in raw the part of o that the tile's own tokens make.  scan_carry_kernel then walks a sequence's tiles in order (a
-// workgroup 16 columns of a head): the products with the carried state and the state itself.  A wave owns 32 rows of S in
+// workgroup 16 or 32 columns of a head): the products with the carried state and the state itself.  A wave owns 32 rows of S in
 // the layout of a matrix instruction's result, which is also its operand in the next tile's product when k is counted in
 // that order; the waves' shares of o meet in LDS.
 //
@@ -177,26 +177,23 @@ __global__ __launch_bounds__(NW * WAVE) void scan_carry_kernel(Op op, float* __r
   }
 }
 
-template <int DP, int NC, class Op>
-int scan_carry_columns(const Op& op, float* state, float* raw, const float* qd, const float* kd, const float* gd, const int* cu_seqlens,
-                       const int* seq_slot, const int* seq_tile0, int B, int n_heads, hipStream_t stream) {
-  const dim3 grid(n_heads, ceil_div(op.dv, 16 * NC), B);
-  if (op.dv % (16 * NC) == 0)
-    scan_carry_kernel<Op, DP / 32, NC, true><<<grid, DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
-                                                                             seq_tile0, n_heads);
-  else
-    scan_carry_kernel<Op, DP / 32, NC, false><<<grid, DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
-                                                                              seq_tile0, n_heads);
-  return launch_status();
-}
-
 // Every workgroup of a head reads the head's scaled queries and keys whole: with 32 columns half as often as with 16, which pays where
-// that still leaves a workgroup and a half for each compute unit (HGRN2, five prompts of 255 to 509 tokens, 32 heads of 128 x 128: 102 -> 83 us).  The sums are the same.
+// the columns are dealt in whole groups of 32 and there is still a workgroup and a half for each compute unit.  The sums are the same.  us of
+// gated linear attention and of lightning's with 16 columns and with 32, 300 tokens a sequence:
+//   6 sequences, 32 heads of 128 x 128 213 185   180 151      12, 32 heads of 64 x 64 154 152   102 103
+//   24, 32 heads of 32 x 32 168 163   85 81                   16, 16 heads of 32 x 96 114 109   69 63
+// and where groups of 32 would stand empty in part:  24, 32 heads of 64 x 16 239 256   112 129
+//   24, 16 heads of 64 x 33 166 174   94 103                  16, 24 heads of 64 x 48 151 154   100 101
 template <int DP, class Op>
 int scan_carry_launch(const Op& op, float* state, float* raw, const float* qd, const float* kd, const float* gd, const int* cu_seqlens,
                       const int* seq_slot, const int* seq_tile0, int B, int n_heads, hipStream_t stream) {
-  if (2L * n_heads * ceil_div(op.dv, 32) * B >= 3L * compute_units())
-    return scan_carry_columns<DP, 2>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, B, n_heads, stream);
-  return scan_carry_columns<DP, 1>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot, seq_tile0, B, n_heads, stream);
+  auto go = [&](auto kernel, int columns) {
+    kernel<<<dim3(n_heads, ceil_div(op.dv, columns), B), DP / 32 * WAVE, 0, stream>>>(op, state, raw, qd, kd, gd, cu_seqlens, seq_slot,
+                                                                                     seq_tile0, n_heads);
+    return launch_status();
+  };
+  if (op.dv % 32 == 0 && 2L * n_heads * (op.dv / 32) * B >= 3L * compute_units()) return go(&scan_carry_kernel<Op, DP / 32, 2, true>, 32);
+  if (op.dv % 16 == 0) return go(&scan_carry_kernel<Op, DP / 32, 1, true>, 16);
+  return go(&scan_carry_kernel<Op, DP / 32, 1, false>, 16);
 }
 }  // namespace
