@@ -581,12 +581,20 @@ def test_the_tiles_are_no_further_off_than_the_walk(H, d, dv, lens):
 
 
 def test_when_the_recurrence_goes_by_tiles():
-    """Few workgroups of the walk and prompts long enough; never key heads that the tiles do not take."""
+    """By tiles where that was measured to be sooner, and only there: steps of (sequences, tokens of each, heads, key and value size) with the
+    us of the walk and of the tiles; never key heads that the tiles do not take.  The longest sequence decides, not the mean."""
     from yalm_amd.ops import kernels
     pay = kernels.hgrn2_tiles_pay
-    assert pay(96, 1, 32, 128, 128) and not pay(95, 1, 32, 128, 128) and pay(1909, 5, 32, 128, 128) and not pay(2340, 9, 32, 128, 128)
-    assert pay(384, 1, 4, 64, 64) and not pay(383, 1, 4, 64, 64) and not pay(3000, 4, 64, 64, 64)
-    assert not pay(5000, 1, 1, 129, 16) and pay(5000, 1, 1, 128, 4000) and kernels.hgrn2_tiles_fit(128) == 128 and kernels.hgrn2_tiles_fit(129) == 0
+    for (B, n, H, d, dv), walk, tiles in (
+            ((1, 64, 32, 128, 128), 22.8, 27.2), ((1, 128, 32, 128, 128), 39.0, 32.1), ((1, 2000, 32, 128, 128), 508.7, 187.2),
+            ((5, 96, 32, 128, 128), 58.9, 78.2), ((5, 500, 32, 128, 128), 254.8, 217.2),
+            ((8, 256, 32, 128, 128), 142.0, 170.5), ((8, 700, 32, 128, 128), 379.2, 451.7), ((10, 96, 16, 128, 128), 58.7, 79.0),
+            ((6, 96, 8, 128, 256), 42.5, 53.4), ((16, 200, 16, 96, 48), 82.1, 116.1), ((1, 96, 4, 64, 64), 20.3, 23.7),
+            ((1, 200, 4, 64, 64), 36.5, 27.6), ((1, 200, 32, 64, 64), 37.3, 30.3), ((5, 200, 32, 64, 64), 43.8, 77.7),
+            ((3, 500, 64, 32, 32), 57.2, 83.2)):
+        assert pay([n] * B, H, d, dv) == (tiles < walk), (B, n, H, d, dv)
+    assert pay([600] + [20] * 7, 32, 128, 128) and not pay([95] * 8, 32, 128, 128)
+    assert not pay([5000], 1, 129, 16) and pay([5000], 1, 128, 4000) and kernels.hgrn2_tiles_fit(128) == 128 and kernels.hgrn2_tiles_fit(129) == 0
 
 
 def test_recurrent_state_is_carried_in_32_bits():
@@ -860,7 +868,7 @@ def test_unequal_batches_with_reuse(folders, name, dtype):
 def test_unequal_batches_whose_recurrence_goes_by_tiles(folders, monkeypatch, name):
     from yalm_amd.ops import kernels
     taken = []
-    monkeypatch.setattr(kernels, "hgrn2_tiles_pay", lambda T, B, n_heads, d, dv: taken.append(T) or kernels.hgrn2_tiles_fit(d) > 0)
+    monkeypatch.setattr(kernels, "hgrn2_tiles_pay", lambda n_tok, n_heads, d, dv: taken.append(n_tok) or kernels.hgrn2_tiles_fit(d) > 0)
     test_unequal_batches_with_reuse(folders, name, "bfloat16")
     assert taken or not any("right" in layer["mixer"] for layer in KC.ALL[name]["layers"])
 

@@ -1463,18 +1463,32 @@ def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_
     return out
 
 
-def hgrn2_tiles_pay(T, B, n_heads, d, dv):
-    """Whether a step of prompts goes tile by tile (hgrn2_tiles) instead of token by token (hgrn2).  The walk takes 0.26 us a token (heads of
-    128 x 128; 0.16 of 64 x 64) while its workgroups, 32 columns of a sequence and head each, are not much more than two a compute
-    unit, and more in proportion behind that; the tiles take 13 to 16 us for every 256 of them and 3 us for each of a sequence's, and all
-    operands pass through memory.  Measured, us, walk and tiles: 32 heads of 128 x 128: one prompt of 64 tokens 22 and 24,
-    100 34 and 28, 2,048 529 and 181; five of 255 to 509 228 and 167; nine of 260 187 and 236, nine of 700 500 and 532; 64 of 33 170
-    and 428; 8 heads, 700 tokens 181 and 57.  Heads of 64 x 64: 4 of them, 100 tokens 21 and 22, 700 112 and 40; eight prompts of 100, 16 heads
-    25 and 32; four of 300, 16 heads of 32 x 64 38 and 40; 4 of 16 x 16, 500 tokens 52 and 33."""
-    groups = B * n_heads * ((dv + 31) // 32)
-    if d <= 64:
-        return hgrn2_tiles_fit(d) > 0 and T >= 384 * B and groups <= 256
-    return hgrn2_tiles_fit(d) > 0 and T >= 96 * B and groups <= 640
+# What hgrn2 (us: a launch, a token of the longest sequence, a token of 32 columns of a head on every compute unit) and hgrn2_tiles (a launch, a
+# tile of a head on every unit, a tile of the longest sequence, a tile of 32 columns on every unit) take, by the padded key size.  Fitted
+# (least squares of the relative errors, which are 5 to 10 %) to 2,117 steps of 1 to 24 sequences of 1 to 2,000 tokens, equal and unequal,
+# and 4 to 64 heads of 16 x 16 to 128 x 256.
+_HGRN2_US = {32: ((5.6, 0.088, 0.027), (18.8, 0.13, 1.62, 8.5)), 64: ((5.9, 0.142, 0.042), (19.2, 10.0, 1.41, 3.96)),
+             128: ((6.9, 0.215, 0.099), (22.0, 12.6, 1.46, 6.1))}
+
+
+def hgrn2_tiles_pay(n_tok, n_heads, d, dv):
+    """Whether a step of prompts of these lengths goes tile by tile (hgrn2_tiles) instead of token by token (hgrn2).  The walk's time is that of
+    the longest sequence's tokens, one behind the other, while its workgroups are few, and of all tokens where they are many; the tiles'
+    that of all tiles, of which every one passes through memory, however long the sequences are.  Of the steps
+    measured 18 of 2,117 are more than 2 % slower so than token by token, 1.1 times at worst; against the better of the two the mean is 0.5 %
+    slower, the worst 1.5 times (unequal sequences of few tokens).  Measured, us, walk and tiles,
+    32 heads of 128 x 128: one prompt of 64 tokens 23 and 27, of 128 39 and 32, of 2,000 509 and 187; five of 96 59 and 78, of 256 139 and
+    126, of 500 255 and 217; eight of 256 142 and 171, of 700 379 and 452; 32 heads of 64 x 64: one of 200 37 and 30, five 44 and 78; 64 of
+    32 x 32: three of 500 57 and 83."""
+    dp = hgrn2_tiles_fit(d)
+    if not dp:
+        return False
+    (walk, token, tokens), (tiles, tile, longest, columns) = _HGRN2_US[dp]
+    n_tiles = sum((n + PAGE - 1) // PAGE for n in n_tok)
+    groups = n_heads * ((dv + 31) // 32) / 256.0
+    by_token = walk + token * max(n_tok) + tokens * sum(n_tok) * groups
+    by_tile = tiles + tile * n_tiles * n_heads / 256.0 + longest * ((max(n_tok) + PAGE - 1) // PAGE) + columns * n_tiles * groups
+    return by_tile < 0.95 * by_token
 
 
 def hgrn2_tiles_fit(d):

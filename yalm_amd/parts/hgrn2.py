@@ -98,9 +98,8 @@ class HGRN2(Part):
         raw = ws.get("hgrn2.raw", (T, self.vv), torch.float32)
         o = ws.get(self.mixed_in, (T, self.vv), h.dtype)
         state = ctx.cache.group_of(line).line_state(line)
-        B = ctx.seq_slot.shape[0]
         if ctx.mode == "prefill" and h.dtype == torch.bfloat16 and not kernels.FORCE_SIMPLE \
-                and kernels.hgrn2_tiles_pay(T, B, self.n_heads, self.key_dim, self.value_dim):
+                and kernels.hgrn2_tiles_pay(ctx.host_n_tokens, self.n_heads, self.key_dim, self.value_dim):
             tiles = ctx.tables["kv_tiles"]
             kernels.hgrn2_tiles(proj, self.f_bias, self.lower, self.w_norm, state, raw, ctx.cu_seqlens, ctx.seq_slot, tiles["seq_tile0"],
                                 tiles["n_tiles"], o, self.n_heads, self.key_dim, self.value_dim, self.eps, ws.get)
