@@ -778,3 +778,22 @@ def test_decode_splits_over_rows_pages_and_heads():
                     assert decode_order(Step, B, heads, kv, n, own=True) == Step.seq_order
                     assert decode_order(Step, B, heads, kv, n) == (None if n > 1 and 128 < per <= 512 else Step.seq_order)
     assert 128 in kernels.MFMA_HEAD_DIMS and 256 in kernels.MFMA_WIDE_HEAD_DIMS
+
+
+# us of a plain product on tiles of 256 x 256, 256 x 192, 256 x 128, 192 x 128, 128 x 128 and 64 x 128, K whole
+SHORT_PRODUCTS = {
+    (2048, 28672, 128): (54.6, 50.6, 60.9, 64.4, 65.4, 80.4), (700, 28672, 128): (22.5, 21.0, 21.2, 22.6, 24.0, 28.2),
+    (1100, 24000, 256): (31.4, 39.7, 33.7, 33.0, 34.5, 48.4), (4096, 6144, 192): (27.5, 27.9, 25.8, 30.1, 30.0, 38.5),
+    (2048, 8192, 64): (14.0, 17.3, 15.4, 15.9, 17.1, 21.3), (300, 32000, 512): (21.6, 28.7, 25.7, 25.0, 27.7, 34.1),
+    (2048, 512, 512): (15.6, 12.7, 10.5, 9.1, 7.7, 6.5), (4096, 1536, 512): (17.7, 15.7, 12.8, 20.7, 15.1, 16.8),
+    (700, 1024, 256): (11.3, 9.2, 7.6, 6.7, 5.8, 4.9), (513, 4096, 960): (22.5, 19.3, 15.0, 12.4, 10.3, 14.3)}
+
+
+def test_products_of_a_short_k_take_tiles_that_suit_them():
+    """What the plan of the products of more than 64 rows picks where a workgroup has few iterations, held to the measured times: within a
+    tenth of the fastest tiling.  (The workspace is too small for slices of K.)"""
+    from yalm_amd.ops import library
+    for (M, N, K), us in SHORT_PRODUCTS.items():
+        choice = library.lib().yalm_gemm_bf16_dma_choice(M, N, K, 0, 0)
+        assert 10 <= choice <= 15 and us[choice % 10] <= 1.1 * min(us), (M, N, K, choice)
+    assert [library.lib().yalm_gemm_bf16_dma_choice(*a) for a in ((64, 64, 64, 0, 0), (65, 64, 72, 0, 0), (65, 64, 64, 0, 3))] == [-1, -1, -1]

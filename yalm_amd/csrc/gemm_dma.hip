@@ -515,23 +515,39 @@ int launch_tiles(const bf16* A, const bf16* W, void* C, int M, int N, int K, Gat
   return launch_status();
 }
 
-// A tiling and what a launch of it takes: `start` us for a workgroup's first loads and its end; an iteration (64 k) of a round on all
-// 256 compute units `full` us, of the last round on the fraction f of them f last + (1 - f) alone (fewer units have more of the memory
-// and clock higher each); and `out` us for a million floats written.  Fitted (least squares of the relative errors, which are 6 to 10
-// %) to 2,362 launches: 12 shapes of 1,024 to 28,672 weight rows and K of 1,024 to 14,336, 129 to 8,192 rows, 1 to 12 slices of K.  What the
-// plan picks by it is 1 % slower than the fastest of them in the mean and 16 % at worst.  Those launches were short bursts.  In the long
+// A tiling and what a launch of it takes, in us: `start` for the first workgroup's loads and the last one's end, `round` more for every
+// round of workgroups on all 256 compute units before the last one; an iteration (64 k) of such a round `full`, of the last round on the
+// fraction f of the units f last + (1 - f) alone (fewer units have more of the memory and clock higher each); and `out` for a million
+// floats written.  Two fits (least squares of the relative errors):
+//  * from K = 1,024 on to 2,362 launches: 12 shapes of 1,024 to 28,672 weight rows and K to 14,336, 129 to 8,192 rows, 1 to 12 slices of K;
+//    errors 6 to 10 %.  What the plan picks by it is 1 % slower than the fastest of them in the mean and 16 % at worst.  Its terms are the fit's,
+//    not the chip's (`out` of 64 x 128 would be stores of 23 TB/s, and rounds start for nothing): bounded to what the chip can
+//    do, with a start a round, it fits as well and picks worse (of 51 products where the two differ 31 are slower, up to 12 %, and 10 faster).
+//  * below it, where a workgroup's few iterations stand behind each other's starts and ends, to 750 launches: 14 shapes of 512 to 32,000 weight
+//    rows and K of 64 to 960, `out` at least 0.3; errors 6 to 12 %, the picks 1 % slower in the mean and, but for one shape (2,048
+//    rows of 4,096 x 512), 12 % at worst.  The first fit gave nearly all of these tiles of 64 x 128: 2,048 rows of 28,672 x 128 81 us
+//    and now 54, 4,096 of 6,144 x 192 41 and 27, 1,100 of 24,000 x 256 49 and 32.
+// Those launches were short bursts.  In the long
 // products of a prompt, layer after layer, the power the chip may take sets its clock, and a narrower tile moves more operands for a product:
 // `warm` is what a product of several rounds, or of more than 1,024 rows, takes longer then (six layers of 7B sizes with 1,536 tokens whose down
 // products went one round of 192 x 128, 170 us for 175 by themselves, took 3 % longer; a step of 28 layers of 3B sizes with 3,641 tokens: q/k/v on 192 x 128
 // 103 us by itself against 116 in two launches, and the step 20,750 us against 20,000).
+struct TileTimes {
+  double start, round, full, last, alone, out;
+};
 struct Tiling {
   int tm, tn;
-  double start, full, last, alone, out, warm;
+  double warm;
+  TileTimes long_k, short_k;
 };
+constexpr int LONG_K = 1024;
 constexpr Tiling TILINGS[] = {
-    {256, 256, 7.74, 1.438, 1.301, 1.069, 0.586, 1.0},   {256, 192, 6.13, 1.170, 1.157, 0.967, 0.531, 1.06},
-    {256, 128, 5.33, 0.827, 0.820, 0.648, 0.734, 1.12},  {192, 128, 4.98, 0.641, 0.656, 0.514, 0.928, 1.12},
-    {128, 128, 3.68, 0.546, 0.567, 0.391, 1.157, 1.12},  {64, 128, 4.22, 0.401, 0.435, 0.305, 0.170, 1.12}};
+    {256, 256, 1.0, {7.74, 0.0, 1.438, 1.301, 1.069, 0.586}, {7.672, 4.099, 1.535, 1.350, 0.956, 0.392}},
+    {256, 192, 1.06, {6.13, 0.0, 1.170, 1.157, 0.967, 0.531}, {6.271, 3.445, 1.241, 1.245, 0.710, 0.416}},
+    {256, 128, 1.12, {5.33, 0.0, 0.827, 0.820, 0.648, 0.734}, {5.429, 1.301, 1.029, 0.847, 0.523, 0.490}},
+    {192, 128, 1.12, {4.98, 0.0, 0.641, 0.656, 0.514, 0.928}, {5.290, 1.983, 0.865, 0.729, 0.351, 0.339}},
+    {128, 128, 1.12, {3.68, 0.0, 0.546, 0.567, 0.391, 1.157}, {4.569, 1.582, 0.653, 0.515, 0.273, 0.334}},
+    {64, 128, 1.12, {4.22, 0.0, 0.401, 0.435, 0.305, 0.170}, {3.931, 1.499, 0.373, 0.338, 0.214, 0.300}}};
 constexpr int N_TILINGS = sizeof(TILINGS) / sizeof(TILINGS[0]);
 
 // What a prompt step's GEMM is launched as: the tiling, the slices of K, and whether whole rounds of 256 x 256
@@ -540,12 +556,13 @@ struct TilePlan {
   int tiling = 0, slices = 1, nt_main = 0;       // nt_main > 0: two launches, the first over nt_main tile columns; `tiling` is the second's
 };
 
-// Estimated time in us of `tiles` workgroups of `iters` k tiles each that write `floats` numbers in all.
-double tiles_time(const Tiling& t, int M, long tiles, int iters, double floats) {
+// Estimated time in us of `tiles` workgroups of `iters` k tiles each that write `floats` numbers in all, of a product of M rows and K.
+double tiles_time(const Tiling& tiling, int M, int K, long tiles, int iters, double floats) {
+  const TileTimes& t = K >= LONG_K ? tiling.long_k : tiling.short_k;
   const long rounds = (tiles - 1) / 256;           // before the last one
   const double f = (double)(tiles - 256 * rounds) / 256.0;
   const double iter = (double)rounds * t.full + f * t.last + (1.0 - f) * t.alone;
-  return t.start + iters * iter * (rounds > 0 || M > 1024 ? t.warm : 1.0) + floats * 1e-6 * t.out;
+  return t.start + rounds * t.round + iters * iter * (rounds > 0 || M > 1024 ? tiling.warm : 1.0) + floats * 1e-6 * t.out;
 }
 
 // Splits K where the tiles alone leave most CUs without work (short prompts, narrow outputs): a second kernel then
@@ -571,7 +588,7 @@ TilePlan tile_plan(int M, int N, int K, long workspace_floats, int consumer) {
       if (want > 1 && (tiles * want > 256 || nk / want < 6 || (long)want * M * N > workspace_floats)) break;
       const int iters = ceil_div(nk, want), s = ceil_div(nk, iters);
       const double adding = consumer == TAKES_READER ? (s - 1) * MN * 4.0 / 5.0e6 : 3.0 + (s + 2) * MN * 4.0 / 4.0e6 - norm_saved;
-      const double t = tiles_time(TILINGS[i], M, tiles * s, iters, MN * s) + (s > 1 ? adding : in_epilogue);
+      const double t = tiles_time(TILINGS[i], M, K, tiles * s, iters, MN * s) + (s > 1 ? adding : in_epilogue);
       if (t < best_t) { best_t = t; best.tiling = i; best.slices = s; best.nt_main = 0; }
     }
   }
@@ -582,8 +599,8 @@ TilePlan tile_plan(int M, int N, int K, long workspace_floats, int consumer) {
   if (nt_main > 0 && nt_main < nt)
     for (int i = 2; i < N_TILINGS; ++i) {
       const long rest = (long)ceil_div(M, TILINGS[i].tm) * (ceil_div(N, STAGES_TN) - 2 * nt_main);
-      const double t = tiles_time(TILINGS[0], M, (long)mt * nt_main, nk, 256.0 * nt_main * M) +
-                       tiles_time(TILINGS[i], M, rest, nk, MN - 256.0 * nt_main * M) + in_epilogue;
+      const double t = tiles_time(TILINGS[0], M, K, (long)mt * nt_main, nk, 256.0 * nt_main * M) +
+                       tiles_time(TILINGS[i], M, K, rest, nk, MN - 256.0 * nt_main * M) + in_epilogue;
       if (t < main_t) { main_t = t; main.tiling = i; main.nt_main = nt_main; }
     }
   // (a second launch waits for the first one's last tile: for a gain of 3 % and more; 6,000 rows of 4,096 x 28,672 1,054 us in one
@@ -631,6 +648,12 @@ long yalm_gemm_bf16_dma_workspace(int M, int N, int K) {
   if (M <= 64 || K < TK || K % TK != 0) return 0;
   const int s = max(tile_plan(M, N, K, (long)1 << 40, TAKES_RESIDUAL).slices, tile_plan(M, N, K, (long)1 << 40, TAKES_READER).slices);
   return s > 1 ? (long)s * M * N : 0;
+}
+
+extern "C" int yalm_gemm_bf16_dma_choice(int M, int N, int K, long workspace_floats, int consumer) {
+  if (M <= 64 || N <= 0 || K < TK || K % TK != 0 || consumer < TAKES_PLAIN || consumer > TAKES_READER) return -1;
+  const TilePlan p = tile_plan(M, N, K, workspace_floats, consumer);
+  return (p.nt_main > 0 ? 1000 : 0) + 10 * p.slices + p.tiling;
 }
 
 // The product's K slices, left unadded, as [*slices][M][N] float32 in the workspace (one slice: the product

@@ -65,6 +65,10 @@ int yalm_gemm_f32_split_choice(int M, int N, int K, int gate);
 // Floats of workspace with which the tiled bfloat16 kernel for more than 64 rows splits K (0: it does
 // not; the output's tiles fill the chip).
 long yalm_gemm_bf16_dma_workspace(int M, int N, int K);
+// How that kernel launches a product, for tests of each way: 10 slices of K + the tiling (0: 256 x 256, 1: 256 x 192, 2: 256 x 128, 3: 192 x
+// 128, 4: 128 x 128, 5: 64 x 128), and 1,000 more where whole rounds of 256 x 256 go in front and that tiling takes the rest; -1: it does not
+// take the shape.  consumer: 0 the epilogue, 1 a product added to the residual stream, 2 a kernel that reads the product anyway.
+int yalm_gemm_bf16_dma_choice(int M, int N, int K, long workspace_floats, int consumer);
 
 // Decode GEMMs from the float32 residual stream, M <= 8 rows (M * (K + 8) * 2 bytes <= 72 KB), bfloat16 weights:
 // C = epilogue(rmsnorm(x, norm_w, eps) * W^T); epilogue 0 (float32 store) or 3 or 5 (gated, as yalm_gemm).
