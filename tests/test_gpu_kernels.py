@@ -288,6 +288,21 @@ def test_gemm_of_every_tiling(M, N, Kd, epi):
     test_gemm_of_prompt_steps(M, N // 2 if epi == "gated" else N, Kd, epi, True)
 
 
+@pytest.mark.parametrize("M,N,tiling", [(200, 16400, 2), (150, 16400, 3), (300, 8208, 4), (150, 4112, 5)])
+def test_no_sum_is_a_chain_of_more_than_512_products(M, N, tiling):
+    """Tiles of 128 columns over 17 k tiles: the running sums of eight tiles, of eight and of one are added, whatever the depth of the ring.  The
+    first product of the first eight is -2^24 and of the second 2^24, beside which the others, 2^-7 each and less than half a unit of that together
+    in any instruction, are lost; the last tile's 64 stand alone and come to 1/2."""
+    from yalm_amd.ops import library
+    k, Kd = K(), 17 * 64
+    assert library.lib().yalm_gemm_bf16_dma_choice(M, N, Kd, 0, 0) == 10 + tiling
+    a, w = torch.full((M, Kd), 2.0 ** -3), torch.full((N, Kd), 2.0 ** -4)
+    a[:, 0], a[:, 512], w[:, 0], w[:, 512] = -2.0 ** 12, 2.0 ** 12, 2.0 ** 12, 2.0 ** 12
+    out = torch.full((M, N), float("nan"), device=DEV)
+    k.gemm(a.bfloat16().to(DEV), w.bfloat16().to(DEV), out, k.EPI_STORE_F32)
+    assert bool((out == 0.5).all()), out.unique()[:4]
+
+
 def test_gemm_of_a_prompt_step_is_the_same_with_and_without_k_slices():
     """A product in K slices agrees with the whole one within float32 rounding, and a launch repeats itself bit
     for bit."""

@@ -131,7 +131,8 @@ __global__ __launch_bounds__(512, 1) void gemm_stages_kernel(const bf16* __restr
                  : : "s"(at), "v"(off[i]), "s"(base), "s"((unsigned)(i * NW * 1024)) : "memory", "m0", "scc");
   };
 
-  // the running sums go into the whole ones every FOLD k tiles: sums of 512 products at a time round as little as the finest slices of K
+  // the running sums go into the whole ones every FOLD k tiles, the last ones included: no sum is a chain of more than 512 products and of one
+  // for every FOLD k tiles, which rounds as little as the finest slices of K
   f32x4 acc[FA][FB], run[FA][FB];
 #pragma unroll
   for (int a = 0; a < FA; ++a)
@@ -208,7 +209,10 @@ __global__ __launch_bounds__(512, 1) void gemm_stages_kernel(const bf16* __restr
     iteration(kt, std::true_type{});
     if (kt % FOLD == FOLD - 1) fold();
   }
-  for (; kt < nk; ++kt) iteration(kt, std::false_type{});
+  for (; kt < nk; ++kt) {
+    iteration(kt, std::false_type{});
+    if (kt % FOLD == FOLD - 1) fold();
+  }
   fold();
   wait_vmcnt<0>();                                 // nothing of this workgroup is on its way into LDS when it ends
 
