@@ -768,7 +768,7 @@ def test_decode_splits_over_rows_pages_and_heads():
                     if pages <= 4:
                         assert n == 1
                     if per > 512:
-                        assert n == (quarters if per < 768 else 1)
+                        assert n == (quarters if per < 768 or (ragged and pages > 64) else 1)
                     elif ragged and (per <= 128 or (per <= 256 and pages > 16)):
                         assert n == max(quarters, decode_splits(heads, kv, hd, B, pages))
                     elif per > 64:
@@ -797,3 +797,20 @@ def test_products_of_a_short_k_take_tiles_that_suit_them():
         choice = library.lib().yalm_gemm_bf16_dma_choice(M, N, K, 0, 0)
         assert 10 <= choice <= 15 and us[choice % 10] <= 1.1 * min(us), (M, N, K, choice)
     assert [library.lib().yalm_gemm_bf16_dma_choice(*a) for a in ((64, 64, 64, 0, 0), (65, 64, 72, 0, 0), (65, 64, 64, 0, 3))] == [-1, -1, -1]
+
+
+# us of the decode attention of bfloat16, 32 heads of 128 in 8 groups, by the number of splits: (rows, their bucket of pages, unequal): {splits: us}
+MANY_ROWS_US = [
+    ((96, 512, True), {1: 237.8, 4: 84.2}),          # one row of 24,000 tokens and 95 of 100 to 600
+    ((96, 128, True), {1: 90.0, 4: 50.5}),           # one of 8,000
+    ((96, 128, True), {1: 81.8, 4: 73.3}),           # eight of 6,000 and 88 of 100 to 600
+    ((96, 64, True), {1: 119.6, 4: 133.3}),          # 200 to 3,200 tokens
+    ((96, 64, True), {1: 41.4, 4: 46.9}),            # one of 2,500 and 95 of 100 to 600
+    ((96, 32, True), {1: 29.1, 4: 35.7}), ((128, 16, True), {1: 30.1, 4: 53.3}),
+    ((96, 16, False), {1: 64.3, 4: 82.5}), ((128, 32, False), {1: 167.1, 2: 182.3})]
+
+
+def test_decode_splits_of_many_rows_are_the_sooner_ones():
+    from yalm_amd.parts.attention import decode_splits
+    for (B, pages, ragged), us in MANY_ROWS_US:
+        assert us[decode_splits(32, 8, 128, B, pages, ragged)] == min(us.values()), (B, pages, ragged)

@@ -62,9 +62,12 @@ def decode_splits(n_heads, n_kv_heads, head_dim, B, max_pages, ragged=False, sha
         quarters = max(1, min((max_pages + 3) // 4, 4))
         # More workgroups than run at once: in quarters the last round is short, which pays while it is nearly empty; from half
         # a round on a split more is only another merge (96 rows of 1,000 tokens 70.2 in one, 82.1 in four; 80 of 3,000 158 and 169;
-        # 128 of 300 31.4, in two 43.2; of 200 to 1,000 tokens 96 rows 48.0 and 65.9).
+        # 128 of 300 31.4, in two 43.2; of 200 to 1,000 tokens 96 rows 48.0 and 65.9).  Of sequences of very unequal lengths the longest is then
+        # one workgroup's alone, its pages one behind the other while the others are long done: up to 64 pages it ends in time (96 rows of 200 to
+        # 3,200 tokens 119.6, in quarters 133.3; one of 2,500 and 95 of 100 to 600 41.4 and 46.9, one of 3,200 the same, one of 4,000 53.4
+        # and 47.2, eight of 4,000 59.9 and 62.4), beyond that not (one of 8,000 90.0 and 50.5, of 24,000 237.8 and 84.2, eight of 6,000 81.8 and 73.3).
         if per > RESIDENT_WORKGROUPS:
-            return quarters if own or 2 * per < 3 * RESIDENT_WORKGROUPS else 1
+            return quarters if own or 2 * per < 3 * RESIDENT_WORKGROUPS or (ragged and max_pages > 64) else 1
         if own or per > 64 or max_pages <= 4:
             even = max(1, min((max_pages + 3) // 4, TARGET_WORKGROUPS // per))
         else:
