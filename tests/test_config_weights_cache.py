@@ -814,3 +814,11 @@ def test_decode_splits_of_many_rows_are_the_sooner_ones():
     from yalm_amd.parts.attention import decode_splits
     for (B, pages, ragged), us in MANY_ROWS_US:
         assert us[decode_splits(32, 8, 128, B, pages, ragged)] == min(us.values()), (B, pages, ragged)
+
+
+def test_decode_splits_of_few_rows_deal_their_pages_evenly():
+    """By the bucket of pages, few rows of one KV group: times over the time in 16, 32 and 64 splits, in the mean of 5 to 16 steps."""
+    from yalm_amd.parts.attention import decode_splits
+    for pages, over in ((64, {15: 1.02, 16: 1.0}), (128, {22: 0.98, 24: 0.95, 32: 1.0}), (256, {31: 0.76, 32: 0.74, 64: 1.0})):
+        n = decode_splits(16, 1, 128, 4, pages)
+        assert over[n] == min(over.values()), (pages, n)

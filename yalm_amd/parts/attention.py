@@ -74,9 +74,13 @@ def decode_splits(n_heads, n_kv_heads, head_dim, B, max_pages, ragged=False, sha
             # Few rows: a wave's pages come one behind the other, 2.3 us each, and a split more costs the merge 0.15 us, which is
             # least at the root of 3.8 pages; three pages of eight a split at the least (one row of 500 tokens in two splits 8.5, in three 7.5,
             # of 1,000 in four 8.4, in six 7.5; three rows of 1,000 9.4 and 8.2; eight of 500 in two 9.2, in three 8.8).
+            # Beyond twelve the nearest multiple of eight, which deals a bucket's pages evenly to the waves (64 pages in 15 splits are 2 % slower than in 16, to
+            # 17 %, over 72 steps of eight shapes of heads; 128 in 22 3 % than in 24, 256 in 31 3 % than in 32).
             # A workgroup on three quarters of the units reads as fast as one on each (one row of 28,000: 24 splits 23.6, 32 24.9).
+            # One group for all heads is cut by the same rule (16 heads of 144, one row of 28,000 tokens in 40 22.9, in 110 and more 33.8).
             most = TARGET_WORKGROUPS // per if per > 8 else TARGET_WORKGROUPS * 3 // 4 // per
-            even = max(1, min((3 * max_pages + 7) // 8, math.isqrt(19 * max_pages // 5), most))
+            root = math.isqrt(19 * max_pages // 5)
+            even = max(1, min((3 * max_pages + 7) // 8, root if root <= 12 else (root + 3) // 8 * 8, most))
         # Sequences of very unequal lengths.  Where the workgroups stand two to a compute unit anyway, one split and
         # the rows in the order that pairs a long sequence with a short one; else splits of the longest sequence's
         # split size (the kernel cuts them so), enough of them that the long sequences' work spreads over the chip.  With a workgroup on more than
