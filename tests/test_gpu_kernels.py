@@ -223,10 +223,9 @@ def test_gemm_store_and_add(M, N, Kd, dtype, simple):
         k.FORCE_SIMPLE = False
 
 
-# (rows, columns or hidden width, K, epilogue): prompt-step shapes, one for every way the launcher of the 256-row
-# tiles goes: tiles of 256, 192 and 128 columns, whole rounds of 256x256 followed by 256x128 tiles for the remaining
-# columns (28,672 columns at 2,048 rows), K split over workgroups (few tiles), one, two and three k tiles (the
-# start and the end of the ring of LDS slots), rows and columns that end inside a tile, many row tiles.
+# (rows, columns or hidden width, K, epilogue): prompt-step shapes with one, two and three k tiles and many, rows and columns that end
+# inside a tile, many row tiles, with the workspace in which K may be split and without.  (Every way the launcher goes, asked for by
+# name: test_gemm_of_every_tiling.)
 PROMPT_GEMMS = [(2048, 6144, 192, "f32"), (2048, 4096, 256, "add"), (1000, 4100, 320, "bf16"),
                 (2048, 14336, 128, "gated"), (2048, 28672, 128, "f32"), (512, 4096, 4096, "add"),
                 (384, 1000, 2048, "gated"), (160, 4096, 2048, "f32"), (8192, 512, 64, "f32"), (300, 700, 128, "add"),
@@ -239,14 +238,14 @@ def test_gemm_of_prompt_steps(M, N, Kd, epi, with_workspace):
     k = K()
     from yalm_amd.parts.swiglu import interleave_gate_up
     a = rnd((M, Kd), 91, torch.bfloat16).to(DEV)
-    if epi == "gated":
+    if epi in ("gated", "gelu"):
         H = N
         wg = rnd((H, Kd), 92, torch.bfloat16, scale=1 / math.sqrt(Kd))
         wu = rnd((H, Kd), 93, torch.bfloat16, scale=1 / math.sqrt(Kd))
         w = interleave_gate_up(wg, wu).to(DEV)
         rows = w.shape[0]
         ad = a.double()
-        act_fn, epi_code = gate("gelu" if M == 384 else "silu")
+        act_fn, epi_code = gate("gelu" if M == 384 or epi == "gelu" else "silu")
         want = (act_fn(ad @ wg.to(DEV).double().T) * (ad @ wu.to(DEV).double().T)).cpu()
     else:
         w = rnd((N, Kd), 92, torch.bfloat16, scale=1 / math.sqrt(Kd)).to(DEV)
@@ -254,7 +253,7 @@ def test_gemm_of_prompt_steps(M, N, Kd, epi, with_workspace):
         want = (a.double() @ w.double().T).cpu()
     floats = k.gemm_workspace_floats(M, rows, Kd) if with_workspace else 0
     ws = torch.full((floats,), float("nan"), device=DEV) if floats else None
-    if epi == "gated":
+    if epi in ("gated", "gelu"):
         out = torch.empty((M, N), dtype=torch.bfloat16, device=DEV)
         k.gemm(a, w, out, epi_code, hidden=N, workspace=ws)
         close(out, want, torch.bfloat16, "gated", factor=2.0)
@@ -273,19 +272,44 @@ def test_gemm_of_prompt_steps(M, N, Kd, epi, with_workspace):
         close(out, want + res.double(), torch.float32, "residual add")
 
 
-# Every tiling of the launcher's plan (rows x columns), with every epilogue: rows and columns that end inside a tile, fewer k tiles than
-# the ring has stages, and whole rounds of 256 x 256 tiles with a second launch of each narrower tiling behind them.  In brackets
-# what the plan takes for plain products.
-@pytest.mark.parametrize("epi", ["f32", "bf16", "add", "gated"])
-@pytest.mark.parametrize("M,N,Kd", [
-    (513, 16416, 320),      # 256 x 256 or 192
-    (256, 16416, 192), (200, 16416, 1024),                                                # 256 x 128
-    (129, 16416, 1024), (150, 4096, 2240), (192, 28640, 64), (191, 4096, 7168),           # 192 x 128, the last one in slices of K
-    (193, 8224, 192), (383, 16416, 128), (129, 4096, 2048), (640, 4128, 1024),            # 128 x 128
-    (129, 96, 448), (385, 4128, 128), (255, 160, 2048), (150, 4128, 2048), (193, 32, 64),  # 64 x 128
-    (1100, 16416, 1024), (1000, 16416, 1024), (768, 28672, 512)])                         # two launches
-def test_gemm_of_every_tiling(M, N, Kd, epi):
-    test_gemm_of_prompt_steps(M, N // 2 if epi == "gated" else N, Kd, epi, True)
+# Every way of the launcher's plan, as yalm_gemm_bf16_dma_choice names it: the tilings whole and in slices of K, and whole rounds of 256 x 256
+# tiles with a second launch of each narrower tiling behind them; rows and columns that end inside a tile, fewer k tiles than the ring
+# has stages and many.  The first shape for products that are stored, the second for those added to the residual stream.
+EVERY_TILING = {
+    "256 x 256": (10, (257, 24608, 192), (257, 24608, 192)), "256 x 256 in slices": (30, (193, 16416, 5120), (129, 16416, 5120)),
+    "256 x 256, one k tile": (10, (2000, 6176, 64), (2000, 6176, 64)),
+    "256 x 192": (11, (257, 21920, 64), (257, 21920, 64)), "256 x 192 in slices": (21, None, (193, 16448, 3072)),
+    "256 x 128": (12, (193, 16416, 64), (193, 16416, 64)), "256 x 128 in slices": (42, (193, 5536, 5120), None),
+    "256 x 128 in three slices": (32, None, (193, 8224, 3072)), "192 x 128": (13, (129, 16448, 64), (129, 16448, 64)),
+    "192 x 128 in slices": (43, (129, 5408, 3072), (129, 5408, 3072)), "128 x 128": (14, (129, 10944, 64), (129, 10944, 64)),
+    "128 x 128 in slices": (44, (130, 32, 1536), (130, 32, 1536)), "64 x 128": (15, (129, 32, 64), (129, 32, 64)),
+    "64 x 128 in slices": (35, (129, 32, 1280), (129, 32, 1280)),
+    "and 256 x 128": (1012, (769, 22944, 768), (769, 22944, 960)), "and 192 x 128": (1013, (769, 21024, 512), (513, 28352, 768)),
+    "and 128 x 128": (1014, (769, 18848, 320), (513, 25536, 512)), "and 64 x 128": (1015, (513, 21824, 320), (769, 16416, 320))}
+
+
+@pytest.mark.parametrize("way,epi", [(way, epi) for way in sorted(EVERY_TILING) for epi in ("f32", "bf16", "add", "gated", "gelu", "biased")
+                                     if EVERY_TILING[way][2 if epi == "add" else 1] is not None])
+def test_gemm_of_every_tiling(way, epi):
+    from yalm_amd.ops import library
+    taken, stored, added = EVERY_TILING[way]
+    M, N, Kd = added if epi == "add" else stored
+    k = K()
+    choice = library.lib().yalm_gemm_bf16_dma_choice(M, N, Kd, k.gemm_workspace_floats(M, N, Kd), 1 if epi == "add" else 0)
+    assert choice == taken, choice
+    if epi != "biased":
+        return test_gemm_of_prompt_steps(M, N // 2 if epi in ("gated", "gelu") else N, Kd, epi, True)
+    from yalm_amd.parts.swiglu import interleave_gate_up
+    H, D = N // 2, 51
+    h, wg, wu = (rnd(size, s, torch.bfloat16, scale=f) for size, s, f in (((M, Kd), 91, 1.0), ((H, Kd), 92, Kd ** -0.5), ((H, Kd), 93, Kd ** -0.5)))
+    bg, bu, x, xb = rnd((H,), 94), rnd((H,), 95), rnd((M, D), 96), rnd((D,), 97)
+    hd, out, xd = h.to(DEV), torch.full((M, H), float("nan"), dtype=torch.bfloat16, device=DEV), x.to(DEV)
+    n = k.gemm_workspace_floats(M, N, Kd)
+    k.gemm_gated_bias(hd, interleave_gate_up(wg, wu).to(DEV), interleave_gate_up(bg[:, None], bu[:, None]).reshape(-1).contiguous().to(DEV), out, xd,
+                      xb.to(DEV), workspace=torch.full((n,), float("nan"), device=DEV) if n else None)
+    g, u = (hd.double() @ w.to(DEV).double().T + b.to(DEV).double() for w, b in ((wg, bg), (wu, bu)))
+    close(out, (R.gelu(g) * u).cpu(), torch.bfloat16, "biased", factor=2.0)
+    assert torch.equal(xd.cpu(), x + xb)
 
 
 @pytest.mark.parametrize("M,N,tiling", [(200, 16400, 2), (150, 16400, 3), (300, 8208, 4), (150, 4112, 5)])
@@ -375,7 +399,7 @@ def test_gemm_random_shapes(with_workspace):
 @pytest.mark.parametrize("M,H,D", [(1, 16, 64), (5, 176, 64), (70, 100, 96), (64, 1000, 264), (3, 14336, 128),
                                    (70, 100, 128), (300, 10300, 64), (260, 1000, 256), (7, 100, 192), (13, 7000, 128),
                                    (16, 13000, 64), (9, 3300, 320), (24, 100, 192), (61, 1000, 128),
-                                   (513, 12820, 64), (2048, 14336, 64)])   # whole rounds of 256x256 tiles + a launch of 256x128
+                                   (513, 12820, 64), (2048, 14336, 64)])   # 192 x 128 and 256 x 256 tiles
 @pytest.mark.parametrize("act", ACTS)
 def test_gemm_gated(M, H, D, dtype, simple, act):
     from yalm_amd.parts.swiglu import interleave_gate_up
