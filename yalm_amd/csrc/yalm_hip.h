@@ -14,12 +14,12 @@ int yalm_abi_version(void);
 
 // x[t, :] = float(table[tokens[t], :]); a negative token gives a row of zeros.
 // reference: copy_embedding_* (src/infer.cu:636-658)
+int yalm_embed(const void* table, int table_dtype, const int* tokens, float* out, int T, int D, int V,
+               hipStream_t stream);
 // x[t] = rmsnorm(float(table[tokens[t]])) with the weights w (float32 [D]), the same into kept (may be null): yalm_embed and yalm_rmsnorm in
 // one launch, with their bits.  D over 1,024 to 8,192, a multiple of 4, every pointer on 16 bytes; else YALM_ERR_ARG.
 int yalm_embed_norm(const void* table, int table_dtype, const int* tokens, const float* w, float eps, float* x, float* kept, int T, int D,
                     int V, hipStream_t stream);
-int yalm_embed(const void* table, int table_dtype, const int* tokens, float* out, int T, int D, int V,
-               hipStream_t stream);
 
 // out[r, :] = x[row(r), :] * rsqrt(mean(x^2) + eps) * w, row(r) = row_index ? row_index[r] : r.
 // x is the float32 residual stream; w may be float32 or bfloat16; out float32 or bfloat16.

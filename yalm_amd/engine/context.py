@@ -64,7 +64,9 @@ class Workspace:
 
 class StepContext:
     """mode: 'prefill' (sequences that start at position 0, whole prompts, packed)
-    or 'decode' (one token per sequence).  Device tensors, all int32:
+    or 'decode' (one token per sequence, no slot in two rows: Engine.step and step_from refuse a batch that names one twice.  The kernels
+    of such a step that carry state rest on it - the recurrences, the convolutions over time and the sinks read a slot's line and write it
+    back without a look at other rows -, and those of attention and its cache writes have been run on such rows only).  Device tensors, all int32:
       tokens[T], tok_seq[T] (row of the batch), tok_pos[T] (position in its sequence),
       seq_slot[B] (-1: padding row), seq_len[B] (length after this step), cu_seqlens[B+1].
     tables: prefill only; {maker's name: {key: int32 device tensor or host value}}, the index tables that parts

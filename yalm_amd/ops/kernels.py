@@ -1498,7 +1498,8 @@ def hgrn2_tiles_fit(d):
 
 def hgrn2_tiles(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, seq_tile0, n_tiles, out, n_heads, d, dv, eps, scratch):
     """hgrn2 for a step of prompts, a tile of 64 tokens at a time on the matrix cores in float32; seq_tile0 and scratch as for
-    gla_tiles."""
+    gla_tiles.  The scratch is 8 dp bytes a token and head (dp: hgrn2_tiles_fit(d), and the last tile of a sequence counts whole), 32 KB a
+    token with 32 heads of 128, of which hgrn2 needs none."""
     T, B = proj.shape[0], seq_slot.shape[0]
     N = 2 * n_heads * d + n_heads * dv
     dp = hgrn2_tiles_fit(d)

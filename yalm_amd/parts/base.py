@@ -10,11 +10,13 @@ it is in.  Kinds of parts and the methods each must have:
                  of its own and its prefix means nothing)
   mixer          cache_request() -> KVRequest | StateRequest | None, or {name: request}: a mixer made of several gets
                  the cache line (line, name) for each of them
-  input_filter   cache_request() as a mixer's; forward(h[T, dim], out[T, dim], ctx, line): what a sublayer reads in h's place
                  forward(h[T, dim], x_f32[T, dim], ctx, line, writes_cache): adds its output to x
                  optional: forward_to(h, y_f32[T, dim], ctx, line, writes_cache), which writes its output to y instead; a
                  `late_bias` (float32 [dim]) that its output lacks and that whoever reads y adds to every row (forward_to
                  is then told so with late_bias_taken=True)
+  input_filter   cache_request() as a mixer's; forward(h[T, dim], out[T, dim], ctx, line): what a sublayer reads in h's place;
+                 fuses_norm(norm, x, ctx): whether forward_prenorm(x_f32, norm, out, ctx, line) takes the norm of the stream in
+                 front of it in this step (the block then names it in that norm's `taken_by`, and nobody prepares its output)
   feed_forward   forward(h[T, dim], x_f32[T, dim], ctx): adds its output to x; optional: forward_to(h, y_f32, ctx)
   block          forward(x_f32[T, dim], ctx, line, writes_cache): one layer on the residual stream;
                  optional: a `next_norm` argument (the norm that reads the stream after this layer, whose
