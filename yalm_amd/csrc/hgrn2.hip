@@ -144,9 +144,10 @@ size_t hgrn2_tiles_lds(int dp) { return ((size_t)4 * GT * (dp + 4) + GNB * dp + 
 // A thread owns one channel of one block of 16 tokens.  LDS (155 KB at DP 128: a workgroup of eight waves a compute unit): four rows
 // a token, first q, 1 - f and f; then q F(block's start, t), (1 - f) F(t, block's end) and, for the halves of a block, q F(half's start, t)
 // in the second and (1 - f) F(t, half's end) in the first, and the same for the quarters of a half.
-// Bound by its phases one behind the other, 15 us a workgroup: the operands' way in 3, their gates 2, the scaled rows through LDS 4, the
-// products 2, the rest barriers and the way out (five prompts of 255 to 509 tokens, 32 heads of 128 x 128, 992 workgroups: 67 us, the
-// walk over the tiles behind it 83, the heads' norm 9; token by token 212 and 16).  Errors against 64 bits, relative, of
+// Bound by its phases one behind the other, 18 us a workgroup: the operands' way in 3, their gates 5 (the walk's own form, two exponentials and
+// two divisions), the scaled rows through LDS 4, the products 2, the rest barriers and the way out (five prompts of 255 to 509 tokens, 32 heads
+// of 128 x 128, 960 workgroups, inside a step: 92 us, the walk over the tiles behind it 100, the heads' norm 10; one behind the other with warm
+// caches 174 in all, token by token 228).  Errors against 64 bits, relative, of
 // the normed heads: ordinary gates 8.4e-8 (token by token 8.5e-8), gates close to one 1.0e-7 (8.2e-7), small ones 6.6e-8 (7.0e-8); of
 // the state 8.2e-8 (1.4e-7), 2.2e-7 (2.8e-6), 3.3e-8 (2.7e-8: there 1 - f is close to one and rounded, which the walk's f (S - v) + v is not).
 template <int DP>
