@@ -530,7 +530,7 @@ int launch_tiles(const bf16* A, const bf16* W, void* C, int M, int N, int K, Gat
 //  * below it, where a workgroup's few iterations stand behind each other's starts and ends, to 750 launches: 14 shapes of 512 to 32,000 weight
 //    rows and K of 64 to 960, `out` at least 0.3; errors 6 to 12 %, the picks 1 % slower in the mean and, but for one shape (2,048
 //    rows of 4,096 x 512), 12 % at worst.  The first fit gave nearly all of these tiles of 64 x 128: 2,048 rows of 28,672 x 128 81 us
-//    and now 54, 4,096 of 6,144 x 192 41 and 27, 1,100 of 24,000 x 256 49 and 32.
+//    and now 54, 4,096 of 6,144 x 192 41 and 27, 1,100 of 24,000 x 256 49 and 31.
 // Those launches were short bursts.  In the long
 // products of a prompt, layer after layer, the power the chip may take sets its clock, and a narrower tile moves more operands for a product:
 // `warm` is what a product of several rounds, or of more than 1,024 rows, takes longer then (six layers of 7B sizes with 1,536 tokens whose down
