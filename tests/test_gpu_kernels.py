@@ -880,6 +880,46 @@ def test_attn_prefill(n_heads, n_kv, hd, window, lens, dtype, simple):
     close(out, packed_attention_reference(q, kk, v, lens, n_heads, n_kv, hd, window), dtype, "prefill attention")
 
 
+@pytest.mark.parametrize("slices", [1, 3])
+@pytest.mark.parametrize("n_heads,n_kv,hd,rd,lens", [
+    (4, 2, 128, 128, [1]), (8, 2, 128, 128, [33]), (8, 2, 128, 64, [64, 1, 15]), (3, 1, 128, 0, [16, 17, 48, 49, 63]),
+    (2, 2, 64, 64, [64]), (6, 3, 64, 6, [31, 32, 1, 64]), (4, 4, 64, 0, [2, 65 - 1])])
+def test_attn_tile(n_heads, n_kv, hd, rd, lens, slices):
+    """Prompts of one tile each in one launch: the bits of the rotation kernel with the attention kernel behind it, in the result
+    and in the pages of the cache, at both ends of a tile and of a wave's 16 queries; a sequence without a slot writes no page."""
+    k = K()
+    PAGE = k.PAGE
+    B, T = len(lens), sum(lens)
+    Q, KV = n_heads * hd, n_kv * hd
+    parts = torch.stack([rnd((T, Q + 2 * KV), 40 + s) for s in range(slices)]).to(DEV)
+    qkv = parts[0] if slices == 1 else parts.reshape(-1)
+    table = make_table(PAGE, hd, rd, 10000.0).to(DEV) if rd else None
+    cu, tile0 = np.concatenate([[0], np.cumsum(lens)]), np.arange(B + 1)
+    seq, pos = np.repeat(np.arange(B), lens), np.concatenate([np.arange(n) for n in lens])
+    slots = [B - b for b in range(B)]
+    if B > 2:
+        slots[1] = -1
+    bt = torch.full((B + 1, 2), -1, dtype=torch.int32)
+    bt[1:, 0] = torch.from_numpy(np.random.default_rng(5).permutation(B + 3)[:B].astype(np.int32))
+    bt = bt.to(DEV)
+
+    def pages():
+        return (torch.zeros((B + 3, n_kv, PAGE, hd), dtype=torch.bfloat16, device=DEV),
+                torch.zeros((B + 3, n_kv, hd, PAGE), dtype=torch.bfloat16, device=DEV))
+    (kp0, vp0), (kp1, vp1) = pages(), pages()
+    q = torch.empty((T, Q), dtype=torch.bfloat16, device=DEV)
+    ks = torch.full((B, n_kv, PAGE, hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    vs = torch.full((B, n_kv, hd, PAGE), float("nan"), dtype=torch.bfloat16, device=DEV)
+    want, got = torch.empty_like(q), torch.full_like(q, float("nan"))
+    k.rope_kv_write(qkv, q, ks, vs, i32(tile0), kp0, vp0, bt, 2, i32(seq), i32(pos), i32(slots), i32(lens), table, n_heads, n_kv,
+                    hd, rd, slices=slices)
+    k.attn_prefill(q, ks, vs, want, i32(cu), i32(tile0), i32(seq), i32(pos), n_heads, n_kv, hd, 0)
+    assert k.attn_tile_fits(qkv, got, kp1, vp1, hd, 0) and not k.attn_tile_fits(qkv, got, kp1, vp1, hd, PAGE - 1)
+    k.attn_tile(qkv, got, kp1, vp1, bt, 2, i32(cu), i32(slots), table, n_heads, n_kv, hd, rd, slices=slices)
+    assert torch.equal(got, want)
+    assert torch.equal(kp0, kp1) and torch.equal(vp0, vp1) and kp0.abs().sum() > 0
+
+
 def masked_attention_float64(q, k, v, n_heads, n_kv, hd, window, bias=None):
     """softmax(q k^T / sqrt(hd) + mask) v for one sequence, all positions at once (float64).  bias ([n_heads,
     distances], optional): bias[h, min(i - j, distances - 1)] is added to the score of query i and key j."""

@@ -175,6 +175,15 @@ int yalm_rope_kv_write_tiles(const float* qkv, void* q_out, void* k_stage, void*
                              int n_kv_heads, int head_dim, int rotary_dim, int n_pages, int page_layout, int slices,
                              int dtype, hipStream_t stream);
 
+// yalm_rope_kv_write and yalm_attn_prefill in one launch, for a step whose prompts are one tile each (n_tiles = B: at most 64
+// tokens a sequence): qkv [slices][T][q + 2 kv] float32 in, out [T, n_heads, hd] bfloat16, keys and values to the first page of each
+// sequence.  bfloat16, heads of 64 and 128, qkv, out and pages on 16 bytes; refuses (YALM_ERR_ARG) anything else.  All keys up
+// to a query's own are seen: for windows of 64 and more, no shape on the scores.
+int yalm_attn_tile(const float* qkv, void* out, void* k_pages, void* v_pages, const int* block_table, int table_stride,
+                   const int* cu_seqlens, const int* seq_slot, const float* cos_sin, int n_positions, int T, int B, int n_tiles,
+                   int n_heads, int n_kv_heads, int head_dim, int rotary_dim, int n_pages, int page_layout, int slices,
+                   hipStream_t stream);
+
 // Causal attention of a step's tokens over the same step's keys (sequences that
 // start at position 0), packed without padding.  window 0 = all keys.
 //   q, out [T, n_heads, hd]; k_stage, v_stage: the staging area rope_kv_write filled

@@ -648,6 +648,57 @@ def rope_kv_write_tiles(qkv, q_out, k_stage, v_stage, cu_seqlens, seq_tile0, k_p
     return True
 
 
+TILE_HEAD_DIMS = (64, 128)      # head sizes that attn_tile is built for
+
+
+def attn_tile_fits(qkv, out, k_pages, v_pages, head_dim, window):
+    """Whether attn_tile takes a step of sequences of one tile each: bfloat16, a window that hides none of a tile's keys, and operands
+    on 16 bytes."""
+    return out.dtype == torch.bfloat16 and not FORCE_SIMPLE and head_dim in TILE_HEAD_DIMS and (window <= 0 or window >= PAGE) and \
+        (qkv.data_ptr() | out.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0
+
+
+def attn_tile(qkv, out, k_pages, v_pages, block_table, ring_pages, cu_seqlens, seq_slot, cos_sin, n_heads, n_kv_heads, head_dim,
+              rotary_dim, slices=1, layout=None):
+    """What rope_kv_write and attn_prefill do with a step of whole prompts of at most 64 tokens each, in one launch: qkv float32
+    (as rope_kv_write takes it) is rotated, keys and values go to the first page of each sequence, and out (bfloat16 [T, n_heads *
+    head_dim]) is the causal attention of every sequence over its own keys.  attn_tile_fits says which steps are taken.  The caller
+    sees to it that no sequence of cu_seqlens is longer than PAGE."""
+    _check_heads(n_heads, n_kv_heads, head_dim)
+    T = out.shape[0]
+    Q, KV = n_heads * head_dim, n_kv_heads * head_dim
+    if slices == 1 and qkv.dim() == 2:
+        p_qkv = _need(qkv, "qkv", torch.float32, (T, Q + 2 * KV))
+    else:
+        p_qkv = _need(qkv, "qkv", torch.float32, (None,))
+        if slices < 1 or qkv.numel() < slices * T * (Q + 2 * KV):
+            raise ValueError("qkv holds %d floats, %d slices of %d rows need %d"
+                             % (qkv.numel(), slices, T, slices * T * (Q + 2 * KV)))
+    p_o = _need(out, "out", torch.bfloat16, (T, Q))
+    B = seq_slot.shape[0]
+    n_pages = k_pages.shape[0]
+    p_kp = _need(k_pages, "k_pages", torch.bfloat16, (n_pages, n_kv_heads, PAGE, head_dim))
+    p_vp = _need(v_pages, "v_pages", torch.bfloat16, (n_pages, n_kv_heads, head_dim, PAGE))
+    p_bt = _need(block_table, "block_table", torch.int32, (None, None))
+    stride = block_table.shape[1]
+    if ring_pages <= 0 or ring_pages > stride:
+        raise ValueError("ring_pages %d does not fit the block table (%d columns)" % (ring_pages, stride))
+    p_cu = _need(cu_seqlens, "cu_seqlens", torch.int32, (B + 1,))
+    p_sl = _need(seq_slot, "seq_slot", torch.int32, (B,))
+    n_pos, p_cs = 0, None
+    if cos_sin is not None:
+        if rotary_dim % 2 != 0 or rotary_dim > head_dim or rotary_dim <= 0:
+            raise ValueError("rotary_dim %d does not fit head_dim %d" % (rotary_dim, head_dim))
+        n_pos = cos_sin.shape[0]
+        p_cs = _need(cos_sin, "cos_sin", torch.float32, (n_pos, rotary_dim // 2, 2))
+    else:
+        rotary_dim = 0
+    library.check(library.lib().yalm_attn_tile(
+        p_qkv, p_o, p_kp, p_vp, p_bt, stride, p_cu, p_sl, p_cs, n_pos, T, B, B, n_heads, n_kv_heads, head_dim, rotary_dim, n_pages,
+        _layout(layout, head_dim), int(slices), _stream()), "attn_tile")
+    return out
+
+
 def prefill_tile_order(n_tokens):
     """The order in which attn_prefill should take the tiles of a step whose sequences bring
     n_tokens tokens each: every second 64-token tile of a sequence (its workgroup covers the

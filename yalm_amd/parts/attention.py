@@ -308,9 +308,32 @@ class GQAttention(Part):
         else:
             qkv = ws.get("attn.qkv", (T, n_qkv), torch.float32)
             self._gemm(ctx, h, self.wqkv, qkv, kernels.EPI_STORE_F32)
-        q = ws.get("attn.q", (T, self.q_dim), act)
         group = ctx.cache.group_of(line)
         k_pages, v_pages = group.line_pages(line)
+        o = ws.get("attn.o", (T, self.q_dim), act)
+        # short prompts, every sequence one tile of keys that nobody reads again in this step: rotation, cache write and attention
+        # are one kernel
+        if prefill and writes_cache and ctx.tables["kv_tiles"]["n_tiles"] == ctx.seq_slot.shape[0] and not self.sinks \
+                and self.score_bias is None and not ctx.line_is_shared(line) \
+                and kernels.attn_tile_fits(qkv, o, k_pages, v_pages, self.head_dim, self.window):
+            kernels.attn_tile(qkv, o, k_pages, v_pages, group.table, group.ring_pages, ctx.cu_seqlens, ctx.seq_slot, pos.table,
+                              self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices)
+        else:
+            self._rotate_and_attend(qkv, slices, o, ctx, group, line, k_pages, v_pages, writes_cache)
+        ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.q_dim) if prefill else None
+        if ready is not None:                     # the product's K slices (or the product) are added with the next norm behind
+            nw2, eps2, h2, ws2 = ready
+            kernels.gemm_add_norm(o, self.wo, x, nw2, eps2, h2, ws2)
+            ctx.normed[id(emit_for)] = (h2, None, None)
+        else:
+            self._gemm(ctx, o, self.wo, x, kernels.EPI_ADD_F32)
+
+    def _rotate_and_attend(self, qkv, slices, o, ctx, group, line, k_pages, v_pages, writes_cache):
+        """From the q/k/v product's sums (or its K slices) to the heads' results o, with keys and values staged for the
+        step's own attention (whole prompts) or read from the cache."""
+        T, act, ws, pos = o.shape[0], o.dtype, ctx.ws, self.position
+        prefill = ctx.mode == "prefill"
+        q = ws.get("attn.q", (T, self.q_dim), act)
         if prefill:
             # the step's own keys and values in page format; a line that later entries read
             # keeps them for those entries
@@ -334,7 +357,6 @@ class GQAttention(Part):
             kernels.rope_kv_write(qkv, q, None, None, None, None, None, None, 0, ctx.tok_seq, ctx.tok_pos,
                                   ctx.seq_slot, ctx.seq_len, pos.table, self.n_heads, self.n_kv_heads, self.head_dim,
                                   pos.rotary_dim, slices=slices)
-        o = ws.get("attn.o", (T, self.q_dim), act)
         if prefill:
             lse = ws.get("attn.lse", (T, self.n_heads), torch.float32) if self.sinks else None
             # with sinks the result is kept unrounded too, so that the row with the sinks mixed in is rounded once
@@ -351,10 +373,3 @@ class GQAttention(Part):
                                       self.n_heads, pos.rotary_dim, self.window, src_f32=o32)
         else:
             self._decode_attention(q, o, ctx, group, line, k_pages, v_pages, writes_cache)
-        ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.q_dim) if prefill else None
-        if ready is not None:                     # the product's K slices (or the product) are added with the next norm behind
-            nw2, eps2, h2, ws2 = ready
-            kernels.gemm_add_norm(o, self.wo, x, nw2, eps2, h2, ws2)
-            ctx.normed[id(emit_for)] = (h2, None, None)
-        else:
-            self._gemm(ctx, o, self.wo, x, kernels.EPI_ADD_F32)
