@@ -329,6 +329,34 @@ def test_a_sequence_at_its_first_token_beside_sequences_that_go_on(folders, name
         helpers.check_logits(np.stack(rows[key]), want, dtype, "%s %s joined at position 0, sequence %s" % (name, dtype, key))
 
 
+@pytest.mark.parametrize("lens", [[1], [16], [17], [9, 7], [5, 1, 11], [64], [65, 64, 3]])
+@pytest.mark.parametrize("name", ["tiny_long", "small_windowed", "tiny_mistral"])
+def test_short_prompts_and_the_steps_behind_them(folders, name, lens):
+    """bfloat16 prompts on both sides of 16 tokens in all (up to there the products prepare the norms) and of 64 a sequence (up to
+    there the attention takes the product's sums), with a head that has the latter's sizes and one that has not, a window that
+    hides keys of a tile and one that does not; the steps behind them read what the prompts have left in the cache."""
+    engine = make_engine(folders, name, "bfloat16", max_tokens=1024)
+    poison = poison_free_pages(engine)
+    lens = [min(n, tiny_configs.ALL[name]["max_position_embeddings"] - 3) for n in lens]
+    requests = [r[1] for r in sorted(helpers.random_requests(tiny_configs.ALL[name], [n + 3 for n in lens], seed=31).items())]
+    slots = engine.start(len(lens))
+    poison(0)
+    first = engine.step(slots, [r[:n] for r, n in zip(requests, lens)], [list(range(n)) for n in lens]).cpu().numpy()
+    rows, at = [], 0
+    for n in lens:
+        rows.append(list(first[at:at + n]))
+        at += n
+    for k in range(3):
+        poison(k + 1)
+        out = engine.step(slots, [[r[n + k]] for r, n in zip(requests, lens)]).cpu().numpy()
+        for i in range(len(lens)):
+            rows[i].append(out[i])
+    engine.release(slots)
+    for i, r in enumerate(requests):
+        helpers.check_logits(np.stack(rows[i]), helpers.plain_logits(folders[name], tuple(r), "bfloat16"), "bfloat16",
+                             "%s prompts %s, sequence %d" % (name, lens, i))
+
+
 def test_a_step_whose_widest_buffer_would_pass_the_checked_size_is_refused(folders):
     from yalm_amd.engine.engine import StepError
     engine = make_engine(folders, "tiny_llama", "float32", max_tokens=1024)

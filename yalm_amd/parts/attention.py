@@ -189,8 +189,8 @@ class GQAttention(Part):
         if not hasattr(norm, "fused") or self.head_dim % 16:
             return False
         T = x.shape[0]
-        if ctx.mode == "prefill":             # takes the norm's output where the product before has left it
-            return kernels.can_add_norm(T, self.dim, self.wo.dtype)
+        if ctx.mode == "prefill":             # takes the norm where the product before has left or prepared it
+            return kernels.can_add_norm(T, self.dim, self.wo.dtype) or kernels.can_chain(T, self.dim, self.wo.dtype)
         if ctx.mode != "decode":
             return False
         if self.wo.dtype == torch.float32:
@@ -201,10 +201,12 @@ class GQAttention(Part):
         """A decode step from the residual stream: norm, q/k/v, rotation and cache write in
         one kernel, attention over the cache, output projection added to x (which may
         prepare the activations of the next norm, emit_for)."""
-        if ctx.mode == "prefill":                 # whole prompts: the norm, unless its output is ready, then the plain way
+        if ctx.mode == "prefill":                 # whole prompts: the norm, unless its output is ready or prepared, then the plain way
             src = ctx.normed.pop(id(norm), None)
             if src is not None and src[1] is None:
                 h = src[0]
+            elif src is not None and kernels.can_chain(x.shape[0], self.dim, self.wo.dtype):
+                return self.forward(src[0], x, ctx, line, writes_cache, emit_for=emit_for, scale_from=src[1:])
             else:
                 h = ctx.ws.get("block.h", (x.shape[0], self.dim), ctx.act_dtype)
                 norm.forward(x, h, ctx)
@@ -290,7 +292,9 @@ class GQAttention(Part):
                             score_bias=self.score_bias,
                             counters=decode_counters(ctx, T, self.n_heads, self.n_kv_heads, n_splits))
 
-    def forward(self, h, x, ctx, line, writes_cache=True, emit_for=None):
+    def forward(self, h, x, ctx, line, writes_cache=True, emit_for=None, scale_from=None):
+        """scale_from: h is a norm that is prepared and not finished (a step of at most CHAIN_MAX_ROWS tokens); the product's
+        sums are scaled row by row."""
         T = h.shape[0]
         act = h.dtype
         ws = ctx.ws
@@ -307,7 +311,10 @@ class GQAttention(Part):
             slices = kernels.gemm_partial(h, self.wqkv, qkv)
         else:
             qkv = ws.get("attn.qkv", (T, n_qkv), torch.float32)
-            self._gemm(ctx, h, self.wqkv, qkv, kernels.EPI_STORE_F32)
+            if scale_from is not None:
+                kernels.gemm_chain(h, self.wqkv, qkv, kernels.EPI_STORE_F32, scale_from=scale_from)
+            else:
+                self._gemm(ctx, h, self.wqkv, qkv, kernels.EPI_STORE_F32)
         group = ctx.cache.group_of(line)
         k_pages, v_pages = group.line_pages(line)
         o = ws.get("attn.o", (T, self.q_dim), act)
@@ -320,8 +327,13 @@ class GQAttention(Part):
                               self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices)
         else:
             self._rotate_and_attend(qkv, slices, o, ctx, group, line, k_pages, v_pages, writes_cache)
-        ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.q_dim) if prefill else None
-        if ready is not None:                     # the product's K slices (or the product) are added with the next norm behind
+        emit = self._emit_args(emit_for, ctx, T, self.dim) if prefill and kernels.can_chain(T, self.q_dim, act) else None
+        ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.q_dim) if prefill and emit is None else None
+        if emit is not None:                      # up to 16 tokens: the product prepares the next norm, as in a decode step
+            nw2, xn2, ss2, eps2 = emit
+            kernels.gemm_chain(o, self.wo, x, kernels.EPI_ADD_F32, emit=(nw2, xn2, ss2))
+            ctx.normed[id(emit_for)] = (xn2, ss2, eps2)
+        elif ready is not None:                   # the product's K slices (or the product) are added with the next norm behind
             nw2, eps2, h2, ws2 = ready
             kernels.gemm_add_norm(o, self.wo, x, nw2, eps2, h2, ws2)
             ctx.normed[id(emit_for)] = (h2, None, None)

@@ -158,7 +158,7 @@ class Part:
         from ..ops import kernels
         if emit_for is None or not hasattr(emit_for, "fused") or width >= 16384:
             return None
-        if ctx.mode != "decode" or not kernels.can_chain(T, width, ctx.act_dtype):
+        if ctx.mode not in ("decode", "prefill") or not kernels.can_chain(T, width, ctx.act_dtype):
             return None
         import torch
         nw, eps = emit_for.fused()

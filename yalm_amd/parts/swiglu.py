@@ -71,8 +71,8 @@ class SwiGLU(Part):
         if not hasattr(norm, "fused") or ctx.mode not in ("decode", "prefill") or self.unit is not None:
             return False
         T = x.shape[0]
-        if ctx.mode == "prefill":             # takes the norm's output where the product before has left it
-            return kernels.can_add_norm(T, self.dim, self.w_down.dtype)
+        if ctx.mode == "prefill":             # takes the norm where the product before has left or prepared it
+            return kernels.can_add_norm(T, self.dim, self.w_down.dtype) or kernels.can_chain(T, self.dim, self.w_down.dtype)
         if self.w_down.dtype == torch.float32:
             return kernels.fuse_norm_pays(T, self.dim, torch.float32, self.w_gate_up.shape[0], gate=True)
         return kernels.can_chain(T, self.dim, self.w_down.dtype) or kernels.can_add_norm(T, self.dim, self.w_down.dtype)
