@@ -182,6 +182,24 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Two of block_sum's sums at once, the same bits, with barriers that leave loads in flight.  `red` holds NW pairs.
+template <int NW>
+__device__ __forceinline__ float2 block_sum2(float a, float b, float2* red) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if (NW == 1) return make_float2(a, b);
+  lds_barrier();
+  if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = make_float2(a, b);
+  lds_barrier();
+  float2 s = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    s.x += red[i].x;
+    s.y += red[i].y;
+  }
+  return s;
+}
+
 // compute units of the current device (asked once: this library drives one device a process)
 inline int compute_units() {
   static int n = 0;

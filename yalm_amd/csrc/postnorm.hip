@@ -22,27 +22,44 @@ __global__ __launch_bounds__(ROW_THREADS) void cast_kernel(const float* __restri
 // next_w the norm that reads the stream next, h[r] = T(x[r] * rsqrt(mean(x[r]^2) + next_eps) * next_w); with PAIR it has the
 // bits of the norm's own kernel (next_vec: rms_row_vec; the row goes through LDS to the threads that sum it there).  Bound by memory in a
 // prompt (x, y, y2 once each way: a second launch for y2 and a norm kernel behind it would read and write x twice more:
-// 1,909 rows of 4,096 24 + 24 + 10 -> 42 us), by the launch in a decode step (three of 4.6 us -> one of 6.5).
+// 1,909 rows of 4,096 24 + 24 + 10 -> 42 us), by the launch in a decode step (three of 4.6 us -> one of 6.5).  Rows of up to 4,096
+// elements keep four a thread, and everything is asked for at once: 1,909 rows 38.5 -> 33.1 us (137 MB), 5 rows 6.5 -> 5.0.
 template <typename W, typename T, int NT, int PER, bool PAIR>
 __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ y, const W* __restrict__ w,
                                                       const float* __restrict__ y2, const W* __restrict__ w2, float eps,
                                                       float* __restrict__ x, T* __restrict__ h, const float* __restrict__ next_w,
                                                       float next_eps, bool next_vec, int D) {
-  // PER > 0: the row fits PER values a thread; y is read once and the new x stays in registers for the second norm
+  // PER > 0: the row fits PER values a thread; y is read once and the new x stays in registers for the second norm.  All that the
+  // row needs is asked for in front of its sums, and the barriers of both sums, which are one, leave it in flight
+  __shared__ float2 red2[NT / WAVE];
   __shared__ float red[NT / WAVE];
   const size_t row = (size_t)blockIdx.x * D;
-  float keep[PER > 0 ? PER : 1], keep2[PER > 0 && PAIR ? PER : 1];
+  constexpr int N = PER > 0 ? PER : 1, N2 = PER > 0 && PAIR ? PER : 1;
+  float keep[N], keep2[N2], had[N], nw[N];
+  W wk[N], wk2[N2];
   float ss = 0.f, sp = 0.f;
   if (PER > 0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
       keep[j] = i < D ? y[row + i] : 0.f;
+      if constexpr (PAIR) keep2[j] = i < D ? y2[row + i] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = min((int)threadIdx.x + j * NT, D - 1);
+      had[j] = x[row + i];
+      wk[j] = w[i];
+      if constexpr (PAIR) wk2[j] = w2[i];
+    }
+    if (next_w != nullptr) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) nw[j] = next_w[min((int)threadIdx.x + j * NT, D - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
       ss += keep[j] * keep[j];
-      if constexpr (PAIR) {
-        keep2[j] = i < D ? y2[row + i] : 0.f;
-        sp += keep2[j] * keep2[j];
-      }
+      if constexpr (PAIR) sp += keep2[j] * keep2[j];
     }
   } else {
     for (int i = threadIdx.x; i < D; i += NT) {
@@ -51,17 +68,16 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
       if constexpr (PAIR) sp += y2[row + i] * y2[row + i];
     }
   }
-  ss = block_sum<NT / WAVE>(ss, red);
-  if constexpr (PAIR) sp = block_sum<NT / WAVE>(sp, red);
-  const float scale = 1.0f / sqrtf(ss / (float)D + eps), scale_p = PAIR ? 1.0f / sqrtf(sp / (float)D + eps) : 0.f;
+  const float2 both = block_sum2<NT / WAVE>(ss, sp, red2);
+  const float scale = 1.0f / sqrtf(both.x / (float)D + eps), scale_p = PAIR ? 1.0f / sqrtf(both.y / (float)D + eps) : 0.f;
   float ss2 = 0.f;
   if (PER > 0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
       if (i < D) {
-        float v = x[row + i] + keep[j] * scale * to_f32(w[i]);
-        if constexpr (PAIR) v += keep2[j] * scale_p * to_f32(w2[i]);
+        float v = had[j] + keep[j] * scale * to_f32(wk[j]);
+        if constexpr (PAIR) v += keep2[j] * scale_p * to_f32(wk2[j]);
         x[row + i] = v;
         keep[j] = v;
         ss2 += v * v;
@@ -92,7 +108,7 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
-      if (i < D) h[row + i] = from_f32<T>(keep[j] * scale2 * next_w[i]);
+      if (i < D) h[row + i] = from_f32<T>(keep[j] * scale2 * nw[j]);
     }
   } else {
     for (int i = threadIdx.x; i < D; i += NT) h[row + i] = from_f32<T>(x[row + i] * scale2 * next_w[i]);   // its own stores
@@ -336,6 +352,7 @@ static int norm_add_launch(const float* y, const void* w, const float* y2, const
                                                           next_vec, D)
   const bool next_vec = rms_row_vec(x, h, D);
   if (D < 2048) NA(256, 8);
+  else if (D <= 4096) NA(1024, 4);
   else if (D <= 8192) NA(1024, 8);
   else NA(1024, 0);
 #undef NA
