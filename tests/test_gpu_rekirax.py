@@ -155,6 +155,32 @@ def test_packing_kernel_of_few_tokens(H, G, d, dv, head_norm):
         assert torch.allclose(a, b, rtol=2e-6, atol=2e-6) and torch.equal(a != 0, b != 0)
 
 
+# Four elements a thread (40 rows) against a workgroup that holds the row in LDS (20): rows at both ends of the kernel's sizes, heads that divide a
+# round of 1,024 elements (their angles asked for once) and that do not
+@pytest.mark.parametrize("H,G,d,dv,head_norm,rot", [(6, 1, 128, 128, False, 64), (6, 1, 128, 132, False, 128), (48, 8, 128, 128, True, 64),
+                                                    (10, 2, 96, 96, False, 64), (14, 2, 100, 60, False, 100), (64, 16, 64, 64, True, 6), (1, 1, 4, 4, False, 2)])
+def test_packing_kernel_four_elements_a_thread(H, G, d, dv, head_norm, rot):
+    from yalm_amd.ops import kernels
+    T, ring, pad = 40, 2, (max(d, dv) + 15) // 16 * 16
+    raw = randn(T, H * d + G * (d + dv), seed=H + d).to(DEV)
+    wq, wk = (1 + randn(n, seed=s, scale=0.2).to(DEV) for s, n in ((1, d if head_norm else H * d), (2, d if head_norm else G * d)))
+    angles = randn(128, rot // 2, seed=4)
+    cos_sin = torch.stack([angles.cos(), angles.sin()], dim=-1).contiguous().to(DEV)
+    table = torch.arange(T * ring, dtype=torch.int32, device=DEV).reshape(T, ring)
+    pos = [(5 * t) % 128 for t in range(T)]
+    out = []
+    for cut in ([(0, 40)], [(0, 20), (20, 40)]):
+        q = torch.full((T, H * pad), float("nan"), device=DEV)
+        kp, vp = torch.zeros(T * ring, G, 64, pad, device=DEV), torch.zeros(T * ring, G, pad, 64, device=DEV)
+        for lo, hi in cut:
+            kernels.qkv_pack(raw[lo:hi], None, wq, wk, 1e-5, None, 1.7, None, 0, None, q[lo:hi], None, None, None, kp, vp, table, ring,
+                             i32(np.arange(hi - lo)), i32(pos[lo:hi]), i32(np.arange(lo, hi)), i32([p + 1 for p in pos[lo:hi]]), H, G, d, dv, pad,
+                             head_norm=head_norm, cos_sin=cos_sin, rot_dims=rot)
+        out.append((q, kp, vp))
+    for a, b in zip(*out):       # the norms' sums in another order: a few roundings of 2^-24 of elements up to 12, two of which a rotation adds
+        assert torch.allclose(a, b, rtol=0, atol=8e-6) and torch.equal(a != 0, b != 0)
+
+
 # The same with the middle in the first product's epilogue: one to 16 rows (K a multiple of 64 and not), to 128, tiles of 128 rows,
 # larger tiles, K in slices and whole; hidden values that end inside a block; streams narrower and wider than what one
 # element a thread covers; and the general kernels

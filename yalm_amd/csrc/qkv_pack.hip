@@ -20,7 +20,8 @@
 namespace {
 // a row of a few hundred numbers takes 256 threads, a real model's thousands 1,024 (a decode step has few tokens, and a
 // thread's loads wait for each other's results in turn: the fewer rounds the better).  Few tokens are dealt to several workgroups each
-// (blockIdx.y), which all read the row and form its sums and write a share of the results (8 tokens of 6,144 numbers 10.1 -> 8.2 us).
+// (blockIdx.y), which all read the row and form its sums and write a share of the results (8 tokens of 6,144 numbers 10.1 -> 8.2 us).  What a thread's
+// first results need beside the row is asked for in front of the sums, which share their barriers (5 tokens 7.7 -> 7.4).
 template <typename T, int PACK_THREADS>
 __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
     const float* __restrict__ qkv, long qkv_row, const float* __restrict__ bias, const float* __restrict__ w_q,
@@ -32,7 +33,7 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
     int n_kv_heads, int d, int dv, int pad, int n_pages, int page_layout, T* __restrict__ v_rows, int head_norm,
     int v_from_k, const float2* __restrict__ cos_sin, int rot_dims, int n_positions) {
   extern __shared__ float row[];                  // [Q + K + V], then a factor for every query and key head
-  __shared__ float red[PACK_THREADS / WAVE];
+  __shared__ float2 red[PACK_THREADS / WAVE];
   const int t = blockIdx.x, tid = threadIdx.x, part = blockIdx.y, parts = gridDim.y;
   const int Q = n_heads * d, K = n_kv_heads * d, V = n_kv_heads * dv, N = Q + K + (v_from_k ? 0 : V);
   float* head_f = row + N;                        // head_norm: 1 / rms of each query head, then of each key head
@@ -68,9 +69,27 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
   for (int k = 0; k < AHEAD; ++k)
     if (tid + k * PACK_THREADS < N) take(tid + k * PACK_THREADS, v[k]);
   for (int i = tid + AHEAD * PACK_THREADS; i < N; i += PACK_THREADS) take(i, src[i] + (bias != nullptr ? bias[i] : 0.f));
-  sq = block_sum<PACK_THREADS / WAVE>(sq, red);
-  sk = block_sum<PACK_THREADS / WAVE>(sk, red);
-  __syncthreads();
+  // the norm weights and the rotation of this thread's first query and key come while the sums are formed
+  const float2* cs = rot_dims > 0 ? cos_sin + (size_t)min(max(pos, 0), n_positions - 1) * (rot_dims / 2) : nullptr;
+  struct Ahead {
+    float w, w_other;                             // of the element, and of the other one of its pair
+    float2 c;
+  };
+  auto ask = [&](const float* w, int head, int e) {
+    Ahead a = {1.0f, 1.0f, make_float2(1.0f, 0.0f)};
+    if (e < d) {
+      const bool turned = e < rot_dims;
+      if (w != nullptr) a.w = w[head_norm ? e : head * d + e];
+      if (w != nullptr && turned) a.w_other = w[head_norm ? e ^ 1 : head * d + (e ^ 1)];
+      if (turned) a.c = cs[e >> 1];
+    }
+    return a;
+  };
+  const int first = part * PACK_THREADS + tid, step = parts * PACK_THREADS;
+  Ahead aq = ask(w_q, first / pad, first < n_heads * pad ? first % pad : d), ak = ask(w_k, first / pad, first < n_kv_heads * pad ? first % pad : d);
+  const float2 both = block_sum2<PACK_THREADS / WAVE>(sq, sk, red);
+  sq = both.x;
+  sk = both.y;
   if (head_norm) {                                // a wave a head: the sum of its squares
     for (int hh = tid / WAVE; hh < n_heads + n_kv_heads; hh += PACK_THREADS / WAVE) {
       float s = 0.f;
@@ -80,22 +99,21 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
     }
     __syncthreads();
   }
-  const float2* cs = rot_dims > 0 ? cos_sin + (size_t)min(max(pos, 0), n_positions - 1) * (rot_dims / 2) : nullptr;
 
   // the queries
   float fq = q_scale;
   if (w_q != nullptr && !head_norm) fq *= 1.0f / sqrtf(sq / (float)Q + eps);
   if (temp_every > 0) fq *= 1.0f + temp_coef * logf((float)((pos + 1) / temp_every) + 1.0f);
-  for (int i = part * PACK_THREADS + tid; i < n_heads * pad; i += parts * PACK_THREADS) {
+  for (int i = first; i < n_heads * pad; i += step) {
     const int h = i / pad, e = i - h * pad;
+    if (i != first) aq = ask(w_q, h, e);
     float v = 0.f;
     if (e < d) {
       const float f = head_norm && w_q != nullptr ? fq * head_f[h] : fq;
-      auto normed = [&](int el) { return row[h * d + el] * f * (w_q != nullptr ? w_q[head_norm ? el : h * d + el] : 1.0f); };
-      v = normed(e);
+      v = row[h * d + e] * f * aq.w;
       if (e < rot_dims) {
-        const float2 c = cs[e >> 1];
-        const float other = normed(e ^ 1);
+        const float2 c = aq.c;
+        const float other = row[h * d + (e ^ 1)] * f * aq.w_other;
         v = (e & 1) ? fmaf(v, c.x, other * c.y) : fmaf(v, c.x, -other * c.y);
       }
     }
@@ -104,16 +122,16 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
 
   const float fk = w_k != nullptr && !head_norm ? 1.0f / sqrtf(sk / (float)K + eps) : 1.0f;
   const float lam = blend == 2 ? lam_p[0] : 0.f;
-  for (int i = part * PACK_THREADS + tid; i < n_kv_heads * pad; i += parts * PACK_THREADS) {
+  for (int i = first; i < n_kv_heads * pad; i += step) {
     const int g = i / pad, e = i - g * pad;
+    if (i != first) ak = ask(w_k, g, e);
     float kv = 0.f, vv = 0.f;
     if (e < d) {
       const float f = head_norm && w_k != nullptr ? head_f[n_heads + g] : fk;
-      auto normed = [&](int el) { return row[Q + g * d + el] * f * (w_k != nullptr ? w_k[head_norm ? el : g * d + el] : 1.0f); };
-      kv = normed(e);
+      kv = row[Q + g * d + e] * f * ak.w;
       if (e < rot_dims) {
-        const float2 c = cs[e >> 1];
-        const float other = normed(e ^ 1);
+        const float2 c = ak.c;
+        const float other = row[Q + g * d + (e ^ 1)] * f * ak.w_other;
         kv = (e & 1) ? fmaf(kv, c.x, other * c.y) : fmaf(kv, c.x, -other * c.y);
       }
     }
@@ -140,9 +158,10 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
   }
 }
 
-// The same work a wave a token, the token's row in registers between its sums and its results: no LDS and no barrier
-// (a workgroup a token spends most of its time waiting at the barriers of its two sums).  For rows whose parts and heads
-// are multiples of four elements (a lane takes four consecutive ones at a time) and at most 256 * NV elements.
+// The same work four elements a thread, the token's row in registers between its sums and its results: one exchange for both sums and
+// no row in LDS.  For rows whose parts and heads are multiples of four elements (a thread takes four consecutive ones at a time) and at most
+// 1,024 * NV elements.  A workgroup of four waves a token: with a wave a token, 24 rounds of a row of 6,144 and its weights were 250
+// registers, two waves a SIMD and too few loads in flight (1,909 tokens 43.8 -> 31.9 us).
 template <typename T> struct Pack4;
 template <> struct Pack4<float> {
   static __device__ __forceinline__ void store(float* p, float a, float b, float c, float d) {
@@ -155,30 +174,42 @@ template <> struct Pack4<bf16> {
     *reinterpret_cast<bf16x4*>(p) = (bf16x4){static_cast<bf16>(a), static_cast<bf16>(b), static_cast<bf16>(c), static_cast<bf16>(d)};
   }
 };
-constexpr int PW_WAVES = 4;
+constexpr int PV_THREADS = 256;
 
 // SHAPED: with norms a head, values that are the keys, or the rotation (the other models run the code without them)
 template <typename T, int NV, bool SHAPED>
-__global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
+__global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
     const float* __restrict__ qkv, long qkv_row, const float* __restrict__ bias, const float* __restrict__ w_q,
     const float* __restrict__ w_k, float eps, float temp_coef, int temp_every, float q_scale, float* __restrict__ v_first,
     int blend, const float* __restrict__ lam_p, T* __restrict__ q_out, T* __restrict__ k_stage, T* __restrict__ v_stage,
     const int* __restrict__ seq_tile0, T* __restrict__ k_pages, T* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_stride, int ring_pages, const int* __restrict__ tok_seq,
-    const int* __restrict__ tok_pos, const int* __restrict__ seq_slot, const int* __restrict__ seq_len, int n_tokens,
+    const int* __restrict__ tok_pos, const int* __restrict__ seq_slot, const int* __restrict__ seq_len,
     int n_heads, int n_kv_heads, int d, int dv, int pad, int n_pages, int page_layout, T* __restrict__ v_rows,
     int head_norm_, int v_from_k_, const float2* __restrict__ cos_sin, int rot_dims_, int n_positions) {
   // head_norm here: d a power of two from 4 to 256, so that a head's elements lie in d / 4 neighbouring lanes of one round
   const int head_norm = SHAPED ? head_norm_ : 0, v_from_k = SHAPED ? v_from_k_ : 0, rot_dims = SHAPED ? rot_dims_ : 0;
-  const int t = blockIdx.x * PW_WAVES + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  if (t >= n_tokens) return;
+  __shared__ float2 red[PV_THREADS / WAVE];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const int pos = tok_pos[t];
+  const int b = tok_seq[t];
   const int Q = n_heads * d, K = n_kv_heads * d, V = n_kv_heads * dv, N = Q + K + (v_from_k ? 0 : V);
   const float* src = qkv + (size_t)t * qkv_row;
+  // Heads that divide a round's elements: a thread has the same place in the head in every round, and its two angles are asked for
+  // once, in front of the row
+  const float2* cs = rot_dims > 0 ? cos_sin + (size_t)min(max(pos, 0), n_positions - 1) * (rot_dims / 2) : nullptr;
+  const bool same_place = (PV_THREADS * 4) % d == 0;
+  float2 turn0 = make_float2(1.0f, 0.0f), turn1 = turn0;
+  if (SHAPED && same_place && cs != nullptr) {
+    const int e = tid * 4 % d;
+    if (e < rot_dims) turn0 = cs[e >> 1];
+    if (e + 2 < rot_dims) turn1 = cs[(e >> 1) + 1];
+  }
   float4 r[NV], wt[NV];                           // the row and the norm weights of its elements: every load asked for at once
   float sq = 0.f, sk = 0.f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int i = (j * WAVE + lane) * 4;
+    const int i = (j * PV_THREADS + tid) * 4;
     wt[j] = make_float4(1.f, 1.f, 1.f, 1.f);
     if (i < Q && w_q != nullptr) wt[j] = *reinterpret_cast<const float4*>(w_q + (head_norm ? i % d : i));
     else if (i >= Q && i < Q + K && w_k != nullptr) wt[j] = *reinterpret_cast<const float4*>(w_k + (head_norm ? (i - Q) % d : i - Q));
@@ -186,7 +217,7 @@ __global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
 
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int i = (j * WAVE + lane) * 4;
+    const int i = (j * PV_THREADS + tid) * 4;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (i < N) {
       v = *reinterpret_cast<const float4*>(src + i);
@@ -208,10 +239,11 @@ __global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
       }
     }
   }
-  sq = wave_sum(sq);
-  sk = wave_sum(sk);
-  const int pos = tok_pos[t];
-  const int b = tok_seq[t];
+  if (!head_norm && (w_q != nullptr || w_k != nullptr)) {
+    const float2 both = block_sum2<PV_THREADS / WAVE>(sq, sk, red);
+    sq = both.x;
+    sk = both.y;
+  }
   const int slot = b >= 0 ? seq_slot[b] : -1;
   float fq = q_scale;
   if (w_q != nullptr && !head_norm) fq *= 1.0f / sqrtf(sq / (float)Q + eps);
@@ -219,16 +251,15 @@ __global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
   const float fk = w_k != nullptr && !head_norm ? 1.0f / sqrtf(sk / (float)K + eps) : 1.0f;
   const float lam = blend == 2 ? lam_p[0] : 0.f;
   const int row = pos & (PAGE - 1);
-  const float2* cs = rot_dims > 0 ? cos_sin + (size_t)min(max(pos, 0), n_positions - 1) * (rot_dims / 2) : nullptr;
   // the lane's four elements e .. e + 3 of a head are two of the rotation's pairs
   auto turn = [&](int e, float& a0, float& a1, float& a2, float& a3) {
     if (e < rot_dims) {
-      const float2 c = cs[e >> 1];
+      const float2 c = same_place ? turn0 : cs[e >> 1];
       const float x = a0 * c.x - a1 * c.y, y = a1 * c.x + a0 * c.y;
       a0 = x, a1 = y;
     }
     if (e + 2 < rot_dims) {
-      const float2 c = cs[(e >> 1) + 1];
+      const float2 c = same_place ? turn1 : cs[(e >> 1) + 1];
       const float x = a2 * c.x - a3 * c.y, y = a3 * c.x + a2 * c.y;
       a2 = x, a3 = y;
     }
@@ -245,7 +276,7 @@ __global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
   T* qo = q_out + (size_t)t * n_heads * pad;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int i = (j * WAVE + lane) * 4;
+    const int i = (j * PV_THREADS + tid) * 4;
     if (i >= N) continue;
     float4 v = r[j];
     if (i < Q) {
@@ -301,8 +332,8 @@ __global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
   const T zero = from_f32<T>(0.f);
   if (pad > d) {
     const int extra = pad - d;
-    for (int i = lane; i < n_heads * extra; i += WAVE) qo[(i / extra) * pad + d + i % extra] = zero;
-    for (int i = lane; i < n_kv_heads * extra; i += WAVE) {
+    for (int i = tid; i < n_heads * extra; i += PV_THREADS) qo[(i / extra) * pad + d + i % extra] = zero;
+    for (int i = tid; i < n_kv_heads * extra; i += PV_THREADS) {
       const int g = i / extra, e = d + i % extra;
       if (tile >= 0) k_stage[((size_t)tile * n_kv_heads + g) * PAGE * pad + (size_t)row * pad + e] = zero;
       if (page >= 0) k_pages[((size_t)page * n_kv_heads + g) * PAGE * pad + page_k_offset(page_layout, row, e, pad)] = zero;
@@ -310,7 +341,7 @@ __global__ __launch_bounds__(PW_WAVES * WAVE) void qkv_pack_wave_kernel(
   }
   if (pad > dv) {
     const int extra = pad - dv;
-    for (int i = lane; i < n_kv_heads * extra; i += WAVE) {
+    for (int i = tid; i < n_kv_heads * extra; i += PV_THREADS) {
       const int g = i / extra, e = dv + i % extra;
       if (v_rows != nullptr) {
         v_rows[(size_t)t * n_kv_heads * pad + g * pad + e] = zero;
@@ -425,29 +456,28 @@ extern "C" int yalm_qkv_pack(const float* qkv, long qkv_row, const float* bias, 
   const int n_row = n_heads * d + n_kv_heads * (d + (v_from_k ? 0 : dv));
   const size_t lds = (size_t)(n_row + n_heads + n_kv_heads) * sizeof(float);
   if (lds > 64 * 1024 || qkv_row < n_row) return YALM_ERR_ARG;
-  // a wave a token where a lane can take four elements at a time and the row fits its registers, and where the tokens
+  // four elements a thread where the row's parts allow it and the row fits the registers, and where the tokens
   // are many: a few tokens are done sooner by 1,024 threads each (8 tokens of 6,144 numbers: 12 against 25 us)
   const bool heads_fit = !head_norm || (d >= 4 && d <= 256 && (d & (d - 1)) == 0);      // a head in neighbouring lanes
-  const bool by_wave = heads_fit && T >= 32 && d % 4 == 0 && dv % 4 == 0 && qkv_row % 4 == 0 && n_row <= 256 * 32 &&
+  const bool by_fours = heads_fit && T >= 32 && d % 4 == 0 && dv % 4 == 0 && qkv_row % 4 == 0 && n_row <= 256 * 32 &&
                        ((((uintptr_t)qkv) | ((uintptr_t)bias) | ((uintptr_t)w_q) | ((uintptr_t)w_k) | ((uintptr_t)v_first) |
                          ((uintptr_t)q_out) | ((uintptr_t)k_stage) | ((uintptr_t)k_pages) | ((uintptr_t)v_rows)) & 15) == 0;
-  if (by_wave) {
-    const int blocks = ceil_div(T, PW_WAVES);
+  if (by_fours) {
     const bool shaped = head_norm || v_from_k || rot_dims > 0;
 #define YALM_PACK_W(TYPE, NV_)                                                                                           \
   do { if (shaped) YALM_PACK_WS(TYPE, NV_, true); else YALM_PACK_WS(TYPE, NV_, false); } while (0)
 #define YALM_PACK_WS(TYPE, NV_, SHAPED_)                                                                                 \
-  qkv_pack_wave_kernel<TYPE, NV_, SHAPED_><<<blocks, PW_WAVES * WAVE, 0, stream>>>(                                               \
+  qkv_pack_vec_kernel<TYPE, NV_, SHAPED_><<<T, PV_THREADS, 0, stream>>>(                                               \
       qkv, qkv_row, bias, w_q, w_k, eps, temp_coef, temp_every, q_scale, v_first, blend, lam, (TYPE*)q_out, (TYPE*)k_stage,        \
       (TYPE*)v_stage, seq_tile0, (TYPE*)k_pages, (TYPE*)v_pages, block_table, table_stride, ring_pages, tok_seq,         \
-      tok_pos, seq_slot, seq_len, T, n_heads, n_kv_heads, d, dv, pad, n_pages, page_layout, (TYPE*)v_rows, head_norm,    \
+      tok_pos, seq_slot, seq_len, n_heads, n_kv_heads, d, dv, pad, n_pages, page_layout, (TYPE*)v_rows, head_norm,       \
       v_from_k, (const float2*)cos_sin, rot_dims, n_positions)
 #define YALM_PACK_WN(TYPE)                                                                                               \
-  if (n_row <= 256 * 4) YALM_PACK_W(TYPE, 4);                                                                            \
-  else if (n_row <= 256 * 8) YALM_PACK_W(TYPE, 8);                                                                       \
-  else if (n_row <= 256 * 16) YALM_PACK_W(TYPE, 16);                                                                     \
-  else if (n_row <= 256 * 24) YALM_PACK_W(TYPE, 24);                                                                     \
-  else YALM_PACK_W(TYPE, 32)
+  if (n_row <= 1024) YALM_PACK_W(TYPE, 1);                                                                               \
+  else if (n_row <= 1024 * 2) YALM_PACK_W(TYPE, 2);                                                                      \
+  else if (n_row <= 1024 * 4) YALM_PACK_W(TYPE, 4);                                                                      \
+  else if (n_row <= 1024 * 6) YALM_PACK_W(TYPE, 6);                                                                      \
+  else YALM_PACK_W(TYPE, 8)
     if (dtype == YALM_F32) {
       YALM_PACK_WN(float);
     } else if (dtype == YALM_BF16) {
