@@ -155,6 +155,31 @@ def test_packing_kernel_of_few_tokens(H, G, d, dv, head_norm):
         assert torch.allclose(a, b, rtol=2e-6, atol=2e-6) and torch.equal(a != 0, b != 0)
 
 
+# The gate of the result beside it along with the recurrence's step: the bits of the two launches, with one and several workgroups a token for
+# the gate, heads whose parts lie on 16 bytes and not, and steps of more tokens than sequences, which are launches of their own
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,H,d,dv,gH,gdv,pad", [([1] * 5, 32, 128, 128, 32, 128, 128), ([1], 3, 16, 16, 5, 24, 32), ([1] * 3, 2, 64, 64, 40, 96, 96),
+                                                    ([1, 1], 4, 32, 32, 7, 20, 32), ([1, 1], 4, 32, 32, 3, 6, 16), ([3, 1], 2, 16, 24, 4, 16, 16)])
+def test_hgrn2_with_the_gate_beside_it(dtype, lens, H, d, dv, gH, gdv, pad):
+    from yalm_amd.ops import kernels
+    B, T, N = len(lens), sum(lens), 2 * H * d + H * dv
+    wide = randn(T, N + gH * gdv, seed=1).to(DEV)             # both read parts of one product's rows
+    proj, g = wide[:, gH * gdv:], wide[:, :gH * gdv]
+    bias, lower, w = randn(H * d, seed=2).to(DEV), torch.rand(H * d, generator=gen(3)).to(DEV), (1 + 0.1 * randn(dv, seed=4)).to(DEV)
+    state, beside = randn(B + 1, H * d * dv, seed=5).to(DEV), randn(T, gH * pad, seed=6).to(dtype).to(DEV)
+    cu, slots = i32(np.concatenate([[0], np.cumsum(lens)])), i32([-1 if B > 2 and b == 1 else B - b for b in range(B)])
+    raw = torch.empty(T, H * dv, device=DEV)
+    got = []
+    for along in (False, True):
+        st, o, out = state.clone(), beside.clone(), torch.full((T, H * dv), float("nan"), dtype=dtype, device=DEV)
+        if not along:
+            kernels.sigmoid_gate(o, g, gH, gdv, pad)
+        kernels.hgrn2(proj, bias, lower, w, st, raw, cu, slots, out, H, d, dv, 1e-5, gate=(o, g, gH, gdv, pad) if along else None)
+        got.append((st, o, out))
+    for a, b in zip(*got):
+        assert torch.equal(a, b) and not torch.equal(got[0][1], beside)
+
+
 # Four elements a thread (40 rows) against a workgroup that holds the row in LDS (20): rows at both ends of the kernel's sizes, heads that divide a
 # round of 1,024 elements (their angles asked for once) and that do not
 @pytest.mark.parametrize("H,G,d,dv,head_norm,rot", [(6, 1, 128, 128, False, 64), (6, 1, 128, 132, False, 128), (48, 8, 128, 128, True, 64),

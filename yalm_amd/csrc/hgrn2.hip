@@ -56,14 +56,45 @@ struct Hgrn2Op {
 // (800 sequences of 8 heads of 16 x 16 9.3 us, with 512 threads each 23.3, those two kernels 13.8).
 constexpr int HS_MAX = 128;
 
+// The gate of a result that stands beside the recurrence's (yalm_sigmoid_gate's: o *= sigmoid(g)), done by further workgroups of a step's
+// launch: both wait for nothing but the product in front, and alone each is a launch of 4.6 us and more that moves next to nothing (five
+// tokens, 32 heads of 128: 5.9 + 4.6 -> 6.4 us).
+template <typename T>
+struct SideGate {
+  T* o;
+  const float* g;
+  long g_stride;
+  int n_heads, dv, pad, blocks;                   // blocks: workgroups a token, behind the heads' (0: none)
+};
+
 template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS) void hgrn2_step_kernel(Hgrn2Op op, float* __restrict__ state, const float* __restrict__ w_norm,
                                                                 T* __restrict__ out, const int* __restrict__ cu_seqlens,
-                                                                const int* __restrict__ seq_slot, int n_heads, int d, int dv, float eps) {
+                                                                const int* __restrict__ seq_slot, int n_heads, int d, int dv, float eps,
+                                                                SideGate<T> gate) {
   constexpr int LANES = 8, GROUPS = THREADS / LANES, NC = 2, NV = HS_MAX / (4 * LANES);
   constexpr int VALUES = THREADS > HS_MAX ? HS_MAX : 0;       // the first of the threads that fetch a token's values
   __shared__ __attribute__((aligned(16))) float s_q[HS_MAX], s_f[HS_MAX], s_v[HS_MAX], s_o[HS_MAX];
   const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, group = tid / LANES, rl = tid % LANES;
+  if (h >= n_heads) {                              // token b's gate, 16 bytes of the result a thread
+    constexpr int VEC = 16 / sizeof(T);
+    const int i = ((h - n_heads) * THREADS + tid) * VEC;
+    if (i >= gate.n_heads * gate.dv) return;
+    T* p = gate.o + ((size_t)b * gate.n_heads + i / gate.dv) * gate.pad + i % gate.dv;
+    const float* g = gate.g + (size_t)b * gate.g_stride + i;
+    typedef __attribute__((ext_vector_type(VEC))) T Vec;
+    Vec v = *reinterpret_cast<const Vec*>(p);
+    float z[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; k += 4) {
+      const float4 z4 = *reinterpret_cast<const float4*>(g + k);
+      z[k] = z4.x, z[k + 1] = z4.y, z[k + 2] = z4.z, z[k + 3] = z4.w;
+    }
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) v[k] = from_f32<T>(to_f32(static_cast<T>(v[k])) / (1.0f + expf(-z[k])));
+    *reinterpret_cast<Vec*>(p) = v;
+    return;
+  }
   const int slot = seq_slot[b], t0 = cu_seqlens[b], t1 = cu_seqlens[b + 1], HV = n_heads * dv;
   const typename Hgrn2Op::Row mine = op.begin(h, min(tid, d - 1), tid < HS_MAX);
   if (slot < 0) {                                  // a padding row: no state is touched, its result is zeros
@@ -429,9 +460,10 @@ extern "C" int yalm_hgrn2_tiles(const float* proj, long proj_row, const float* f
   return heads_norm_launch(raw, w_norm, nullptr, 0, out, T, n_heads, dv, eps, out_dtype, stream);
 }
 
-extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state,
-                          float* raw, const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads,
-                          int d, int dv, float eps, int out_dtype, hipStream_t stream) {
+static int hgrn2_gated(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state,
+                       float* raw, const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads, int d, int dv, float eps,
+                       void* gate_o, const float* gate, long gate_stride, int gate_heads, int gate_dv, int gate_pad, int out_dtype,
+                       hipStream_t stream) {
   if (T <= 0 || B <= 0) return YALM_OK;
   if (n_heads <= 0 || d <= 0 || d > 256 || dv <= 0) return YALM_ERR_ARG;
   if (out_dtype != YALM_F32 && out_dtype != YALM_BF16) return YALM_ERR_DTYPE;
@@ -439,12 +471,26 @@ extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias,
   const Hgrn2Op op = {proj, f_bias, lower, n_heads * d, (int)proj_row, d, dv, n_heads * dv};
   // one token a sequence, as the numbers say (the kernel walks whatever cu_seqlens holds; eight tokens of one sequence and none of seven
   // others, which no step of the engine is, take it 12 us and diag_scan_kernel 6)
-  if (T == B && n_heads <= 65535 && B <= 65535 && d <= HS_MAX && dv <= HS_MAX && d % 4 == 0 && dv % 4 == 0 && ((uintptr_t)state & 15) == 0) {
-    const dim3 grid(n_heads, B);
-#define STEP(T_, THREADS_) \
-  hgrn2_step_kernel<T_, THREADS_><<<grid, THREADS_, 0, stream>>>(op, state, w_norm, (T_*)out, cu_seqlens, seq_slot, n_heads, d, dv, eps)
+  const bool step = T == B && n_heads <= 65535 && B <= 65535 && d <= HS_MAX && dv <= HS_MAX && d % 4 == 0 && dv % 4 == 0 && ((uintptr_t)state & 15) == 0;
+  // the gate goes along where a thread's part of it lies on 16 bytes; else it is a launch of its own
+  const int vec = out_dtype == YALM_BF16 ? 8 : 4, threads = dv <= 32 ? 128 : dv <= 64 ? 256 : 512;
+  int blocks = 0;
+  if (gate_o != nullptr) {
+    if (gate_heads <= 0 || gate_dv <= 0 || gate_pad < gate_dv || gate_stride < (long)gate_heads * gate_dv) return YALM_ERR_ARG;
+    if (step && gate_dv % vec == 0 && gate_pad % vec == 0 && gate_stride % 4 == 0 && (((uintptr_t)gate_o | (uintptr_t)gate) & 15) == 0) {
+      blocks = ceil_div((long)gate_heads * gate_dv, (long)threads * vec);
+    } else {
+      const int rc = yalm_sigmoid_gate(gate_o, gate, gate_stride, T, gate_heads, gate_dv, gate_pad, out_dtype, stream);
+      if (rc != YALM_OK) return rc;
+    }
+  }
+  if (step) {
+    const dim3 grid(n_heads + blocks, B);
+#define STEP(T_, THREADS_)                                                                                                                   \
+  hgrn2_step_kernel<T_, THREADS_><<<grid, THREADS_, 0, stream>>>(op, state, w_norm, (T_*)out, cu_seqlens, seq_slot, n_heads, d, dv, eps, \
+                                                                 SideGate<T_>{(T_*)gate_o, gate, gate_stride, gate_heads, gate_dv, gate_pad, blocks})
 #define STEP_OF(T_) \
-  if (dv <= 32) STEP(T_, 128); else if (dv <= 64) STEP(T_, 256); else STEP(T_, 512)
+  if (threads == 128) STEP(T_, 128); else if (threads == 256) STEP(T_, 256); else STEP(T_, 512)
     if (out_dtype == YALM_F32) { STEP_OF(float); }
     else { STEP_OF(bf16); }
 #undef STEP_OF
@@ -465,4 +511,20 @@ extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias,
 #undef SCAN
   if (rc != YALM_OK) return rc;
   return heads_norm_launch(raw, w_norm, nullptr, 0, out, T, n_heads, dv, eps, out_dtype, stream);
+}
+
+extern "C" int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state,
+                          float* raw, const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads,
+                          int d, int dv, float eps, int out_dtype, hipStream_t stream) {
+  return hgrn2_gated(proj, proj_row, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, T, B, n_heads, d, dv, eps, nullptr, nullptr, 0,
+                     0, 0, 0, out_dtype, stream);
+}
+
+extern "C" int yalm_hgrn2_gated(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state,
+                                float* raw, const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads, int d, int dv,
+                                float eps, void* gate_o, const float* gate, long gate_stride, int gate_heads, int gate_dv, int gate_pad,
+                                int out_dtype, hipStream_t stream) {
+  if (gate_o == nullptr || gate == nullptr) return YALM_ERR_ARG;
+  return hgrn2_gated(proj, proj_row, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, T, B, n_heads, d, dv, eps, gate_o, gate,
+                     gate_stride, gate_heads, gate_dv, gate_pad, out_dtype, stream);
 }

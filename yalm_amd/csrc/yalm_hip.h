@@ -508,6 +508,10 @@ int yalm_loop_pack(float* x, const float* x0, const float* start, void* both, in
 int yalm_hgrn2(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state, float* raw,
                const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads, int d, int dv, float eps,
                int out_dtype, hipStream_t stream);
+// The same, and yalm_sigmoid_gate on a result of as many tokens beside it (gate_o of `out_dtype`): one launch in a step of one token a sequence.
+int yalm_hgrn2_gated(const float* proj, long proj_row, const float* f_bias, const float* lower, const float* w_norm, float* state, float* raw,
+                     const int* cu_seqlens, const int* seq_slot, void* out, int T, int B, int n_heads, int d, int dv, float eps, void* gate_o,
+                     const float* gate, long gate_stride, int gate_heads, int gate_dv, int gate_pad, int out_dtype, hipStream_t stream);
 // The same for steps of prompts, a tile of 64 tokens at a time (seq_tile0, n_tiles and scratch as for yalm_gla_tiles, DP =
 // yalm_hgrn2_tiles_fit(d); 0: key heads of d are not taken).
 int yalm_hgrn2_tiles_fit(int d);

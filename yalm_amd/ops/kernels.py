@@ -1493,11 +1493,13 @@ def hgrn2_state_elements(n_heads, d, dv):
     return n_heads * d * dv
 
 
-def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_heads, d, dv, eps):
+def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_heads, d, dv, eps, gate=None):
     """The HGRN2 recurrence over a step's tokens.  proj float32 [T, 2 H d + H dv] (rows may be parts of wider ones) = z_q | z_f | v; q = silu(z_q), f = lower
     + (1 - lower) sigmoid(z_f + f_bias); per head S <- diag(f) S + (1 - f) v^T, o = S^T q; out [T, H dv] = o over its root
     mean square a head, times w_norm [dv].  state float32 [slots, H dv d] (a head's S column by column) is read and left
-    advanced; raw float32 [T, H dv] is scratch.  Sequence b's tokens are cu_seqlens[b] .. cu_seqlens[b + 1] - 1."""
+    advanced; raw float32 [T, H dv] is scratch.  Sequence b's tokens are cu_seqlens[b] .. cu_seqlens[b + 1] - 1.
+    gate = (o, g, n_heads, dv, pad): sigmoid_gate of these (o [T, ...] in out's dtype) is done on the way, in the same launch where the step
+    has one token a sequence."""
     T = proj.shape[0]
     B = seq_slot.shape[0]
     N = 2 * n_heads * d + n_heads * dv
@@ -1505,12 +1507,19 @@ def hgrn2(proj, f_bias, lower, w_norm, state, raw, cu_seqlens, seq_slot, out, n_
         raise ValueError("hgrn2: key heads of %d (at most %d)" % (d, HGRN2_MAX_KEY_DIM))
     if proj.dtype != torch.float32 or proj.dim() != 2 or proj.shape[1] != N or proj.stride(1) != 1 or not proj.is_cuda:
         raise ValueError("hgrn2: the projections are float32 [%d, %d] on the device, rows contiguous" % (T, N))
-    library.check(library.lib().yalm_hgrn2(
+    more = ()
+    if gate is not None:
+        o, g, heads, width, pad = gate
+        if g.dtype != torch.float32 or g.dim() != 2 or g.shape != (T, heads * width) or g.stride(1) != 1 or not g.is_cuda:
+            raise ValueError("hgrn2: the gates beside it are float32 [%d, %d] on the device, rows contiguous" % (T, heads * width))
+        more = (_need(o, "o", out.dtype, (T, heads * pad)), g.data_ptr(), int(g.stride(0)), heads, width, pad)
+    run = library.lib().yalm_hgrn2 if gate is None else library.lib().yalm_hgrn2_gated
+    library.check(run(
         proj.data_ptr(), int(proj.stride(0)), _need(f_bias, "f_bias", torch.float32, (n_heads * d,)),
         _need(lower, "lower", torch.float32, (n_heads * d,)), _need(w_norm, "w_norm", torch.float32, (dv,)),
         _need(state, "state", torch.float32, (None, n_heads * d * dv)), _need(raw, "raw", torch.float32, (T, n_heads * dv)),
         _need(cu_seqlens, "cu_seqlens", torch.int32, (B + 1,)), _need(seq_slot, "seq_slot", torch.int32, (B,)),
-        _need(out, "out", None, (T, n_heads * dv)), T, B, n_heads, d, dv, float(eps), dtype_code(out.dtype), _stream()), "hgrn2")
+        _need(out, "out", None, (T, n_heads * dv)), T, B, n_heads, d, dv, float(eps), *more, dtype_code(out.dtype), _stream()), "hgrn2")
     return out
 
 

@@ -103,6 +103,7 @@ _SIGNATURES = {
     "yalm_loop_pack": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
     "yalm_hgrn2_tiles_fit": (_I, [_I]),
     "yalm_hgrn2_tiles": (_I, [_P, ctypes.c_long, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I, _P]),
+    "yalm_hgrn2_gated": (_I, [_P, ctypes.c_long, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, ctypes.c_long, _I, _I, _I, _I, _P]),
     "yalm_hgrn2": (_I, [_P, ctypes.c_long, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P]),
     "yalm_head_gate": (_I, [_P, _P, ctypes.c_long, _F, _P, ctypes.c_long, _I, _I, _I, _I, _P]),
     "yalm_softcap": (_I, [_P, ctypes.c_long, _F, _P]),

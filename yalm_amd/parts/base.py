@@ -250,8 +250,9 @@ class JoinableMixer(Part):
 
     mixed_in = "joinable.o"           # the step's buffer in which `mixed` leaves its result, until the next mixer that uses it runs
 
-    def mixed(self, h, ctx, line, writes_cache=True, proj=None):
-        """What the last product reads."""
+    def mixed(self, h, ctx, line, writes_cache=True, proj=None, gate_left=None):
+        """What the last product reads.  gate_left (a list; of mixers that say `leaves_gate`): the gate on the result may be left to
+        the caller, as the arguments of kernels.sigmoid_gate in that list."""
         import torch
         from ..ops import kernels
         T = h.shape[0]
@@ -259,7 +260,7 @@ class JoinableMixer(Part):
             proj = ctx.ws.get("joinable.proj", (T, self.n_in), torch.float32)
             self._gemm(ctx, h, self.w_in, proj, kernels.EPI_STORE_F32)
         o = ctx.ws.get(self.mixed_in, (T, self.n_out), h.dtype)
-        self.between(h, proj, o, ctx, line, writes_cache)
+        self.between(h, proj, o, ctx, line, writes_cache, **({} if gate_left is None else {"gate_left": gate_left}))
         return o
 
     def _run(self, h, x, ctx, line, writes_cache, epilogue, proj=None):

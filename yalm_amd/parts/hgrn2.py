@@ -88,7 +88,9 @@ class HGRN2(Part):
 
     mixed_in = "hgrn2.o"
 
-    def mixed(self, h, ctx, line, writes_cache=True, proj=None):
+    takes_gate = True                 # mixed takes the gate of a result beside it (kernels.sigmoid_gate's arguments) along
+
+    def mixed(self, h, ctx, line, writes_cache=True, proj=None, gate=None):
         """As JoinableMixer has it."""
         T = h.shape[0]
         ws = ctx.ws
@@ -101,15 +103,17 @@ class HGRN2(Part):
         if ctx.mode == "prefill" and h.dtype == torch.bfloat16 and not kernels.FORCE_SIMPLE \
                 and kernels.hgrn2_tiles_pay(ctx.host_n_tokens, self.n_heads, self.key_dim, self.value_dim):
             tiles = ctx.tables["kv_tiles"]
+            if gate is not None:
+                kernels.sigmoid_gate(*gate)
             kernels.hgrn2_tiles(proj, self.f_bias, self.lower, self.w_norm, state, raw, ctx.cu_seqlens, ctx.seq_slot, tiles["seq_tile0"],
                                 tiles["n_tiles"], o, self.n_heads, self.key_dim, self.value_dim, self.eps, ws.get)
         else:                 # float32 as the compute dtype: prompts go token by token too, so that their bits stay what they were
-            self._walk(proj, state, raw, o, ctx)
+            self._walk(proj, state, raw, o, ctx, gate)
         return o
 
     def _run(self, h, x, ctx, line, epilogue, proj=None):
         self._gemm(ctx, self.mixed(h, ctx, line, proj=proj), self.wo, x, epilogue)
 
-    def _walk(self, proj, state, raw, o, ctx):
+    def _walk(self, proj, state, raw, o, ctx, gate=None):
         kernels.hgrn2(proj, self.f_bias, self.lower, self.w_norm, state, raw, ctx.cu_seqlens, ctx.seq_slot, o, self.n_heads,
-                      self.key_dim, self.value_dim, self.eps)
+                      self.key_dim, self.value_dim, self.eps, gate=gate)

@@ -227,7 +227,9 @@ class ShapedAttention(JoinableMixer):
     def slopes(self):
         return getattr(self.position, "slopes", None)
 
-    def between(self, h, proj, o, ctx, line, writes_cache, scale=1.0):
+    leaves_gate = True                # between leaves a gate of elements to whoever asks for it
+
+    def between(self, h, proj, o, ctx, line, writes_cache, scale=1.0, gate_left=None):
         T = h.shape[0]
         joint = o                         # where the result belongs: maybe columns of a wider row
         act, ws = h.dtype, ctx.ws
@@ -280,4 +282,8 @@ class ShapedAttention(JoinableMixer):
         if self.gate == "heads":
             kernels.head_gate(o, proj[:, self.n_proj:self.n_proj + H], H, scale, joint)
         elif self.gate == "elements":
-            kernels.sigmoid_gate(o, proj[:, self.n_proj:], H, self.value_dim, P)
+            gate = (o, proj[:, self.n_proj:], H, self.value_dim, P)
+            if gate_left is None:
+                kernels.sigmoid_gate(*gate)
+            else:
+                gate_left.append(gate)

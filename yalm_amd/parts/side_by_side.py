@@ -133,8 +133,11 @@ class SideBySide(Part):
                 and kernels.gemm_pair_fits(
                 ctx.ws.get(self.left.mixed_in, (T, self.left.wo.shape[1]), h.dtype), self.left.wo,
                 ctx.ws.get(self.right.mixed_in, (T, self.right.wo.shape[1]), h.dtype), self.right.wo):
-            o = self.left.mixed(h, ctx, (line, "left"), writes_cache, **front[0])
-            o2 = self.right.mixed(h, ctx, (line, "right"), writes_cache, **front[1])
+            # the left result's gate waits for nothing that the right one does not wait for, and goes along with it
+            together = getattr(self.left, "leaves_gate", False) and getattr(self.right, "takes_gate", False)
+            left_over = [] if together else None
+            o = self.left.mixed(h, ctx, (line, "left"), writes_cache, **front[0], **({"gate_left": left_over} if together else {}))
+            o2 = self.right.mixed(h, ctx, (line, "right"), writes_cache, **front[1], **({"gate": left_over[0]} if left_over else {}))
             kernels.gemm_pair(o, self.left.wo, y, o2, self.right.wo, y2)
         else:
             self.left.forward_to(h, y, ctx, (line, "left"), writes_cache, **front[0])
