@@ -161,7 +161,8 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
 // The same work four elements a thread, the token's row in registers between its sums and its results: one exchange for both sums and
 // no row in LDS.  For rows whose parts and heads are multiples of four elements (a thread takes four consecutive ones at a time) and at most
 // 1,024 * NV elements.  A workgroup of four waves a token: with a wave a token, 24 rounds of a row of 6,144 and its weights were 250
-// registers, two waves a SIMD and too few loads in flight (1,909 tokens 43.8 -> 31.9 us).
+// registers, two waves a SIMD and too few loads in flight (1,909 tokens inside a step 43.8 -> 31.9 us; 32
+// tokens alone 19.5 -> 6.8, 2,048 33.9 -> 24.5; rows of 1,536 5.3 -> 3.5 and 8.3 -> 8.1).  Rows of up to 256 are a wave's (2,048 of them 4.2 us, with four waves 5.5).
 template <typename T> struct Pack4;
 template <> struct Pack4<float> {
   static __device__ __forceinline__ void store(float* p, float a, float b, float c, float d) {
@@ -174,10 +175,9 @@ template <> struct Pack4<bf16> {
     *reinterpret_cast<bf16x4*>(p) = (bf16x4){static_cast<bf16>(a), static_cast<bf16>(b), static_cast<bf16>(c), static_cast<bf16>(d)};
   }
 };
-constexpr int PV_THREADS = 256;
 
 // SHAPED: with norms a head, values that are the keys, or the rotation (the other models run the code without them)
-template <typename T, int NV, bool SHAPED>
+template <typename T, int NV, bool SHAPED, int PV_THREADS>
 __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
     const float* __restrict__ qkv, long qkv_row, const float* __restrict__ bias, const float* __restrict__ w_q,
     const float* __restrict__ w_k, float eps, float temp_coef, int temp_every, float q_scale, float* __restrict__ v_first,
@@ -464,20 +464,21 @@ extern "C" int yalm_qkv_pack(const float* qkv, long qkv_row, const float* bias, 
                          ((uintptr_t)q_out) | ((uintptr_t)k_stage) | ((uintptr_t)k_pages) | ((uintptr_t)v_rows)) & 15) == 0;
   if (by_fours) {
     const bool shaped = head_norm || v_from_k || rot_dims > 0;
-#define YALM_PACK_W(TYPE, NV_)                                                                                           \
-  do { if (shaped) YALM_PACK_WS(TYPE, NV_, true); else YALM_PACK_WS(TYPE, NV_, false); } while (0)
-#define YALM_PACK_WS(TYPE, NV_, SHAPED_)                                                                                 \
-  qkv_pack_vec_kernel<TYPE, NV_, SHAPED_><<<T, PV_THREADS, 0, stream>>>(                                               \
+#define YALM_PACK_W(TYPE, NV_, TH_)                                                                                      \
+  do { if (shaped) YALM_PACK_WS(TYPE, NV_, true, TH_); else YALM_PACK_WS(TYPE, NV_, false, TH_); } while (0)
+#define YALM_PACK_WS(TYPE, NV_, SHAPED_, TH_)                                                                               \
+  qkv_pack_vec_kernel<TYPE, NV_, SHAPED_, TH_><<<T, TH_, 0, stream>>>(                                               \
       qkv, qkv_row, bias, w_q, w_k, eps, temp_coef, temp_every, q_scale, v_first, blend, lam, (TYPE*)q_out, (TYPE*)k_stage,        \
       (TYPE*)v_stage, seq_tile0, (TYPE*)k_pages, (TYPE*)v_pages, block_table, table_stride, ring_pages, tok_seq,         \
       tok_pos, seq_slot, seq_len, n_heads, n_kv_heads, d, dv, pad, n_pages, page_layout, (TYPE*)v_rows, head_norm,       \
       v_from_k, (const float2*)cos_sin, rot_dims, n_positions)
 #define YALM_PACK_WN(TYPE)                                                                                               \
-  if (n_row <= 1024) YALM_PACK_W(TYPE, 1);                                                                               \
-  else if (n_row <= 1024 * 2) YALM_PACK_W(TYPE, 2);                                                                      \
-  else if (n_row <= 1024 * 4) YALM_PACK_W(TYPE, 4);                                                                      \
-  else if (n_row <= 1024 * 6) YALM_PACK_W(TYPE, 6);                                                                      \
-  else YALM_PACK_W(TYPE, 8)
+  if (n_row <= 256) YALM_PACK_W(TYPE, 1, 64);                                                                            \
+  else if (n_row <= 1024) YALM_PACK_W(TYPE, 1, 256);                                                                             \
+  else if (n_row <= 1024 * 2) YALM_PACK_W(TYPE, 2, 256);                                                                      \
+  else if (n_row <= 1024 * 4) YALM_PACK_W(TYPE, 4, 256);                                                                      \
+  else if (n_row <= 1024 * 6) YALM_PACK_W(TYPE, 6, 256);                                                                      \
+  else YALM_PACK_W(TYPE, 8, 256)
     if (dtype == YALM_F32) {
       YALM_PACK_WN(float);
     } else if (dtype == YALM_BF16) {
