@@ -31,9 +31,20 @@ from .base import Part, build_part, part
 TARGET_WORKGROUPS = 256
 RESIDENT_WORKGROUPS = 512       # decode-attention workgroups that the chip holds at once (two a compute unit)
 # A prompt step of fewer tokens rotates and stores token by token: the kernel that works a page-shaped tile at a
-# time has a workgroup per (tile, head), too few to fill the chip below this (64 tokens: 4.78 against 4.46 ms a
-# step, 128: 5.75 against 5.48, 256: 6.87 against 6.76, 384: the same)
+# time has a workgroup per (tile, head), too few to fill the chip below this.  It then takes its 12 us (two slices of K 15) however few tokens
+# there are, which the other one reaches later the fewer heads a token has.  us token by token and by tiles, 32 heads of 128 in 8
+# groups: one slice 320 tokens 10.6 11.8, 400 12.6 12.4, 512 15.0 12.7; two 400 12.9 15.6, 512 15.4 16.3, 640 22.2 20.5; four 400 20.8 23.7, 512
+# 26.4 24.8; 24 heads much the same (one slice 400 12.0 11.8, two 512 14.6 15.4, four 400 15.7 20.2, 512 24.6 23.4).  32 groups: 512 tokens 33.5 14.0, two slices 58.1 24.4;
+# heads of 64: 11.6 7.6, two slices 11.7 9.0
 ROPE_TILES_MIN_TOKENS = 320
+
+
+def rope_by_tiles(T, n_heads, n_kv_heads, head_dim, slices):
+    """Whether a step of whole prompts rotates and stores by tiles of 64 positions: with wide heads of which a q/k/v row has at most
+    64 from 400 tokens on, of several slices from 512."""
+    if head_dim < 128 or n_heads + 2 * n_kv_heads > 64:
+        return T >= ROPE_TILES_MIN_TOKENS
+    return T >= (ROPE_TILES_MIN_TOKENS * 5 // 4 if slices == 1 else ROPE_TILES_MIN_TOKENS * 8 // 5)
 
 
 def kv_tiles(n_tok):
@@ -357,7 +368,7 @@ class GQAttention(Part):
         else:
             kst = vst = seq_tile0 = None
         if writes_cache:
-            done = prefill and T >= ROPE_TILES_MIN_TOKENS and kernels.rope_kv_write_tiles(
+            done = prefill and rope_by_tiles(T, self.n_heads, self.n_kv_heads, self.head_dim, slices) and kernels.rope_kv_write_tiles(
                 qkv, q, kst, vst, ctx.cu_seqlens, seq_tile0, k_pages, v_pages, group.table, group.ring_pages,
                 ctx.seq_slot, ctx.seq_len, pos.table, self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim,
                 slices=slices)
