@@ -63,7 +63,7 @@ def test_packing_kernel(dtype, H, G, d, dv, temp, blend, by_tiles):
     and transposed a tile at a time."""
     from yalm_amd.ops import kernels
     from yalm_amd.parts.attention import kv_tiles
-    n_tok = [3, 70, 1]                            # 74 tokens: enough for the kernel that works a wave a token
+    n_tok = [3, 70, 1]                            # 74 tokens: enough for the kernel that keeps rows in registers
     T = sum(n_tok)
     Q, K, V = H * d, G * d, G * dv
     N = Q + K + V

@@ -130,7 +130,7 @@ def test_middle_of_a_gated_feed_forward_with_biases(T, F, D, kind, dtype):
     assert torch.allclose(out2.float().cpu().to(F64), act0 * z.to(F64)[:, F:], rtol=tol, atol=tol)
 
 
-# Few tokens are dealt to several workgroups each (20 rows), many take a wave each (40): the results agree, and every element is there.
+# Few tokens are dealt to several workgroups each (20 rows), many four waves each (40): the results agree, and every element is there.
 # Rows of 1,024 and of 256 threads, more key heads than query heads' share, heads that end inside a round
 @pytest.mark.parametrize("H,G,d,dv,head_norm", [(32, 8, 128, 128, False), (32, 8, 128, 64, True), (6, 2, 64, 48, False), (3, 3, 20, 28, False),
                                                 (44, 44, 32, 16, True)])
