@@ -457,7 +457,9 @@ extern "C" int yalm_qkv_pack(const float* qkv, long qkv_row, const float* bias, 
   const size_t lds = (size_t)(n_row + n_heads + n_kv_heads) * sizeof(float);
   if (lds > 64 * 1024 || qkv_row < n_row) return YALM_ERR_ARG;
   // four elements a thread where the row's parts allow it and the row fits the registers, and where the tokens
-  // are many: a few tokens are done sooner by 1,024 threads each (8 tokens of 6,144 numbers: 12 against 25 us)
+  // are many.  A few tokens alone take much the same either way (5 of 6,144 numbers 6.8 us with the row in LDS and 6.6 in registers, with
+  // norms a head 7.3 and 8.2, rows of 8,192 8.3 and 10.9, of 1,536 4.9 and 3.5); inside a step, where the row and the weights come from
+  // memory, the shares of several workgroups are sooner (requests of 255 to 509 tokens and 12 steps on four Rekirax layers 12.18 ms and 12.33)
   const bool heads_fit = !head_norm || (d >= 4 && d <= 256 && (d & (d - 1)) == 0);      // a head in neighbouring lanes
   const bool by_fours = heads_fit && T >= 32 && d % 4 == 0 && dv % 4 == 0 && qkv_row % 4 == 0 && n_row <= 256 * 32 &&
                        ((((uintptr_t)qkv) | ((uintptr_t)bias) | ((uintptr_t)w_q) | ((uintptr_t)w_k) | ((uintptr_t)v_first) |
