@@ -206,6 +206,58 @@ def test_packing_kernel_four_elements_a_thread(H, G, d, dv, head_norm, rot):
         assert torch.allclose(a, b, rtol=0, atol=8e-6) and torch.equal(a != 0, b != 0)
 
 
+# Many tokens are taken four waves each; their norms' sums are added as one wave adds them, 256 elements after 256 in every lane: ones behind a
+# square of 2^24 are lost one by one in that order, and in any other some of them are added up first
+@pytest.mark.parametrize("H,G,d", [(16, 16, 64), (16, 16, 128), (32, 8, 128), (64, 32, 64), (8, 8, 256)])
+def test_packing_kernel_adds_squares_in_one_order(H, G, d):
+    from yalm_amd.ops import kernels
+    T, Q, K = 64, H * d, G * d
+    raw = torch.zeros(T, Q + 2 * K)
+    for t in range(T):                            # each token in a lane of its own
+        for part, width in ((0, Q), (Q, K)):
+            at = list(range(part + (4 * t - part) % 256, part + width, 256))
+            raw[t, at[0]] = 4096.0
+            raw[t, at[1:]] = 1.0
+    raw = raw.to(DEV)
+    table = torch.zeros(1, 1, dtype=torch.int32, device=DEV)
+    q, k = torch.empty(T, Q, device=DEV), torch.empty(1, G, 64, d, device=DEV)
+    kp, vp = torch.empty(1, G, 64, d, device=DEV), torch.empty(1, G, d, 64, device=DEV)
+    ones = torch.ones(max(Q, K), device=DEV)
+    kernels.qkv_pack(raw, None, ones[:Q], ones[:K], 1e-5, None, 1.0, None, 0, None, q, k, torch.empty(1, G, d, 64, device=DEV), i32([0, 1]), kp, vp,
+                     table, 1, i32([0] * T), i32(range(T)), i32([0]), i32([T]), H, G, d, d, d)
+    for got, width in ((q, Q), (k[0].permute(1, 0, 2).reshape(T, K), K)):
+        rms = np.float32(1.0) / np.sqrt(np.float32(2.0 ** 24 / width) + np.float32(1e-5))
+        assert (got.max(dim=1).values.cpu().numpy() == np.float32(4096.0) * rms).all()
+
+
+# Which of a rotation's two products is rounded before the other joins it: the sine's in keys and in float32, the cosine's in bfloat16 queries
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,d,rot", [(4, 2, 128, 128), (20, 4, 64, 64), (14, 2, 100, 100)])
+def test_packing_kernel_rounds_rotations_one_way(dtype, H, G, d, rot):
+    from yalm_amd.ops import kernels
+    T, pad = 640, (d + 15) // 16 * 16
+    tiles = T // 64
+    raw = randn(T, H * d + 2 * G * d, seed=8)
+    angles = randn(T, rot // 2, seed=9)
+    cos_sin = torch.stack([angles.cos(), angles.sin()], dim=-1).contiguous()
+    table = torch.arange(tiles, dtype=torch.int32, device=DEV).reshape(1, tiles)
+    q, k, v = (torch.empty(s, dtype=dtype, device=DEV) for s in ((T, H * pad), (tiles, G, 64, pad), (tiles, G, pad, 64)))
+    kp, vp = torch.empty_like(k), torch.empty_like(v)
+    kernels.qkv_pack(raw.to(DEV), None, None, None, 1e-5, None, 1.0, None, 0, None, q, k, v, i32([0, tiles]), kp, vp, table, tiles, i32([0] * T),
+                     i32(range(T)), i32([0]), i32([T]), H, G, d, d, pad, cos_sin=cos_sin.to(DEV), rot_dims=rot)
+
+    def turned(x, late):                          # a product of two floats is exact in float64
+        x, c = x.to(F64).reshape(T, -1, d // 2, 2), cos_sin.to(F64)[:, None]
+        a0, a1, cos, sin = x[..., 0], x[..., 1], c[..., 0], c[..., 1]
+        if late:
+            x = torch.stack([(a0 * cos).float() - a1 * sin, (a1 * cos).float() + a0 * sin], dim=-1)
+        else:
+            x = torch.stack([a0 * cos - (a1 * sin).float(), a1 * cos + (a0 * sin).float()], dim=-1)
+        return x.float().to(dtype).reshape(T, -1, d)
+    assert torch.equal(q.cpu().reshape(T, H, pad)[..., :d], turned(raw[:, :H * d], dtype == torch.bfloat16))
+    assert torch.equal(k.cpu().permute(0, 2, 1, 3).reshape(T, G, pad)[..., :d], turned(raw[:, H * d:(H + G) * d], False))
+
+
 # The same with the middle in the first product's epilogue: one to 16 rows (K a multiple of 64 and not), to 128, tiles of 128 rows,
 # larger tiles, K in slices and whole; hidden values that end inside a block; streams narrower and wider than what one
 # element a thread covers; and the general kernels

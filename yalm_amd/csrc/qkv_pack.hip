@@ -159,7 +159,9 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
 }
 
 // The same work four elements a thread, the token's row in registers between its sums and its results: one exchange for both sums and
-// no row in LDS.  For rows whose parts and heads are multiples of four elements (a thread takes four consecutive ones at a time) and at most
+// no row in LDS.  The sums are formed as one wave alone forms them, 256 elements after 256 in every lane, whatever the number of waves: the
+// bits of a row's norm do not hang on it (what the waves hand each other is a sum of four squares an element's thread; the exchange is
+// level with one of the waves' sums: 1,909 rows of 6,144 20.9 and 21.1 us).  For rows whose parts and heads are multiples of four elements (a thread takes four consecutive ones at a time) and at most
 // 1,024 * NV elements.  A workgroup of four waves a token: with a wave a token, 24 rounds of a row of 6,144 and its weights were 250
 // registers, two waves a SIMD and too few loads in flight (1,909 tokens inside a step 43.8 -> 31.9 us; 32
 // tokens alone 19.5 -> 6.8, 2,048 33.9 -> 24.5; rows of 1,536 5.3 -> 3.5 and 8.3 -> 8.1).  Rows of up to 256 are a wave's (2,048 of them 4.2 us, with four waves 5.5).
@@ -189,8 +191,10 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
     int head_norm_, int v_from_k_, const float2* __restrict__ cos_sin, int rot_dims_, int n_positions) {
   // head_norm here: d a power of two from 4 to 256, so that a head's elements lie in d / 4 neighbouring lanes of one round
   const int head_norm = SHAPED ? head_norm_ : 0, v_from_k = SHAPED ? v_from_k_ : 0, rot_dims = SHAPED ? rot_dims_ : 0;
-  __shared__ float2 red[PV_THREADS / WAVE];
-  const int t = blockIdx.x, tid = threadIdx.x;
+  constexpr int WAVES = PV_THREADS / WAVE, ROUNDS = NV * WAVES;      // a round: 256 elements in their order
+  constexpr int AT_ONCE = ROUNDS < 8 ? ROUNDS : 8;
+  __shared__ float round_ss[WAVES > 1 ? ROUNDS : 1][WAVE], sums[2];
+  const int t = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int pos = tok_pos[t];
   const int b = tok_seq[t];
   const int Q = n_heads * d, K = n_kv_heads * d, V = n_kv_heads * dv, N = Q + K + (v_from_k ? 0 : V);
@@ -206,6 +210,7 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
     if (e + 2 < rot_dims) turn1 = cs[(e >> 1) + 1];
   }
   float4 r[NV], wt[NV];                           // the row and the norm weights of its elements: every load asked for at once
+  const bool row_norm = !head_norm && (w_q != nullptr || w_k != nullptr);
   float sq = 0.f, sk = 0.f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -226,8 +231,12 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
         v.x += b4.x; v.y += b4.y; v.z += b4.z; v.w += b4.w;
       }
       const float ss = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-      if (i < Q) sq += ss;
-      else if (i < Q + K) sk += ss;
+      if constexpr (WAVES > 1) {
+        if (row_norm) round_ss[j * WAVES + wave][lane] = ss;
+      } else {
+        if (i < Q) sq += ss;
+        else if (i < Q + K) sk += ss;
+      }
     }
     r[j] = v;
     if constexpr (SHAPED) {
@@ -239,10 +248,32 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
       }
     }
   }
-  if (!head_norm && (w_q != nullptr || w_k != nullptr)) {
-    const float2 both = block_sum2<PV_THREADS / WAVE>(sq, sk, red);
-    sq = both.x;
-    sk = both.y;
+  if (row_norm) {                                 // the rounds are added in their order, lane by lane, as one wave alone does it
+    if constexpr (WAVES > 1) {
+      lds_barrier();
+      if (wave < 2) {                             // the first wave the queries', the second the keys'
+        const int lo = wave == 0 ? 0 : Q, hi = wave == 0 ? Q : Q + K;
+        float s = 0.f;
+        for (int j0 = lo / (WAVE * 4); j0 * WAVE * 4 < hi; j0 += AT_ONCE) {
+          float part[AT_ONCE];
+#pragma unroll
+          for (int u = 0; u < AT_ONCE; ++u) part[u] = round_ss[min(j0 + u, ROUNDS - 1)][lane];
+#pragma unroll
+          for (int u = 0; u < AT_ONCE; ++u) {
+            const int i = ((j0 + u) * WAVE + lane) * 4;
+            s += i >= lo && i < hi ? part[u] : 0.f;
+          }
+        }
+        s = wave_sum(s);
+        if (lane == 0) sums[wave] = s;
+      }
+      lds_barrier();
+      sq = sums[0];
+      sk = sums[1];
+    } else {
+      sq = wave_sum(sq);
+      sk = wave_sum(sk);
+    }
   }
   const int slot = b >= 0 ? seq_slot[b] : -1;
   float fq = q_scale;
@@ -251,18 +282,17 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
   const float fk = w_k != nullptr && !head_norm ? 1.0f / sqrtf(sk / (float)K + eps) : 1.0f;
   const float lam = blend == 2 ? lam_p[0] : 0.f;
   const int row = pos & (PAGE - 1);
-  // the lane's four elements e .. e + 3 of a head are two of the rotation's pairs
-  auto turn = [&](int e, float& a0, float& a1, float& a2, float& a3) {
-    if (e < rot_dims) {
-      const float2 c = same_place ? turn0 : cs[e >> 1];
-      const float x = a0 * c.x - a1 * c.y, y = a1 * c.x + a0 * c.y;
-      a0 = x, a1 = y;
-    }
-    if (e + 2 < rot_dims) {
-      const float2 c = same_place ? turn1 : cs[(e >> 1) + 1];
-      const float x = a2 * c.x - a3 * c.y, y = a3 * c.x + a2 * c.y;
-      a2 = x, a3 = y;
-    }
+  // the lane's four elements e .. e + 3 of a head are two of the rotation's pairs.  Which product is rounded before the other joins it
+  // is said here and not left to the compiler: the sine's, and of bfloat16 queries the cosine's
+  auto turn_pair = [](bool q, const float2& c, float& a0, float& a1) {
+    float x, y;
+    if (q && sizeof(T) == 2) x = fmaf(-a1, c.y, a0 * c.x), y = fmaf(a0, c.y, a1 * c.x);
+    else x = fmaf(a0, c.x, -(a1 * c.y)), y = fmaf(a1, c.x, a0 * c.y);
+    a0 = x, a1 = y;
+  };
+  auto turn = [&](bool q, int e, float& a0, float& a1, float& a2, float& a3) {
+    if (e < rot_dims) turn_pair(q, same_place ? turn0 : cs[e >> 1], a0, a1);
+    if (e + 2 < rot_dims) turn_pair(q, same_place ? turn1 : cs[(e >> 1) + 1], a2, a3);
   };
   long page = -1, tile = -1;
   if (slot >= 0 && pos >= 0 && k_pages != nullptr) {
@@ -283,13 +313,13 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
       const int h = i / d, e = i - h * d;
       const float4 w4 = wt[j];
       float a0 = v.x * fq * w4.x, a1 = v.y * fq * w4.y, a2 = v.z * fq * w4.z, a3 = v.w * fq * w4.w;
-      if constexpr (SHAPED) turn(e, a0, a1, a2, a3);
+      if constexpr (SHAPED) turn(true, e, a0, a1, a2, a3);
       Pack4<T>::store(qo + h * pad + e, a0, a1, a2, a3);
     } else if (i < Q + K) {
       const int ik = i - Q, g = ik / d, e = ik - g * d;
       const float4 w4 = wt[j];
       float a0 = v.x * fk * w4.x, a1 = v.y * fk * w4.y, a2 = v.z * fk * w4.z, a3 = v.w * fk * w4.w;
-      if constexpr (SHAPED) turn(e, a0, a1, a2, a3);
+      if constexpr (SHAPED) turn(false, e, a0, a1, a2, a3);
       if (SHAPED && v_from_k) {                             // the key as projected is the value
         if (v_rows != nullptr) {
           Pack4<T>::store(v_rows + (size_t)t * n_kv_heads * pad + g * pad + e, v.x, v.y, v.z, v.w);
