@@ -258,6 +258,30 @@ def test_packing_kernel_rounds_rotations_one_way(dtype, H, G, d, rot):
     assert torch.equal(k.cpu().permute(0, 2, 1, 3).reshape(T, G, pad)[..., :d], turned(raw[:, H * d:(H + G) * d], False))
 
 
+# Short rows of many tokens are taken by one wave or two each, of few by four: the same bits on both sides of every change
+@pytest.mark.parametrize("T", [1024, 1025, 1537, 3073])
+@pytest.mark.parametrize("H,G,d,rot", [(4, 1, 64, 64), (6, 1, 128, 0), (5, 1, 148, 20), (12, 2, 128, 128)])
+def test_packing_kernel_of_short_rows_and_many_tokens(T, H, G, d, rot):
+    from yalm_amd.ops import kernels
+    ring, pad = (T + 63) // 64, (d + 15) // 16 * 16
+    raw = randn(T, (H + 2 * G) * d, seed=H).to(DEV)
+    wq, wk = (1 + randn(n, seed=s, scale=0.2).to(DEV) for s, n in ((1, H * d), (2, G * d)))
+    angles = randn(T, max(rot, 2) // 2, seed=4)
+    cos_sin = torch.stack([angles.cos(), angles.sin()], dim=-1).contiguous().to(DEV) if rot else None
+    table = torch.arange(ring, dtype=torch.int32, device=DEV).reshape(1, ring)
+    out = []
+    for size in (T, 400):                         # 32 tokens and more in every share
+        q = torch.full((T, H * pad), float("nan"), device=DEV)
+        kp, vp = torch.zeros(ring, G, 64, pad, device=DEV), torch.zeros(ring, G, pad, 64, device=DEV)
+        for lo in range(0, T, size):
+            n = min(size, T - lo)
+            kernels.qkv_pack(raw[lo:lo + n], None, wq, wk, 1e-5, None, 1.7, None, 0, None, q[lo:lo + n], None, None, None, kp, vp, table, ring,
+                             i32([0] * n), i32(range(lo, lo + n)), i32([0]), i32([T]), H, G, d, d, pad, cos_sin=cos_sin, rot_dims=rot)
+        out.append((q, kp, vp))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
 # The same with the middle in the first product's epilogue: one to 16 rows (K a multiple of 64 and not), to 128, tiles of 128 rows,
 # larger tiles, K in slices and whole; hidden values that end inside a block; streams narrower and wider than what one
 # element a thread covers; and the general kernels

@@ -164,7 +164,10 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
 // level with one of the waves' sums: 1,909 rows of 6,144 20.9 and 21.1 us).  For rows whose parts and heads are multiples of four elements (a thread takes four consecutive ones at a time) and at most
 // 1,024 * NV elements.  A workgroup of four waves a token: with a wave a token, 24 rounds of a row of 6,144 and its weights were 250
 // registers, two waves a SIMD and too few loads in flight (1,909 tokens inside a step 43.8 -> 31.9 us; 32
-// tokens alone 19.5 -> 6.8, 2,048 33.9 -> 24.5; rows of 1,536 5.3 -> 3.5 and 8.3 -> 8.1).  Rows of up to 256 are a wave's (2,048 of them 4.2 us, with four waves 5.5).
+// tokens alone 19.5 -> 6.8, 2,048 33.9 -> 24.5; rows of 1,536 5.3 -> 3.5 and 8.3 -> 8.1).  Rows of up to 256 are a wave's (2,048 of them 4.2 us, with four waves 5.5), and so are those of up to
+// 2,048 where tokens are many: each of the four has next to nothing to load and the chip holds 2,048 workgroups of four.  us with four waves, two
+// and one, rows of 384: 1,000 tokens 4.5 4.1 4.3, 1,909 6.0 5.0 4.6, 4,000 9.7 7.5 6.2; of 1,024 4.8 4.6 5.0, 6.8 6.2 6.6, 11.5 9.5 9.0; of 1,344
+// 5.7 5.7 7.1, 9.6 7.9 8.9, 14.4 12.8 11.7; of 2,048 7.3 7.7 9.8, 11.4 10.1 11.0, 18.4 16.9 15.9; of 2,304 and more four are the soonest or level.
 template <typename T> struct Pack4;
 template <> struct Pack4<float> {
   static __device__ __forceinline__ void store(float* p, float a, float b, float c, float d) {
@@ -291,8 +294,13 @@ __global__ __launch_bounds__(PV_THREADS) void qkv_pack_vec_kernel(
     a0 = x, a1 = y;
   };
   auto turn = [&](bool q, int e, float& a0, float& a1, float& a2, float& a3) {
-    if (e < rot_dims) turn_pair(q, same_place ? turn0 : cs[e >> 1], a0, a1);
-    if (e + 2 < rot_dims) turn_pair(q, same_place ? turn1 : cs[(e >> 1) + 1], a2, a3);
+    if (same_place) {                             // two ways, so that this one waits for no load (and for no store in front of it)
+      if (e < rot_dims) turn_pair(q, turn0, a0, a1);
+      if (e + 2 < rot_dims) turn_pair(q, turn1, a2, a3);
+    } else {
+      if (e < rot_dims) turn_pair(q, cs[e >> 1], a0, a1);
+      if (e + 2 < rot_dims) turn_pair(q, cs[(e >> 1) + 1], a2, a3);
+    }
   };
   long page = -1, tile = -1;
   if (slot >= 0 && pos >= 0 && k_pages != nullptr) {
@@ -506,10 +514,13 @@ extern "C" int yalm_qkv_pack(const float* qkv, long qkv_row, const float* bias, 
       v_from_k, (const float2*)cos_sin, rot_dims, n_positions)
 #define YALM_PACK_WN(TYPE)                                                                                               \
   if (n_row <= 256) YALM_PACK_W(TYPE, 1, 64);                                                                            \
-  else if (n_row <= 1024) YALM_PACK_W(TYPE, 1, 256);                                                                             \
-  else if (n_row <= 1024 * 2) YALM_PACK_W(TYPE, 2, 256);                                                                      \
-  else if (n_row <= 1024 * 4) YALM_PACK_W(TYPE, 4, 256);                                                                      \
-  else if (n_row <= 1024 * 6) YALM_PACK_W(TYPE, 6, 256);                                                                      \
+  else if (n_row <= 1024 && T > 1024) YALM_PACK_W(TYPE, 4, 64);                                                          \
+  else if (n_row <= 1024) YALM_PACK_W(TYPE, 1, 256);                                                                     \
+  else if (n_row <= 1024 * 2 && T > 3072) YALM_PACK_W(TYPE, 8, 64);                                                      \
+  else if (n_row <= 1024 * 2 && T > 1536) YALM_PACK_W(TYPE, 4, 128);                                                     \
+  else if (n_row <= 1024 * 2) YALM_PACK_W(TYPE, 2, 256);                                                                 \
+  else if (n_row <= 1024 * 4) YALM_PACK_W(TYPE, 4, 256);                                                                 \
+  else if (n_row <= 1024 * 6) YALM_PACK_W(TYPE, 6, 256);                                                                 \
   else YALM_PACK_W(TYPE, 8, 256)
     if (dtype == YALM_F32) {
       YALM_PACK_WN(float);
