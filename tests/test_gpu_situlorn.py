@@ -100,6 +100,13 @@ def test_norm_add_pair_has_the_bits_of_its_three_steps(R_, D, dtype, off):
     assert torch.equal(one, both) and torch.equal(h1, h2)
 
 
+# the ends of the narrow forms, and of wide pairs both ways of asking for what stands behind the sums
+@pytest.mark.parametrize("R_,D", [(3, 255), (2, 256), (2, 257), (256, 4100), (257, 4100), (257, 8192)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_norm_add_pair_has_these_bits_in_all_its_forms(R_, D, dtype):
+    test_norm_add_pair_has_the_bits_of_its_three_steps(R_, D, dtype, 0)
+
+
 @pytest.mark.parametrize("R_,F", [(1, 4), (7, 112), (20, 1500), (3, 8200), (2, 40001)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_polynorm(R_, F, out_dtype):

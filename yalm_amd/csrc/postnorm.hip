@@ -23,14 +23,18 @@ __global__ __launch_bounds__(ROW_THREADS) void cast_kernel(const float* __restri
 // bits of the norm's own kernel (next_vec: rms_row_vec; the row goes through LDS to the threads that sum it there).  Bound by memory in a
 // prompt (x, y, y2 once each way: a second launch for y2 and a norm kernel behind it would read and write x twice more:
 // 1,909 rows of 4,096 24 + 24 + 10 -> 42 us), by the launch in a decode step (three of 4.6 us -> one of 6.5).  Rows of up to 4,096
-// elements keep four a thread, and everything is asked for at once: 1,909 rows 38.5 -> 33.1 us (137 MB), 5 rows 6.5 -> 5.0.
-template <typename W, typename T, int NT, int PER, bool PAIR>
+// elements keep four a thread, and everything is asked for at once: 1,909 rows 38.5 -> 33.1 us (137 MB), 5 rows 6.5 -> 5.0.  Not
+// for a pair of wider rows than that with more rows than compute units: 80 to 86 registers leave a unit one workgroup of two (1,909 rows of 5,120
+// 51.3 us, asked for behind the sums 43.7; 300 rows 11.8 and 10.4; 5 rows 5.3 and 5.8).  Narrow rows have no more rounds a thread than they
+// fill (1,909 rows of 256 6.8 -> 5.0, of 1,024 10.5 -> 9.4).
+template <typename W, typename T, int NT, int PER, bool PAIR, bool AHEAD>
 __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ y, const W* __restrict__ w,
                                                       const float* __restrict__ y2, const W* __restrict__ w2, float eps,
                                                       float* __restrict__ x, T* __restrict__ h, const float* __restrict__ next_w,
                                                       float next_eps, bool next_vec, int D) {
-  // PER > 0: the row fits PER values a thread; y is read once and the new x stays in registers for the second norm.  All that the
-  // row needs is asked for in front of its sums, and the barriers of both sums, which are one, leave it in flight
+  // PER > 0: the row fits PER values a thread; y is read once and the new x stays in registers for the second norm.  AHEAD: all that
+  // the row needs is asked for in front of its sums, and the barriers of both sums, which are one, leave it in flight
+  static_assert(PER > 0 || !AHEAD, "a row that is not kept is not asked for");
   __shared__ float2 red2[NT / WAVE];
   __shared__ float red[NT / WAVE];
   const size_t row = (size_t)blockIdx.x * D;
@@ -45,16 +49,18 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
       keep[j] = i < D ? y[row + i] : 0.f;
       if constexpr (PAIR) keep2[j] = i < D ? y2[row + i] : 0.f;
     }
+    if constexpr (AHEAD) {
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int i = min((int)threadIdx.x + j * NT, D - 1);
-      had[j] = x[row + i];
-      wk[j] = w[i];
-      if constexpr (PAIR) wk2[j] = w2[i];
-    }
-    if (next_w != nullptr) {
+      for (int j = 0; j < PER; ++j) {
+        const int i = min((int)threadIdx.x + j * NT, D - 1);
+        had[j] = x[row + i];
+        wk[j] = w[i];
+        if constexpr (PAIR) wk2[j] = w2[i];
+      }
+      if (next_w != nullptr) {
 #pragma unroll
-      for (int j = 0; j < PER; ++j) nw[j] = next_w[min((int)threadIdx.x + j * NT, D - 1)];
+        for (int j = 0; j < PER; ++j) nw[j] = next_w[min((int)threadIdx.x + j * NT, D - 1)];
+      }
     }
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
@@ -68,16 +74,23 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
       if constexpr (PAIR) sp += y2[row + i] * y2[row + i];
     }
   }
-  const float2 both = block_sum2<NT / WAVE>(ss, sp, red2);
-  const float scale = 1.0f / sqrtf(both.x / (float)D + eps), scale_p = PAIR ? 1.0f / sqrtf(both.y / (float)D + eps) : 0.f;
+  if constexpr (AHEAD) {
+    const float2 both = block_sum2<NT / WAVE>(ss, sp, red2);
+    ss = both.x;
+    sp = both.y;
+  } else {
+    ss = block_sum<NT / WAVE>(ss, red);
+    if constexpr (PAIR) sp = block_sum<NT / WAVE>(sp, red);
+  }
+  const float scale = 1.0f / sqrtf(ss / (float)D + eps), scale_p = PAIR ? 1.0f / sqrtf(sp / (float)D + eps) : 0.f;
   float ss2 = 0.f;
   if (PER > 0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
       if (i < D) {
-        float v = had[j] + keep[j] * scale * to_f32(wk[j]);
-        if constexpr (PAIR) v += keep2[j] * scale_p * to_f32(wk2[j]);
+        float v = (AHEAD ? had[j] : x[row + i]) + keep[j] * scale * to_f32(AHEAD ? wk[j] : w[i]);
+        if constexpr (PAIR) v += keep2[j] * scale_p * to_f32(AHEAD ? wk2[j] : w2[i]);
         x[row + i] = v;
         keep[j] = v;
         ss2 += v * v;
@@ -108,7 +121,7 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * NT;
-      if (i < D) h[row + i] = from_f32<T>(keep[j] * scale2 * nw[j]);
+      if (i < D) h[row + i] = from_f32<T>(keep[j] * scale2 * (AHEAD ? nw[j] : next_w[i]));
     }
   } else {
     for (int i = threadIdx.x; i < D; i += NT) h[row + i] = from_f32<T>(x[row + i] * scale2 * next_w[i]);   // its own stores
@@ -347,14 +360,17 @@ extern "C" int yalm_cast(const float* x, void* out, long n, int out_dtype, hipSt
 template <typename W, typename T, bool PAIR>
 static int norm_add_launch(const float* y, const void* w, const float* y2, const void* w2, float eps, float* x, void* h,
                            const float* next_w, float next_eps, int R, int D, hipStream_t stream) {
-#define NA(NT_, PER_) \
-  norm_add_kernel<W, T, NT_, PER_, PAIR><<<R, NT_, 0, stream>>>(y, (const W*)w, y2, (const W*)w2, eps, x, (T*)h, next_w, next_eps, \
-                                                          next_vec, D)
+#define NA(NT_, PER_, AHEAD_) \
+  norm_add_kernel<W, T, NT_, PER_, PAIR, AHEAD_><<<R, NT_, 0, stream>>>(y, (const W*)w, y2, (const W*)w2, eps, x, (T*)h, next_w, next_eps, \
+                                                                  next_vec, D)
   const bool next_vec = rms_row_vec(x, h, D);
-  if (D < 2048) NA(256, 8);
-  else if (D <= 4096) NA(1024, 4);
-  else if (D <= 8192) NA(1024, 8);
-  else NA(1024, 0);
+  if (D <= 256) NA(256, 1, true);
+  else if (D <= 1024) NA(256, 4, true);
+  else if (D < 2048) NA(256, 8, true);
+  else if (D <= 4096) NA(1024, 4, true);
+  else if (D > 8192) NA(1024, 0, false);
+  else if (PAIR && R > 256) NA(1024, 8, false);
+  else NA(1024, 8, true);
 #undef NA
   return launch_status();
 }
