@@ -357,6 +357,20 @@ def test_short_prompts_and_the_steps_behind_them(folders, name, lens):
                              "%s prompts %s, sequence %d" % (name, lens, i))
 
 
+def test_more_short_prompts_than_one_launch_takes(folders):
+    """65,536 prompts of one token each, with heads that the launch for one-tile prompts is built for: one sequence more than it
+    takes.  What follows a token hangs on the token alone, so equal prompts have equal rows."""
+    n, kinds = 65536, 8
+    engine = make_engine(folders, "tiny_long", "bfloat16", max_tokens=n * 64, max_batch=n)
+    slots = engine.start(n)
+    out = engine.step(slots, [[3 + i % kinds] for i in range(n)])
+    for k in range(kinds):
+        rows = out[k::kinds]
+        assert torch.equal(rows, rows[:1].expand_as(rows))
+        helpers.check_logits(rows[:1].cpu().numpy(), helpers.plain_logits(folders["tiny_long"], (3 + k,), "bfloat16"), "bfloat16",
+                             "%d prompts, token %d" % (n, 3 + k))
+
+
 def test_a_step_whose_widest_buffer_would_pass_the_checked_size_is_refused(folders):
     from yalm_amd.engine.engine import StepError
     engine = make_engine(folders, "tiny_llama", "float32", max_tokens=1024)

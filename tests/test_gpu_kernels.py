@@ -920,6 +920,25 @@ def test_attn_tile(n_heads, n_kv, hd, rd, lens, slices):
     assert torch.equal(kp0, kp1) and torch.equal(vp0, vp1) and kp0.abs().sum() > 0
 
 
+def test_attn_tile_says_which_steps_it_takes():
+    """Operands off 16 bytes, more sequences than a launch has room for and more tiles than sequences are left to the kernels
+    that it stands for."""
+    k = K()
+    hd, B = 64, 3
+    qkv, kp = torch.zeros(1 + B * 3 * hd, device=DEV), torch.zeros(B, 1, k.PAGE, hd, dtype=torch.bfloat16, device=DEV)
+    vp, out = torch.zeros(B, 1, hd, k.PAGE, dtype=torch.bfloat16, device=DEV), torch.zeros(1 + B * hd, dtype=torch.bfloat16, device=DEV)
+
+    def fits(x=qkv[:-1], o=out[:-1], *rest):
+        return k.attn_tile_fits(x, o, kp, vp, hd, 0, *rest)
+    assert fits() and not fits(qkv[1:]) and not fits(o=out[1:])
+    assert k.attn_tile_fits(qkv, out, kp, vp, hd, 0, 65535) and not k.attn_tile_fits(qkv, out, kp, vp, hd, 0, 65536)
+    table, cu = torch.arange(B, dtype=torch.int32, device=DEV).reshape(B, 1), i32([0, 1, 2, 3])
+    with pytest.raises(RuntimeError):
+        k.attn_tile(qkv[:-1].view(B, 3 * hd), out[:-1].view(B, hd), kp, vp, table, 1, cu, i32([0, 1, 2]), None, 1, 1, hd, 0, n_tiles=B + 1)
+    k.attn_tile(qkv[:-1].view(B, 3 * hd), out[:-1].view(B, hd), kp, vp, table, 1, cu, i32([0, 1, 2]), None, 1, 1, hd, 0, n_tiles=B)
+    assert out.abs().sum() == 0
+
+
 def masked_attention_float64(q, k, v, n_heads, n_kv, hd, window, bias=None):
     """softmax(q k^T / sqrt(hd) + mask) v for one sequence, all positions at once (float64).  bias ([n_heads,
     distances], optional): bias[h, min(i - j, distances - 1)] is added to the score of query i and key j."""

@@ -651,19 +651,24 @@ def rope_kv_write_tiles(qkv, q_out, k_stage, v_stage, cu_seqlens, seq_tile0, k_p
 TILE_HEAD_DIMS = (64, 128)      # head sizes that attn_tile is built for
 
 
-def attn_tile_fits(qkv, out, k_pages, v_pages, head_dim, window):
-    """Whether attn_tile takes a step of sequences of one tile each: bfloat16, a window that hides none of a tile's keys, and operands
-    on 16 bytes."""
+TILE_MAX_SEQS = 65535           # sequences that it takes in a step (the launch's second dimension)
+
+
+def attn_tile_fits(qkv, out, k_pages, v_pages, head_dim, window, n_seqs=1):
+    """Whether attn_tile takes a step of n_seqs sequences of one tile each: bfloat16, a window that hides none of a tile's keys, and
+    operands on 16 bytes."""
     return out.dtype == torch.bfloat16 and not FORCE_SIMPLE and head_dim in TILE_HEAD_DIMS and (window <= 0 or window >= PAGE) and \
+        n_seqs <= TILE_MAX_SEQS and \
         (qkv.data_ptr() | out.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0
 
 
 def attn_tile(qkv, out, k_pages, v_pages, block_table, ring_pages, cu_seqlens, seq_slot, cos_sin, n_heads, n_kv_heads, head_dim,
-              rotary_dim, slices=1, layout=None):
+              rotary_dim, slices=1, layout=None, n_tiles=None):
     """What rope_kv_write and attn_prefill do with a step of whole prompts of at most 64 tokens each, in one launch: qkv float32
     (as rope_kv_write takes it) is rotated, keys and values go to the first page of each sequence, and out (bfloat16 [T, n_heads *
-    head_dim]) is the causal attention of every sequence over its own keys.  attn_tile_fits says which steps are taken.  The caller
-    sees to it that no sequence of cu_seqlens is longer than PAGE."""
+    head_dim]) is the causal attention of every sequence over its own keys.  attn_tile_fits says which steps are taken.  n_tiles: the
+    tiles of the step's sequences; a step of more tiles than sequences is refused (None: the caller sees to it that no sequence
+    of cu_seqlens is longer than PAGE)."""
     _check_heads(n_heads, n_kv_heads, head_dim)
     T = out.shape[0]
     Q, KV = n_heads * head_dim, n_kv_heads * head_dim
@@ -694,7 +699,7 @@ def attn_tile(qkv, out, k_pages, v_pages, block_table, ring_pages, cu_seqlens, s
     else:
         rotary_dim = 0
     library.check(library.lib().yalm_attn_tile(
-        p_qkv, p_o, p_kp, p_vp, p_bt, stride, p_cu, p_sl, p_cs, n_pos, T, B, B, n_heads, n_kv_heads, head_dim, rotary_dim, n_pages,
+        p_qkv, p_o, p_kp, p_vp, p_bt, stride, p_cu, p_sl, p_cs, n_pos, T, B, B if n_tiles is None else int(n_tiles), n_heads, n_kv_heads, head_dim, rotary_dim, n_pages,
         _layout(layout, head_dim), int(slices), _stream()), "attn_tile")
     return out
 

@@ -331,11 +331,11 @@ class GQAttention(Part):
         o = ws.get("attn.o", (T, self.q_dim), act)
         # short prompts, every sequence one tile of keys that nobody reads again in this step: rotation, cache write and attention
         # are one kernel
-        if prefill and writes_cache and ctx.tables["kv_tiles"]["n_tiles"] == ctx.seq_slot.shape[0] and not self.sinks \
-                and self.score_bias is None and not ctx.line_is_shared(line) \
-                and kernels.attn_tile_fits(qkv, o, k_pages, v_pages, self.head_dim, self.window):
+        n_seqs, n_tiles = ctx.seq_slot.shape[0], ctx.tables["kv_tiles"]["n_tiles"] if prefill else 0
+        if prefill and writes_cache and n_tiles == n_seqs and not self.sinks and self.score_bias is None and not ctx.line_is_shared(line) \
+                and kernels.attn_tile_fits(qkv, o, k_pages, v_pages, self.head_dim, self.window, n_seqs):
             kernels.attn_tile(qkv, o, k_pages, v_pages, group.table, group.ring_pages, ctx.cu_seqlens, ctx.seq_slot, pos.table,
-                              self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices)
+                              self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices, n_tiles=n_tiles)
         else:
             self._rotate_and_attend(qkv, slices, o, ctx, group, line, k_pages, v_pages, writes_cache)
         emit = self._emit_args(emit_for, ctx, T, self.dim) if prefill and kernels.can_chain(T, self.q_dim, act) else None
