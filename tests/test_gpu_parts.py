@@ -370,6 +370,68 @@ def test_toy_mixer_and_architecture_from_outside(tmp_path, mixer, window, sinks)
         unregister_part("mixer", "toy_running_mean_on_device")
 
 
+class MixedBlocksConfig:
+    """Layers whose products prepare the norm that reads the stream next, in front of layers that take a finished norm only."""
+
+    def __init__(self, d):
+        self.d = d
+
+    @classmethod
+    def from_dict(cls, d):
+        return cls(d)
+
+    def to_dict(self):
+        return dict(self.d)
+
+    def to_spec(self):
+        from yalm_amd.config import LayerSpec, ModelSpec, PartSpec
+        D, eps = self.d["width"], {"eps": 1e-5}
+
+        def norm(name):
+            return PartSpec("rmsnorm", eps, prefix=name + ".")
+        pos = PartSpec("rope", {"head_dim": 64, "rotary_dim": 64, "theta": 100.0, "scaling": None, "weight_rows": "interleaved"})
+        attention = PartSpec("gqa_attention", {"n_heads": 2, "n_kv_heads": 1, "head_dim": 64, "position": pos}, prefix="attn.")
+        recurrence = PartSpec("hgrn2", {"n_heads": 2, "key_dim": 32, "value_dim": 32}, prefix="rec.")
+        layers = []
+        for i, kind in enumerate(self.d["blocks"]):
+            mlp = PartSpec("swiglu", {"hidden": 96}, prefix="ff.")
+            if kind == "prenorm_residual":
+                members = dict(mixer_norm=norm("n1"), mixer=attention, feed_forward_norm=norm("n2"), feed_forward=mlp)
+            elif kind == "parallel_residual":
+                members = dict(norm=norm("n1"), mixer=attention, feed_forward=mlp)
+            else:
+                members = dict(mixer_norm=norm("n1"), mixer=recurrence, mixer_out_norm=norm("n1b"), feed_forward_norm=norm("n2"),
+                               feed_forward=mlp, feed_forward_out_norm=norm("n2b"))
+            layers.append(LayerSpec(kind, parts=members, prefix="m.%d." % i))
+        return ModelSpec("MixedBlocks", D, 61, 200, PartSpec("token_embedding", {"vocab_size": 61}, prefix="emb."), layers, norm("last"),
+                         PartSpec("lm_head", {"vocab_size": 61, "tied": True}))
+
+
+@pytest.mark.parametrize("second", ["sandwich_residual", "parallel_residual", "prenorm_residual"])
+def test_a_norm_that_is_prepared_reaches_no_layer_that_takes_finished_ones(tmp_path, monkeypatch, second):
+    """bfloat16 prompts of up to 16 tokens and the steps behind them, with products that prepare the next norm and with none that do."""
+    from yalm_amd import Engine, Model, register_architecture, write_random_model
+    from yalm_amd.config import unregister_architecture
+    from yalm_amd.ops import kernels
+    register_architecture("MixedBlocks", MixedBlocksConfig, replace=True)
+    try:
+        d = {"architectures": ["MixedBlocks"], "width": 128, "blocks": ["prenorm_residual", second, "prenorm_residual", second]}
+        model = Model.from_folder(write_random_model(str(tmp_path / "mixed"), d, seed=6), dtype=torch.bfloat16, device=DEV)
+        rows = []
+        for chain in (True, False):
+            if not chain:
+                monkeypatch.setattr(kernels, "can_chain", lambda M, K, dtype: False)
+            engine, got = Engine(model, max_tokens=1024, use_graphs=False), []
+            slots = engine.start(2)
+            got.append(engine.step(slots, [[5, 9, 60, 3, 3, 17, 44], [8, 0]], [list(range(7)), [0, 1]]).cpu().numpy())
+            for tok in (31, 7):
+                got.append(engine.step(slots, [[tok], [tok + 1]]).cpu().numpy())
+            rows.append(np.concatenate(got))
+        helpers.check_logits(rows[0], rows[1], "bfloat16", "norms prepared, %s behind" % second)
+    finally:
+        unregister_architecture("MixedBlocks")
+
+
 # ---------------------------------------------------------------------------
 # a toy feed-forward with routing and a toy position encoding, in a second toy architecture
 # ---------------------------------------------------------------------------

@@ -234,12 +234,12 @@ class SandwichResidualBlock(Part):
         import torch
         T = x.shape[0]
         y = ctx.ws.get("block.y", (T, self.dim), torch.float32)
-        h = ctx.ws.get("block.h", (T, self.dim), ctx.act_dtype)
         left = ctx.normed.pop(id(self.mixer_norm), None)
-        if left is None:
-            self.mixer_norm.forward(x, h, ctx)
-        else:                                             # the layer before has left this norm's output
+        if left is not None and left[1] is None:          # the layer before has left this norm's output
             h = left[0]
+        else:
+            h = ctx.ws.get("block.h", (T, self.dim), ctx.act_dtype)
+            self.mixer_norm.forward(x, h, ctx)
         bias = getattr(self.mixer, "late_bias", None)
         self.mixer.forward_to(h, y, ctx, line, writes_cache, **({} if bias is None else {"late_bias_taken": True}))
         after = next_norm if self.feed_forward is None else self.feed_forward_norm
