@@ -384,7 +384,7 @@ class MixedBlocksConfig:
         return dict(self.d)
 
     def to_spec(self):
-        from yalm_amd.config import LayerSpec, ModelSpec, PartSpec
+        from yalm_amd.config import LayerSpec, ModelSpec, PartSpec, ScheduleEntry
         D, eps = self.d["width"], {"eps": 1e-5}
 
         def norm(name):
@@ -393,6 +393,7 @@ class MixedBlocksConfig:
         attention = PartSpec("gqa_attention", {"n_heads": 2, "n_kv_heads": 1, "head_dim": 64, "position": pos}, prefix="attn.")
         recurrence = PartSpec("hgrn2", {"n_heads": 2, "key_dim": 32, "value_dim": 32}, prefix="rec.")
         layers = []
+        readers = [ScheduleEntry(i, 0, writes_cache=False) for i in range(self.d.get("readers", 0))]      # of the first layer's keys and values
         for i, kind in enumerate(self.d["blocks"]):
             mlp = PartSpec("swiglu", {"hidden": 96}, prefix="ff.")
             if kind == "prenorm_residual":
@@ -404,32 +405,81 @@ class MixedBlocksConfig:
                                feed_forward=mlp, feed_forward_out_norm=norm("n2b"))
             layers.append(LayerSpec(kind, parts=members, prefix="m.%d." % i))
         return ModelSpec("MixedBlocks", D, 61, 200, PartSpec("token_embedding", {"vocab_size": 61}, prefix="emb."), layers, norm("last"),
-                         PartSpec("lm_head", {"vocab_size": 61, "tied": True}))
+                         PartSpec("lm_head", {"vocab_size": 61, "tied": True}),
+                         schedule=[ScheduleEntry(i, i) for i in range(len(layers))] + readers if readers else None)
+
+
+@pytest.fixture
+def mixed_blocks(tmp_path):
+    """make(blocks, ...): a bfloat16 model of such layers, 128 wide."""
+    from yalm_amd import Model, register_architecture, write_random_model
+    from yalm_amd.config import unregister_architecture
+
+    def make(blocks, **more):
+        d = {"architectures": ["MixedBlocks"], "width": 128, "blocks": blocks, **more}
+        return Model.from_folder(write_random_model(str(tmp_path / "mixed"), d, seed=6), dtype=torch.bfloat16, device=DEV)
+    register_architecture("MixedBlocks", MixedBlocksConfig, replace=True)
+    yield make
+    unregister_architecture("MixedBlocks")
+
+
+@pytest.mark.parametrize("n_tok,tiles,prepared", [([9], 3, 5), ([16], 3, 5), ([9, 8], 3, 0), ([64], 3, 0), ([65], 0, 0), ([3, 65], 0, 0)])
+def test_short_prompts_take_the_launches_that_are_made_for_them(mixed_blocks, monkeypatch, n_tok, tiles, prepared):
+    """Three layers: the one-tile attention in each up to 64 tokens a sequence; up to 16 tokens in all every norm but the first layer's
+    first and the last, which the head does for the rows that are asked for, is prepared by the product in front of it."""
+    from yalm_amd import Engine
+    from yalm_amd.ops import kernels
+    calls = {"attn_tile": 0, "prepared": 0}
+    attn_tile, gemm_chain = kernels.attn_tile, kernels.gemm_chain
+
+    def count_tile(*a, **kw):
+        calls["attn_tile"] += 1
+        return attn_tile(*a, **kw)
+
+    def count_chain(*a, **kw):
+        calls["prepared"] += kw.get("emit") is not None
+        return gemm_chain(*a, **kw)
+    engine = Engine(mixed_blocks(["prenorm_residual"] * 3), max_tokens=1024)
+    monkeypatch.setattr(kernels, "attn_tile", count_tile)
+    monkeypatch.setattr(kernels, "gemm_chain", count_chain)
+    engine.step(engine.start(len(n_tok)), [list(range(2, 2 + min(n, 50))) + [7] * max(0, n - 50) for n in n_tok])
+    assert calls == {"attn_tile": tiles, "prepared": prepared}
+
+
+@pytest.mark.parametrize("n_tok", [[9], [64, 20]])
+def test_keys_that_a_later_layer_reads_are_not_left_out_by_one_tile_attention(mixed_blocks, monkeypatch, n_tok):
+    """A layer whose line is read again in the step keeps its keys and values for the reader (two launches); the layer behind it,
+    whose line nobody reads, takes one.  The bits of a step that takes two everywhere."""
+    from yalm_amd import Engine
+    from yalm_amd.ops import kernels
+    model, rows, taken = mixed_blocks(["prenorm_residual"] * 2, readers=1), [], []
+    attn_tile = kernels.attn_tile
+    monkeypatch.setattr(kernels, "attn_tile", lambda *a, **kw: (taken.append(1), attn_tile(*a, **kw))[1])
+    for one_launch in (True, False):
+        if not one_launch:
+            monkeypatch.setattr(kernels, "attn_tile_fits", lambda *a: False)
+        engine = Engine(model, max_tokens=1024)
+        tokens = [[(5 * i + k) % 61 for k in range(n)] for i, n in enumerate(n_tok)]
+        rows.append(engine.step(engine.start(len(n_tok)), tokens, [list(range(n)) for n in n_tok]).clone())
+    assert len(taken) == 1 and torch.equal(*rows)
 
 
 @pytest.mark.parametrize("second", ["sandwich_residual", "parallel_residual", "prenorm_residual"])
-def test_a_norm_that_is_prepared_reaches_no_layer_that_takes_finished_ones(tmp_path, monkeypatch, second):
+def test_a_norm_that_is_prepared_reaches_no_layer_that_takes_finished_ones(mixed_blocks, monkeypatch, second):
     """bfloat16 prompts of up to 16 tokens and the steps behind them, with products that prepare the next norm and with none that do."""
-    from yalm_amd import Engine, Model, register_architecture, write_random_model
-    from yalm_amd.config import unregister_architecture
+    from yalm_amd import Engine
     from yalm_amd.ops import kernels
-    register_architecture("MixedBlocks", MixedBlocksConfig, replace=True)
-    try:
-        d = {"architectures": ["MixedBlocks"], "width": 128, "blocks": ["prenorm_residual", second, "prenorm_residual", second]}
-        model = Model.from_folder(write_random_model(str(tmp_path / "mixed"), d, seed=6), dtype=torch.bfloat16, device=DEV)
-        rows = []
-        for chain in (True, False):
-            if not chain:
-                monkeypatch.setattr(kernels, "can_chain", lambda M, K, dtype: False)
-            engine, got = Engine(model, max_tokens=1024, use_graphs=False), []
-            slots = engine.start(2)
-            got.append(engine.step(slots, [[5, 9, 60, 3, 3, 17, 44], [8, 0]], [list(range(7)), [0, 1]]).cpu().numpy())
-            for tok in (31, 7):
-                got.append(engine.step(slots, [[tok], [tok + 1]]).cpu().numpy())
-            rows.append(np.concatenate(got))
-        helpers.check_logits(rows[0], rows[1], "bfloat16", "norms prepared, %s behind" % second)
-    finally:
-        unregister_architecture("MixedBlocks")
+    model, rows = mixed_blocks(["prenorm_residual", second, "prenorm_residual", second]), []
+    for chain in (True, False):
+        if not chain:
+            monkeypatch.setattr(kernels, "can_chain", lambda M, K, dtype: False)
+        engine, got = Engine(model, max_tokens=1024, use_graphs=False), []
+        slots = engine.start(2)
+        got.append(engine.step(slots, [[5, 9, 60, 3, 3, 17, 44], [8, 0]], [list(range(7)), [0, 1]]).cpu().numpy())
+        for tok in (31, 7):
+            got.append(engine.step(slots, [[tok], [tok + 1]]).cpu().numpy())
+        rows.append(np.concatenate(got))
+    helpers.check_logits(rows[0], rows[1], "bfloat16", "norms prepared, %s behind" % second)
 
 
 # ---------------------------------------------------------------------------

@@ -121,6 +121,7 @@ def decode_counters(ctx, B, n_heads, n_kv_heads, n_splits):
 @part("mixer", "gqa_attention")
 class GQAttention(Part):
     prompt_tables = (kv_tiles,)
+    takes_prepared_prompts = True
 
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
@@ -269,7 +270,7 @@ class GQAttention(Part):
                                   self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices)
         o = ctx.ws.get("attn.o", (T, self.q_dim), self.wo.dtype)
         self._decode_attention(q, o, ctx, group, line, k_pages, v_pages, True)
-        emit = self._emit_args(emit_for, ctx, T, self.dim)
+        emit = self._emit_args(emit_for, ctx, x)
         prepared = self._add_emit_args(emit_for, ctx, T, self.dim, self.q_dim) if emit is None else None
         ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.q_dim) if emit is None and prepared is None else None
         if emit is not None and kernels.can_chain(T, self.q_dim, o.dtype):
@@ -338,7 +339,7 @@ class GQAttention(Part):
                               self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices, n_tiles=n_tiles)
         else:
             self._rotate_and_attend(qkv, slices, o, ctx, group, line, k_pages, v_pages, writes_cache)
-        emit = self._emit_args(emit_for, ctx, T, self.dim) if prefill and kernels.can_chain(T, self.q_dim, act) else None
+        emit = self._emit_args(emit_for, ctx, x) if prefill and kernels.can_chain(T, self.q_dim, act) else None
         ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.q_dim) if prefill and emit is None else None
         if emit is not None:                      # up to 16 tokens: the product prepares the next norm, as in a decode step
             nw2, xn2, ss2, eps2 = emit

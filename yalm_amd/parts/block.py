@@ -23,6 +23,9 @@ class PreNormResidualBlock(Part):
         if layer_spec.part("mixer_input") is not None:
             self.mixer_input = build_part("input_filter", layer_spec.mixer_input, dim, p)
             self.mixer_norm.taken_by = self.mixer_input
+        self.mixer_norm.read_by = self.mixer if self.mixer_input is None else None
+        if self.feed_forward is not None:
+            self.feed_forward_norm.read_by = self.feed_forward
 
     def children(self):
         return [c for c in (self.mixer_norm, self.mixer_input, self.mixer, self.feed_forward_norm, self.feed_forward)

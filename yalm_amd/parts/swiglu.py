@@ -33,6 +33,8 @@ def interleave_gate_up(gate, up):
 
 @part("feed_forward", "swiglu")
 class SwiGLU(Part):
+    takes_prepared_prompts = True
+
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
         self.hidden = int(spec.params["hidden"])
@@ -96,7 +98,7 @@ class SwiGLU(Part):
             h = ctx.ws.get("block.h", (T, self.dim), ctx.act_dtype)
             norm.forward(x, h, ctx)
             self._gemm(ctx, h, self.w_gate_up, mid, self.gated, hidden=self.hidden)
-        emit = self._emit_args(emit_for, ctx, T, self.dim)
+        emit = self._emit_args(emit_for, ctx, x)
         prepared = self._add_emit_args(emit_for, ctx, T, self.dim, self.hidden) if emit is None else None
         ready = self._add_norm_args(emit_for, ctx, T, self.dim, self.hidden) if emit is None and prepared is None else None
         if emit is not None and kernels.can_chain(T, self.hidden, mid.dtype):
