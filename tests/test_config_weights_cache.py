@@ -822,3 +822,12 @@ def test_decode_splits_of_few_rows_deal_their_pages_evenly():
     for pages, over in ((64, {15: 1.02, 16: 1.0}), (128, {22: 0.98, 24: 0.95, 32: 1.0}), (256, {31: 0.76, 32: 0.74, 64: 1.0})):
         n = decode_splits(16, 1, 128, 4, pages)
         assert over[n] == min(over.values()), (pages, n)
+
+
+def test_when_short_prompts_take_one_launch():
+    """Up to a number of slices times tokens; groups of more than six heads while the chip has room for them."""
+    from yalm_amd.parts.attention import one_tile_pays
+    assert one_tile_pays(1, 64, 32, 8, 128, 5) and one_tile_pays(1, 48, 16, 4, 128, 10) and not one_tile_pays(1, 64, 16, 8, 128, 8)
+    assert one_tile_pays(1, 64, 32, 8, 64, 15) and not one_tile_pays(1, 64, 32, 8, 64, 16)
+    assert one_tile_pays(40, 64, 64, 8, 128, 1) and not one_tile_pays(41, 64, 64, 8, 128, 1) and not one_tile_pays(24, 64, 64, 8, 128, 2)
+    assert one_tile_pays(256, 64, 48, 8, 128, 1) and one_tile_pays(256, 64, 64, 8, 64, 1)

@@ -920,6 +920,11 @@ def test_attn_tile(n_heads, n_kv, hd, rd, lens, slices):
     assert torch.equal(kp0, kp1) and torch.equal(vp0, vp1) and kp0.abs().sum() > 0
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,rd,lens,slices", [(16, 1, 128, 128, [33, 64], 2), (71, 1, 64, 64, [5, 64, 17], 1), (32, 2, 128, 64, [40], 8)])
+def test_attn_tile_of_wide_groups_and_many_slices(n_heads, n_kv, hd, rd, lens, slices):
+    test_attn_tile(n_heads, n_kv, hd, rd, lens, slices)
+
+
 def test_attn_tile_says_which_steps_it_takes():
     """Operands off 16 bytes, more sequences than a launch has room for and more tiles than sequences are left to the kernels
     that it stands for."""

@@ -20,6 +20,7 @@ __device__ __forceinline__ int v_place(int el, int row) { return row ^ ((el >> 4
 //   33 tokens, 1 slice 8.9 5.5   2 slices 9.1 6.1   4 slices 9.9 7.6   8 slices 11.2 9.7        9 tokens, 24 heads 8.0 5.1
 //   64 tokens, 2 slices 9.7 7.6   4 slices 11.0 9.9   8 slices 11.9 14.4       4 x 40 tokens, 1 slice 13.8 6.5   4 slices 14.6 10.0
 //   8 x 50, 24 heads 18.7 7.7   40 x 50, 24 heads 37.7 26.6   128 x 64, 2 slices 170 167      heads of 64: 30 tokens 7.5 4.1   100 x 50 46 34
+// Where it is behind (many slices of long prompts, many sequences of wide groups) its caller takes the two (one_tile_pays in parts/attention.py).
 template <int HD>
 __global__ __launch_bounds__(HD * 8) void attn_tile_kernel(
     const float* __restrict__ qkv, bf16* __restrict__ out, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages,

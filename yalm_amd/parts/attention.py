@@ -47,6 +47,24 @@ def rope_by_tiles(T, n_heads, n_kv_heads, head_dim, slices):
     return T >= (ROPE_TILES_MIN_TOKENS * 5 // 4 if slices == 1 else ROPE_TILES_MIN_TOKENS * 8 // 5)
 
 
+def one_tile_pays(n_seqs, longest, n_heads, n_kv_heads, head_dim, slices):
+    """Whether a step of prompts of one tile each, the longest of `longest` tokens, is sooner done by kernels.attn_tile than by the rotation and
+    the attention behind each other.  A workgroup takes in all slices of its rows, 98 KB for 64 tokens of heads of 128, at what a compute unit takes in
+    (1 us), which the two launches spread over the chip; the launch less is worth 2 to 4 us inside a step, and 19 where the host is what
+    the step waits for.  us a layer that the one launch takes more inside steps of eight layers:
+      heads of 128, 32 + 8 at K 4,096: 64 tokens of 5 slices -2.1; 24 + 8 at K 8,192: 64 of 6 -1.8; 16 + 8 at 8,192: 48 of 8 -2.3, 64 of 8 0.3
+                   8 + 2 at 8,192: 48 of 16 -5.4, 64 of 16 3.3; 16 + 4 at 12,288: 33 of 10 -2.3, 48 of 10 -0.6, 64 of 10 2.1
+      heads of 64, 32 + 8 at 8,192: 64 of 10 -4.4; 8 + 2 at 8,192: 64 of 16 -12
+    Every head of a group takes in the group's keys and values, with more than six heads most of the work once the chip is full.  us, the two launches and
+    the one, back to back without a step around them:
+      heads of 128, 64 + 8: 16 x 64 38.4 32.1, two slices 46.2 45.8; 24 x 64 48.3 46.2, 59.5 66.7; 64 x 64 108 117, 142 166
+                   32 + 2:  32 x 64 35.6 27.9; 128 x 64 99.6 102, 130 141; 200 x 20 88.9 97.5   48 + 8: 256 x 64 325 288, two slices 426 413
+      heads of 64, 64 + 8: 256 x 64 228 172, two slices 299 256"""
+    if head_dim >= 128 and n_heads > 6 * n_kv_heads and n_heads * n_seqs * slices > 2560:
+        return False
+    return slices * longest * head_dim <= 480 * 128
+
+
 def kv_tiles(n_tok):
     """The index tables a step of whole prompts needs for attention over its own keys and values, which are
     staged in page-shaped tiles of 64 positions: seq_tile0[B + 1], the first tile of each sequence (n_tiles in
@@ -334,7 +352,8 @@ class GQAttention(Part):
         # are one kernel
         n_seqs, n_tiles = ctx.seq_slot.shape[0], ctx.tables["kv_tiles"]["n_tiles"] if prefill else 0
         if prefill and writes_cache and n_tiles == n_seqs and not self.sinks and self.score_bias is None and not ctx.line_is_shared(line) \
-                and kernels.attn_tile_fits(qkv, o, k_pages, v_pages, self.head_dim, self.window, n_seqs):
+                and kernels.attn_tile_fits(qkv, o, k_pages, v_pages, self.head_dim, self.window, n_seqs) \
+                and one_tile_pays(n_seqs, ctx.max_position + 1, self.n_heads, self.n_kv_heads, self.head_dim, slices):
             kernels.attn_tile(qkv, o, k_pages, v_pages, group.table, group.ring_pages, ctx.cu_seqlens, ctx.seq_slot, pos.table,
                               self.n_heads, self.n_kv_heads, self.head_dim, pos.rotary_dim, slices=slices, n_tiles=n_tiles)
         else:
