@@ -831,3 +831,11 @@ def test_when_short_prompts_take_one_launch():
     assert one_tile_pays(1, 64, 32, 8, 64, 15) and not one_tile_pays(1, 64, 32, 8, 64, 16)
     assert one_tile_pays(40, 64, 64, 8, 128, 1) and not one_tile_pays(41, 64, 64, 8, 128, 1) and not one_tile_pays(24, 64, 64, 8, 128, 2)
     assert one_tile_pays(256, 64, 48, 8, 128, 1) and one_tile_pays(256, 64, 64, 8, 64, 1)
+
+
+@pytest.mark.parametrize("n_heads,n_kv_heads,head_dim,slices,first", [
+    (32, 8, 128, 1, 384), (32, 8, 128, 2, 536), (32, 8, 128, 4, 447), (24, 8, 128, 1, 414), (32, 16, 128, 1, 320), (8, 2, 128, 1, 1536),
+    (32, 8, 64, 4, 320), (32, 8, 256, 1, 384), (16, 8, 144, 4, 334)])
+def test_from_how_many_tokens_on_prompts_rotate_by_tiles(n_heads, n_kv_heads, head_dim, slices, first):
+    from yalm_amd.parts.attention import rope_by_tiles
+    assert rope_by_tiles(first, n_heads, n_kv_heads, head_dim, slices) and not rope_by_tiles(first - 1, n_heads, n_kv_heads, head_dim, slices)

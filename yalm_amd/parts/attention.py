@@ -31,20 +31,29 @@ from .base import Part, build_part, part
 TARGET_WORKGROUPS = 256
 RESIDENT_WORKGROUPS = 512       # decode-attention workgroups that the chip holds at once (two a compute unit)
 # A prompt step of fewer tokens rotates and stores token by token: the kernel that works a page-shaped tile at a
-# time has a workgroup per (tile, head), too few to fill the chip below this.  It then takes its 12 us (two slices of K 15) however few tokens
-# there are, which the other one reaches later the fewer heads a token has.  us token by token and by tiles, 32 heads of 128 in 8
-# groups: one slice 320 tokens 10.6 11.8, 400 12.6 12.4, 512 15.0 12.7; two 400 12.9 15.6, 512 15.4 16.3, 640 22.2 20.5; four 400 20.8 23.7, 512
-# 26.4 24.8; 24 heads much the same (one slice 400 12.0 11.8, two 512 14.6 15.4, four 400 15.7 20.2, 512 24.6 23.4).  32 groups: 512 tokens 33.5 14.0, two slices 58.1 24.4;
-# heads of 64: 11.6 7.6, two slices 11.7 9.0
+# time has a workgroup per (tile, head), too few to fill the chip below this
 ROPE_TILES_MIN_TOKENS = 320
 
 
 def rope_by_tiles(T, n_heads, n_kv_heads, head_dim, slices):
-    """Whether a step of whole prompts rotates and stores by tiles of 64 positions: with wide heads of which a q/k/v row has at most
-    64 from 400 tokens on, of several slices from 512."""
-    if head_dim < 128 or n_heads + 2 * n_kv_heads > 64:
+    """Whether a step of whole prompts of T tokens rotates and stores by tiles of 64 positions.  With heads of 128 and more that takes the same
+    time for few tokens as for some hundreds (12 us, two slices of K 15, four 16 to 25, heads of 256 20 and more), while token by token goes with the
+    heads, a key and value head (whose values are stored turned) like ten of queries.  The two meet where tokens times such heads reach
+    what is asked for here.  us token by token and by tiles:
+      heads of 128, one slice    32 + 8: 360 tokens 11.7 11.9, 400 12.7 12.4   32 + 16: 320 15.7 11.3   48 + 8: 320 11.8 12.4, 360 13.0 12.2
+                                 32 + 4: 576 12.0 12.4, 640 13.0 12.4   8 + 8: 448 11.3 11.7, 512 12.5 11.8   8 + 2: 1,024 9.4 11.7, 1,500 11.9 11.9
+        two slices               32 + 8: 512 15.6 16.4, 640 20.8 20.1   32 + 16: 320 15.9 15.5   16 + 8: 576 14.9 15.5, 640 16.0 15.5
+        four and eight slices    32 + 8: 448 23.1 24.2, 512 26.5 24.9   eight 512 35.2 39.1, 640 43.2 41.9   64 + 8: 320 24.1 24.8, 360 27.5 25.1
+      heads of 144, one slice    32 + 8: 384 12.9 13.0   24 + 8: 448 14.1 13.2   two 32 + 8: 448 16.2 18.1   four 320 25.3 25.1, 384 30.6 26.3
+      heads of 256, one slice    32 + 8: 448 19.0 21.2, 576 23.2 21.7   four 400 46.5 43.7   16 + 4: 768 17.1 20.8, 1,500 49.0 31.7
+    Heads below 128 go by tiles from 320 tokens on (64: 512 tokens 11.6 7.6, two slices 11.7 9.0)."""
+    if T < ROPE_TILES_MIN_TOKENS or head_dim < 128:
         return T >= ROPE_TILES_MIN_TOKENS
-    return T >= (ROPE_TILES_MIN_TOKENS * 5 // 4 if slices == 1 else ROPE_TILES_MIN_TOKENS * 8 // 5)
+    if head_dim == 128:
+        meet = 43000 if slices == 1 else 60000 if slices == 2 else 50000
+    else:                 # for the narrowest of these: wider ones meet later
+        meet = 43000 if slices <= 2 else 32000
+    return T * (n_heads + 10 * n_kv_heads) >= meet
 
 
 def one_tile_pays(n_seqs, longest, n_heads, n_kv_heads, head_dim, slices):
