@@ -333,8 +333,8 @@ def test_a_sequence_at_its_first_token_beside_sequences_that_go_on(folders, name
 @pytest.mark.parametrize("name", ["tiny_long", "small_windowed", "tiny_mistral"])
 def test_short_prompts_and_the_steps_behind_them(folders, name, lens):
     """bfloat16 prompts on both sides of 16 tokens in all (up to there the products prepare the norms) and of 64 a sequence (up to
-    there the attention takes the product's sums), with a head that has the latter's sizes and one that has not, a window that
-    hides keys of a tile and one that does not; the steps behind them read what the prompts have left in the cache."""
+    there the attention takes the product's sums), with heads that the latter is built for, without a window and with one that hides
+    nothing in a tile, and heads of 32, which it is not built for; the steps behind them read what the prompts have left in the cache."""
     engine = make_engine(folders, name, "bfloat16", max_tokens=1024)
     poison = poison_free_pages(engine)
     lens = [min(n, tiny_configs.ALL[name]["max_position_embeddings"] - 3) for n in lens]
@@ -355,6 +355,32 @@ def test_short_prompts_and_the_steps_behind_them(folders, name, lens):
     for i, r in enumerate(requests):
         helpers.check_logits(np.stack(rows[i]), helpers.plain_logits(folders[name], tuple(r), "bfloat16"), "bfloat16",
                              "%s prompts %s, sequence %d" % (name, lens, i))
+
+
+@pytest.mark.parametrize("head_dim,window,taken", [(128, 40, False), (64, 63, False), (64, 64, True)])
+def test_short_prompts_whose_window_hides_keys_of_a_tile(tmp_path, monkeypatch, head_dim, window, taken):
+    """Heads that the launch for one-tile prompts is built for, with windows on both sides of a tile; the sequences go on across the
+    window."""
+    from yalm_amd.engine import Engine, Model
+    from yalm_amd.ops import kernels
+    cfg = dict(tiny_configs.SMALL_WINDOWED, head_dim=head_dim, sliding_window=window)
+    folder = helpers.make_folder(tmp_path, "window", cfg, seed=14)
+    calls, attn_tile = [], kernels.attn_tile
+    monkeypatch.setattr(kernels, "attn_tile", lambda *a, **kw: (calls.append(1), attn_tile(*a, **kw))[1])
+    engine = Engine(Model.from_folder(folder, dtype=torch.bfloat16, device="cuda:0"), max_tokens=1024)
+    lens = [64, 50, 9]
+    requests = [r[1] for r in sorted(helpers.random_requests(cfg, [n + 4 for n in lens], seed=32).items())]
+    slots = engine.start(len(lens))
+    first = engine.step(slots, [r[:n] for r, n in zip(requests, lens)], [list(range(n)) for n in lens]).cpu().numpy()
+    rows = [[first[sum(lens[:i]):sum(lens[:i + 1])]] for i in range(len(lens))]
+    for k in range(4):
+        out = engine.step(slots, [[r[n + k]] for r, n in zip(requests, lens)]).cpu().numpy()
+        for i in range(len(lens)):
+            rows[i].append(out[i:i + 1])
+    assert len(calls) == (cfg["num_hidden_layers"] if taken else 0)
+    for i, r in enumerate(requests):
+        helpers.check_logits(np.concatenate(rows[i]), helpers.plain_logits(folder, tuple(r), "bfloat16"), "bfloat16",
+                             "heads of %d, window %d, sequence %d" % (head_dim, window, i))
 
 
 def test_more_short_prompts_than_one_launch_takes(folders):

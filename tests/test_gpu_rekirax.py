@@ -282,6 +282,28 @@ def test_packing_kernel_of_short_rows_and_many_tokens(T, H, G, d, rot):
         assert torch.equal(a, b)
 
 
+# Norms over heads that are a whole wave's elements, or nearly the whole row: one wave a token (rows of up to 256, and longer ones of many tokens)
+@pytest.mark.parametrize("H,G,d,T", [(2, 1, 64, 40), (1, 1, 4, 33), (1, 1, 256, 1030), (6, 1, 256, 3080), (2, 1, 256, 40)])
+def test_packing_kernel_norms_heads_in_one_wave(H, G, d, T):
+    from yalm_amd.ops import kernels
+    ring = (T + 63) // 64
+    raw = randn(T, (H + 2 * G) * d, seed=d).to(DEV)
+    wq, wk = (1 + randn(d, seed=s, scale=0.2).to(DEV) for s in (1, 2))
+    table = torch.arange(ring, dtype=torch.int32, device=DEV).reshape(1, ring)
+    out = []
+    for size in (T, 30):                          # 30 tokens and fewer: a workgroup that holds the row in LDS
+        pad = (d + 15) // 16 * 16
+        q = torch.full((T, H * pad), float("nan"), device=DEV)
+        kp, vp = torch.zeros(ring, G, 64, pad, device=DEV), torch.zeros(ring, G, pad, 64, device=DEV)
+        for lo in range(0, T, size):
+            n = min(size, T - lo)
+            kernels.qkv_pack(raw[lo:lo + n], None, wq, wk, 1e-5, None, 1.7, None, 0, None, q[lo:lo + n], None, None, None, kp, vp, table, ring,
+                             i32([0] * n), i32(range(lo, lo + n)), i32([0]), i32([T]), H, G, d, d, pad, head_norm=True)
+        out.append((q, kp, vp))
+    for a, b in zip(*out):       # a head's squares in another order: three roundings of 2^-24 of elements up to 15 (4.5 normed, times 1.8 and 1.7)
+        assert torch.allclose(a, b, rtol=1e-6, atol=4e-6) and torch.equal(a != 0, b != 0)
+
+
 # The same with the middle in the first product's epilogue: one to 16 rows (K a multiple of 64 and not), to 128, tiles of 128 rows,
 # larger tiles, K in slices and whole; hidden values that end inside a block; streams narrower and wider than what one
 # element a thread covers; and the general kernels
