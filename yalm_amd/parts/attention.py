@@ -148,7 +148,6 @@ def decode_counters(ctx, B, n_heads, n_kv_heads, n_splits):
 @part("mixer", "gqa_attention")
 class GQAttention(Part):
     prompt_tables = (kv_tiles,)
-    takes_prepared_prompts = True
 
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
@@ -166,6 +165,7 @@ class GQAttention(Part):
             raise ValueError("n_heads %d is no multiple of n_kv_heads %d" % (self.n_heads, self.n_kv_heads))
         if self.head_dim % 2 or self.head_dim > kernels.MAX_HEAD_DIM:
             raise ValueError("head_dim %d is not supported (even, at most %d)" % (self.head_dim, kernels.MAX_HEAD_DIM))
+        self.takes_prepared_prompts = self.head_dim % 16 == 0
         self.q_dim = self.n_heads * self.head_dim
         self.kv_dim = self.n_kv_heads * self.head_dim
         self.position = build_part("position", p["position"], dim, prefix)

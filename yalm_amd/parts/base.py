@@ -31,9 +31,9 @@ also leave, in ctx.normed[id(next_norm)], either (xn, ss, eps): the activations 
 multiplied by that norm's weights and the partial sums of squares [rows, parts] (its residual-add GEMM,
 or the kernel that adds that GEMM's K slices, writes them: decode steps of up to 128 rows), or
 (h, None, None): the norm's finished output (more rows, and steps of whole prompts), which the next
-consumer takes instead of reading the residual stream.  In a step of whole prompts the first form (up to 16
-tokens) reaches only a part that says `takes_prepared_prompts` and whose fuses_norm takes the norm in that step; the
-block names the part that reads a norm in that norm's `read_by`.
+consumer takes instead of reading the residual stream.  In a step of whole prompts the first form reaches only a part
+that says `takes_prepared_prompts`: wherever kernels.can_chain takes the step (up to 16 tokens), its fuses_norm does and its
+forward_prenorm takes that form.  The block names the part that reads a norm in that norm's `read_by`.
 
 A part whose launches in a decode step depend on host values (it reads ctx.host_*, or sizes that
 change from step to step) says so with the class attribute `graph_safe = False`; the layers around
@@ -154,8 +154,6 @@ class Part:
         n = kernels.gemm_workspace_floats(a.shape[0], w.shape[0], a.shape[1]) if a.dtype == torch.bfloat16 else 0
         return ctx.ws.get("gemm.partial", (n,), torch.float32) if n and ctx is not None else None
 
-    takes_prepared_prompts = False    # whether forward_prenorm takes a norm that is prepared and not finished in steps of whole prompts too
-
     def _emit_args(self, emit_for, ctx, x):
         """Operands for a GEMM that adds to the stream x [T, dim] and also prepares the activations of the norm
         `emit_for` (the next norm on the residual stream), or None if that cannot be done."""
@@ -166,8 +164,7 @@ class Part:
         if ctx.mode not in ("decode", "prefill") or not kernels.can_chain(T, width, ctx.act_dtype):
             return None
         if ctx.mode == "prefill":                 # not for the head, which picks rows of a prompt, nor for whoever norms the stream itself
-            reader = getattr(emit_for, "read_by", None)
-            if not getattr(reader, "takes_prepared_prompts", False) or not reader.fuses_norm(emit_for, x, ctx):
+            if not getattr(getattr(emit_for, "read_by", None), "takes_prepared_prompts", False):
                 return None
         import torch
         nw, eps = emit_for.fused()

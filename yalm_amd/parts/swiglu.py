@@ -33,8 +33,6 @@ def interleave_gate_up(gate, up):
 
 @part("feed_forward", "swiglu")
 class SwiGLU(Part):
-    takes_prepared_prompts = True
-
     def __init__(self, spec, dim, prefix):
         super().__init__(spec, dim, prefix)
         self.hidden = int(spec.params["hidden"])
@@ -46,6 +44,7 @@ class SwiGLU(Part):
         self.unit = None if unit == (0.0, 1.0, 0.0) else unit          # the epilogue's constants, where they are not silu's
         if self.unit is not None and (self.activation != "silu" or unit[0] <= 0.0):
             raise ValueError("feed-forward: alpha and up_shift go with silu and a positive limit")
+        self.takes_prepared_prompts = self.unit is None
         # the tensors' names behind the part's prefix (parameter `tensors`: {gate, up, down})
         self.names = {"gate": "gate_proj.weight", "up": "up_proj.weight", "down": "down_proj.weight"}
         self.names.update(spec.params.get("tensors") or {})
