@@ -163,8 +163,8 @@ __global__ __launch_bounds__(PACK_THREADS) void qkv_pack_kernel(
 // bits of a row's norm do not hang on it (what the waves hand each other is a sum of four squares an element's thread; the exchange is
 // level with one of the waves' sums: 1,909 rows of 6,144 20.9 and 21.1 us).  For rows whose parts and heads are multiples of four elements (a thread takes four consecutive ones at a time) and at most
 // 1,024 * NV elements.  A workgroup of four waves a token: with a wave a token, 24 rounds of a row of 6,144 and its weights were 250
-// registers, two waves a SIMD and too few loads in flight (1,909 tokens inside a step 43.8 -> 31.9 us; 32
-// tokens alone 19.5 -> 6.8, 2,048 33.9 -> 24.5; rows of 1,536 5.3 -> 3.5 and 8.3 -> 8.1).  Rows of up to 256 are a wave's (2,048 of them 4.2 us, with four waves 5.5), and so are those of up to
+// registers, two waves a SIMD and too few loads in flight (1,909 tokens inside a step 43.8 -> 31.1 us; 32
+// tokens alone 19.8 -> 7.2, 1,909 29.5 -> 21; rows of 1,536 7.3 -> 4.9 and 10.5 -> 9.1).  Rows of up to 256 are a wave's (2,048 of them 4.2 us, with four waves 5.5), and so are those of up to
 // 2,048 where tokens are many: each of the four has next to nothing to load and the chip holds 2,048 workgroups of four.  us with four waves, two
 // and one, rows of 384: 1,000 tokens 4.5 4.1 4.3, 1,909 6.0 5.0 4.6, 4,000 9.7 7.5 6.2; of 1,024 4.8 4.6 5.0, 6.8 6.2 6.6, 11.5 9.5 9.0; of 1,344
 // 5.7 5.7 7.1, 9.6 7.9 8.9, 14.4 12.8 11.7; of 2,048 7.3 7.7 9.8, 11.4 10.1 11.0, 18.4 16.9 15.9; of 2,304 and more four are the soonest or level.
